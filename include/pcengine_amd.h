@@ -445,6 +445,32 @@ int pce_conv_fwd_os(const void *in_feats, const void *weight, const void *weight
                     int64_t n_in, int64_t n_out, int32_t c_in, int32_t c_out, int32_t kv,
                     const int32_t *nbr_dev, const pce_epilogue_t *epilogue, pce_stream_t stream);
 
+/* The same for wide fp16 layers, over blocks of rows with equal neighbour patterns: the rows of every 8192 consecutive
+ * ones are visited sorted by their patterns, a block of 16 leaves out the offsets none of its rows has, and the tiles
+ * are dealt to the compute units by cost.
+ *
+ * pce_osb_order derives the order and the work lists from a neighbour table (output-major for a layer, input-major for
+ * the transposed layer over the same map), once per table: order_dev of pce_osb_order_elems(n_rows) ints, kv <= 27;
+ * two launches, no wait.  mask_dev (optional): the rows' patterns where they are known, e.g. order_dev + n_rows of
+ * pce_row_order; mid (or -1): an offset every row counts as having (the centre, which those patterns leave out).
+ * pce_conv_osb_takes(dtype, c_in, c_out, kv): fp16, c_in a multiple of 32 from 64 on, c_out a multiple of 8 from 72 to
+ * 1024, kv from 2 to 27.  weight_packed from pce_pack_weights; ws of pce_conv_osb_workspace_bytes(n_out, c_out) bytes,
+ * its contents do not outlive the call's work on the stream; all pointers 16-byte aligned; at most 3.75 GiB of features.
+ * n_pairs: the map's pairs without the centre ones (an estimate of the work of a tile), -1 = unknown.
+ * The sums of a row do not depend on the order of the rows, except that a layer whose tiles do not fill the last round
+ * of workgroups adds up some tiles in several parts. */
+int64_t pce_osb_order_elems(int64_t n_rows);
+int pce_osb_order(const int32_t *nbr_dev, const int32_t *mask_dev, int32_t mid, int32_t kv, int64_t n_rows, int32_t *order_dev,
+                  int64_t order_elems, pce_stream_t stream);
+int pce_conv_osb_takes(int32_t dtype, int32_t c_in, int32_t c_out, int32_t kv);
+int64_t pce_conv_osb_workspace_bytes(int64_t n_out, int32_t c_out);
+/* 1 where it is the fastest dataflow of a submanifold layer (mid >= 0): asked before pce_select_dataflow, which knows the
+ * dataflows that need no block order. */
+int pce_conv_osb_leads(int64_t n_out, int64_t n_pairs, int32_t c_in, int32_t c_out, int32_t kv, int32_t mid, int32_t dtype);
+int pce_conv_fwd_osb(const void *in_feats, const void *weight_packed, void *out_feats, int32_t dtype, int64_t n_in, int64_t n_out,
+                     int64_t n_pairs, int32_t c_in, int32_t c_out, int32_t kv, const int32_t *nbr_dev, const int32_t *order_dev, void *ws, int64_t ws_bytes,
+                     const pce_epilogue_t *epilogue, pce_stream_t stream);
+
 /* Output-stationary over ordered rows, for narrow layers on clouds where most voxels have few
  * neighbours (surfaces: 0.2 pairs per voxel on a 64 x 2048 LiDAR scan at 0.1 m).
  *

@@ -144,6 +144,13 @@ _SIGNATURES = {
     "pce_conv_fwd_os": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int32, c_int32, c_int32, c_void_p, POINTER(Epilogue), c_void_p]),
     "pce_conv_fwd_oso": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32,
                                    c_void_p, c_void_p, POINTER(c_int64), POINTER(Epilogue), c_void_p]),
+    "pce_osb_order_elems": (c_int64, [c_int64]),
+    "pce_osb_order": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int64, c_void_p, c_int64, c_void_p]),
+    "pce_conv_osb_takes": (c_int32, [c_int32, c_int32, c_int32, c_int32]),
+    "pce_conv_osb_leads": (c_int32, [c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, c_int32]),
+    "pce_conv_osb_workspace_bytes": (c_int64, [c_int64, c_int32]),
+    "pce_conv_fwd_osb": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int64, c_int32, c_int32, c_int32, c_void_p,
+                                   c_void_p, c_void_p, c_int64, POINTER(Epilogue), c_void_p]),
     "pce_row_order": (c_int32, [c_void_p, c_int32, c_int64, c_int32, c_void_p, c_int64, POINTER(c_int64), c_void_p]),
     "pce_row_order_elems": (c_int64, [c_int64]),
     "pce_conv_fwd_dense": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int32, c_int32, POINTER(Epilogue), c_void_p]),

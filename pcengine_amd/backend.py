@@ -21,6 +21,7 @@ import torch
 from . import _lib
 from ._lib import Geom, DATAFLOW_FOD, DATAFLOW_GMS, DATAFLOW_OS, DATAFLOW_FDS, DATAFLOW_OSO, PCE_F16, PCE_F32, QUANTUM, CSR_CODE
 
+_OSB_MAX_BYTES = 0xF0000000      # features the block output-stationary kernel addresses
 CODE_A, CODE_B = 94273, 311  # packed 3-vectors, script/utils.py:233-242
 
 
@@ -714,6 +715,50 @@ def row_order(km: KernelMap) -> torch.Tensor:
     return km.order
 
 
+def block_order(km: KernelMap, transposed: bool = False) -> torch.Tensor:
+    """Row order of the block output-stationary kernel (``pce_osb_order``), cached on the map per direction: two
+    launches, no wait of the host.  Another stream than the one that built it waits for it."""
+    cached = km.__dict__.setdefault("_blocks", {})
+    entry = cached.get(transposed)
+    if entry is None:
+        nbr, n = (km.nbr_in, km.n_in) if transposed else (km.nbr_out, km.n_out)
+        lib = _lib.load()
+        elems = lib.pce_osb_order_elems(n)
+        # a map of a planned pyramid lives as long as the forward's arena; any other may outlive it
+        planned = "_arena" in km.__dict__
+        order = (_new if planned else torch.empty)(elems, dtype=torch.int32, device=nbr.device)
+        # the row order of the ordered dataflow, where the map came with one, holds the rows' patterns already
+        known = None if transposed or km.order is None else km.order.data_ptr() + 4 * n
+        mid = _mid(km.ks) if km.subm and not transposed else -1
+        s = _stream(nbr.device)
+        _lib.check(lib.pce_osb_order(nbr.data_ptr(), known, mid, km.kv, n, order.data_ptr(), elems, s))
+        event = None
+        if not planned:
+            event = torch.cuda.Event()
+            event.record(torch.cuda.current_stream(nbr.device))
+        entry = cached[transposed] = (order, s, event)
+    order, s, event = entry
+    if event is not None and s != _stream(order.device):
+        current = torch.cuda.current_stream(order.device)
+        current.wait_event(event)
+        order.record_stream(current)
+    return order
+
+
+_osb_takes_cache = {}
+
+
+def osb_takes(kv: int, c_in: int, c_out: int, dtype: torch.dtype) -> bool:
+    """Layers the block output-stationary kernel takes (``pce_conv_osb_takes``)."""
+    if dtype != torch.float16:
+        return False
+    key = (kv, c_in, c_out)
+    ans = _osb_takes_cache.get(key)
+    if ans is None:
+        ans = _osb_takes_cache[key] = bool(_lib.load().pce_conv_osb_takes(PCE_F16, c_in, c_out, kv))
+    return ans
+
+
 _oso_takes_cache = {}
 
 
@@ -744,6 +789,10 @@ def select_dataflow(km: KernelMap, c_in: int, c_out: int, dtype: torch.dtype, tr
     lib = _lib.load()
     n_out = km.n_in if transposed else km.n_out
     n_in = km.n_out if transposed else km.n_in
+    # (the transposed layer over a submanifold map of odd kernel sizes is a plain layer, see conv_forward)
+    if osb_takes(km.kv, c_in, c_out, dtype) and km.subm and (not transposed or all(k % 2 == 1 for k in km.ks)) and \
+            lib.pce_conv_osb_leads(n_out, km.M, c_in, c_out, km.kv, _mid(km.ks), PCE_F16):
+        return DATAFLOW_OS
     df = lib.pce_select_dataflow(n_in, n_out, km.M, c_in, c_out, km.kv, _mid(km.ks) if km.subm else -1, int(bool(transposed)),
                                  PCE_F16 if dtype == torch.float16 else PCE_F32)
     if not km.has_pairs and df not in (DATAFLOW_OSO, DATAFLOW_OS):
@@ -954,6 +1003,16 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
                 t[_mid(km.ks)] = torch.arange(km.n_in, dtype=torch.int32, device=t.device)
                 km._nbr_in_t = t.view(-1)
             nbr = km._nbr_in_t
+        elif osb_takes(kv, c_in, c_out, feats.dtype) and n_in * (ld_in or c_in) * 2 < _OSB_MAX_BYTES and \
+                (feats.data_ptr() | out.data_ptr() | ((epi.bias or 0) | (epi.residual or 0) if epi is not None else 0)) % 16 == 0:
+            if packed is None:
+                packed = pack_weights(weight)
+            order = block_order(km, transposed)
+            ws_bytes = lib.pce_conv_osb_workspace_bytes(n_out, c_out)
+            ws = _staging(ws_bytes, torch.uint8, dev)
+            _lib.check(lib.pce_conv_fwd_osb(feats.data_ptr(), packed.data_ptr(), out.data_ptr(), dt, n_in, n_out, km.M, c_in, c_out, kv,
+                                            nbr.data_ptr(), order.data_ptr(), ws.data_ptr(), ws_bytes, epi, s))
+            return out
         _lib.check(lib.pce_conv_fwd_os(feats.data_ptr(), weight.data_ptr(), _ptr(packed), out.data_ptr(), dt, n_in, n_out,
                                        c_in, c_out, kv, nbr.data_ptr(), epi, s))
     else:
