@@ -172,6 +172,19 @@ int pce_voxelize_emit(const void *ws_dev, int64_t n_points, int64_t n_voxels,
                       const int32_t *coords_min3_host, const int32_t *coords_max3_host,
                       int32_t batch_index, int32_t *coords_out_dev, int32_t *index_out_dev,
                       int32_t *inverse_out_dev, pce_stream_t stream);
+/* The same as sparse_quantize returns it: coords_out[n_voxels,3] and 64-bit indices. */
+int pce_voxelize_emit3(const void *ws_dev, int64_t n_points, int64_t n_voxels,
+                       const int32_t *coords_min3_host, const int32_t *coords_max3_host, int32_t *coords_out_dev,
+                       int64_t *index_out_dev, int64_t *inverse_out_dev, pce_stream_t stream);
+
+/* ---- collation -------------------------------------------------------------------------------- *
+ * The coordinates of a batch (sparse_collate, script/utils.py:167-196): sample k's rows[k] rows of (x, y, z) at
+ * coords_dev[k] become out_dev[total,4] = (k, x, y, z), in order; upper3_host receives the maxima of the three
+ * columns (one wait of the host).  At least one row in all. */
+#define PCE_MAX_COLLATE 64
+int64_t pce_collate_workspace_bytes(void);
+int pce_collate(const int32_t *const *coords_dev, const int64_t *rows, int32_t samples, int32_t *out_dev, void *ws_dev,
+                int64_t ws_bytes, int32_t *upper3_host, pce_stream_t stream);
 
 /* ---- kernel map ------------------------------------------------------------------------------ *
  * Replaces the four _queryhash_* kernels, exclusive_scan_for_kernel_quantified, mapping_counter and

@@ -19,6 +19,7 @@ DATAFLOW_FOD, DATAFLOW_GMS, DATAFLOW_OS, DATAFLOW_FDS, DATAFLOW_OSO = 0, 1, 2, 3
 QUANTUM = 128
 KMAP_NO_GRID = 1
 KMAP_TABLE_ONLY = 2
+MAX_COLLATE = 64         # PCE_MAX_COLLATE
 ABI_VERSION = 200        # PCE_ABI_VERSION of include/pcengine_amd.h
 CSR_CODE = 1186111
 
@@ -109,6 +110,10 @@ _SIGNATURES = {
                                POINTER(c_int32), POINTER(c_int32), c_void_p]),
     "pce_voxelize_emit": (c_int32, [c_void_p, c_int64, c_int64, POINTER(c_int32), POINTER(c_int32), c_int32, c_void_p, c_void_p,
                                     c_void_p, c_void_p]),
+    "pce_voxelize_emit3": (c_int32, [c_void_p, c_int64, c_int64, POINTER(c_int32), POINTER(c_int32), c_void_p, c_void_p, c_void_p,
+                                     c_void_p]),
+    "pce_collate_workspace_bytes": (c_int64, []),
+    "pce_collate": (c_int32, [POINTER(c_void_p), POINTER(c_int64), c_int32, c_void_p, c_void_p, c_int64, POINTER(c_int32), c_void_p]),
     "pce_col_sums_workspace_bytes": (c_int64, [c_int64, c_int32]),
     "pce_col_sums": (c_int32, [c_void_p, c_void_p, c_int32, c_int64, c_int32, c_void_p, c_int64, c_void_p, c_void_p]),
     "pce_col_affine": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_int32,

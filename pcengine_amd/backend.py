@@ -242,12 +242,13 @@ def build_out_coords_chain(in_coords: torch.Tensor, geoms: Sequence[Geom], batch
     return [pieces[4 * l + 2][:4 * n_out[l]].view(n_out[l], 4) for l in range(levels)]
 
 
-def voxelize(points: torch.Tensor, voxel_size, batch_index: int = 0, return_index: bool = False,
+def voxelize(points: torch.Tensor, voxel_size, batch_index: Optional[int] = 0, return_index: bool = False,
              return_inverse: bool = False):
     """Voxelisation on the GPU (sparse_quantize of script/utils.py:33-55): ``points`` [P,3] float32 or
     float64 on the device -> coords int32 [V,4] = (batch_index, x, y, z) of the unique voxels in
     ascending (x,y,z) order, optionally the first point of every voxel (int32 [V]) and the voxel of
-    every point (int32 [P]).  Also returns the integer coordinate bounds (min, max) as lists."""
+    every point (int32 [P]).  Also returns the integer coordinate bounds (min, max) as lists.
+    ``batch_index=None``: coords int32 [V,3] without the batch column, and int64 indices."""
     lib = _lib.load()
     _require_cuda(points, "points")
     if points.dim() != 2 or points.shape[1] != 3 or points.dtype not in (torch.float32, torch.float64):
@@ -268,11 +269,16 @@ def voxelize(points: torch.Tensor, voxel_size, batch_index: int = 0, return_inde
     dt = _lib.PCE_F32 if points.dtype == torch.float32 else _lib.PCE_F64
     _lib.check(lib.pce_voxelize(points.data_ptr(), dt, n, vs, ws.data_ptr(), ws_bytes, n_vox, cmin, cmax, s))
     v = n_vox.value
-    coords = torch.empty((v, 4), dtype=torch.int32, device=dev)
-    index = torch.empty(v, dtype=torch.int32, device=dev) if return_index else None
-    inverse = torch.empty(n, dtype=torch.int32, device=dev) if return_inverse else None
-    _lib.check(lib.pce_voxelize_emit(ws.data_ptr(), n, v, cmin, cmax, int(batch_index), coords.data_ptr(), _ptr(index),
-                                     _ptr(inverse), s))
+    plain = batch_index is None
+    itype = torch.int64 if plain else torch.int32
+    coords = torch.empty((v, 3 if plain else 4), dtype=torch.int32, device=dev)
+    index = torch.empty(v, dtype=itype, device=dev) if return_index else None
+    inverse = torch.empty(n, dtype=itype, device=dev) if return_inverse else None
+    if plain:
+        _lib.check(lib.pce_voxelize_emit3(ws.data_ptr(), n, v, cmin, cmax, coords.data_ptr(), _ptr(index), _ptr(inverse), s))
+    else:
+        _lib.check(lib.pce_voxelize_emit(ws.data_ptr(), n, v, cmin, cmax, int(batch_index), coords.data_ptr(), _ptr(index),
+                                         _ptr(inverse), s))
     outs = [coords]
     if return_index:
         outs.append(index)
@@ -280,6 +286,28 @@ def voxelize(points: torch.Tensor, voxel_size, batch_index: int = 0, return_inde
         outs.append(inverse)
     outs.append((list(cmin), list(cmax)))
     return tuple(outs)
+
+
+def collate_coords(coords: Sequence[torch.Tensor]):
+    """(int32 [N, 4] = (sample, x, y, z), maxima of x, y, z as a list) of the samples' int32 [n, 3] coordinates in one
+    launch, or None where the kernel does not take them (other layouts, devices or dtypes, no rows, many samples)."""
+    first = coords[0]
+    if len(coords) > _lib.MAX_COLLATE or not all(c.is_cuda and c.device == first.device and c.dtype == torch.int32 and c.dim() == 2
+                                                 and c.shape[1] == 3 and c.is_contiguous() for c in coords):
+        return None
+    rows = [c.shape[0] for c in coords]
+    total = sum(rows)
+    if total == 0:
+        return None
+    lib = _lib.load()
+    out = torch.empty((total, 4), dtype=torch.int32, device=first.device)
+    ws_bytes = lib.pce_collate_workspace_bytes()
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=first.device)
+    src = (_lib.ctypes.c_void_p * len(rows))(*[c.data_ptr() for c in coords])
+    upper = (_lib.c_int32 * 3)()
+    _lib.check(lib.pce_collate(src, (_lib.c_int64 * len(rows))(*rows), len(rows), out.data_ptr(), ws.data_ptr(), ws_bytes, upper,
+                               _stream(first.device)))
+    return out, list(upper)
 
 
 class _MapJob:

@@ -65,8 +65,7 @@ def sparse_quantize(coords, voxel_size: Union[float, Tuple[float, ...]] = 1, *, 
     assert isinstance(voxel_size, tuple) and len(voxel_size) == 3
     if isinstance(coords, torch.Tensor) and coords.is_cuda:
         from . import backend
-        res = backend.voxelize(coords, voxel_size, 0, return_index=return_index, return_inverse=return_inverse)
-        outs = [res[0][:, 1:].contiguous()] + [t.long() for t in res[1:-1]]
+        outs = list(backend.voxelize(coords, voxel_size, None, return_index=return_index, return_inverse=return_inverse)[:-1])
         return outs[0] if len(outs) == 1 else outs
     q = np.floor(coords / np.array(voxel_size)).astype(np.int32)
     _, idx, inv = np.unique(ravel_hash(q), return_index=True, return_inverse=True)
@@ -148,12 +147,17 @@ def sparse_collate(inputs: List[spTensor]) -> spTensor:
         if sample.stride != stride:
             raise AssertionError((sample.stride, stride))
         sizes.append(sample.coords.shape[0])
-    spatial = torch.cat([sample.coords.int() for sample in inputs], dim=0)
-    index = torch.repeat_interleave(torch.arange(len(inputs), dtype=torch.int32, device=spatial.device),
-                                    torch.tensor(sizes, device=spatial.device))
-    coords = torch.cat((index.unsqueeze(1), spatial), dim=1)
+    from . import backend
+    joined = backend.collate_coords([sample.coords for sample in inputs])
+    if joined is not None:
+        coords, upper = joined
+    else:
+        spatial = torch.cat([sample.coords.int() for sample in inputs], dim=0)
+        index = torch.repeat_interleave(torch.arange(len(inputs), dtype=torch.int32, device=spatial.device),
+                                        torch.tensor(sizes, device=spatial.device))
+        coords = torch.cat((index.unsqueeze(1), spatial), dim=1)
+        upper = [int(v) for v in spatial.amax(dim=0).tolist()]
     feats = torch.cat([sample.feats for sample in inputs], dim=0)
-    upper = [int(v) for v in spatial.amax(dim=0).tolist()]
     return spTensor(coords=coords, feats=feats, stride=stride, batchsize=len(inputs), buffer=None,
                     coords_min=[0, 0, 0], coords_max=upper)
 
