@@ -354,6 +354,11 @@ typedef struct pce_epilogue {
 int64_t pce_packed_weight_bytes(int32_t dtype, int32_t kv, int32_t c_in, int32_t c_out);
 int pce_pack_weights(const void *weight, int32_t dtype, int32_t kv, int32_t c_in, int32_t c_out,
                      void *packed_dev, pce_stream_t stream);
+/* Weights of a training step in one launch: w [kv][c_in][c_out] of dtype_w to `out` in dtype (fp32 may become fp16), with
+ * transpose every offset's matrix transposed ([kv][c_out][c_in]), with flip the offsets reversed; for fp16 also the
+ * packed copy of `out` (pce_packed_weight_bytes of its shape, 16-byte aligned; NULL for fp32).  out must not overlap w. */
+int pce_prepare_weights(const void *w, int32_t dtype_w, int32_t dtype, int32_t kv, int32_t c_in, int32_t c_out,
+                        int32_t transpose, int32_t flip, void *out, void *packed_dev, pce_stream_t stream);
 
 /* Fetch-on-demand: pairs (imap, omap, kpos, qkpos) and qsum = qkpos[kv] on the host.
  * fp16 needs an fp32 accumulation scratch of pce_conv_fod_workspace_bytes(); fp32 needs none. */

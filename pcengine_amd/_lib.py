@@ -132,6 +132,7 @@ _SIGNATURES = {
     "pce_conv_fod_workspace_bytes": (c_int64, [c_int64, c_int32, c_int32]),
     "pce_packed_weight_bytes": (c_int64, [c_int32, c_int32, c_int32, c_int32]),
     "pce_pack_weights": (c_int32, [c_void_p, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p]),
+    "pce_prepare_weights": (c_int32, [c_void_p] + [c_int32] * 7 + [c_void_p, c_void_p, c_void_p]),
     "pce_conv_fwd_fds": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32,
                                    c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, POINTER(c_int32), POINTER(c_int32), c_void_p, c_void_p,
                                    c_int64, c_int64, c_void_p, c_int64, POINTER(Epilogue), c_void_p]),

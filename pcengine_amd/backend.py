@@ -848,6 +848,32 @@ def pack_weights(weight: torch.Tensor) -> Optional[torch.Tensor]:
     return packed
 
 
+def prepare_weights(weight: torch.Tensor, dtype: torch.dtype, transpose: bool = False, flip: bool = False):
+    """(kernel, packed copy or None) of a layer of a training step in one launch: ``weight`` [kv, c_in, c_out] (or
+    [c_in, c_out]) in ``dtype``, every offset's matrix transposed and / or the offsets in reverse order on request."""
+    half = dtype == torch.float16
+    if not weight.is_cuda or weight.numel() == 0 or not (weight.dtype == dtype and (half or dtype == torch.float32)
+                                                         or half and weight.dtype == torch.float32):
+        w = weight.to(dtype)
+        w = w.transpose(-2, -1) if transpose else w
+        w = (w.flip(0) if flip and w.dim() == 3 else w).contiguous()
+        return w, pack_weights(w) if half else None
+    weight = weight.contiguous()
+    if weight.dtype == dtype and not (transpose or flip):
+        return weight, pack_weights(weight)
+    lib = _lib.load()
+    kv = weight.shape[0] if weight.dim() == 3 else 1
+    c_in, c_out = weight.shape[-2:]
+    rows, cols = (c_out, c_in) if transpose else (c_in, c_out)
+    out = torch.empty(weight.shape[:-2] + (rows, cols), dtype=dtype, device=weight.device)
+    packed = None
+    if half:
+        packed = torch.empty(lib.pce_packed_weight_bytes(PCE_F16, kv, rows, cols), dtype=torch.uint8, device=weight.device)
+    _lib.check(lib.pce_prepare_weights(weight.data_ptr(), _dtype_code(weight), PCE_F16 if half else PCE_F32, kv, c_in, c_out,
+                                       int(transpose), int(flip), out.data_ptr(), _ptr(packed), _stream(weight.device)))
+    return out, packed
+
+
 def _act_code(act) -> Tuple[int, float]:
     """``act``: None, 'relu', or ('leaky_relu', negative_slope) -> (PCE_ACT_*, slope)."""
     if act is None:
@@ -1208,19 +1234,24 @@ def dense_wgrad(feats: torch.Tensor, grad_out: torch.Tensor) -> torch.Tensor:
 
 
 def conv_backward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, grad_out: torch.Tensor, transposed: bool = False,
-                  need_feats: bool = True, need_weight: bool = True, dataflow: Optional[int] = None):
+                  need_feats: bool = True, need_weight: bool = True, dataflow: Optional[int] = None,
+                  weight_dtype: Optional[torch.dtype] = None):
     """(grad_feats, grad_weight) of ``conv_forward``.  The feature gradient is the convolution of
     ``grad_out`` with the per-offset transposed kernel over the same pairs with the roles swapped,
     run by the forward kernels; the kernel gradient comes from ``pce_conv_wgrad`` (fp32 sums,
-    returned in the kernel's dtype)."""
+    returned in ``weight_dtype``, by default the kernel's)."""
     gf = gw = None
-    w3 = weight if weight.dim() == 3 else weight.unsqueeze(0)
     if need_feats:
-        wt = w3.transpose(1, 2).contiguous()
-        df = dataflow if dataflow is not None else select_dataflow(km, wt.shape[1], wt.shape[2], wt.dtype, not transposed)
-        gf = conv_forward(grad_out.contiguous(), wt, km, df, transposed=not transposed, packed=pack_weights(wt))
+        w3 = weight if weight.dim() == 3 else weight.unsqueeze(0)
+        c_out, c_in = w3.shape[1:]
+        df = dataflow if dataflow is not None else select_dataflow(km, c_in, c_out, w3.dtype, not transposed)
+        # over a map that is its own mirror image the swapped layer is the plain one with the offsets reversed (see
+        # conv_forward): they are reversed in the launch that transposes them
+        mirror = not transposed and km.subm and all(k % 2 == 1 for k in km.ks)
+        wt, packed = prepare_weights(w3, w3.dtype, transpose=True, flip=mirror)
+        gf = conv_forward(grad_out.contiguous(), wt, km, df, transposed=not transposed and not mirror, packed=packed)
     if need_weight:
-        gw = conv_wgrad(feats, grad_out, km, transposed).to(weight.dtype).reshape(weight.shape)
+        gw = conv_wgrad(feats, grad_out, km, transposed).to(weight_dtype or weight.dtype).reshape(weight.shape)
     return gf, gw
 
 

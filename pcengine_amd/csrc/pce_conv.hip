@@ -43,6 +43,48 @@ __global__ void __launch_bounds__(256) pack_weights_kernel(const half_t *__restr
   *reinterpret_cast<half8 *>(&P[e * 8]) = v;
 }
 
+// ---- weights of a training step -----------------------------------------------------------------
+// One launch turns a kernel [kv][c_in][c_out] into what a convolution takes: in the features' type, for the feature
+// gradient with every offset's matrix transposed (and the offsets reversed where the map is its own mirror image), and
+// for fp16 the packed copy beside it.  A workgroup takes a 32 x 32 tile of one offset through LDS, so that rows are
+// read and written along memory in either orientation (row stride 33: no bank conflicts down a column).  Bound by
+// launches: a 27 x 256 x 256 kernel is 10 MB in and out.  As a cast, a transposing copy, a reversal and one or two packing
+// launches the same took a step of a U-Net on a 100 k-voxel scan 1740 us in 330 launches, now 525 in 99.
+template <typename TS, typename TD>
+__global__ void __launch_bounds__(256) prepare_weights_kernel(const TS *__restrict__ W, TD *__restrict__ out, half_t *__restrict__ P,
+                                                              int kv, int c_in, int c_out, int transpose, int flip,
+                                                              int k8_total, int n_pad, int bi, int bo) {
+  __shared__ TD tile[32][33];   // [row k][column n] of the result
+  const int kp = blockIdx.x / (bi * bo), rest = blockIdx.x % (bi * bo);
+  const int i0 = (rest / bo) * 32, o0 = (rest % bo) * 32;   // input and output channels of the tile
+  const int x = threadIdx.x & 31, y0 = threadIdx.x >> 5;
+#pragma unroll
+  for (int y = y0; y < 32; y += 8) {
+    TD v = (TD)0.f;
+    if (i0 + y < c_in && o0 + x < c_out) v = (TD)W[((long long)kp * c_in + i0 + y) * c_out + o0 + x];
+    if (transpose)
+      tile[x][y] = v;
+    else
+      tile[y][x] = v;
+  }
+  __syncthreads();
+  const int rows = transpose ? c_out : c_in, cols = transpose ? c_in : c_out;
+  const int k0 = transpose ? o0 : i0, n0 = transpose ? i0 : o0;
+  const int dst = flip ? kv - 1 - kp : kp;
+#pragma unroll
+  for (int y = y0; y < 32; y += 8)
+    if (k0 + y < rows && n0 + x < cols) out[((long long)dst * rows + k0 + y) * cols + n0 + x] = tile[y][x];
+  if (sizeof(TD) == 2 && P && threadIdx.x < 128) {
+    const int k8 = k0 / 8 + y0;
+    if (k8 < k8_total && n0 + x < n_pad) {
+      half8 v;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = (half_t)tile[y0 * 8 + j][x];   // zeros outside the kernel, as the tile holds them
+      *reinterpret_cast<half8 *>(&P[(((long long)dst * k8_total + k8) * n_pad + n0 + x) * 8]) = v;
+    }
+  }
+}
+
 // Workgroup barrier that orders LDS accesses only.  __syncthreads() also waits for every outstanding
 // global load; here loads for later use (feature rows, partial rows) stay in flight across the
 // barrier and are waited for where their registers are first read.
@@ -1466,6 +1508,32 @@ extern "C" int pce_pack_weights(const void *w, int32_t dtype, int32_t kv, int32_
   hipLaunchKernelGGL(pack_weights_kernel, dim3((unsigned)pce_div_up(total, 256)), dim3(256), 0, (hipStream_t)stream,
                      (const half_t *)w, (half_t *)packed, kv, c_in, c_out, k8, n_pad);
   PCE_LAUNCH_CHECK("pack_weights");
+  return PCE_OK;
+}
+
+extern "C" int pce_prepare_weights(const void *w, int32_t dtype_w, int32_t dtype, int32_t kv, int32_t c_in, int32_t c_out,
+                                   int32_t transpose, int32_t flip, void *out, void *packed, pce_stream_t stream) {
+  if (!w || !out || kv <= 0 || c_in <= 0 || c_out <= 0) PCE_FAIL(PCE_EINVAL, "pce_prepare_weights: bad argument");
+  if ((dtype_w != PCE_F16 && dtype_w != PCE_F32) || (dtype != dtype_w && dtype != PCE_F16))
+    PCE_FAIL(PCE_EINVAL, "pce_prepare_weights: dtype %d from %d", (int)dtype, (int)dtype_w);
+  if ((dtype == PCE_F16) != (packed != nullptr)) PCE_FAIL(PCE_EINVAL, "pce_prepare_weights: fp16 weights and only these have a packed copy");
+  if (!aligned16(packed)) PCE_FAIL(PCE_EINVAL, "pce_prepare_weights: packed copy is not 16-byte aligned");
+  const int bi = (c_in + 31) / 32, bo = (c_out + 31) / 32;
+  const int k = transpose ? c_out : c_in, n = transpose ? c_in : c_out;
+  const int k8_total = (k + 7) / 8, n_pad = (n + 31) / 32 * 32;
+  const long long blocks = (long long)kv * bi * bo;
+  if (blocks >= (1ll << 31)) PCE_FAIL(PCE_ECAPACITY, "pce_prepare_weights: %lld workgroups exceed the grid limit", blocks);
+#define PCE_PREP(TS_, TD_)                                                                                                       \
+  hipLaunchKernelGGL((prepare_weights_kernel<TS_, TD_>), dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (const TS_ *)w, \
+                     (TD_ *)out, (half_t *)packed, kv, c_in, c_out, transpose, flip, k8_total, n_pad, bi, bo)
+  if (dtype_w == PCE_F16)
+    PCE_PREP(half_t, half_t);
+  else if (dtype == PCE_F16)
+    PCE_PREP(float, half_t);
+  else
+    PCE_PREP(float, float);
+#undef PCE_PREP
+  PCE_LAUNCH_CHECK("prepare_weights");
   return PCE_OK;
 }
 

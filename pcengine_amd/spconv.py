@@ -157,15 +157,16 @@ def _pick_dataflow(km: backend.KernelMap, requested: str, c_in: int, c_out: int,
 
 class _ConvFunction(torch.autograd.Function):
     """conv (+ bias) with gradients for features, kernel and bias (conv_d1 / conv_d2,
-    script/spconv.py:110-288)."""
+    script/spconv.py:110-288).  The kernel may be wider than the features: it is converted in the launch that
+    packs it, and its gradient is returned as the fp32 sums."""
 
     @staticmethod
     def forward(ctx, feats, kernel, bias, km, df, transposed, buffer):
-        k = kernel.detach()
+        k, packed = backend.prepare_weights(kernel.detach(), feats.dtype)
         out = backend.conv_forward(feats.detach(), k, km, df, transposed=transposed, buffer=buffer,
-                                   packed=backend.pack_weights(k), bias=None if bias is None else bias.detach())
-        ctx.save_for_backward(feats, kernel)
-        ctx.km, ctx.transposed, ctx.has_bias = km, transposed, bias is not None
+                                   packed=packed, bias=None if bias is None else bias.detach())
+        ctx.save_for_backward(feats, kernel if kernel.dtype == feats.dtype else k)
+        ctx.km, ctx.transposed, ctx.has_bias, ctx.kernel_dtype = km, transposed, bias is not None, kernel.dtype
         return out
 
     @staticmethod
@@ -173,7 +174,8 @@ class _ConvFunction(torch.autograd.Function):
         feats, kernel = ctx.saved_tensors
         grad_out = grad_out.contiguous()
         gf, gw = backend.conv_backward(feats.detach(), kernel.detach(), ctx.km, grad_out, transposed=ctx.transposed,
-                                       need_feats=ctx.needs_input_grad[0], need_weight=ctx.needs_input_grad[1])
+                                       need_feats=ctx.needs_input_grad[0], need_weight=ctx.needs_input_grad[1],
+                                       weight_dtype=ctx.kernel_dtype)
         gb = grad_out.sum(0) if (ctx.has_bias and ctx.needs_input_grad[2]) else None
         return gf, gw, gb, None, None, None, None
 
@@ -183,10 +185,10 @@ class _DenseFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, feats, kernel, bias):
-        k = kernel.detach()
-        out = backend.dense_forward(feats.detach(), k, backend.pack_weights(k), bias=None if bias is None else bias.detach())
-        ctx.save_for_backward(feats, kernel)
-        ctx.has_bias = bias is not None
+        k, packed = backend.prepare_weights(kernel.detach(), feats.dtype)
+        out = backend.dense_forward(feats.detach(), k, packed, bias=None if bias is None else bias.detach())
+        ctx.save_for_backward(feats, kernel if kernel.dtype == feats.dtype else k)
+        ctx.has_bias, ctx.kernel_dtype = bias is not None, kernel.dtype
         return out
 
     @staticmethod
@@ -195,10 +197,10 @@ class _DenseFunction(torch.autograd.Function):
         grad_out = grad_out.contiguous()
         gf = gw = None
         if ctx.needs_input_grad[0]:
-            kt = kernel.detach().t().contiguous()
-            gf = backend.dense_forward(grad_out, kt, backend.pack_weights(kt))
+            kt, packed = backend.prepare_weights(kernel.detach(), kernel.dtype, transpose=True)
+            gf = backend.dense_forward(grad_out, kt, packed)
         if ctx.needs_input_grad[1]:
-            gw = backend.dense_wgrad(feats.detach(), grad_out).to(kernel.dtype)
+            gw = backend.dense_wgrad(feats.detach(), grad_out).to(ctx.kernel_dtype)
         gb = grad_out.sum(0) if (ctx.has_bias and ctx.needs_input_grad[2]) else None
         return gf, gw, gb
 
@@ -233,10 +235,9 @@ def _run(input: spTensor, km: backend.KernelMap, kernel, in_channel, out_channel
     feats = input.feats
     if _wants_grad(feats, kernel, bias):
         _no_out_with_grad(out)
-        k = kernel if kernel.dtype == feats.dtype else kernel.to(feats.dtype)
         b = bias if bias is None or bias.dtype == feats.dtype else bias.to(feats.dtype)
         df = _pick_dataflow(km, dataflow, in_channel, out_channel, feats.dtype, transposed)
-        out = _ConvFunction.apply(feats, k, b, km, df, transposed, input.buffer)
+        out = _ConvFunction.apply(feats, kernel, b, km, df, transposed, input.buffer)
         return _apply_unfused(out, residual, act)
     if kernel.dtype != feats.dtype:
         kernel, packed = kernel.to(feats.dtype), None
@@ -529,9 +530,8 @@ def conv_func(input: spTensor, in_channel, out_channel, kernel, kernel_size_code
         # 1x1 stride 1: plain matrix product, coordinates unchanged, no map (script/spconv.py:297-304)
         if _wants_grad(input.feats, kernel, bias):
             _no_out_with_grad(out)
-            k = kernel if kernel.dtype == input.feats.dtype else kernel.to(input.feats.dtype)
             b = bias if bias is None or bias.dtype == input.feats.dtype else bias.to(input.feats.dtype)
-            return input._like(_apply_unfused(_DenseFunction.apply(input.feats, k, b), residual, act))
+            return input._like(_apply_unfused(_DenseFunction.apply(input.feats, kernel, b), residual, act))
         if kernel.dtype != input.feats.dtype:
             kernel, packed = kernel.to(input.feats.dtype), None
         out_feats = backend.dense_forward(input.feats, kernel.detach(), packed, bias=bias, residual=residual, act=act)
