@@ -462,6 +462,14 @@ int pce_conv_fwd_os(const void *in_feats, const void *weight, const void *weight
                     void *out_feats, int32_t dtype,
                     int64_t n_in, int64_t n_out, int32_t c_in, int32_t c_out, int32_t kv,
                     const int32_t *nbr_dev, const pce_epilogue_t *epilogue, pce_stream_t stream);
+/* The same with a workspace (16-byte aligned), in which fp32 layers of few rows keep partial sums over shares of the
+ * offsets.  pce_conv_os_workspace_bytes gives its size; 0: the layer needs none and runs as pce_conv_fwd_os without
+ * packed weights. */
+int64_t pce_conv_os_workspace_bytes(int32_t dtype, int64_t n_out, int32_t c_in, int32_t c_out, int32_t kv);
+int pce_conv_fwd_os_parts(const void *in_feats, const void *weight, void *out_feats, int32_t dtype,
+                          int64_t n_in, int64_t n_out, int32_t c_in, int32_t c_out, int32_t kv,
+                          const int32_t *nbr_dev, void *workspace_dev, int64_t workspace_bytes,
+                          const pce_epilogue_t *epilogue, pce_stream_t stream);
 
 /* The same for wide fp16 layers, over blocks of rows with equal neighbour patterns: the rows of every 8192 consecutive
  * ones are visited sorted by their patterns, a block of 16 leaves out the offsets none of its rows has, and the tiles

@@ -148,6 +148,9 @@ _SIGNATURES = {
                                    c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64,
                                    POINTER(Epilogue), c_void_p]),
     "pce_conv_fwd_os": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int32, c_int32, c_int32, c_void_p, POINTER(Epilogue), c_void_p]),
+    "pce_conv_os_workspace_bytes": (c_int64, [c_int32, c_int64, c_int32, c_int32, c_int32]),
+    "pce_conv_fwd_os_parts": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int32, c_int32, c_int32, c_void_p, c_void_p,
+                                        c_int64, POINTER(Epilogue), c_void_p]),
     "pce_conv_fwd_oso": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32,
                                    c_void_p, c_void_p, POINTER(c_int64), POINTER(Epilogue), c_void_p]),
     "pce_osb_order_elems": (c_int64, [c_int64]),

@@ -945,14 +945,19 @@ def dense_forward(feats: torch.Tensor, weight: torch.Tensor, packed: Optional[to
 def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataflow: int, transposed: bool = False,
                  buffer: Optional[torch.Tensor] = None, packed: Optional[torch.Tensor] = None,
                  out: Optional[torch.Tensor] = None, bias: Optional[torch.Tensor] = None,
-                 residual: Optional[torch.Tensor] = None, act=None, route_single_pairs: bool = True) -> torch.Tensor:
+                 residual: Optional[torch.Tensor] = None, act=None, route_single_pairs: bool = True,
+                 split_offsets: bool = True) -> torch.Tensor:
     """One forward convolution over an existing map with the chosen dataflow:
     ``act(conv(feats) + bias + residual)``, the last three optional and applied inside the kernels
     (``act``: None, 'relu' or ('leaky_relu', slope)).
 
     ``out`` (optional) is a preallocated [n_out, c_out] tensor of the feature dtype: with it, a
     large enough ``buffer`` and a dataflow other than plain fetch-on-demand the call allocates
-    nothing, so a loop of layers can be captured into a HIP graph."""
+    nothing, so a loop of layers can be captured into a HIP graph.
+
+    ``split_offsets``: output-stationary fp32 layers of few rows may add up shares of the offsets.  The layers of a
+    training step don't: a last bit there decides which side of a ReLU an activation is on, 0.5 % of a gradient at the
+    deep levels of a small scan, and a run that is continued should go on as it began."""
     lib = _lib.load()
     _require_cuda(feats, "feats")
     # the deferred-scatter and output-stationary kernels take column slices of wider matrices in place (the halves
@@ -1067,8 +1072,16 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
             _lib.check(lib.pce_conv_fwd_osb(feats.data_ptr(), packed.data_ptr(), out.data_ptr(), dt, n_in, n_out, km.M, c_in, c_out, kv,
                                             nbr.data_ptr(), order.data_ptr(), ws.data_ptr(), ws_bytes, epi, s))
             return out
-        _lib.check(lib.pce_conv_fwd_os(feats.data_ptr(), weight.data_ptr(), _ptr(packed), out.data_ptr(), dt, n_in, n_out,
-                                       c_in, c_out, kv, nbr.data_ptr(), epi, s))
+        need = lib.pce_conv_os_workspace_bytes(dt, n_out, c_in, c_out, kv) if split_offsets else 0
+        if need > 0:
+            ws = buffer
+            if ws is None or ws.numel() * ws.element_size() < need or ws.device != dev or not ws.is_contiguous() or ws.data_ptr() % 16:
+                ws = _staging(need, torch.uint8, dev)
+            _lib.check(lib.pce_conv_fwd_os_parts(feats.data_ptr(), weight.data_ptr(), out.data_ptr(), dt, n_in, n_out, c_in, c_out, kv,
+                                                 nbr.data_ptr(), ws.data_ptr(), need, epi, s))
+        else:
+            _lib.check(lib.pce_conv_fwd_os(feats.data_ptr(), weight.data_ptr(), _ptr(packed), out.data_ptr(), dt, n_in, n_out,
+                                           c_in, c_out, kv, nbr.data_ptr(), epi, s))
     else:
         raise NotImplementedError(f"unknown dataflow {dataflow}")
     if slice_out is not None:
@@ -1249,7 +1262,8 @@ def conv_backward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, grad
         # conv_forward): they are reversed in the launch that transposes them
         mirror = not transposed and km.subm and all(k % 2 == 1 for k in km.ks)
         wt, packed = prepare_weights(w3, w3.dtype, transpose=True, flip=mirror)
-        gf = conv_forward(grad_out.contiguous(), wt, km, df, transposed=not transposed and not mirror, packed=packed)
+        gf = conv_forward(grad_out.contiguous(), wt, km, df, transposed=not transposed and not mirror, packed=packed,
+                          split_offsets=False)
     if need_weight:
         gw = conv_wgrad(feats, grad_out, km, transposed).to(weight_dtype or weight.dtype).reshape(weight.shape)
     return gf, gw

@@ -418,6 +418,11 @@ __global__ void __launch_bounds__(256, ((TMODE >= 0 && sizeof(T) == 2 && NB <= 2
     arow = (mode == MODE_DENSE) ? orow : -1;
     w_begin = (mode == MODE_DENSE) ? a.w_fixed : 0;
     w_end = (mode == MODE_DENSE) ? a.w_fixed + 1 : a.kv;
+    if (mode == MODE_OS && a.parts > 1) {   // this workgroup's share of the offsets, its sums go to the share's own rows
+      w_begin = a.kv * (int)blockIdx.y / a.parts;
+      w_end = a.kv * ((int)blockIdx.y + 1) / a.parts;
+      a.out = (float *)a.out + (long long)blockIdx.y * a.n_rows * a.c_out;
+    }
   } else {
     // indicator: which offset owns this tile = number of segment ends at or before its first row
     long long q0 = tile * 128;
@@ -1103,28 +1108,39 @@ static int launch_os_pipe(TileArgs a, long long tiles, hipStream_t s) {
   return PCE_OK;
 }
 
+#define OS_WORKGROUPS 512   // two per compute unit
+
 static unsigned xcd_grid(TileArgs *a, long long tiles, int slabs) {
   a->slabs = slabs;
   a->items = tiles * slabs;
   return (unsigned)(pce_div_up(a->items, PCE_XCDS) * PCE_XCDS);
 }
 
+// 32-column blocks of a column slab: up to four (every slab gathers the rows again).  In fp32 a wavefront multiplies 32
+// rows by 128 columns at 14 us per 256 input channels whatever the number of rows, so where the tiles leave the chip
+// without two workgroups per compute unit the slabs get narrower, with the same sums: the centre GEMMs of a U-Net's deep
+// levels on a small scan (8 to 16 workgroups before) 23-30 us -> 11, 128 -> 128 on 30 k LiDAR rows 41.6 us -> 33.0, 256 -> 256
+// on 4 k dense rows 86 -> 75, and nothing slower from 16 to 512 channels.  The fp16 instruction is 16 times faster and the gathers decide there.
+static int tile_blocks(int elem, long long tiles, int c_out) {
+  const int nb = (c_out + 31) / 32;
+  if (elem == 2 || nb == 1) return nb < 4 ? nb : 4;
+  if (nb >= 4 && tiles * ((nb + 3) / 4) >= OS_WORKGROUPS) return 4;
+  if (nb < 4 && tiles >= OS_WORKGROUPS) return nb;
+  return nb >= 4 && tiles * ((nb + 1) / 2) >= OS_WORKGROUPS ? 2 : 1;
+}
+
 template <typename T, bool FAST, int TMODE, int TEPI>
 static void launch_tile_nb(TileArgs a, long long tiles, hipStream_t s) {
-  int nb = (a.c_out + 31) / 32;
-  if (nb >= 4) {
-    unsigned grid = xcd_grid(&a, tiles, (a.c_out + 127) / 128);
-    hipLaunchKernelGGL((tile_gemm_kernel<T, 4, FAST, TMODE, TEPI>), dim3(grid), dim3(256), 0, s, a);
-  } else if (nb == 3) {
-    unsigned grid = xcd_grid(&a, tiles, 1);
-    hipLaunchKernelGGL((tile_gemm_kernel<T, 3, FAST, TMODE, TEPI>), dim3(grid), dim3(256), 0, s, a);
-  } else if (nb == 2) {
-    unsigned grid = xcd_grid(&a, tiles, 1);
-    hipLaunchKernelGGL((tile_gemm_kernel<T, 2, FAST, TMODE, TEPI>), dim3(grid), dim3(256), 0, s, a);
-  } else {
-    unsigned grid = xcd_grid(&a, tiles, 1);
-    hipLaunchKernelGGL((tile_gemm_kernel<T, 1, FAST, TMODE, TEPI>), dim3(grid), dim3(256), 0, s, a);
-  }
+  const int nb = tile_blocks(sizeof(T), tiles, a.c_out);
+  const dim3 grid(xcd_grid(&a, tiles, (a.n_pad / 32 + nb - 1) / nb), a.parts > 1 ? a.parts : 1);
+  if (nb == 4)
+    hipLaunchKernelGGL((tile_gemm_kernel<T, 4, FAST, TMODE, TEPI>), grid, dim3(256), 0, s, a);
+  else if (nb == 3)
+    hipLaunchKernelGGL((tile_gemm_kernel<T, 3, FAST, TMODE, TEPI>), grid, dim3(256), 0, s, a);
+  else if (nb == 2)
+    hipLaunchKernelGGL((tile_gemm_kernel<T, 2, FAST, TMODE, TEPI>), grid, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((tile_gemm_kernel<T, 1, FAST, TMODE, TEPI>), grid, dim3(256), 0, s, a);
 }
 
 template <typename T>
@@ -1990,6 +2006,84 @@ static int os_impl(const void *in, const void *w, const void *wp, void *out, int
   a.mode = MODE_OS;
   a.epi = EPI_ROWS;
   return launch_tile<T>(a, pce_div_up(n_out, 128), s);
+}
+
+// Output-stationary fp32 layers of few rows: a tile walks its offsets one after the other (10 us each at 256 -> 256
+// channels), so a few tiles take as long as many.  The offsets are shared out among `parts` workgroups per tile and
+// column slab, as many as make two workgroups per compute unit; every share stores its fp32 sums and os_parts_kernel adds
+// them up in the order of the offsets and finishes the rows.  The partial sums are at most 512 tiles of 128 x 32 (8 MB).
+// Where a tile has less to do than about six offsets of 128 channels the second launch costs what the shares give.
+// Layers of a U-Net on a 28 k-voxel surface scan whose tiles make 8 to 88 workgroups: 5.2 ms in 29 launches -> 0.9 ms in 60;
+// a forward of it 4.64 -> 2.32 ms, of the wide one on 8 k voxels 4.64 -> 2.94.
+static int os_parts(int dtype, long long n_out, int c_in, int c_out, int kv) {
+  if (dtype != PCE_F32 || n_out <= 0 || (long long)kv * c_in < 768) return 1;
+  const long long tiles = pce_div_up(n_out, 128);
+  const int nb = tile_blocks(4, tiles, c_out);
+  const long long parts = OS_WORKGROUPS / (tiles * (((c_out + 31) / 32 + nb - 1) / nb));
+  return parts < 2 ? 1 : parts < kv ? (int)parts : kv;
+}
+
+template <int VEC>
+__global__ void __launch_bounds__(256) os_parts_kernel(const float *__restrict__ part, int parts, long long n_rows, int c_out,
+                                                       float *__restrict__ out, int ldo, const float *__restrict__ bias,
+                                                       const float *__restrict__ res, int act, float slope) {
+  typedef typename VecOf<float, VEC>::type V;
+  const int row_vecs = c_out / VEC;
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x, total = n_rows * row_vecs;
+  if (i >= total) return;
+  const long long row = i / row_vecs;
+  const int col = (int)(i - row * row_vecs) * VEC;
+  const V *src = reinterpret_cast<const V *>(part) + i;
+  V sum = src[0];
+#pragma unroll 8
+  for (int p = 1; p < parts; ++p) sum += src[p * total];
+  if (bias) sum += *reinterpret_cast<const V *>(bias + col);
+  if (res) sum += *reinterpret_cast<const V *>(res + row * c_out + col);
+  float *v = reinterpret_cast<float *>(&sum);
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) v[j] = act_apply(v[j], act, slope);
+  *reinterpret_cast<V *>(out + row * ldo + col) = sum;
+}
+
+extern "C" int64_t pce_conv_os_workspace_bytes(int32_t dtype, int64_t n_out, int32_t c_in, int32_t c_out, int32_t kv) {
+  const int parts = c_in > 0 && c_out > 0 && kv > 0 ? os_parts(dtype, n_out, c_in, c_out, kv) : 1;
+  return parts > 1 ? (int64_t)parts * n_out * c_out * 4 : 0;
+}
+
+extern "C" int pce_conv_fwd_os_parts(const void *in, const void *w, void *out, int32_t dtype, int64_t n_in, int64_t n_out,
+                                     int32_t c_in, int32_t c_out, int32_t kv, const int32_t *nbr, void *ws, int64_t ws_bytes,
+                                     const pce_epilogue_t *epilogue, pce_stream_t stream) {
+  int rc = check_common("pce_conv_fwd_os_parts", in, w, out, dtype, n_in, n_out, c_in, c_out, kv, -1);
+  if (rc) return rc;
+  if (!nbr) PCE_FAIL(PCE_EINVAL, "pce_conv_fwd_os_parts: null neighbour table");
+  const int64_t need = pce_conv_os_workspace_bytes(dtype, n_out, c_in, c_out, kv);
+  if (need == 0) return pce_conv_fwd_os(in, w, nullptr, out, dtype, n_in, n_out, c_in, c_out, kv, nbr, epilogue, stream);
+  if (!ws || !aligned16(ws) || ws_bytes < need)
+    PCE_FAIL(PCE_EINVAL, "pce_conv_fwd_os_parts: workspace of %lld bytes, 16-byte aligned, expected", (long long)need);
+  Epi e;
+  if ((rc = read_epilogue("pce_conv_fwd_os_parts", epilogue, out, &e, c_in, c_out))) return rc;
+  hipStream_t s = (hipStream_t)stream;
+  TileArgs a = base_args<float>(in, w, nullptr, kv, c_in, c_out, e.lda);
+  set_out<float>(&a, ws, false);
+  a.nbr = nbr;
+  a.n_rows = n_out;
+  a.mode = MODE_OS;
+  a.epi = EPI_ROWS;
+  a.parts = os_parts(dtype, n_out, c_in, c_out, kv);
+  if ((rc = launch_tile<float>(a, pce_div_up(n_out, 128), s))) return rc;
+  const int ldo = e.ldo > 0 ? e.ldo : c_out;
+  const bool vec = c_out % 4 == 0 && ldo % 4 == 0 && aligned16(out) && aligned16(e.bias) && aligned16(e.res);
+  const long long total = (long long)n_out * (vec ? c_out / 4 : c_out);
+#define PCE_PARTS(VEC_)                                                                                              \
+  hipLaunchKernelGGL((os_parts_kernel<VEC_>), dim3((unsigned)pce_div_up(total, 256)), dim3(256), 0, s, (const float *)ws, \
+                     a.parts, (long long)n_out, c_out, (float *)out, ldo, (const float *)e.bias, (const float *)e.res, e.act, e.slope)
+  if (vec)
+    PCE_PARTS(4);
+  else
+    PCE_PARTS(1);
+#undef PCE_PARTS
+  PCE_LAUNCH_CHECK("os_parts");
+  return PCE_OK;
 }
 
 extern "C" int pce_conv_fwd_os(const void *in, const void *w, const void *wp, void *out, int32_t dtype, int64_t n_in,

@@ -58,6 +58,7 @@ struct TileArgs {
   long long n_rows;  // MODE_DENSE / MODE_OS: rows of the output
   long long items;   // (tile, column slab) work items of the launch
   int slabs;         // column slabs per tile
+  int parts;         // MODE_OS: shares of the offsets, blockIdx.y; the sums of share p at out + p * n_rows * c_out (0, 1: one)
   int kv, c_in, c_out;
   int lda, ldo;      // elements between consecutive rows of A and of `out` (rows of buf, res and out_alt are dense)
   int w_fixed;

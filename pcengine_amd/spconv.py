@@ -164,7 +164,7 @@ class _ConvFunction(torch.autograd.Function):
     def forward(ctx, feats, kernel, bias, km, df, transposed, buffer):
         k, packed = backend.prepare_weights(kernel.detach(), feats.dtype)
         out = backend.conv_forward(feats.detach(), k, km, df, transposed=transposed, buffer=buffer,
-                                   packed=packed, bias=None if bias is None else bias.detach())
+                                   packed=packed, bias=None if bias is None else bias.detach(), split_offsets=False)
         ctx.save_for_backward(feats, kernel if kernel.dtype == feats.dtype else k)
         ctx.km, ctx.transposed, ctx.has_bias, ctx.kernel_dtype = km, transposed, bias is not None, kernel.dtype
         return out
