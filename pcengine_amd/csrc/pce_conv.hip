@@ -411,6 +411,7 @@ __global__ void __launch_bounds__(256, ((TMODE >= 0 && sizeof(T) == 2 && NB <= 2
 
   int arow = -1, orow = -1;
   int w_begin, w_end;
+  char *out = (char *)a.out;
   long long row = tile * 128 + wave * 32 + l32;
   if (mode == MODE_DENSE || mode == MODE_OS) {
     bool ok = row < a.n_rows;
@@ -418,10 +419,10 @@ __global__ void __launch_bounds__(256, ((TMODE >= 0 && sizeof(T) == 2 && NB <= 2
     arow = (mode == MODE_DENSE) ? orow : -1;
     w_begin = (mode == MODE_DENSE) ? a.w_fixed : 0;
     w_end = (mode == MODE_DENSE) ? a.w_fixed + 1 : a.kv;
-    if (mode == MODE_OS && a.parts > 1) {   // this workgroup's share of the offsets, its sums go to the share's own rows
+    if (sizeof(T) == 4 && mode == MODE_OS && a.parts > 1) {   // a share of the offsets, its sums to the share's own rows
       w_begin = a.kv * (int)blockIdx.y / a.parts;
       w_end = a.kv * ((int)blockIdx.y + 1) / a.parts;
-      a.out = (float *)a.out + (long long)blockIdx.y * a.n_rows * a.c_out;
+      out += (long long)blockIdx.y * a.n_rows * a.c_out * 4;
     }
   } else {
     // indicator: which offset owns this tile = number of segment ends at or before its first row
@@ -542,14 +543,14 @@ __global__ void __launch_bounds__(256, ((TMODE >= 0 && sizeof(T) == 2 && NB <= 2
   }
   if (FAST || a.o_vec) {
     if (f32out)
-      store_rows_via_lds<float, NB>(V, Pl[wave], (float *)a.out, orow, a, n0, lane, l32, g, a.stream);
+      store_rows_via_lds<float, NB>(V, Pl[wave], (float *)out, orow, a, n0, lane, l32, g, a.stream);
     else
-      store_rows_via_lds<half_t, NB>(V, Pl[wave], (half_t *)a.out, orow, a, n0, lane, l32, g, a.stream);
+      store_rows_via_lds<half_t, NB>(V, Pl[wave], (half_t *)out, orow, a, n0, lane, l32, g, a.stream);
   } else {
     if (f32out)
-      store_row_pieces_slow<float, NB>(V, (float *)a.out, orow, a, n0, g);
+      store_row_pieces_slow<float, NB>(V, (float *)out, orow, a, n0, g);
     else
-      store_row_pieces_slow<half_t, NB>(V, (half_t *)a.out, orow, a, n0, g);
+      store_row_pieces_slow<half_t, NB>(V, (half_t *)out, orow, a, n0, g);
   }
 }
 
