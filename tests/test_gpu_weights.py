@@ -1,4 +1,4 @@
-"""The one-launch weight preparation of a training step and the kernel gradient's deal of tiles."""
+"""The one-launch weight preparation of a training step and the kernel gradient over every kind of pair list."""
 import pytest
 import torch
 
@@ -55,9 +55,9 @@ class _Pairs:
     ([300 + 37 * i for i in range(13)] + [0] + [700] * 13, 5000, True, 130, 257),   # several blocks of channels
     ([40] * 125, 500, False, 24, 8),                            # more offsets than lanes
     ([300000, 5, 0, 260000], 3000, False, 32, 32),              # runs of many tiles
-    ([90000, 5, 0, 130, 180000, 0, 1], 3000, False, 72, 24),    # dealt by region: empty and one-tile offsets among long ones
+    ([90000, 5, 0, 130, 180000, 0, 1], 3000, False, 72, 24),    # empty and one-tile offsets among long ones
     ([20000] * 13 + [0] + [20000] * 13, 20001, True, 16, 100),  # ... with a centre
-    ([3000] * 130, 4000, False, 72, 16),                        # ... and more offsets than are kept in LDS
+    ([3000] * 130, 4000, False, 72, 16),                        # more offsets than any kernel map of the networks
 ])
 def test_kernel_gradient_covers_every_pair(dtype, counts, n, centre, ci, co):
     km = _Pairs(counts, n, centre)
