@@ -30,8 +30,11 @@ __device__ constexpr int osb_key_bit27(int kp) {
 
 // One workgroup per window: the rows' patterns (known, or 27 table reads per row), then a radix sort of (key, row) in LDS,
 // three passes of 9 bits.  The key is the rank of the pattern in the reflected Gray code, in which
-// consecutive patterns differ in one bit.  Bound by the LDS counters of the ranking, not by memory: 33 us for the 680 k
-// rows of 83 windows, once per map.
+// consecutive patterns differ in one bit.  The sort is stable by construction: a wavefront ranks its entries of a digit by
+// ballots (the lanes of one LDS atomic have no promised order), so the order of a cloud is the same in every run, and the
+// entries behind the last row of the cloud, which share their key with a pattern of offset 0 alone, stay behind every row.
+// Bound by the ballots and the LDS counters, not by memory: with the plan 36 us for 72 k rows of a random cloud as for
+// 100 k of a scan (ranked by LDS atomics, whose lanes met at few counters: 36 and 43).
 __global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(const int *__restrict__ nbr, const unsigned *__restrict__ known,
                                                                       unsigned centre, int kv, int n, int *__restrict__ perm,
                                                                       unsigned *__restrict__ bmask) {
@@ -85,12 +88,15 @@ __global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(const int 
     keys[li] = ok ? k : (1u << 27) - 1;
     rows[li] = (unsigned short)li;
   }
+  // where a digit's counter of a wavefront lies: the counters one wavefront updates fall into different banks
+  auto counter = [](int d, int w) { return d * WAVES + ((w + (d >> 2)) & (WAVES - 1)); };
   for (int shift = 0; shift < 3 * BITS; shift += BITS) {
     for (int i = t; i < BINS * WAVES; i += OSB_ORDER_THREADS) hist[i] = 0;
     __syncthreads();
     unsigned key[PER], pos[PER];
     unsigned short rw[PER];
-    // rank among the wavefront's entries of one digit: a counter per (digit, wavefront), its updates in issue order
+    // rank among the wavefront's entries of one digit: the lanes below with the same digit, behind those of the entries
+    // before (a counter per (digit, wavefront), updated by the first lane of a digit)
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int at = (wave * PER + i) * 64 + lane;
@@ -98,7 +104,22 @@ __global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(const int 
       rw[i] = rows[at];
     }
 #pragma unroll
-    for (int i = 0; i < PER; ++i) pos[i] = atomicAdd(&hist[((key[i] >> shift) & (BINS - 1)) * WAVES + wave], 1u);
+    for (int i = 0; i < PER; ++i) {
+      const unsigned d = (key[i] >> shift) & (BINS - 1);
+      unsigned long long peers = ~0ull;
+#pragma unroll
+      for (int b = 0; b < BITS; ++b) {
+        const unsigned mine = (unsigned)((int)(d << (31 - b)) >> 31);   // the bit of this lane, in all bits
+        peers &= ~(__ballot(mine != 0) ^ (mine | (unsigned long long)mine << 32));
+      }
+      const int before = __popcll(peers & ((1ull << lane) - 1));
+      unsigned *count = &hist[counter(d, wave)];
+      pos[i] = *count + before;
+      __builtin_amdgcn_wave_barrier();
+      if (before == 0) *count = pos[i] + __popcll(peers);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
     __syncthreads();
     // exclusive scan over (digit, wavefront)
     constexpr int HP = BINS * WAVES / OSB_ORDER_THREADS;
@@ -106,7 +127,7 @@ __global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(const int 
 #pragma unroll
     for (int j = 0; j < HP; ++j) {
       v[j] = sum;
-      sum += hist[t * HP + j];
+      sum += hist[counter((t * HP + j) / WAVES, (t * HP + j) % WAVES)];
     }
     unsigned inc = sum;
 #pragma unroll
@@ -119,12 +140,12 @@ __global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(const int 
     unsigned base = inc - sum;
     for (int w = 0; w < wave; ++w) base += wave_sum[w];
 #pragma unroll
-    for (int j = 0; j < HP; ++j) hist[t * HP + j] = base + v[j];
+    for (int j = 0; j < HP; ++j) hist[counter((t * HP + j) / WAVES, (t * HP + j) % WAVES)] = base + v[j];
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const unsigned d = (key[i] >> shift) & (BINS - 1);
-      const unsigned p = hist[d * WAVES + wave] + pos[i];
+      const unsigned p = hist[counter(d, wave)] + pos[i];
       keys[p] = key[i];
       rows[p] = rw[i];
     }
