@@ -13,6 +13,7 @@ Torch is used for device memory and the current stream only.
 """
 from __future__ import annotations
 
+import threading
 from dataclasses import dataclass, field
 from typing import List, Optional, Sequence, Tuple
 
@@ -22,6 +23,7 @@ from . import _lib
 from ._lib import Geom, DATAFLOW_FOD, DATAFLOW_GMS, DATAFLOW_OS, DATAFLOW_FDS, DATAFLOW_OSO, PCE_F16, PCE_F32, QUANTUM, CSR_CODE
 
 _OSB_MAX_BYTES = 0xF0000000      # features the block output-stationary kernel addresses
+OSB_MAX_KV = 27                  # ... and the largest kernel volume it takes
 CODE_A, CODE_B = 94273, 311  # packed 3-vectors, script/utils.py:233-242
 
 
@@ -633,8 +635,24 @@ class PyramidPlan:
             raise PlanNotApplicable()
         _lib.check(rc)
         self.n_cap, self.n_batch, self.device = int(n_cap), int(n_batch), device
-        self.arena = torch.empty(self.plan.arena_bytes, dtype=torch.uint8, device=device)
+        # behind the library's arrays a place for what layers build on first use and keep on a map (_build_kept)
+        end, places = self.plan.arena_bytes, []
+        for i, (ks, stride, _, _, _, subm) in enumerate(self.args):
+            m, want = self.plan.map[i], {}
+            if m.kv <= OSB_MAX_KV:
+                want["blocks", False] = lib.pce_osb_order_elems(m.cap_out)
+                if reqs[i].want_nbr_in:
+                    want["blocks", True] = lib.pce_osb_order_elems(m.cap_in)
+            if not subm and ks == stride:       # an input row is in one pair at most
+                want["route", False] = lib.pce_pair_route_elems(m.cap_in, m.cap_out)
+                want["route", True] = lib.pce_pair_route_elems(m.cap_in, m.cap_in)
+            places.append({})
+            for key, elems in want.items():
+                places[i][key] = (end // 4, elems)
+                end += -(-elems * 4 // 256) * 256
+        self.arena = torch.empty(end, dtype=torch.uint8, device=device)
         self.arena32 = self.arena.view(torch.int32)
+        self.places = [{key: self.arena32[at:at + elems] for key, (at, elems) in p.items()} for p in places]
 
     def build(self, in_coords: torch.Tensor):
         """(coordinates of every level, the maps in request order) for one cloud.  Raises ``PlanNotApplicable`` when
@@ -678,7 +696,7 @@ class PyramidPlan:
             km._cmin, km._cmax = cmin, cmax_out
             km.kpos_host = (_lib.c_int32 * (kv + 1))(*meta[kv:2 * kv + 1])
             km.qkpos_host = (_lib.c_int32 * (kv + 1))(*meta[2 * kv + 1:3 * kv + 2])
-            km._arena = self.arena
+            km._arena, km._places = self.arena, self.places[i]
             maps.append(km)
         return coords, maps
 
@@ -706,20 +724,58 @@ def ensure_csr(km: KernelMap) -> None:
         km.imap, km.omap = full.imap, full.omap
 
 
+_first_use = threading.Lock()
+
+
+def _build_kept(km: KernelMap, kept: dict, what: str, transposed: bool, elems: int, device, build) -> torch.Tensor:
+    """An int32 array that a layer builds on first use and that stays with its map in ``kept[transposed]``, made by
+    ``build(array)`` on the current stream.  It lives as long as the map: in the allocation of the map's plan where that
+    holds a place for it, else in memory of its own, never in a forward's arena (a map outlives forwards).  Under capture
+    nothing is kept: the kernels of a capture have not run yet, so an array built there belongs to the graph alone."""
+    with _first_use:
+        if transposed in kept:
+            return _kept(kept[transposed], device)
+        capturing = torch.cuda.is_current_stream_capturing()
+        place = None if capturing else km.__dict__.get("_places", {}).get((what, transposed))
+        array = place[:elems] if place is not None and place.numel() >= elems else torch.empty(elems, dtype=torch.int32, device=device)
+        build(array)
+        if not capturing:
+            event = torch.cuda.Event()
+            event.record(torch.cuda.current_stream(device))
+            kept[transposed] = (array, _stream(device), event)
+        return array
+
+
+def _kept(entry, device) -> torch.Tensor:
+    """The array of an entry that ``_build_kept`` made; another stream than the one that built it waits for it (not under
+    capture: what a graph reads from other streams is the program's to order before a replay, as for its inputs)."""
+    array, built_on, event = entry
+    if built_on != _stream(device) and not torch.cuda.is_current_stream_capturing():
+        current = torch.cuda.current_stream(device)
+        current.wait_event(event)
+        array.record_stream(current)
+    return array
+
+
 def pair_route(km: KernelMap, transposed: bool = False) -> torch.Tensor:
     """Routing array of a layer without centre offset, cached on the map (``pce_pair_route``): the number of output
     rows whose pair count is not one, the destination of every pair (the output row where the pair is the row's
     only one, else ``n_out`` + its partial-row slot) and the list of those rows.  ``transposed``: the array of
     the transposed layer, whose output rows are the map's input rows."""
-    route = km.route_t if transposed else km.route
-    if route is None:
-        ensure_csr(km)
-        lib = _lib.load()
-        omap, oslot, ocsr, n_out = (km.imap, km.islot, km.icsr, km.n_in) if transposed else (km.omap, km.oslot, km.ocsr, km.n_out)
-        elems = lib.pce_pair_route_elems(km.M, n_out)
-        route = _new(elems, torch.int32, omap.device)
+    kept = km.__dict__.setdefault("_routes", {})
+    if transposed in kept:
+        return _kept(kept[transposed], km.out_coords.device)
+    ensure_csr(km)
+    lib = _lib.load()
+    omap, oslot, ocsr, n_out = (km.imap, km.islot, km.icsr, km.n_in) if transposed else (km.omap, km.oslot, km.ocsr, km.n_out)
+    elems = lib.pce_pair_route_elems(km.M, n_out)
+
+    def build(route):
         _lib.check(lib.pce_pair_route(omap.data_ptr(), oslot.data_ptr(), ocsr.data_ptr(), km.M, n_out,
                                       route.data_ptr(), elems, _stream(omap.device)))
+
+    route = _build_kept(km, kept, "route", transposed, elems, omap.device, build)
+    if transposed in kept:
         if transposed:
             km.route_t = route
         else:
@@ -745,32 +801,21 @@ def row_order(km: KernelMap) -> torch.Tensor:
 
 def block_order(km: KernelMap, transposed: bool = False) -> torch.Tensor:
     """Row order of the block output-stationary kernel (``pce_osb_order``), cached on the map per direction: two
-    launches, no wait of the host.  Another stream than the one that built it waits for it."""
-    cached = km.__dict__.setdefault("_blocks", {})
-    entry = cached.get(transposed)
-    if entry is None:
-        nbr, n = (km.nbr_in, km.n_in) if transposed else (km.nbr_out, km.n_out)
-        lib = _lib.load()
-        elems = lib.pce_osb_order_elems(n)
-        # a map of a planned pyramid lives as long as the forward's arena; any other may outlive it
-        planned = "_arena" in km.__dict__
-        order = (_new if planned else torch.empty)(elems, dtype=torch.int32, device=nbr.device)
+    launches, no wait of the host."""
+    nbr, n = (km.nbr_in, km.n_in) if transposed else (km.nbr_out, km.n_out)
+    kept = km.__dict__.setdefault("_blocks", {})
+    if transposed in kept:
+        return _kept(kept[transposed], nbr.device)
+    lib = _lib.load()
+    elems = lib.pce_osb_order_elems(n)
+
+    def build(order):
         # the row order of the ordered dataflow, where the map came with one, holds the rows' patterns already
         known = None if transposed or km.order is None else km.order.data_ptr() + 4 * n
         mid = _mid(km.ks) if km.subm and not transposed else -1
-        s = _stream(nbr.device)
-        _lib.check(lib.pce_osb_order(nbr.data_ptr(), known, mid, km.kv, n, order.data_ptr(), elems, s))
-        event = None
-        if not planned:
-            event = torch.cuda.Event()
-            event.record(torch.cuda.current_stream(nbr.device))
-        entry = cached[transposed] = (order, s, event)
-    order, s, event = entry
-    if event is not None and s != _stream(order.device):
-        current = torch.cuda.current_stream(order.device)
-        current.wait_event(event)
-        order.record_stream(current)
-    return order
+        _lib.check(lib.pce_osb_order(nbr.data_ptr(), known, mid, km.kv, n, order.data_ptr(), elems, _stream(nbr.device)))
+
+    return _build_kept(km, kept, "blocks", transposed, elems, nbr.device, build)
 
 
 _osb_takes_cache = {}
