@@ -481,7 +481,8 @@ int pce_conv_fwd_os_parts(const void *in_feats, const void *weight, void *out_fe
  * pce_row_order; mid (or -1): an offset every row counts as having (the centre, which those patterns leave out).
  * pce_conv_osb_takes(dtype, c_in, c_out, kv): fp16, c_in a multiple of 32 from 64 on, c_out a multiple of 8 from 72 to
  * 1024, kv from 2 to 27.  weight_packed from pce_pack_weights; ws of pce_conv_osb_workspace_bytes(n_out, c_out) bytes,
- * its contents do not outlive the call's work on the stream; all pointers 16-byte aligned; at most 3.75 GiB of features.
+ * its contents do not outlive the call's work on the stream, or NULL where pce_conv_osb_scratch_bytes says 0 (no tile of
+ * the layer is cut); all pointers 16-byte aligned; at most 3.75 GiB of features.
  * n_pairs: the map's pairs without the centre ones (an estimate of the work of a tile), -1 = unknown.
  * The sums of a row do not depend on the order of the rows, except that a layer whose tiles do not fill the last round
  * of workgroups adds up some tiles in several parts. */
@@ -490,6 +491,7 @@ int pce_osb_order(const int32_t *nbr_dev, const int32_t *mask_dev, int32_t mid, 
                   int64_t order_elems, pce_stream_t stream);
 int pce_conv_osb_takes(int32_t dtype, int32_t c_in, int32_t c_out, int32_t kv);
 int64_t pce_conv_osb_workspace_bytes(int64_t n_out, int32_t c_out);
+int64_t pce_conv_osb_scratch_bytes(int64_t n_out, int64_t n_pairs, int32_t c_in, int32_t c_out, int32_t kv);
 /* 1 where it is the fastest dataflow of a submanifold layer (mid >= 0): asked before pce_select_dataflow, which knows the
  * dataflows that need no block order. */
 int pce_conv_osb_leads(int64_t n_out, int64_t n_pairs, int32_t c_in, int32_t c_out, int32_t kv, int32_t mid, int32_t dtype);

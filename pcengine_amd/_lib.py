@@ -158,6 +158,7 @@ _SIGNATURES = {
     "pce_conv_osb_takes": (c_int32, [c_int32, c_int32, c_int32, c_int32]),
     "pce_conv_osb_leads": (c_int32, [c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, c_int32]),
     "pce_conv_osb_workspace_bytes": (c_int64, [c_int64, c_int32]),
+    "pce_conv_osb_scratch_bytes": (c_int64, [c_int64, c_int64, c_int32, c_int32, c_int32]),
     "pce_conv_fwd_osb": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int64, c_int32, c_int32, c_int32, c_void_p,
                                    c_void_p, c_void_p, c_int64, POINTER(Epilogue), c_void_p]),
     "pce_row_order": (c_int32, [c_void_p, c_int32, c_int64, c_int32, c_void_p, c_int64, POINTER(c_int64), c_void_p]),

@@ -598,6 +598,16 @@ def _staging(numel: int, dtype, device) -> torch.Tensor:
     return torch.empty(max(int(numel), 1), dtype=dtype, device=device)
 
 
+def _scratch(buffer: Optional[torch.Tensor], need: int, device) -> Optional[torch.Tensor]:
+    """``need`` bytes for one call: the caller's buffer where it serves, else staging memory; None for none."""
+    if need <= 0:
+        return None
+    if buffer is not None and buffer.numel() * buffer.element_size() >= need and buffer.device == device and \
+            buffer.is_contiguous() and buffer.data_ptr() % 16 == 0:
+        return buffer
+    return _staging(need, torch.uint8, device)
+
+
 class PlanNotApplicable(Exception):
     """The native planner does not take this pyramid (a level that is not a bitmap chain, an unsorted cloud): the
     caller builds map by map."""
@@ -998,7 +1008,8 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
 
     ``out`` (optional) is a preallocated [n_out, c_out] tensor of the feature dtype: with it, a
     large enough ``buffer`` and a dataflow other than plain fetch-on-demand the call allocates
-    nothing, so a loop of layers can be captured into a HIP graph.
+    nothing once the arrays it keeps on the map (row order, block order, pair route) are built, so a
+    loop of layers can be captured into a HIP graph.
 
     ``split_offsets``: output-stationary fp32 layers of few rows may add up shares of the offsets.  The layers of a
     training step don't: a last bit there decides which side of a ReLU an activation is on, 0.5 % of a gradient at the
@@ -1112,16 +1123,14 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
             if packed is None:
                 packed = pack_weights(weight)
             order = block_order(km, transposed)
-            ws_bytes = lib.pce_conv_osb_workspace_bytes(n_out, c_out)
-            ws = _staging(ws_bytes, torch.uint8, dev)
+            need = lib.pce_conv_osb_scratch_bytes(n_out, km.M, c_in, c_out, kv)
+            ws = _scratch(buffer, need, dev)
             _lib.check(lib.pce_conv_fwd_osb(feats.data_ptr(), packed.data_ptr(), out.data_ptr(), dt, n_in, n_out, km.M, c_in, c_out, kv,
-                                            nbr.data_ptr(), order.data_ptr(), ws.data_ptr(), ws_bytes, epi, s))
+                                            nbr.data_ptr(), order.data_ptr(), _ptr(ws), need, epi, s))
             return out
         need = lib.pce_conv_os_workspace_bytes(dt, n_out, c_in, c_out, kv) if split_offsets else 0
         if need > 0:
-            ws = buffer
-            if ws is None or ws.numel() * ws.element_size() < need or ws.device != dev or not ws.is_contiguous() or ws.data_ptr() % 16:
-                ws = _staging(need, torch.uint8, dev)
+            ws = _scratch(buffer, need, dev)
             _lib.check(lib.pce_conv_fwd_os_parts(feats.data_ptr(), weight.data_ptr(), out.data_ptr(), dt, n_in, n_out, c_in, c_out, kv,
                                                  nbr.data_ptr(), ws.data_ptr(), need, epi, s))
         else:

@@ -713,6 +713,13 @@ static bool osb_cuts(int64_t n_out, int64_t n_pairs, int c_in, int kv, long long
   return steps >= 24 && items < 16 * 8 * OSB_SLOTS;
 }
 
+extern "C" int64_t pce_conv_osb_scratch_bytes(int64_t n_out, int64_t n_pairs, int32_t c_in, int32_t c_out, int32_t kv) {
+  if (n_out <= 0 || c_out <= 0) return 0;
+  int cb, slabs;
+  osb_shape(n_out, c_out, &cb, &slabs);
+  return osb_cuts(n_out, n_pairs, c_in, kv, pce_div_up(n_out, OSB_ROWS) * slabs) ? pce_conv_osb_workspace_bytes(n_out, c_out) : 0;
+}
+
 extern "C" int pce_conv_fwd_osb(const void *in, const void *wp, void *out, int32_t dtype, int64_t n_in, int64_t n_out, int64_t n_pairs,
                                 int32_t c_in, int32_t c_out, int32_t kv, const int32_t *nbr, const int32_t *order, void *ws, int64_t ws_bytes,
                                 const pce_epilogue_t *epilogue, pce_stream_t stream) {
@@ -732,10 +739,11 @@ extern "C" int pce_conv_fwd_osb(const void *in, const void *wp, void *out, int32
   const int64_t a_bytes = ((n_in - 1) * (int64_t)a.lda + c_in) * 2;
   if (a_bytes >= (int64_t)OSB_MISSING || n_out >= (1ll << 31) / OSB_MAX_SLABS - OSB_WINDOW)
     PCE_FAIL(PCE_ECAPACITY, "pce_conv_fwd_osb: %lld bytes of features, %lld rows", (long long)a_bytes, (long long)n_out);
-  if (!ws || !aligned16(ws) || ws_bytes < pce_conv_osb_workspace_bytes(n_out, c_out))
-    PCE_FAIL(PCE_EWORKSPACE, "pce_conv_fwd_osb: workspace of %lld bytes, needs %lld", (long long)ws_bytes, (long long)pce_conv_osb_workspace_bytes(n_out, c_out));
   int cb, slabs;
   osb_shape(n_out, c_out, &cb, &slabs);
+  const bool cuts = osb_cuts(n_out, n_pairs, c_in, kv, pce_div_up(n_out, OSB_ROWS) * slabs);
+  if (ws ? !aligned16(ws) || ws_bytes < pce_conv_osb_workspace_bytes(n_out, c_out) : cuts)
+    PCE_FAIL(PCE_EWORKSPACE, "pce_conv_fwd_osb: workspace of %lld bytes, needs %lld", (long long)ws_bytes, (long long)pce_conv_osb_workspace_bytes(n_out, c_out));
   const long long tiles = pce_div_up(n_out, OSB_ROWS);
   OsbArgs o = {};
   o.perm = order;
@@ -744,7 +752,7 @@ extern "C" int pce_conv_fwd_osb(const void *in, const void *wp, void *out, int32
   o.cap = (int)osb_plan_cap(tiles, slabs);
   o.part = (float *)ws;
   o.a_bytes = (unsigned)a_bytes;
-  o.whole = !osb_cuts(n_out, n_pairs, c_in, kv, tiles * slabs);
+  o.whole = !cuts;
   a.slabs = slabs;
   hipStream_t s = (hipStream_t)stream;
   const unsigned grid = (unsigned)(8 * o.cap);
