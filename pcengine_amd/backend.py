@@ -292,10 +292,13 @@ def voxelize(points: torch.Tensor, voxel_size, batch_index: Optional[int] = 0, r
 
 def collate_coords(coords: Sequence[torch.Tensor]):
     """(int32 [N, 4] = (sample, x, y, z), maxima of x, y, z as a list) of the samples' int32 [n, 3] coordinates in one
-    launch, or None where the kernel does not take them (other layouts, devices or dtypes, no rows, many samples)."""
+    launch, or None where the kernel does not take them (other layouts or dtypes, another device than the current one, no
+    rows, many samples)."""
     first = coords[0]
-    if len(coords) > _lib.MAX_COLLATE or not all(c.is_cuda and c.device == first.device and c.dtype == torch.int32 and c.dim() == 2
-                                                 and c.shape[1] == 3 and c.is_contiguous() for c in coords):
+    if len(coords) > _lib.MAX_COLLATE or not first.is_cuda or first.device.index != torch.cuda.current_device():
+        return None
+    if not all(c.device == first.device and c.dtype == torch.int32 and c.dim() == 2 and c.shape[1] == 3 and c.is_contiguous()
+               for c in coords):
         return None
     rows = [c.shape[0] for c in coords]
     total = sum(rows)
