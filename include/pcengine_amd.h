@@ -69,9 +69,11 @@ enum {
   PCE_DATAFLOW_OS = 2,  /* output-stationary fetch-on-demand: no atomics, no staging buffer */
   PCE_DATAFLOW_FDS = 3, /* fetch-on-demand with deferred scatter: pair tiles write partial rows to a
                            staging buffer, the centre GEMM's epilogue sums them per output row */
-  PCE_DATAFLOW_OSO = 4  /* output-stationary over rows ordered by their neighbour pattern (pce_row_order):
+  PCE_DATAFLOW_OSO = 4, /* output-stationary over rows ordered by their neighbour pattern (pce_row_order):
                            fp16 layers up to 64 channels and of 64 / 96 -> 65..128 and 128 -> 65..96 channels, submanifold
                            or strided; fp32 submanifold layers up to 32 channels; one launch, no partial rows */
+  PCE_DATAFLOW_OSB = 5  /* the same over blocks of rows with equal patterns, for wide fp16 layers (pce_conv_fwd_osb);
+                             answered by pce_select_layer only */
 };
 
 #define PCE_QUANTUM 128        /* rows per tile of the pair list; qkpos granularity (backend/hash.cu:203-205) */
@@ -492,8 +494,8 @@ int pce_osb_order(const int32_t *nbr_dev, const int32_t *mask_dev, int32_t mid, 
 int pce_conv_osb_takes(int32_t dtype, int32_t c_in, int32_t c_out, int32_t kv);
 int64_t pce_conv_osb_workspace_bytes(int64_t n_out, int32_t c_out);
 int64_t pce_conv_osb_scratch_bytes(int64_t n_out, int64_t n_pairs, int32_t c_in, int32_t c_out, int32_t kv);
-/* 1 where it is the fastest dataflow of a submanifold layer (mid >= 0): asked before pce_select_dataflow, which knows the
- * dataflows that need no block order. */
+/* 1 where it is the fastest dataflow of a submanifold layer (mid >= 0).  pce_select_dataflow knows the dataflows that
+ * need no block order only; pce_select_layer asks for both. */
 int pce_conv_osb_leads(int64_t n_out, int64_t n_pairs, int32_t c_in, int32_t c_out, int32_t kv, int32_t mid, int32_t dtype);
 int pce_conv_fwd_osb(const void *in_feats, const void *weight_packed, void *out_feats, int32_t dtype, int64_t n_in, int64_t n_out,
                      int64_t n_pairs, int32_t c_in, int32_t c_out, int32_t kv, const int32_t *nbr_dev, const int32_t *order_dev, void *ws, int64_t ws_bytes,
@@ -631,6 +633,13 @@ int pce_conv_wgrad(const void *in_feats, const void *grad_out, int32_t dtype, in
  * class, PCEngine/script/spconv.py:94-124: D1 or D2 by the tag the model file sets.) */
 int pce_select_dataflow(int64_t n_in, int64_t n_out, int64_t n_pairs, int32_t c_in, int32_t c_out,
                         int32_t kv, int32_t mid, int32_t transposed, int32_t dtype);
+
+/* The same with PCE_DATAFLOW_OSB among the answers: a submanifold layer (a transposed one over a map of odd kernel sizes,
+ * which is a plain layer, included) where pce_conv_osb_leads() is 1 and dense rows of the features lie within what
+ * pce_conv_fwd_osb addresses.  Where strided rows do not, or a pointer is not 16-byte aligned, the answer of
+ * pce_select_dataflow is the one to take. */
+int pce_select_layer(int64_t n_in, int64_t n_out, int64_t n_pairs, int32_t c_in, int32_t c_out,
+                     int32_t kv, int32_t mid, int32_t transposed, int32_t dtype);
 
 /* 1 when pce_conv_fwd_oso takes a layer of this dtype, these widths, kernel volume and centre offset (it checks
  * alignment and the packed weights besides), else 0. */

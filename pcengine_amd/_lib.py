@@ -15,7 +15,7 @@ MEASURE_LIB_PATH = os.path.join(_HERE, "lib", "libpcengine_amd_measure.so")
 
 PCE_OK, PCE_EINVAL, PCE_ECAPACITY, PCE_EHIP, PCE_EWORKSPACE, PCE_ECOORD = range(6)
 PCE_F16, PCE_F32, PCE_F64 = 0, 1, 2
-DATAFLOW_FOD, DATAFLOW_GMS, DATAFLOW_OS, DATAFLOW_FDS, DATAFLOW_OSO = 0, 1, 2, 3, 4
+DATAFLOW_FOD, DATAFLOW_GMS, DATAFLOW_OS, DATAFLOW_FDS, DATAFLOW_OSO, DATAFLOW_OSB = 0, 1, 2, 3, 4, 5
 QUANTUM = 128
 KMAP_NO_GRID = 1
 KMAP_TABLE_ONLY = 2
@@ -170,6 +170,7 @@ _SIGNATURES = {
     "pce_pyramid_plan": (c_int32, [c_int64, c_int32, POINTER(Geom), c_int32, POINTER(PyrRequest), c_int32, POINTER(PyrPlan)]),
     "pce_pyramid_build": (c_int32, [POINTER(PyrPlan), c_void_p, c_int64, c_void_p, c_int64, c_void_p]),
     "pce_select_dataflow": (c_int32, [c_int64, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32]),
+    "pce_select_layer": (c_int32, [c_int64, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32]),
     "pce_conv_oso_takes": (c_int32, [c_int32, c_int32, c_int32, c_int32, c_int32]),
 }
 

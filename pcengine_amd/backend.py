@@ -20,7 +20,7 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 
 from . import _lib
-from ._lib import Geom, DATAFLOW_FOD, DATAFLOW_GMS, DATAFLOW_OS, DATAFLOW_FDS, DATAFLOW_OSO, PCE_F16, PCE_F32, QUANTUM, CSR_CODE
+from ._lib import Geom, DATAFLOW_FOD, DATAFLOW_GMS, DATAFLOW_OS, DATAFLOW_FDS, DATAFLOW_OSO, DATAFLOW_OSB, PCE_F16, PCE_F32, QUANTUM, CSR_CODE
 
 _OSB_MAX_BYTES = 0xF0000000      # features the block output-stationary kernel addresses
 OSB_MAX_KV = 27                  # ... and the largest kernel volume it takes
@@ -871,22 +871,25 @@ def ensure_nbr(km: KernelMap, transposed: bool) -> None:
         km.order_nonzero, km.order_single = full.order_nonzero, full.order_single
 
 
-def select_dataflow(km: KernelMap, c_in: int, c_out: int, dtype: torch.dtype, transposed: bool = False) -> int:
+def pick_dataflow(km: KernelMap, c_in: int, c_out: int, dtype: torch.dtype, transposed: bool = False, blocks: bool = True) -> int:
+    """The dataflow of a layer over this map.  ``DATAFLOW_OSB`` where the block kernel leads: ``conv_forward`` takes it then,
+    or, where its rows or pointers do not fit that kernel, what this answers without ``blocks``."""
     lib = _lib.load()
-    n_out = km.n_in if transposed else km.n_out
-    n_in = km.n_out if transposed else km.n_in
-    # (the transposed layer over a submanifold map of odd kernel sizes is a plain layer, see conv_forward)
-    if osb_takes(km.kv, c_in, c_out, dtype) and km.subm and (not transposed or all(k % 2 == 1 for k in km.ks)) and \
-            lib.pce_conv_osb_leads(n_out, km.M, c_in, c_out, km.kv, _mid(km.ks), PCE_F16):
-        return DATAFLOW_OS
-    df = lib.pce_select_dataflow(n_in, n_out, km.M, c_in, c_out, km.kv, _mid(km.ks) if km.subm else -1, int(bool(transposed)),
-                                 PCE_F16 if dtype == torch.float16 else PCE_F32)
-    if not km.has_pairs and df not in (DATAFLOW_OSO, DATAFLOW_OS):
+    n_in, n_out = (km.n_out, km.n_in) if transposed else (km.n_in, km.n_out)
+    select = lib.pce_select_layer if blocks else lib.pce_select_dataflow
+    df = select(n_in, n_out, km.M, c_in, c_out, km.kv, _mid(km.ks) if km.subm else -1, int(bool(transposed)),
+                PCE_F16 if dtype == torch.float16 else PCE_F32)
+    if not km.has_pairs and df not in (DATAFLOW_OSO, DATAFLOW_OS, DATAFLOW_OSB):
         # a map built without pair lists (its layers were expected to read the neighbour table only): rather than
         # build them now, the layer takes the table-reading dataflow that is closest (a band of densities where the
         # ordered dataflow is within a tenth of deferred scatter)
         df = DATAFLOW_OSO if oso_takes(km, c_in, c_out, dtype, transposed) else DATAFLOW_OS
     return df
+
+
+def select_dataflow(km: KernelMap, c_in: int, c_out: int, dtype: torch.dtype, transposed: bool = False) -> int:
+    df = pick_dataflow(km, c_in, c_out, dtype, transposed)
+    return DATAFLOW_OS if df == DATAFLOW_OSB else df
 
 
 def pack_weights(weight: torch.Tensor) -> Optional[torch.Tensor]:
@@ -1021,7 +1024,7 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
     _require_cuda(feats, "feats")
     # the deferred-scatter and output-stationary kernels take column slices of wider matrices in place (the halves
     # of a concatenated skip connection); everything else gets dense rows
-    strided_ok = dataflow in (DATAFLOW_FDS, DATAFLOW_OS, DATAFLOW_OSO)
+    strided_ok = dataflow in (DATAFLOW_FDS, DATAFLOW_OS, DATAFLOW_OSO, DATAFLOW_OSB)
     ld_in = _row_stride(feats) if strided_ok else -1
     if ld_in < 0:
         feats, ld_in = feats.contiguous(), 0
@@ -1061,6 +1064,13 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
             slice_out, ld_out = out, 0
             out = _new((n_out, c_out), feats.dtype, dev)
     epi, _keep = _epilogue(feats, n_out, c_out, bias, residual, act, ld_in, ld_out)
+    blocks = False
+    if dataflow == DATAFLOW_OS or dataflow == DATAFLOW_OSB:
+        # (not the transposed layer over a submanifold map of even kernel sizes: its table is made below)
+        blocks = not (transposed and km.subm) and osb_takes(kv, c_in, c_out, feats.dtype) and n_in * (ld_in or c_in) * 2 < _OSB_MAX_BYTES \
+            and (feats.data_ptr() | out.data_ptr() | ((epi.bias or 0) | (epi.residual or 0) if epi is not None else 0)) % 16 == 0
+        if dataflow == DATAFLOW_OSB:
+            dataflow = DATAFLOW_OS if blocks else pick_dataflow(km, c_in, c_out, feats.dtype, transposed, blocks=False)
     if dataflow == DATAFLOW_FOD:
         imap, omap = (km.omap, km.imap) if transposed else (km.imap, km.omap)
         ws_bytes = lib.pce_conv_fod_workspace_bytes(n_out, c_out, dt)
@@ -1121,8 +1131,7 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
                 t[_mid(km.ks)] = torch.arange(km.n_in, dtype=torch.int32, device=t.device)
                 km._nbr_in_t = t.view(-1)
             nbr = km._nbr_in_t
-        elif osb_takes(kv, c_in, c_out, feats.dtype) and n_in * (ld_in or c_in) * 2 < _OSB_MAX_BYTES and \
-                (feats.data_ptr() | out.data_ptr() | ((epi.bias or 0) | (epi.residual or 0) if epi is not None else 0)) % 16 == 0:
+        elif blocks:
             if packed is None:
                 packed = pack_weights(weight)
             order = block_order(km, transposed)
@@ -1131,7 +1140,7 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
             _lib.check(lib.pce_conv_fwd_osb(feats.data_ptr(), packed.data_ptr(), out.data_ptr(), dt, n_in, n_out, km.M, c_in, c_out, kv,
                                             nbr.data_ptr(), order.data_ptr(), _ptr(ws), need, epi, s))
             return out
-        need = lib.pce_conv_os_workspace_bytes(dt, n_out, c_in, c_out, kv) if split_offsets else 0
+        need = lib.pce_conv_os_workspace_bytes(dt, n_out, c_in, c_out, kv) if split_offsets and dt == PCE_F32 else 0
         if need > 0:
             ws = _scratch(buffer, need, dev)
             _lib.check(lib.pce_conv_fwd_os_parts(feats.data_ptr(), weight.data_ptr(), out.data_ptr(), dt, n_in, n_out, c_in, c_out, kv,
@@ -1314,7 +1323,7 @@ def conv_backward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, grad
     if need_feats:
         w3 = weight if weight.dim() == 3 else weight.unsqueeze(0)
         c_out, c_in = w3.shape[1:]
-        df = dataflow if dataflow is not None else select_dataflow(km, c_in, c_out, w3.dtype, not transposed)
+        df = dataflow if dataflow is not None else pick_dataflow(km, c_in, c_out, w3.dtype, not transposed)
         # over a map that is its own mirror image the swapped layer is the plain one with the offsets reversed (see
         # conv_forward): they are reversed in the launch that transposes them
         mirror = not transposed and km.subm and all(k % 2 == 1 for k in km.ks)

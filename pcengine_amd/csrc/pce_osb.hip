@@ -699,6 +699,14 @@ extern "C" int pce_conv_osb_leads(int64_t n_out, int64_t n_pairs, int32_t c_in, 
   return 1;
 }
 
+extern "C" int pce_select_layer(int64_t n_in, int64_t n_out, int64_t n_pairs, int32_t c_in, int32_t c_out, int32_t kv, int32_t mid,
+                                int32_t transposed, int32_t dtype) {
+  if (mid >= 0 && (!transposed || kv % 2 == 1) && n_in * c_in * 2 < (int64_t)OSB_MISSING &&
+      pce_conv_osb_leads(n_out, n_pairs, c_in, c_out, kv, mid, dtype))
+    return PCE_DATAFLOW_OSB;
+  return pce_select_dataflow(n_in, n_out, n_pairs, c_in, c_out, kv, mid, transposed, dtype);
+}
+
 extern "C" int64_t pce_conv_osb_workspace_bytes(int64_t n_out, int32_t c_out) {
   int cb, slabs;
   osb_shape(n_out, c_out, &cb, &slabs);
