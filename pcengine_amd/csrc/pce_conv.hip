@@ -1121,18 +1121,35 @@ static unsigned xcd_grid(TileArgs *a, long long tiles, int slabs) {
 // rows by 128 columns at 14 us per 256 input channels whatever the number of rows, so where the tiles leave the chip
 // without two workgroups per compute unit the slabs get narrower, with the same sums: the centre GEMMs of a U-Net's deep
 // levels on a small scan (8 to 16 workgroups before) 23-30 us -> 11, 128 -> 128 on 30 k LiDAR rows 41.6 us -> 33.0, 256 -> 256
-// on 4 k dense rows 86 -> 75, and nothing slower from 16 to 512 channels.  The fp16 instruction is 16 times faster and the gathers decide there.
-static int tile_blocks(int elem, long long tiles, int c_out) {
+// on 4 k dense rows 86 -> 75.  The fp16 instruction is 16 times faster and the gathers decide there.
+static int narrow_blocks(long long tiles, int c_out) {
   const int nb = (c_out + 31) / 32;
-  if (elem == 2 || nb == 1) return nb < 4 ? nb : 4;
   if (nb >= 4 && tiles * ((nb + 3) / 4) >= OS_WORKGROUPS) return 4;
   if (nb < 4 && tiles >= OS_WORKGROUPS) return nb;
   return nb >= 4 && tiles * ((nb + 1) / 2) >= OS_WORKGROUPS ? 2 : 1;
 }
 
+// Not where the widest slabs fill whole rounds of the compute units and narrower ones only add gathers: a slab counted as
+// its blocks and a fifth of one for its rows, in rounds of a workgroup per compute unit.  Plain products of 96 input
+// channels and more, an eighth apart: 250 wide slabs 128 -> 128 on 32 k rows 17.6 us (narrow 19.2), 256 -> 256 on 16 k 29.6
+// (31.9), 512 -> 512 on 8 k 52.4 (56.1), 96 -> 96 on 32 k 12.5 (13.0), but 500 of 128 -> 128 on 64 k 30.0 (28.7) and 250 of 48 -> 96
+// 9.3 (8.5); output-stationary layers of several slabs: 471 of 384 -> 384 on 20 k rows 1446 (1626), but 247 of 128 -> 128 on 31 k,
+// one slab each, 288 (271).  Up to 96 columns at nearly two rounds: 64 -> 64 on 60 k rows 11.6 (11.9), but 16 -> 96 9.7 (8.3); 16 -> 48 on 2 k to 65 k
+// rows 7.2-7.8 (7.4-8.2).
+static int tile_blocks(int elem, long long tiles, const TileArgs &a) {
+  const int nb = (a.c_out + 31) / 32, widest = nb < 4 ? nb : 4;
+  if (elem == 2) return widest;
+  const int narrow = narrow_blocks(tiles, a.c_out);
+  if (narrow == widest || a.parts > 1 || (a.mode == MODE_OS && nb <= 4)) return narrow;
+  if (a.mode != MODE_OS && nb < 4 && (a.c_in >= 32 ? 8 * tiles >= 7 * OS_WORKGROUPS : nb == 2)) return widest;
+  if (a.c_in < 96) return narrow;
+  auto cost = [&](int blocks) { return pce_div_up(tiles * ((nb + blocks - 1) / blocks), OS_WORKGROUPS / 2) * (5 * blocks + 1); };
+  return a.mode == MODE_OS ? (cost(widest) < cost(narrow) ? widest : narrow) : (9 * cost(widest) <= 8 * cost(narrow) ? widest : narrow);
+}
+
 template <typename T, bool FAST, int TMODE, int TEPI>
 static void launch_tile_nb(TileArgs a, long long tiles, hipStream_t s) {
-  const int nb = tile_blocks(sizeof(T), tiles, a.c_out);
+  const int nb = tile_blocks(sizeof(T), tiles, a);
   const dim3 grid(xcd_grid(&a, tiles, (a.n_pad / 32 + nb - 1) / nb), a.parts > 1 ? a.parts : 1);
   if (nb == 4)
     hipLaunchKernelGGL((tile_gemm_kernel<T, 4, FAST, TMODE, TEPI>), grid, dim3(256), 0, s, a);
@@ -2019,7 +2036,7 @@ static int os_impl(const void *in, const void *w, const void *wp, void *out, int
 static int os_parts(int dtype, long long n_out, int c_in, int c_out, int kv) {
   if (dtype != PCE_F32 || n_out <= 0 || (long long)kv * c_in < 768) return 1;
   const long long tiles = pce_div_up(n_out, 128);
-  const int nb = tile_blocks(4, tiles, c_out);
+  const int nb = narrow_blocks(tiles, c_out);
   const long long parts = OS_WORKGROUPS / (tiles * (((c_out + 31) / 32 + nb - 1) / nb));
   return parts < 2 ? 1 : parts < kv ? (int)parts : kv;
 }
