@@ -53,3 +53,32 @@ def test_layer_the_block_kernel_cannot_read():
         got, km = through(feats)
         assert "_blocks" not in km.__dict__ and km.has_csr
         assert ((got.float() - want.float()).norm() / want.float().norm()).item() < 2e-3
+
+
+def test_selector_on_measured_wide_layers():
+    """fp16 layers timed with every dataflow; us in brackets: block kernel, the one it stands against."""
+    lib = _lib.load()
+    FDS, OSO, OSB = _lib.DATAFLOW_FDS, _lib.DATAFLOW_OSO, _lib.DATAFLOW_OSB
+    for n, rho, c_in, c_out, want in [
+            (12036, 7.5, 384, 384, FDS),       # random clouds: 112, 76
+            (11437, 9.4, 512, 512, FDS),       # 155, 123
+            (18729, 9.8, 384, 256, FDS),       # 114, 94
+            (20202, 7.2, 256, 128, FDS),       # 51, 43
+            (32025, 5.4, 192, 128, FDS),       # 58, 45
+            (113177, 2.9, 256, 128, FDS),      # 111, 82
+            (199899, 3.7, 384, 384, FDS),      # 1.13 of it
+            (82198, 4.2, 96, 96, OSO),         # 1.22 of it
+            (66200, 8.9, 96, 96, OSO),         # a level of a scan: 58, 55
+            (12063, 11.6, 512, 512, FDS),      # a level of indoor scenes: 3 to 5 % behind
+            (821, 6.5, 192, 192, OSB),         # 0.81 of it
+            (12036, 7.5, 128, 192, OSB),       # equal
+            (28103, 10.1, 256, 256, OSB),      # 0.87 of it
+            (60159, 7.7, 192, 192, OSB),       # 0.68
+            (66200, 8.9, 256, 256, OSB),       # a level of a scan: 0.67
+            (679728, 5.2, 192, 192, OSB),      # indoor scenes: 0.42
+            (276205, 8.7, 384, 256, OSB),      # 0.42
+            (69431, 9.9, 512, 512, OSB),       # 0.52
+            (806, 13.1, 256, 256, OSB),        # 0.83
+            (261532, 7.8, 64, 96, OSB),        # 0.84 of the ordered rows
+            (106646, 5.5, 64, 128, OSB)]:      # 0.82
+        assert lib.pce_select_layer(n, n, round(n * rho), c_in, c_out, 27, 13, 0, _lib.PCE_F16) == want, (n, rho, c_in, c_out)
