@@ -407,6 +407,79 @@ struct OsbOut {
   }
 };
 
+// Zeros stand for a row's missing neighbour in the matrix products, and zero times a weight that is not finite is NaN.  Where a
+// sum of the wavefront is NaN and one of its weights is not finite, the NaN sums of rows that miss such an offset are formed
+// again, neighbour by neighbour.  `all`: the offsets the sums run over.  Costs a comparison per sum otherwise.
+template <int CB>
+__device__ __forceinline__ void osb_redo_nan(f32x4 (&acc)[OSB_RB][CB], const TileArgs &a, unsigned all, const int *rows, int nw, int lane) {
+  bool nan = false;
+#pragma unroll
+  for (int rb = 0; rb < OSB_RB; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) nan |= acc[rb][cb][i] != acc[rb][cb][i];
+  if (!__any(nan)) return;
+  const int l16 = lane & 15, q = lane >> 4, n = (int)a.n_rows;
+  const half8 *wp = (const half8 *)a.Wp;
+  unsigned bad = 0;   // the offsets with a weight that is not finite in this wavefront's columns
+  for (unsigned rest = all; rest; rest &= rest - 1) {
+    const int kp = __ffs(rest) - 1;
+    bool here = false;
+    for (int k8 = q; k8 < a.k8_total; k8 += 4)
+      for (int cb = 0; cb < CB; ++cb) {
+        const int c = nw + cb * 16 + l16;
+        const half8 w = wp[((long long)kp * a.k8_total + k8) * a.n_pad + (c < a.n_pad ? c : a.n_pad - 1)];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) here |= !(fabsf((float)w[j]) <= 65504.f);
+      }
+    if (__any(here)) bad |= 1u << kp;
+  }
+  if (!bad) return;
+#pragma clang loop unroll(disable)
+  for (int e = 0; e < OSB_RB * CB * 4; ++e) {
+    float v = 0.f;
+    int at = e;   // (opaque, here and below: otherwise the comparisons are made once and fill the scalar registers)
+    asm volatile("" : "+v"(at));
+#pragma unroll
+    for (int rb = 0; rb < OSB_RB; ++rb)
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v = (rb * CB + cb) * 4 + i == at ? acc[rb][cb][i] : v;
+    const int row = rows[e / (4 * CB) * 16 + l16], c = nw + e / 4 % CB * 16 + q * 4 + e % 4;
+    const bool mine = v != v && row >= 0 && c < a.c_out;
+    if (!__any(mine)) continue;
+    bool misses = false, live = mine;
+    float sum = 0.f;
+    for (int pass = 0; pass < 2; ++pass) {   // those offsets first: a sum they make NaN is done
+      for (unsigned rest = pass == 0 ? bad : all & ~bad; rest && __any(live); rest &= rest - 1) {
+        const int kp = __ffs(rest) - 1;
+        const int nb = live ? a.nbr[(long long)kp * n + row] : -1;
+        if (pass == 0) misses |= nb < 0;
+        if (nb >= 0) {
+          const half8 *f = (const half8 *)((const half_t *)a.A + (long long)nb * a.lda), *w = wp + (long long)kp * a.k8_total * a.n_pad + c;
+          for (int k8 = 0; k8 < a.k8_total; ++k8) {
+            const half8 x = f[k8], y = w[(long long)k8 * a.n_pad];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) sum += (float)x[j] * (float)y[j];
+          }
+          live = !(sum != sum);
+        }
+      }
+      live = live && misses;
+    }
+    v = mine && misses ? sum : v;
+    asm volatile("" : "+v"(at));
+#pragma unroll
+    for (int rb = 0; rb < OSB_RB; ++rb)
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[rb][cb][i] = (rb * CB + cb) * 4 + i == at ? v : acc[rb][cb][i];
+  }
+}
+
 // Bound by the matrix cores and by what keeps them from running: the gathers' L2 latency and the LDS reads (a wavefront
 // reads 1 KB per 16-row block and step for CB matrix instructions of 16 clocks; four of them share the LDS port, so below
 // CB = 4 the reads alone take as long as the instructions).  A tile of 128 rows holds its sums in registers (8 * CB
@@ -615,6 +688,7 @@ __global__ void __launch_bounds__(256, 2) osb_kernel(TileArgs a, OsbArgs o) {
 #undef OSB_ISSUE_A
 #undef OSB_SRC
 #undef OSB_NEXT
+  osb_redo_nan<CB>(acc, a, all, rows, nw, lane);
   if (parts > 1) {
     // partial sums as they lie in the registers: [slot][wavefront][block][column block][lane] of 16 bytes
     f32x4 *dst = (f32x4 *)o.part + ((long long)slot * 4 + wave) * (OSB_RB * CB * 64) + lane;
