@@ -648,24 +648,27 @@ class PyramidPlan:
             raise PlanNotApplicable()
         _lib.check(rc)
         self.n_cap, self.n_batch, self.device = int(n_cap), int(n_batch), device
-        # behind the library's arrays a place for what layers build on first use and keep on a map (_build_kept)
-        end, places = self.plan.arena_bytes, []
+        # behind the library's arrays a place (first element, elements) for each array that layers build on first use and
+        # keep on a map (_build_kept)
+        end, self.places, blocks = self.plan.arena_bytes // 4, [], {}
         for i, (ks, stride, _, _, _, subm) in enumerate(self.args):
-            m, want = self.plan.map[i], {}
+            m, places = self.plan.map[i], {}
+            want = []
             if m.kv <= OSB_MAX_KV:
-                want["blocks", False] = lib.pce_osb_order_elems(m.cap_out)
-                if reqs[i].want_nbr_in:
-                    want["blocks", True] = lib.pce_osb_order_elems(m.cap_in)
+                for transposed, rows in ((False, m.cap_out), (True, m.cap_in if reqs[i].want_nbr_in else 0)):
+                    if rows not in blocks:
+                        blocks[rows] = lib.pce_osb_order_elems(rows)
+                    want.append((("blocks", transposed), blocks[rows]))
             if not subm and ks == stride:       # an input row is in one pair at most
-                want["route", False] = lib.pce_pair_route_elems(m.cap_in, m.cap_out)
-                want["route", True] = lib.pce_pair_route_elems(m.cap_in, m.cap_in)
-            places.append({})
-            for key, elems in want.items():
-                places[i][key] = (end // 4, elems)
-                end += -(-elems * 4 // 256) * 256
-        self.arena = torch.empty(end, dtype=torch.uint8, device=device)
+                want += [(("route", False), lib.pce_pair_route_elems(m.cap_in, m.cap_out)),
+                         (("route", True), lib.pce_pair_route_elems(m.cap_in, m.cap_in))]
+            for key, elems in want:
+                if elems > 0:
+                    places[key] = (end, elems)
+                    end += -(-elems // 64) * 64
+            self.places.append(places)
+        self.arena = torch.empty(4 * end, dtype=torch.uint8, device=device)
         self.arena32 = self.arena.view(torch.int32)
-        self.places = [{key: self.arena32[at:at + elems] for key, (at, elems) in p.items()} for p in places]
 
     def build(self, in_coords: torch.Tensor):
         """(coordinates of every level, the maps in request order) for one cloud.  Raises ``PlanNotApplicable`` when
@@ -709,7 +712,7 @@ class PyramidPlan:
             km._cmin, km._cmax = cmin, cmax_out
             km.kpos_host = (_lib.c_int32 * (kv + 1))(*meta[kv:2 * kv + 1])
             km.qkpos_host = (_lib.c_int32 * (kv + 1))(*meta[2 * kv + 1:3 * kv + 2])
-            km._arena, km._places = self.arena, self.places[i]
+            km._arena, km._places = self.arena, (a32, self.places[i])
             maps.append(km)
         return coords, maps
 
@@ -749,8 +752,9 @@ def _build_kept(km: KernelMap, kept: dict, what: str, transposed: bool, elems: i
         if transposed in kept:
             return _kept(kept[transposed], device)
         capturing = torch.cuda.is_current_stream_capturing()
-        place = None if capturing else km.__dict__.get("_places", {}).get((what, transposed))
-        array = place[:elems] if place is not None and place.numel() >= elems else torch.empty(elems, dtype=torch.int32, device=device)
+        arena, places = (None, {}) if capturing else km.__dict__.get("_places", (None, {}))
+        at, room = places.get((what, transposed), (0, 0))
+        array = arena[at:at + elems] if elems <= room else torch.empty(elems, dtype=torch.int32, device=device)
         build(array)
         if not capturing:
             event = torch.cuda.Event()
