@@ -759,36 +759,41 @@ extern "C" int pce_conv_osb_takes(int32_t dtype, int32_t c_in, int32_t c_out, in
 // Pairs per row from which this kernel leads on deferred scatter.  Its time hardly depends on them, as long as the patterns
 // are as mixed as those of a random cloud (a tile then meets 21 to 24 of 27 offsets; on walls and scans fewer, so it leads
 // earlier there): it follows the rows and the product of the widths, while deferred scatter's follows the pairs.  The line is
-// where the two met on random clouds of 0.6 k to 0.8 M rows, 1 to 13 pairs per row and fourteen pairs of widths: highest at
-// 12 k to 20 k rows, where deferred scatter's launches are long enough and its partial rows still in the caches, lower for
-// fewer rows (one launch against several) and for more (partial rows in memory), and the higher the more input channels are
-// gathered for each offset.  Crossings, rows: 128 -> 192 7 at 15 k, 4 at 40 k, below 1.8 from 95 k; 192 -> 192 4 at 2 k, 9 at 15 k, 5 at
-// 40 k; 256 -> 256 10 at 15 k, 6 at 60 k, below 1.8 from 150 k; 512 -> 512 10 to 13 up to 30 k, 6 to 7 beyond.  Of 2963 layers on
-// random clouds, LiDAR and indoor pyramids 1148 take this kernel: 10 of them 2 to 9 % slower than the other choice, the mean
-// 1.5 times faster.
+// where the two met on random clouds of 0.6 k to 0.8 M rows, 1 to 13 pairs per row and 26 pairs of widths: highest at 12 k to
+// 20 k rows, where deferred scatter's launches are long enough and its partial rows still in the caches, lower for fewer rows
+// (one launch against several) and for more (partial rows in memory), and the higher the more input channels are gathered
+// for each offset.  Crossings: 128 -> 192 7 at 15 k rows, 4 at 40 k, below 1.8 from 95 k; 192 -> 192 4 at 2 k, 9 at 15 k, 5
+// at 40 k; 256 -> 256 10 at 15 k, 6 at 60 k, below 1.8 from 150 k; 512 -> 512 10 to 13 up to 30 k, 6 to 7 beyond.  Of 3920
+// layers on random clouds, LiDAR and indoor pyramids 1660 take this kernel: 19 of them 2 to 16 % slower than the other
+// choice, the mean 1.53 times faster.
 static double osb_from(double n, int c_in, int c_out) {
   const double prod = (double)c_in * c_out;
-  double from = 7.5 + 4.0 * log2(c_in / 128.0);
-  from = from < 6.0 ? 6.0 : from > 13.0 ? 13.0 : from;
-  const bool narrow = c_out <= 128 && c_in >= 160;   // much to gather, short partial rows
+  const int c = (c_in + OSB_KC - 1) / OSB_KC * OSB_KC;   // channels it multiplies
+  double from = 7.5 + 4.0 * log2(c / 128.0);
+  from = from < 7.5 ? 7.5 : from > 13.0 || prod >= 262144 ? 13.0 : from;
+  const bool narrow = c_out <= 128 && c >= 160;          // much to gather, short partial rows
   if (n < 12000)
-    from *= pow(n / 12000, prod >= 131072 ? 0.05 : c_in >= 384 ? 0.2 : 0.25);
+    from *= pow(n / 12000, prod >= 131072 ? 0.05 : c >= 384 ? 0.2 : 0.25);
   else if (n > 20000)
-    from *= pow(20000 / n, narrow ? 0.35 : c_in >= 384 ? 0.55 : c_in >= 256 ? 0.6 : 0.7);
-  const double least = c_out <= 128 ? 1.85 : c_in > 256 && prod > 65536 ? 1.5 + (prod - 65536) / 36000 : 1.5;
+    from *= pow(20000 / n, narrow ? (c_in < 192 ? 0.35 : 0.4) : c >= 384 ? 0.55 : c >= 256 ? 0.6 : 0.7);
+  if (c >= 256 && c_out >= 2 * c && c_out <= 512) from *= 0.8;   // long partial rows
+  double least = c_out <= 128 ? 1.85 : (c > 256 && prod > 65536) || prod > 131072 ? 1.8 + (prod - 65536) / 38000 : 1.5;
+  if (least > 9.5) least = 9.5;
   return from > least ? from : least;
 }
 
 // Submanifold layers this kernel leads on: from osb_from() on against deferred scatter, and wherever the general selector
 // would take the dense tiles, which multiply every offset (128 -> 128 at 7 pairs per row on 20 k rows 0.76 of their time, at
-// 19 on 27 k 0.85).  On the widths the ordered rows of the K-stepped kernel take as well: to 128 columns from five pairs per
+// 19 on 27 k 0.85; not with 64 and 96 channels on 12 k to 50 k rows with 11 and more: 64 -> 192
+// at 12 on 16 k rows 1.21).  On the widths the ordered rows of the K-stepped kernel take as well: to 128 columns from five pairs per
 // row on 60 k rows and more (0.65-0.95 of their time), to fewer from five to twelve on a million pairs and more (0.78-0.98;
 // 96 -> 96 with 0.4 to 0.9 million 1.05-1.26), from 112 channels where the dense tiles are the other choice.
 extern "C" int pce_conv_osb_leads(int64_t n_out, int64_t n_pairs, int32_t c_in, int32_t c_out, int32_t kv, int32_t mid, int32_t dtype) {
   if (n_out <= 0 || mid < 0 || !pce_conv_osb_takes(dtype, c_in, c_out, kv)) return 0;
   const double n = (double)n_out, rho = (double)n_pairs / n;
   const bool dense = pce_select_dataflow(n_out, n_out, n_pairs, c_in, c_out, kv, mid, 0, dtype) == PCE_DATAFLOW_OS;
-  if (!pce_conv_oso_takes(dtype, c_in, c_out, kv, mid)) return dense || rho >= osb_from(n, c_in, c_out);
+  if (!pce_conv_oso_takes(dtype, c_in, c_out, kv, mid))
+    return dense ? c_in >= 128 || rho < 11.0 || n_out < 12000 || n_out >= 50000 : rho >= osb_from(n, c_in, c_out);
   if (c_in >= 112) return dense && (n_out >= 60000 || (n_out >= 25000 && rho >= 9.0));
   return c_out >= 128 ? n_out >= 60000 && rho >= 5.0 : rho >= 5.0 && rho <= 12.0 && n_pairs >= 1000000;
 }

@@ -1,4 +1,4 @@
-"""Weights that are not finite reach the rows that have such an offset's neighbour and no others (block kernel)."""
+"""Weights and features that are not finite reach the rows that have such an offset or neighbour and no others (block kernel)."""
 import pytest
 import torch
 
@@ -58,3 +58,15 @@ def test_layer_of_many_pairs():
     got = backend.conv_forward(f, w, km, DATAFLOW_OS)
     has = km.nbr_out.view(27, -1)[2] >= 0
     assert torch.equal(got.isinf().all(dim=1), has) and bool(got[~has].isfinite().all())
+
+
+@pytest.mark.parametrize("c_in,c_out", [(64, 96), (96, 192), (128, 256)])
+def test_features(c_in, c_out):
+    km = gpu_map(synth.random_cloud(seed=3, n=1500, extent=14), (3, 3, 3), batchsize=1)
+    f = torch.as_tensor(synth.features(1, km.n_in, c_in), device=DEV).half()
+    f[5, 3], f[6, c_in - 1], f[900] = float("inf"), float("-inf"), float("nan")
+    w = torch.as_tensor(synth.weights(2, 27, c_in, c_out), device=DEV).half()
+    w[w == 0] = 0.5
+    got, want = backend.conv_forward(f, w, km, DATAFLOW_OS), reference(f, w, km, False)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert bool(want.isinf().any()) and bool(want.isfinite().any())

@@ -70,6 +70,9 @@ def test_selector_on_measured_wide_layers():
             (82198, 4.2, 96, 96, OSO),         # 1.22 of it
             (66200, 8.9, 96, 96, OSO),         # a level of a scan: 58, 55
             (12063, 11.6, 512, 512, FDS),      # a level of indoor scenes: 3 to 5 % behind
+            (155843, 3.6, 256, 1024, FDS),     # 1260, 1084
+            (302352, 7.7, 768, 512, FDS),      # 4814, 3833
+            (16369, 12.1, 64, 192, _lib.DATAFLOW_OS),   # 36, 30 for the dense tiles
             (821, 6.5, 192, 192, OSB),         # 0.81 of it
             (12036, 7.5, 128, 192, OSB),       # equal
             (28103, 10.1, 256, 256, OSB),      # 0.87 of it
@@ -78,6 +81,8 @@ def test_selector_on_measured_wide_layers():
             (679728, 5.2, 192, 192, OSB),      # indoor scenes: 0.42
             (276205, 8.7, 384, 256, OSB),      # 0.42
             (69431, 9.9, 512, 512, OSB),       # 0.52
+            (69431, 9.9, 768, 512, OSB),       # 0.60
+            (16455, 10.9, 256, 512, OSB),      # 0.73
             (806, 13.1, 256, 256, OSB),        # 0.83
             (261532, 7.8, 64, 96, OSB),        # 0.84 of the ordered rows
             (106646, 5.5, 64, 128, OSB)]:      # 0.82
