@@ -757,19 +757,19 @@ def _build_kept(km: KernelMap, kept: dict, what: str, transposed: bool, elems: i
         array = arena[at:at + elems] if elems <= room else torch.empty(elems, dtype=torch.int32, device=device)
         build(array)
         if not capturing:
-            event = torch.cuda.Event()
-            event.record(torch.cuda.current_stream(device))
-            kept[transposed] = (array, _stream(device), event)
+            kept[transposed] = (array, _stream(device))
         return array
 
 
 def _kept(entry, device) -> torch.Tensor:
-    """The array of an entry that ``_build_kept`` made; another stream than the one that built it waits for it (not under
-    capture: what a graph reads from other streams is the program's to order before a replay, as for its inputs)."""
-    array, built_on, event = entry
+    """The array of an entry that ``_build_kept`` made.  Another stream than the one that built it waits for what that one
+    has been given so far (an event recorded behind every build would cost each forward 5 us per map); not under capture:
+    what a graph reads from other streams is the program's to order before a replay, as for its inputs."""
+    array, built_on = entry
     if built_on != _stream(device) and not torch.cuda.is_current_stream_capturing():
         current = torch.cuda.current_stream(device)
-        current.wait_event(event)
+        # (an ExternalStream of handle 0 would be a new stream of torch's pool)
+        current.wait_stream(torch.cuda.ExternalStream(built_on, device=device) if built_on else torch.cuda.default_stream(device))
         array.record_stream(current)
     return array
 

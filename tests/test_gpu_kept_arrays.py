@@ -57,30 +57,27 @@ def test_a_tensor_goes_through_a_planned_network_again():
         assert any("_blocks" in km.__dict__ for km in b.kmaps.values())
 
 
+@pytest.mark.parametrize("on_default", [False, True])
 @pytest.mark.parametrize("planned", [False, True])
-def test_another_stream_waits_for_the_order(planned):
+def test_another_stream_waits_for_the_order(planned, on_default):
     coords = synth.random_cloud(seed=9, n=60000, extent=44)
     km = _planned_map(coords)[0] if planned else gpu_map(coords, (3, 3, 3), batchsize=1)
-    n = km.n_out
-    f = torch.as_tensor(synth.features(1, n, 128), device=DEV).half()
+    f = torch.as_tensor(synth.features(1, km.n_out, 128), device=DEV).half()
     w = torch.as_tensor(synth.weights(2, 27, 128, 128), device=DEV).half()
-    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    packed = backend.pack_weights(w)
+    first, second = torch.cuda.default_stream() if on_default else torch.cuda.Stream(), torch.cuda.Stream()
     torch.cuda.synchronize()
     with torch.cuda.stream(first):
+        torch.cuda._sleep(20000000)          # the order is far from ready when the layer is queued
         backend.block_order(km)
-    built_on, event = km._blocks[False][1:]
-    assert built_on == first.cuda_stream
-    waited = []
-    orig = torch.cuda.Stream.wait_event
-    try:
-        torch.cuda.Stream.wait_event = lambda self, e: (waited.append((self.cuda_stream, e)), orig(self, e))[1]
-        with torch.cuda.stream(second):
-            got = backend.conv_forward(f, w, km, DATAFLOW_OS)
-    finally:
-        torch.cuda.Stream.wait_event = orig
-    assert waited == [(second.cuda_stream, event)]
+    assert km._blocks[False][1] == first.cuda_stream
+    with torch.cuda.stream(second):
+        got = backend.conv_forward(f, w, km, DATAFLOW_OS, packed=packed)
+        queued = torch.cuda.Event()
+        queued.record()
+    assert not queued.query()                # it waits on the GPU, the host did not
     torch.cuda.synchronize()
-    assert torch.equal(got, backend.conv_forward(f, w, km, DATAFLOW_OS))
+    assert torch.equal(got, backend.conv_forward(f, w, km, DATAFLOW_OS, packed=packed))
 
 
 @pytest.mark.parametrize("warm", [False, True])
