@@ -750,7 +750,7 @@ def _build_kept(km: KernelMap, kept: dict, what: str, transposed: bool, elems: i
     nothing is kept: the kernels of a capture have not run yet, so an array built there belongs to the graph alone."""
     with _first_use:
         if transposed in kept:
-            return _kept(kept[transposed], device)
+            return _kept(kept[transposed])
         capturing = torch.cuda.is_current_stream_capturing()
         arena, places = (None, {}) if capturing else km.__dict__.get("_places", (None, {}))
         at, room = places.get((what, transposed), (0, 0))
@@ -761,11 +761,12 @@ def _build_kept(km: KernelMap, kept: dict, what: str, transposed: bool, elems: i
         return array
 
 
-def _kept(entry, device) -> torch.Tensor:
+def _kept(entry) -> torch.Tensor:
     """The array of an entry that ``_build_kept`` made.  Another stream than the one that built it waits for what that one
     has been given so far (an event recorded behind every build would cost each forward 5 us per map); not under capture:
     what a graph reads from other streams is the program's to order before a replay, as for its inputs."""
     array, built_on = entry
+    device = array.device
     if built_on != _stream(device) and not torch.cuda.is_current_stream_capturing():
         current = torch.cuda.current_stream(device)
         # (an ExternalStream of handle 0 would be a new stream of torch's pool)
@@ -781,7 +782,7 @@ def pair_route(km: KernelMap, transposed: bool = False) -> torch.Tensor:
     the transposed layer, whose output rows are the map's input rows."""
     kept = km.__dict__.setdefault("_routes", {})
     if transposed in kept:
-        return _kept(kept[transposed], km.out_coords.device)
+        return _kept(kept[transposed])
     ensure_csr(km)
     lib = _lib.load()
     omap, oslot, ocsr, n_out = (km.imap, km.islot, km.icsr, km.n_in) if transposed else (km.omap, km.oslot, km.ocsr, km.n_out)
@@ -819,10 +820,10 @@ def row_order(km: KernelMap) -> torch.Tensor:
 def block_order(km: KernelMap, transposed: bool = False) -> torch.Tensor:
     """Row order of the block output-stationary kernel (``pce_osb_order``), cached on the map per direction: two
     launches, no wait of the host."""
-    nbr, n = (km.nbr_in, km.n_in) if transposed else (km.nbr_out, km.n_out)
     kept = km.__dict__.setdefault("_blocks", {})
     if transposed in kept:
-        return _kept(kept[transposed], nbr.device)
+        return _kept(kept[transposed])
+    nbr, n = (km.nbr_in, km.n_in) if transposed else (km.nbr_out, km.n_out)
     lib = _lib.load()
     elems = lib.pce_osb_order_elems(n)
 
