@@ -565,7 +565,7 @@ _arena: Optional[ForwardArena] = None
 
 
 class allocate_from:
-    """Context manager: inside it the outputs, routing arrays and staging buffers of the forward operators of this
+    """Context manager: inside it the outputs and staging buffers of the forward operators of this
     module come from ``arena`` (a ``ForwardArena``) and not from ``torch.empty``.  Not for concurrent use."""
 
     def __init__(self, arena: Optional[ForwardArena]):
@@ -754,7 +754,7 @@ def _build_kept(km: KernelMap, kept: dict, what: str, transposed: bool, elems: i
         capturing = torch.cuda.is_current_stream_capturing()
         arena, places = (None, {}) if capturing else km.__dict__.get("_places", (None, {}))
         at, room = places.get((what, transposed), (0, 0))
-        array = arena[at:at + elems] if elems <= room else torch.empty(elems, dtype=torch.int32, device=device)
+        array = arena[at:at + elems] if 0 < elems <= room else torch.empty(elems, dtype=torch.int32, device=device)
         build(array)
         if not capturing:
             kept[transposed] = (array, _stream(device))
@@ -876,25 +876,28 @@ def ensure_nbr(km: KernelMap, transposed: bool) -> None:
         km.order_nonzero, km.order_single = full.order_nonzero, full.order_single
 
 
-def pick_dataflow(km: KernelMap, c_in: int, c_out: int, dtype: torch.dtype, transposed: bool = False, blocks: bool = True) -> int:
-    """The dataflow of a layer over this map.  ``DATAFLOW_OSB`` where the block kernel leads: ``conv_forward`` takes it then,
-    or, where its rows or pointers do not fit that kernel, what this answers without ``blocks``."""
+class _BlocksLead(int):
+    """``DATAFLOW_OS`` as the selector's answer where the block kernel leads: ``conv_forward`` takes that kernel then, or,
+    where the layer's rows or pointers do not fit it, what the selector says without it."""
+
+
+BLOCKS_LEAD = _BlocksLead(DATAFLOW_OS)
+
+
+def select_dataflow(km: KernelMap, c_in: int, c_out: int, dtype: torch.dtype, transposed: bool = False, blocks: bool = True) -> int:
     lib = _lib.load()
     n_in, n_out = (km.n_out, km.n_in) if transposed else (km.n_in, km.n_out)
     select = lib.pce_select_layer if blocks else lib.pce_select_dataflow
     df = select(n_in, n_out, km.M, c_in, c_out, km.kv, _mid(km.ks) if km.subm else -1, int(bool(transposed)),
                 PCE_F16 if dtype == torch.float16 else PCE_F32)
-    if not km.has_pairs and df not in (DATAFLOW_OSO, DATAFLOW_OS, DATAFLOW_OSB):
+    if df == DATAFLOW_OSB:
+        return BLOCKS_LEAD
+    if not km.has_pairs and df not in (DATAFLOW_OSO, DATAFLOW_OS):
         # a map built without pair lists (its layers were expected to read the neighbour table only): rather than
         # build them now, the layer takes the table-reading dataflow that is closest (a band of densities where the
         # ordered dataflow is within a tenth of deferred scatter)
         df = DATAFLOW_OSO if oso_takes(km, c_in, c_out, dtype, transposed) else DATAFLOW_OS
     return df
-
-
-def select_dataflow(km: KernelMap, c_in: int, c_out: int, dtype: torch.dtype, transposed: bool = False) -> int:
-    df = pick_dataflow(km, c_in, c_out, dtype, transposed)
-    return DATAFLOW_OS if df == DATAFLOW_OSB else df
 
 
 def pack_weights(weight: torch.Tensor) -> Optional[torch.Tensor]:
@@ -1029,7 +1032,7 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
     _require_cuda(feats, "feats")
     # the deferred-scatter and output-stationary kernels take column slices of wider matrices in place (the halves
     # of a concatenated skip connection); everything else gets dense rows
-    strided_ok = dataflow in (DATAFLOW_FDS, DATAFLOW_OS, DATAFLOW_OSO, DATAFLOW_OSB)
+    strided_ok = dataflow in (DATAFLOW_FDS, DATAFLOW_OS, DATAFLOW_OSO)
     ld_in = _row_stride(feats) if strided_ok else -1
     if ld_in < 0:
         feats, ld_in = feats.contiguous(), 0
@@ -1070,12 +1073,12 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
             out = _new((n_out, c_out), feats.dtype, dev)
     epi, _keep = _epilogue(feats, n_out, c_out, bias, residual, act, ld_in, ld_out)
     blocks = False
-    if dataflow == DATAFLOW_OS or dataflow == DATAFLOW_OSB:
+    if dataflow == DATAFLOW_OS:
         # (not the transposed layer over a submanifold map of even kernel sizes: its table is made below)
         blocks = not (transposed and km.subm) and osb_takes(kv, c_in, c_out, feats.dtype) and n_in * (ld_in or c_in) * 2 < _OSB_MAX_BYTES \
             and (feats.data_ptr() | out.data_ptr() | ((epi.bias or 0) | (epi.residual or 0) if epi is not None else 0)) % 16 == 0
-        if dataflow == DATAFLOW_OSB:
-            dataflow = DATAFLOW_OS if blocks else pick_dataflow(km, c_in, c_out, feats.dtype, transposed, blocks=False)
+        if dataflow is BLOCKS_LEAD and not blocks:
+            dataflow = select_dataflow(km, c_in, c_out, feats.dtype, transposed, blocks=False)
     if dataflow == DATAFLOW_FOD:
         imap, omap = (km.omap, km.imap) if transposed else (km.imap, km.omap)
         ws_bytes = lib.pce_conv_fod_workspace_bytes(n_out, c_out, dt)
@@ -1328,7 +1331,7 @@ def conv_backward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, grad
     if need_feats:
         w3 = weight if weight.dim() == 3 else weight.unsqueeze(0)
         c_out, c_in = w3.shape[1:]
-        df = dataflow if dataflow is not None else pick_dataflow(km, c_in, c_out, w3.dtype, not transposed)
+        df = dataflow if dataflow is not None else select_dataflow(km, c_in, c_out, w3.dtype, not transposed)
         # over a map that is its own mirror image the swapped layer is the plain one with the offsets reversed (see
         # conv_forward): they are reversed in the launch that transposes them
         mirror = not transposed and km.subm and all(k % 2 == 1 for k in km.ks)

@@ -487,9 +487,10 @@ __device__ __forceinline__ void osb_redo_nan(f32x4 (&acc)[OSB_RB][CB], const Til
 // once per 128 rows.  Two workgroups per compute unit; the four wavefronts of one share the rows and split the columns: the
 // weights of a wavefront are its own, go straight to registers and need no LDS.  Chunks of 64 channels outside, offsets inside:
 // the same rows' 128-byte pieces are gathered for 27 offsets in a row and stay in the L2.
-// fp16, pairs per row in brackets, against the dataflow that was taken before: 256 -> 256 on 72 k rows (7) 184 us
-// against 278 (deferred scatter); the layers of the eight indoor scenes' network 15.6 ms against 25.1; 45-55 % of the
-// matrix rate while two workgroups are resident.
+// fp16, pairs per row in brackets, against the dataflow that was taken before: 256 -> 256 on 72 k rows (9) 180 us against 278
+// (deferred scatter), matrix cores busy for 59 % of the cycles a compute unit has workgroups and 49 % of the launch (the
+// blocks multiply 2.0 times the useful products); the layers of the eight indoor scenes' network 15.7 ms
+// against 25.
 // TAIL: the last chunk of input channels has 32 of them.
 template <int CB, bool TAIL>
 __global__ void __launch_bounds__(256, 2) osb_kernel(TileArgs a, OsbArgs o) {

@@ -107,8 +107,8 @@ class SparseResUNet(nn.Module):
         """Build the kernel maps of every forward through the native planner (``spconv.MapPlanner``): one allocation,
         kept and reused from cloud to cloud, and two library calls for the whole pyramid.  The maps of a cloud then
         live until the next forward of this module; leave it off where maps must outlive that (a tensor whose
-        ``kmaps`` are reused after another cloud went through the network).  In inference the layer outputs, routing
-        arrays and the staging buffer then come from one allocation as well (``backend.ForwardArena``): from the
+        ``kmaps`` are reused after another cloud went through the network).  In inference the layer outputs
+        and the staging buffer then come from one allocation as well (``backend.ForwardArena``): from the
         second forward over clouds of one size on, a forward allocates no device memory, and the tensor it returns is
         valid until the next forward."""
         from .spconv import MapPlanner

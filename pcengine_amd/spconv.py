@@ -151,7 +151,7 @@ def _pick_dataflow(km: backend.KernelMap, requested: str, c_in: int, c_out: int,
     key = (c_in, c_out, dtype, transposed)
     df = picks.get(key)
     if df is None:
-        df = picks[key] = backend.pick_dataflow(km, c_in, c_out, dtype, transposed)
+        df = picks[key] = backend.select_dataflow(km, c_in, c_out, dtype, transposed)
     return df
 
 
@@ -252,7 +252,7 @@ def _run(input: spTensor, km: backend.KernelMap, kernel, in_channel, out_channel
     out = backend.conv_forward(feats, kernel.detach(), km, df, transposed=transposed, buffer=input.buffer, packed=packed,
                                out=out, bias=bias, residual=residual, act=act)
     if layer_log is not None:
-        layer_log.append((feats.shape[0], out.shape[0], km.M, in_channel, out_channel, DATAFLOW_OS if df == backend.DATAFLOW_OSB else df))
+        layer_log.append((feats.shape[0], out.shape[0], km.M, in_channel, out_channel, df))
     return out
 
 
