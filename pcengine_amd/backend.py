@@ -757,20 +757,23 @@ def _build_kept(km: KernelMap, kept: dict, what: str, transposed: bool, elems: i
         array = arena[at:at + elems] if 0 < elems <= room else torch.empty(elems, dtype=torch.int32, device=device)
         build(array)
         if not capturing:
-            kept[transposed] = (array, _stream(device))
+            kept[transposed] = [array, _stream(device), None]
         return array
 
 
 def _kept(entry) -> torch.Tensor:
-    """The array of an entry that ``_build_kept`` made.  Another stream than the one that built it waits for what that one
-    has been given so far (an event recorded behind every build would cost each forward 5 us per map); not under capture:
-    what a graph reads from other streams is the program's to order before a replay, as for its inputs."""
-    array, built_on = entry
+    """The array of an entry that ``_build_kept`` made.  Other streams than the one that built it wait for what that one had
+    been given when the first of them came (an event recorded behind every build would cost each forward 5 us per map);
+    not under capture: what a graph reads from other streams is the program's to order before a replay, as for its inputs."""
+    array, built_on, done = entry
     device = array.device
     if built_on != _stream(device) and not torch.cuda.is_current_stream_capturing():
+        if done is None:
+            # (an ExternalStream of handle 0 would be a new stream of torch's pool)
+            builder = torch.cuda.ExternalStream(built_on, device=device) if built_on else torch.cuda.default_stream(device)
+            done = entry[2] = builder.record_event()
         current = torch.cuda.current_stream(device)
-        # (an ExternalStream of handle 0 would be a new stream of torch's pool)
-        current.wait_stream(torch.cuda.ExternalStream(built_on, device=device) if built_on else torch.cuda.default_stream(device))
+        current.wait_event(done)
         array.record_stream(current)
     return array
 

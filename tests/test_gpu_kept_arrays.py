@@ -77,6 +77,13 @@ def test_another_stream_waits_for_the_order(planned, on_default):
         queued.record()
     assert not queued.query()                # it waits on the GPU, the host did not
     torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        torch.cuda._sleep(20000000)
+    with torch.cuda.stream(second):          # later layers do not wait for what the builder's stream does by then
+        again = backend.conv_forward(f, w, km, DATAFLOW_OS, packed=packed)
+        second.synchronize()
+    assert not first.query()
+    assert torch.equal(again, got)
     assert torch.equal(got, backend.conv_forward(f, w, km, DATAFLOW_OS, packed=packed))
 
 
