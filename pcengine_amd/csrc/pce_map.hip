@@ -1025,35 +1025,68 @@ extern "C" int pce_outcoords_chain_planned(const int32_t *in_coords, int64_t n_i
 // index[v] is the first point (smallest point index) that falls into voxel v and inverse[p] the
 // voxel of point p (numpy.unique's return_index / return_inverse).
 //
-// Two ways to the same arrays.  Boxes of up to VOX_WORDS_PER_POINT bitmap words per point: one bit per cell, a scan of
-// the words' counts, and every point's voxel is the rank of its bit (three short passes).  Emptier boxes: keys
-// code << idx_bits | point index are sorted; the sort is stable, so only the code's bits are passed over.
-// 217 k points of a 64-ring scan in 60 M cells: 30 us of kernels against 108 with the sort.
+// Two ways to the same arrays.  Usually through bitmaps: the box is cut into blocks of VOX_CELLS consecutive codes, one bit
+// each in a map of the box; the occupied blocks, at most one per point, get a bitmap of their cells each, in the order of
+// their rank, and the voxel of a point is the rank of its cell's bit in those.  A box of no more blocks than points needs no map
+// of them: its blocks are numbered as they lie.  The box is worked out on the device, so all of this is queued before the
+// host waits, once, for the box and the number of voxels: 60 us of kernels for 172 k points of a 64-ring scan in 238 M cells
+// (one bit per cell of the whole box: 45, and as much as the sort in 1.9 G cells; sorted: 150, and two waits).
+// Boxes too empty even for a bit per block: keys code << idx_bits | point index are sorted; the sort is stable, so only the
+// code's bits are passed over.
 #define VOX_LIMIT (1 << 30)
-#define VOX_WORDS_PER_POINT 16
+#define VOX_SUB 16           // words per counted block of a bitmap: a line of 64 bytes
+#define VOX_CELLS (32 * VOX_SUB)
+#define VOX_TILE 4096        // words a workgroup counts at a time: 256 blocks
+#define VOX_WORDS_PER_POINT 16   // words of the box's map per point, what the sort's arrays are too
 #define VOX_WORDS_MAX (1ll << 26)
+#define VOX_POINTS_MAX (1ll << 26)   // more points are sorted: the blocks' cells take 64 bytes a point, the sort 24
 #define VOX_BLOCKS 512       // workgroups that read the points; each leaves its bounds in a line of its own
 
 struct VoxLayout {
-  int64_t off_q, off_scan, off_bounds, off_keys_a, off_keys_b, off_hist, off_flags, off_bits, off_count, off_first, total;
+  int64_t off_q, off_scan, off_bounds, off_box, off_keys_a, off_keys_b, off_hist, off_flags, off_first, total;
+  int64_t off_bits[2], off_count[2], off_tiles[2], words[2];   // the box's map and the cells of its occupied blocks
 };
 
-static int64_t vox_words_cap(int64_t n) {
+__host__ __device__ static inline int64_t vox_words_cap(int64_t n) {
+  if (n > VOX_POINTS_MAX) return 0;
   int64_t words = VOX_WORDS_PER_POINT * n + 65536;
   return words < VOX_WORDS_MAX ? words : VOX_WORDS_MAX;
 }
 
+// the words that are cleared and counted
+__host__ __device__ static inline int64_t vox_padded(int64_t words) { return (words + VOX_TILE - 1) / VOX_TILE * VOX_TILE; }
+
+enum { VOX_SORT = 0, VOX_BLOCKS_ALL = 1, VOX_BLOCKS_MAPPED = 2 };
+
+struct VoxGrid {
+  int lo[3];
+  long long ey, ez;  // extents of y and z
+  int idx_bits;
+};
+
+// what the device works out: the box of the points and the number of voxels (the bitmap's)
+struct VoxBox {
+  int lo[3], hi[3];
+  int bad, total;
+  int way;
+  long long words[2];   // of the map of the box and of the blocks' cells
+  VoxGrid g;
+};
+
 static void vox_layout(int64_t n, VoxLayout *L) {
-  int64_t nblocks = pce_div_up(n, SORT_KEYS_PER_BLOCK), words = vox_words_cap(n);
+  int64_t nblocks = pce_div_up(n, SORT_KEYS_PER_BLOCK);
+  L->words[0] = vox_padded(vox_words_cap(n));
+  L->words[1] = L->words[0] ? vox_padded(VOX_SUB * n) : 0;
   int64_t o = 0;
   L->off_q = o;
   o += pce_align_up(n * 16, 256);
   L->off_scan = o;
   int64_t scan_n = 256 * nblocks + 1 > n + 1 ? 256 * nblocks + 1 : n + 1;
-  scan_n = scan_n > words ? scan_n : words;
   o += pce_align_up(scan_tmp_ints(scan_n) * 4, 256);
   L->off_bounds = o;  // int[VOX_BLOCKS][8]
   o += VOX_BLOCKS * 32;
+  L->off_box = o;
+  o += pce_align_up(sizeof(VoxBox), 256);
   // the sort's arrays and the bitmap's share the rest
   const int64_t rest = o;
   L->off_keys_a = o;
@@ -1066,18 +1099,22 @@ static void vox_layout(int64_t n, VoxLayout *L) {
   o += pce_align_up((n + 1) * 4, 256);
   const int64_t sort_end = o;
   o = rest;
-  L->off_bits = o;
-  o += pce_align_up(words * 4, 256);
-  L->off_count = o;
-  o += pce_align_up(words * 4, 256);
+  for (int k = 0; k < 2; ++k) {
+    L->off_bits[k] = o;
+    o += L->words[k] * 4;
+    L->off_count[k] = o;
+    o += pce_align_up(L->words[k] / VOX_SUB * 4, 256);
+    L->off_tiles[k] = o;
+    o += pce_align_up(L->words[k] / VOX_TILE * 4, 256);
+  }
   L->off_first = o;
   o += pce_align_up(n * 4, 256);
   L->total = o > sort_end ? o : sort_end;
 }
 
 // bounds[block]: min xyz, max xyz, status (a point is not finite or its voxel index exceeds +-2^30).
-// Bound by the 28 bytes a point takes; the bounds go to the host as they are: atomics on one line took 180 of the
-// kernel's 187 us on 217 k points.
+// Bound by the 28 bytes a point takes; a workgroup leaves its bounds in a line of its own: atomics on one line took 180 of
+// the kernel's 187 us on 217 k points.
 template <typename F>
 __global__ void __launch_bounds__(256) vox_quantize_kernel(const F *__restrict__ pts, long long n, double vx, double vy,
                                                            double vz, int4 *__restrict__ q, int *__restrict__ bounds) {
@@ -1116,37 +1153,187 @@ __global__ void __launch_bounds__(256) vox_quantize_kernel(const F *__restrict__
   }
 }
 
-struct VoxGrid {
-  int lo[3];
-  long long ey, ez;  // extents of y and z
-  int idx_bits;
-};
-
 __device__ __forceinline__ unsigned long long vox_code(const int4 c, const VoxGrid &g) {
   return ((unsigned long long)(c.x - g.lo[0]) * g.ey + (c.y - g.lo[1])) * g.ez + (c.z - g.lo[2]);
 }
 
-__global__ void __launch_bounds__(256) vox_mark_kernel(const int4 *__restrict__ q, long long n, VoxGrid g,
-                                                       unsigned *__restrict__ bits, int *__restrict__ first) {
+// the box of the points: cell codes, the way it takes and the words of the bitmap that depends on the box alone
+__host__ __device__ static inline int vox_box(int64_t n, const int *lo, const int *hi, VoxGrid *g, int *code_bits, int64_t *words) {
+  g->idx_bits = 1;
+  while ((1ll << g->idx_bits) < n) ++g->idx_bits;
+  double cells = 1.0;   // extents of up to 2^31 each: the product is formed in floating point to stay clear of overflow
+  for (int a = 0; a < 3; ++a) {
+    g->lo[a] = lo[a];
+    cells *= (double)((long long)hi[a] - lo[a] + 1);
+  }
+  g->ey = (long long)hi[1] - lo[1] + 1;
+  g->ez = (long long)hi[2] - lo[2] + 1;
+  *code_bits = 1;
+  while (*code_bits < 64 && cells > (double)(1ull << *code_bits)) ++*code_bits;
+  *words = 0;
+  if (!(cells < 32.0 * VOX_CELLS * (double)(vox_words_cap(n) - 1))) return VOX_SORT;
+  const bool all = cells < (double)VOX_CELLS * (double)(n - 1);
+  *words = (int64_t)(cells / (all ? 32.0 : 32.0 * VOX_CELLS)) + 1;
+  return all ? VOX_BLOCKS_ALL : VOX_BLOCKS_MAPPED;
+}
+
+// the bits in front of bit `at` of a counted bitmap
+__device__ __forceinline__ int vox_rank(const uint4 *__restrict__ bits, const int *__restrict__ count, const int *__restrict__ tiles, long long at) {
+  const long long sub = at / VOX_CELLS;
+  const int word = (int)(at >> 5) & (VOX_SUB - 1);
+  const unsigned below = (1u << (at & 31)) - 1;
+  uint4 w[VOX_SUB / 4];
+#pragma unroll
+  for (int j = 0; j < VOX_SUB / 4; ++j) w[j] = bits[sub * (VOX_SUB / 4) + j];
+  int v = tiles[sub / 256] + count[sub];
+#pragma unroll
+  for (int j = 0; j < VOX_SUB; ++j) {
+    const unsigned x = j % 4 == 0 ? w[j / 4].x : j % 4 == 1 ? w[j / 4].y : j % 4 == 2 ? w[j / 4].z : w[j / 4].w;
+    v += __popc(x & (j < word ? ~0u : j == word ? below : 0u));
+  }
+  return v;
+}
+
+// Every workgroup reduces the bounds to the box; the first one writes it down, all clear the bitmaps (the second one for as
+// many blocks as there are points).  Bound by their bytes.
+__global__ void __launch_bounds__(256) vox_clear_kernel(const int *__restrict__ bounds, int readers, long long n, VoxBox *__restrict__ out,
+                                                        uint4 *__restrict__ map, uint4 *__restrict__ cells) {
+  __shared__ int part[4][7];
+  __shared__ VoxBox box;
+  int v[7] = {VOX_LIMIT, VOX_LIMIT, VOX_LIMIT, VOX_LIMIT, VOX_LIMIT, VOX_LIMIT, 0};   // minima of c and of -c, -1 where bad
+  for (int b = threadIdx.x; b < readers; b += 256) {
+    const int4 x = ((const int4 *)bounds)[2 * b], y = ((const int4 *)bounds)[2 * b + 1];
+    const int k[7] = {x.x, x.y, x.z, -x.w, -y.x, -y.y, y.z ? -1 : 0};
+#pragma unroll
+    for (int a = 0; a < 7; ++a) v[a] = k[a] < v[a] ? k[a] : v[a];
+  }
+#pragma unroll
+  for (int a = 0; a < 7; ++a) {
+    for (int d = 32; d >= 1; d >>= 1) {
+      const int o = __shfl_xor(v[a], d, PCE_WAVE);
+      v[a] = o < v[a] ? o : v[a];
+    }
+    if (__lane_id() == 0) part[threadIdx.x >> 6][a] = v[a];
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int m[7];
+#pragma unroll
+    for (int a = 0; a < 7; ++a) {
+      m[a] = part[0][a];
+      for (int w = 1; w < 4; ++w) m[a] = part[w][a] < m[a] ? part[w][a] : m[a];
+    }
+    for (int a = 0; a < 3; ++a) {
+      box.lo[a] = m[a];
+      box.hi[a] = -m[3 + a];
+    }
+    box.bad = m[6];
+    box.total = 0;
+    int code_bits;
+    int64_t words;
+    box.way = vox_box(n, box.lo, box.hi, &box.g, &code_bits, &words);
+    box.words[0] = box.way == VOX_BLOCKS_MAPPED ? words : 0;
+    box.words[1] = box.way == VOX_BLOCKS_ALL ? words : 0;
+    if (blockIdx.x == 0) *out = box;
+  }
+  __syncthreads();
+  const long long map_quads = vox_padded(box.words[0]) / 4, quads = map_quads + vox_padded(box.words[0] ? VOX_SUB * n : box.words[1]) / 4;
+  for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < quads; i += (long long)gridDim.x * 256)
+    (i < map_quads ? map + i : cells + (i - map_quads))[0] = make_uint4(0, 0, 0, 0);
+}
+
+// the blocks of the box that hold a point (a block that others have marked already is only read)
+__global__ void __launch_bounds__(256) vox_mark_kernel(const int4 *__restrict__ q, long long n, const VoxBox *__restrict__ box,
+                                                       unsigned *__restrict__ map) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const unsigned long long code = vox_code(q[i], g);
-  atomicOr(&bits[code >> 5], 1u << (code & 31));
+  if (i >= n || box->way != VOX_BLOCKS_MAPPED) return;
+  const unsigned long long block = vox_code(q[i], box->g) / VOX_CELLS;
+  if (!((map[block >> 5] >> (block & 31)) & 1u)) atomicOr(&map[block >> 5], 1u << (block & 31));
+}
+
+// the cells that hold a point, in the bitmaps of the blocks; q[i].w = number of the point's block
+__global__ void __launch_bounds__(256) vox_cells_kernel(int4 *__restrict__ q, long long n, const VoxBox *__restrict__ box,
+                                                        const uint4 *__restrict__ map, const int *__restrict__ count,
+                                                        const int *__restrict__ tiles, unsigned *__restrict__ cells, int *__restrict__ first) {
+  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n || box->way == VOX_SORT) return;
+  const unsigned long long code = vox_code(q[i], box->g);
+  const int block = box->way == VOX_BLOCKS_ALL ? (int)(code / VOX_CELLS) : vox_rank(map, count, tiles, (long long)(code / VOX_CELLS));
+  const long long bit = (long long)block * VOX_CELLS + (long long)(code % VOX_CELLS);
+  atomicOr(&cells[bit >> 5], 1u << (bit & 31));
+  q[i].w = block;
   first[i] = 0x7FFFFFFF;   // one per voxel at most
 }
 
-// the voxel of a point is the rank of its bit; all points of a voxel write the same coordinates.
+// count[block of VOX_SUB words]: the bits of its tile in front of it; tiles[tile]: the bits of the tile.  Bound by the
+// bitmap's bytes.
+__global__ void __launch_bounds__(256) vox_count_kernel(const uint4 *__restrict__ bits, const long long *__restrict__ words,
+                                                        int *__restrict__ count, int *__restrict__ tiles) {
+  __shared__ int sub[VOX_TILE / VOX_SUB];
+  const int n_tiles = (int)(vox_padded(*words) / VOX_TILE);
+  for (int tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
+    uint4 w[VOX_TILE / 1024];
+#pragma unroll
+    for (int i = 0; i < VOX_TILE / 1024; ++i) w[i] = bits[(long long)tile * (VOX_TILE / 4) + i * 256 + threadIdx.x];
+#pragma unroll
+    for (int i = 0; i < VOX_TILE / 1024; ++i) {
+      int c = __popc(w[i].x) + __popc(w[i].y) + __popc(w[i].z) + __popc(w[i].w);
+      c += __shfl_xor(c, 1, PCE_WAVE);
+      c += __shfl_xor(c, 2, PCE_WAVE);
+      if ((threadIdx.x & 3) == 0) sub[i * 64 + threadIdx.x / 4] = c;
+    }
+    __syncthreads();
+    int total;
+    count[(long long)tile * 256 + threadIdx.x] = block_exclusive_scan(sub[threadIdx.x], &total);
+    if (threadIdx.x == 0) tiles[tile] = total;
+  }
+}
+
+// tiles[tile]: the bits in front of the tile; one workgroup, four tiles a thread and round.  MAP 0: the box's map, whose
+// bits are the blocks of the other bitmap; 1: that one, whose bits are the voxels.  A launch of its own (3 us): the last
+// workgroup of vox_count_kernel doing it made that one 30 us longer, a release of the caches per workgroup.
+template <int MAP>
+__global__ void __launch_bounds__(1024) vox_total_kernel(VoxBox *__restrict__ box, int4 *__restrict__ tiles) {
+  __shared__ int wsum[16];
+  const int n_tiles = (int)(vox_padded(box->words[MAP]) / VOX_TILE), wave = threadIdx.x >> 6;
+  int run = 0;
+  for (int t0 = 0; t0 < n_tiles; t0 += 4096) {
+    const int t = t0 + 4 * threadIdx.x;
+    int4 v = make_int4(0, 0, 0, 0);
+    if (t < n_tiles) v = tiles[t / 4];
+    v.y = t + 1 < n_tiles ? v.y : 0;
+    v.z = t + 2 < n_tiles ? v.z : 0;
+    v.w = t + 3 < n_tiles ? v.w : 0;
+    const int sum = v.x + v.y + v.z + v.w, inc = wave_inclusive_scan(sum);
+    if ((threadIdx.x & 63) == 63) wsum[wave] = inc;
+    __syncthreads();
+    int base = run + inc - sum;
+    for (int w = 0; w < 16; ++w) {
+      base += w < wave ? wsum[w] : 0;
+      run += wsum[w];
+    }
+    if (t < n_tiles) tiles[t / 4] = make_int4(base, base + v.x, base + v.x + v.y, base + v.x + v.y + v.z);
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    if (MAP == 1)
+      box->total = run;
+    else if (box->way == VOX_BLOCKS_MAPPED)
+      box->words[1] = (long long)VOX_SUB * run;
+  }
+}
+
+// the voxel of a point is the rank of its cell; all points of a voxel write the same coordinates.
 // STRIDE: ints per row of `coords` (4: batch, x, y, z; 3: x, y, z)
 template <int STRIDE, typename I>
 __global__ void __launch_bounds__(256) vox_rank_kernel(const int4 *__restrict__ q, long long n, VoxGrid g,
-                                                       const unsigned *__restrict__ bits, const int *__restrict__ count,
-                                                       int batch, int *__restrict__ coords, int *__restrict__ first,
-                                                       I *__restrict__ inverse) {
+                                                       const uint4 *__restrict__ cells, const int *__restrict__ count,
+                                                       const int *__restrict__ tiles, int batch, int *__restrict__ coords,
+                                                       int *__restrict__ first, I *__restrict__ inverse) {
   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int4 c = q[i];
-  const unsigned long long code = vox_code(c, g);
-  const int v = count[code >> 5] + __popc(bits[code >> 5] & ((1u << (code & 31)) - 1));
+  const int v = vox_rank(cells, count, tiles, (long long)c.w * VOX_CELLS + (long long)(vox_code(c, g) % VOX_CELLS));
   if (inverse) inverse[i] = (I)v;
   if (first) atomicMin(&first[v], (int)i);
   if (coords) {
@@ -1211,24 +1398,6 @@ __global__ void __launch_bounds__(256) vox_emit_kernel(const unsigned long long 
   }
 }
 
-// the box of the points: cell codes, and the bitmap words where it takes the bitmap (0: it is sorted)
-static void vox_box(int64_t n, const int *lo, const int *hi, VoxGrid *g, int *code_bits, int64_t *words) {
-  g->idx_bits = 1;
-  while ((1ll << g->idx_bits) < n) ++g->idx_bits;
-  double cells = 1.0;   // extents of up to 2^31 each: the product is formed in floating point to stay clear of overflow
-  for (int a = 0; a < 3; ++a) {
-    g->lo[a] = lo[a];
-    cells *= (double)((long long)hi[a] - lo[a] + 1);
-  }
-  g->ey = (long long)hi[1] - lo[1] + 1;
-  g->ez = (long long)hi[2] - lo[2] + 1;
-  *code_bits = 1;
-  while (*code_bits < 64 && cells > (double)(1ull << *code_bits)) ++*code_bits;
-  // the last word stays empty: after the scan it holds the number of voxels
-  *words = cells < 32.0 * (double)(vox_words_cap(n) - 1) ? (int64_t)(cells / 32.0) + 2 : 0;
-  if (*words > vox_words_cap(n)) *words = 0;
-}
-
 extern "C" int64_t pce_voxelize_workspace_bytes(int64_t n_points) {
   if (n_points <= 0) return -1;
   VoxLayout L;
@@ -1260,18 +1429,37 @@ extern "C" int pce_voxelize(const void *points, int32_t dtype, int64_t n_points,
     hipLaunchKernelGGL(vox_quantize_kernel<double>, dim3(readers), dim3(256), 0, s, (const double *)points,
                        (long long)n_points, voxel_size[0], voxel_size[1], voxel_size[2], q, bounds);
   PCE_LAUNCH_CHECK("vox_quantize");
-  int host[VOX_BLOCKS][8];
-  PCE_HIP(hipMemcpyAsync(host, bounds, (size_t)readers * sizeof(host[0]), hipMemcpyDeviceToHost, s));
-  PCE_HIP(hipStreamSynchronize(s));
-  int lo[3] = {VOX_LIMIT, VOX_LIMIT, VOX_LIMIT}, hi[3] = {-VOX_LIMIT, -VOX_LIMIT, -VOX_LIMIT}, bad = 0;
-  for (unsigned b = 0; b < readers; ++b) {
-    for (int a = 0; a < 3; ++a) {
-      lo[a] = host[b][a] < lo[a] ? host[b][a] : lo[a];
-      hi[a] = host[b][3 + a] > hi[a] ? host[b][3 + a] : hi[a];
+  VoxBox *box = (VoxBox *)(w + L.off_box);
+  uint4 *bits[2] = {(uint4 *)(w + L.off_bits[0]), (uint4 *)(w + L.off_bits[1])};
+  int *count[2] = {(int *)(w + L.off_count[0]), (int *)(w + L.off_count[1])};
+  int *tiles[2] = {(int *)(w + L.off_tiles[0]), (int *)(w + L.off_tiles[1])};
+  hipLaunchKernelGGL(vox_clear_kernel, dim3(1024), dim3(256), 0, s, (const int *)bounds, (int)readers, (long long)n_points, box, bits[0], bits[1]);
+  PCE_LAUNCH_CHECK("vox_clear");
+  if (L.words[0]) {
+    hipLaunchKernelGGL(vox_mark_kernel, dim3(blocks), dim3(256), 0, s, (const int4 *)q, (long long)n_points, (const VoxBox *)box, (unsigned *)bits[0]);
+    PCE_LAUNCH_CHECK("vox_mark");
+    for (int k = 0; k < 2; ++k) {
+      if (k == 1) {
+        hipLaunchKernelGGL(vox_cells_kernel, dim3(blocks), dim3(256), 0, s, q, (long long)n_points, (const VoxBox *)box, (const uint4 *)bits[0],
+                           (const int *)count[0], (const int *)tiles[0], (unsigned *)bits[1], (int *)(w + L.off_first));
+        PCE_LAUNCH_CHECK("vox_cells");
+      }
+      const int64_t most = L.words[k] / VOX_TILE;
+      hipLaunchKernelGGL(vox_count_kernel, dim3((unsigned)(most < 1024 ? most : 1024)), dim3(256), 0, s, (const uint4 *)bits[k],
+                         (const long long *)&box->words[k], count[k], tiles[k]);
+      PCE_LAUNCH_CHECK("vox_count");
+      if (k == 0)
+        hipLaunchKernelGGL(vox_total_kernel<0>, dim3(1), dim3(1024), 0, s, box, (int4 *)tiles[k]);
+      else
+        hipLaunchKernelGGL(vox_total_kernel<1>, dim3(1), dim3(1024), 0, s, box, (int4 *)tiles[k]);
+      PCE_LAUNCH_CHECK("vox_total");
     }
-    bad |= host[b][6];
   }
-  if (bad) PCE_FAIL(PCE_ECOORD, "pce_voxelize: a point is not finite or its voxel index exceeds +-2^30");
+  VoxBox host;
+  PCE_HIP(hipMemcpyAsync(&host, box, sizeof(host), hipMemcpyDeviceToHost, s));
+  PCE_HIP(hipStreamSynchronize(s));
+  if (host.bad) PCE_FAIL(PCE_ECOORD, "pce_voxelize: a point is not finite or its voxel index exceeds +-2^30");
+  const int *lo = host.lo, *hi = host.hi;
   for (int a = 0; a < 3; ++a) {
     coords_min_host[a] = lo[a];
     coords_max_host[a] = hi[a];
@@ -1279,20 +1467,12 @@ extern "C" int pce_voxelize(const void *points, int32_t dtype, int64_t n_points,
   VoxGrid g;
   int code_bits;
   int64_t words;
-  vox_box(n_points, lo, hi, &g, &code_bits, &words);
+  const int way = vox_box(n_points, lo, hi, &g, &code_bits, &words);
   if (code_bits + g.idx_bits > 64)
     PCE_FAIL(PCE_ECAPACITY, "pce_voxelize: %lld x %lld x %lld cells with %lld points do not fit a 64-bit sort key",
              (long long)hi[0] - lo[0] + 1, g.ey, g.ez, (long long)n_points);
-  int total = 0;
-  if (words) {
-    unsigned *bits = (unsigned *)(w + L.off_bits);
-    int *count = (int *)(w + L.off_count);
-    if ((rc = fill_u32(bits, words, 0u, s))) return rc;
-    hipLaunchKernelGGL(vox_mark_kernel, dim3(blocks), dim3(256), 0, s, (const int4 *)q, (long long)n_points, g, bits, (int *)(w + L.off_first));
-    PCE_LAUNCH_CHECK("vox_mark");
-    if ((rc = scan_exclusive2(count, words, nullptr, 0, scan_tmp, s, bits))) return rc;
-    PCE_HIP(hipMemcpyAsync(&total, count + (words - 1), sizeof(int), hipMemcpyDeviceToHost, s));
-  } else {
+  int total = host.total;
+  if (way == VOX_SORT) {
     unsigned long long *ka = (unsigned long long *)(w + L.off_keys_a), *kb = (unsigned long long *)(w + L.off_keys_b);
     int *flags = (int *)(w + L.off_flags);
     hipLaunchKernelGGL(vox_keys_kernel, dim3(blocks), dim3(256), 0, s, (const int4 *)q, (long long)n_points, g, ka);
@@ -1305,8 +1485,8 @@ extern "C" int pce_voxelize(const void *points, int32_t dtype, int64_t n_points,
     if ((rc = scan_exclusive(flags, n_points + 1, scan_tmp, s))) return rc;
     if (sorted != ka) PCE_HIP(hipMemcpyAsync(ka, sorted, (size_t)n_points * 8, hipMemcpyDeviceToDevice, s));
     PCE_HIP(hipMemcpyAsync(&total, flags + n_points, sizeof(int), hipMemcpyDeviceToHost, s));
+    PCE_HIP(hipStreamSynchronize(s));
   }
-  PCE_HIP(hipStreamSynchronize(s));
   *n_voxels_host = total;
   return PCE_OK;
 }
@@ -1322,14 +1502,14 @@ static int vox_emit(const void *ws, int64_t n_points, int64_t n_voxels, const in
   VoxGrid g;
   int code_bits;
   int64_t words;
-  vox_box(n_points, lo, hi, &g, &code_bits, &words);
+  const int way = vox_box(n_points, lo, hi, &g, &code_bits, &words);
   char *w = (char *)ws;
   const unsigned blocks = (unsigned)pce_div_up(n_points, 256);
-  if (words) {
+  if (way != VOX_SORT) {
     int *first = (int *)(w + L.off_first);
     hipLaunchKernelGGL((vox_rank_kernel<STRIDE, I>), dim3(blocks), dim3(256), 0, s, (const int4 *)(w + L.off_q), (long long)n_points, g,
-                       (const unsigned *)(w + L.off_bits), (const int *)(w + L.off_count), (int)batch_index, coords,
-                       index ? first : nullptr, inverse);
+                       (const uint4 *)(w + L.off_bits[1]), (const int *)(w + L.off_count[1]), (const int *)(w + L.off_tiles[1]),
+                       (int)batch_index, coords, index ? first : nullptr, inverse);
     PCE_LAUNCH_CHECK("vox_rank");
     if (index) {
       hipLaunchKernelGGL((vox_first_kernel<I>), dim3((unsigned)pce_div_up(n_voxels, 256)), dim3(256), 0, s, (const int *)first,

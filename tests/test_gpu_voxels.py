@@ -42,6 +42,17 @@ def test_voxelize_both_ways(n, side, dtype):
     assert np.array_equal(index.cpu().numpy(), first) and np.array_equal(inv.cpu().numpy(), inverse)
 
 
+# boxes on both sides of the largest map, 16384 (16 n + 65536 - 1) cells: 1024^3 is that for two points, 1291^3 is the first
+# cube that is not for 4097; 1 200 000 points in as many blocks are more than one round of the kernel that adds up the tiles
+@pytest.mark.parametrize("n,side", [(2, 1024), (2, 1025), (300, 130), (4097, 1290), (4097, 1291), (70001, 900), (1200000, 1800)])
+def test_voxelize_large_boxes(n, side):
+    pts = _points(n, side, np.float32, n + side)
+    want, first, inverse = orc.sparse_quantize(pts, (0.5, 0.5, 0.5))
+    coords, index, inv = utils.sparse_quantize(torch.as_tensor(pts, device=DEV), 0.5, return_index=True, return_inverse=True)
+    assert np.array_equal(coords.cpu().numpy(), want)
+    assert np.array_equal(index.cpu().numpy(), first) and np.array_equal(inv.cpu().numpy(), inverse)
+
+
 @pytest.mark.parametrize("rows", [[1], [3, 0, 5], [256, 257, 1], [70000, 1, 12345], [7] * 64, [7] * 65])
 def test_collate(rows):
     rng = np.random.default_rng(len(rows))
