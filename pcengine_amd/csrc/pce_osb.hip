@@ -350,57 +350,63 @@ __device__ __forceinline__ int osb_slot(int r, int p) { return p ^ ((r >> 1) & 7
                : "=&v"(F_[0]), "=&v"(F_[1]) : "v"(ra0), "v"(ra1), "n"((RB_) * 16 * OSB_KC * 2) : "memory")
 #define OSB_WAIT(F_, N_) asm volatile("s_waitcnt lgkmcnt(" #N_ ")" : "+v"(F_[0]), "+v"(F_[1]) : : "memory")
 
-// four rows of columns of a lane: bias, residual and activation on f32x4 pieces
+// Sums of 16-row blocks -> finished rows in memory.  They go through the wavefront's LDS region in fp32, so that bias,
+// residual and activation are applied to the eight consecutive columns a lane stores, and a residual is read as whole lines
+// the way the rows are written (as 32 bytes of 16 rows an instruction, each block waited for: 566 us, 523 so), up to
+// OSB_AHEAD blocks before it is added.
+#define OSB_AHEAD 4
 template <int CB>
 struct OsbOut {
-  f32x4 bias[CB];
+  static constexpr int LD = CB * 16 + 4;             // floats per row of the region
+  static constexpr int PPR = CB * 2;                 // 16-byte pieces of a finished row
+  static constexpr int ITS = (16 * PPR + 63) / 64;
+  half8 bias[ITS], res[OSB_AHEAD][ITS];
   ActK act;
-  __device__ __forceinline__ void init(const TileArgs &a, int nw, int q) {
-    act = act_coeffs(a.act, a.slope, a.act != PCE_ACT_NONE);
+  static __device__ __forceinline__ int row(int it, int lane) { return (it * 64 + lane) / PPR; }
+  static __device__ __forceinline__ int col(int it, int lane) { return (it * 64 + lane) % PPR * 8; }
+  // rows: the output rows of the tile's blocks (-1: none)
+  __device__ __forceinline__ void request(int rb, const int *rows, const TileArgs &a, int nw, int lane) {
+    if (!a.res) return;
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      const int c = nw + cb * 16 + q * 4;
-      VecOfC<half_t, 4>::type b = {0, 0, 0, 0};
-      if (a.bias && c < a.c_out) b = *reinterpret_cast<const VecOfC<half_t, 4>::type *>((const half_t *)a.bias + c);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) bias[cb][i] = (float)b[i];
+    for (int it = 0; it < ITS; ++it) {
+      const int r = row(it, lane), c = nw + col(it, lane), dst = rows[rb * 16 + (r & 15)];
+      const bool ok = r < 16 && dst >= 0 && c < a.c_out;
+      res[rb % OSB_AHEAD][it] = *reinterpret_cast<const half8 *>((const half_t *)a.res + (ok ? (long long)dst * a.c_out + c : 0ll));
     }
   }
-  // sums of one 16-row block -> rows in memory, through the wavefront's LDS region as whole lines
-  __device__ __forceinline__ void store(const f32x4 (&acc)[CB], int orow, const TileArgs &a, int nw, half_t *region, int lane) {
-    typedef VecOfC<half_t, 4>::type half4;
-    constexpr int LD = CB * 16 + 8, PPR = CB * 2;
+  __device__ __forceinline__ void init(int blocks, const int *rows, const TileArgs &a, int nw, int lane) {
+    act = act_coeffs(a.act, a.slope, a.act != PCE_ACT_NONE);
+#pragma unroll
+    for (int rb = 0; rb < OSB_AHEAD; ++rb)
+      if (rb < blocks) request(rb, rows, a, nw, lane);
+#pragma unroll
+    for (int it = 0; it < ITS; ++it) {
+      const int c = nw + col(it, lane);
+      half8 b = {0, 0, 0, 0, 0, 0, 0, 0};
+      if (a.bias && c < a.c_out) b = *reinterpret_cast<const half8 *>((const half_t *)a.bias + c);
+      bias[it] = b;
+    }
+  }
+  __device__ __forceinline__ void store(const f32x4 (&acc)[CB], int rb, const int *rows, const TileArgs &a, int nw, float *region, int lane) {
     const int l16 = lane & 15, q = lane >> 4;
-    half4 r[CB];
-    if (a.res) {
 #pragma unroll
-      for (int cb = 0; cb < CB; ++cb) {
-        const int c = nw + cb * 16 + q * 4;
-        const bool ok = orow >= 0 && c < a.c_out;
-        r[cb] = *reinterpret_cast<const half4 *>((const half_t *)a.res + (ok ? (long long)orow * a.c_out + c : 0ll));
-      }
-    }
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      half4 y;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float v = acc[cb][i] + bias[cb][i];
-        if (a.res) v += (float)r[cb][i];
-        y[i] = (half_t)act_apply(v, act);
-      }
-      *reinterpret_cast<half4 *>(region + l16 * LD + cb * 16 + q * 4) = y;
-    }
+    for (int cb = 0; cb < CB; ++cb) *reinterpret_cast<f32x4 *>(region + l16 * LD + cb * 16 + q * 4) = acc[cb];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int it = 0; it < (16 * PPR + 63) / 64; ++it) {
-      const int e = it * 64 + lane, row = e / PPR, p = e - row * PPR;
-      const int dst = __shfl(orow, row & 15, PCE_WAVE);
-      const int c = nw + p * 8;
-      if (row < 16 && dst >= 0 && c < a.c_out)
-        store_maybe_stream(reinterpret_cast<half8 *>((half_t *)a.out + (long long)dst * a.ldo + c),
-                           *reinterpret_cast<const half8 *>(region + row * LD + p * 8), a.stream);
+    for (int it = 0; it < ITS; ++it) {
+      const int r = row(it, lane), c = nw + col(it, lane), dst = rows[rb * 16 + (r & 15)];
+      const float *from = region + (r & 15) * LD + col(it, lane);
+      const f32x4 v[2] = {*reinterpret_cast<const f32x4 *>(from), *reinterpret_cast<const f32x4 *>(from + 4)};
+      half8 y;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float x = v[i / 4][i % 4] + (float)bias[it][i];
+        if (a.res) x += (float)res[rb % OSB_AHEAD][it][i];
+        y[i] = (half_t)act_apply(x, act);
+      }
+      if (r < 16 && dst >= 0 && c < a.c_out)
+        store_maybe_stream(reinterpret_cast<half8 *>((half_t *)a.out + (long long)dst * a.ldo + c), y, a.stream);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -541,18 +547,26 @@ __global__ void __launch_bounds__(256, 2) osb_kernel(TileArgs a, OsbArgs o) {
     const long long p = (long long)tile * OSB_ROWS + r;
     const int row = p < n ? o.perm[p] : -1;
     if (half == 0) rows[r] = row;
-    // every table read of the thread is requested before the first one is used
-    int nb[(OSB_MAX_KV + 1) / 2];
+    // The offsets some row of the tile has go to the two halves of the workgroup in turn; every table read of the thread is
+    // requested before the first one is used.  The other offsets' entries are not read (of 27 offsets a tile of the 951 k-row
+    // level of the indoor scenes has 7: 614 us with all of them, 566 without).
+    int nb[(OSB_MAX_KV + 1) / 2], kp[(OSB_MAX_KV + 1) / 2];
+    unsigned left = all;
 #pragma unroll
     for (int i = 0; i < (OSB_MAX_KV + 1) / 2; ++i) {
-      const int kp = 2 * i + half;
-      nb[i] = a.nbr[(long long)(kp < a.kv ? kp : 0) * n + (row >= 0 ? row : 0)];
+      const unsigned b0 = left & (0u - left);
+      left ^= b0;
+      const unsigned b1 = left & (0u - left);
+      left ^= b1;
+      const unsigned mine = half ? b1 : b0;
+      kp[i] = mine ? __ffs(mine) - 1 : -1;
+      if (b0) nb[i] = a.nbr[(long long)(mine ? kp[i] : 0) * n + (row >= 0 ? row : 0)];
     }
+    const int at = (r & ~31) + (r & 7) * 4 + ((r >> 3) & 3);
 #pragma unroll
-    for (int i = 0; i < (OSB_MAX_KV + 1) / 2; ++i) {
-      const int kp = 2 * i + half;
-      src[kp][(r & ~31) + (r & 7) * 4 + ((r >> 3) & 3)] = row >= 0 && kp < a.kv && nb[i] >= 0 ? (unsigned)nb[i] * (unsigned)(a.lda * 2) : OSB_MISSING;
-    }
+    for (int i = 0; i < (OSB_MAX_KV + 1) / 2; ++i)
+      if (kp[i] >= 0) src[kp[i]][at] = row >= 0 && nb[i] >= 0 ? (unsigned)nb[i] * (unsigned)(a.lda * 2) : OSB_MISSING;
+    if (half) src[OSB_MAX_KV][at] = OSB_MISSING;   // what the steps behind the last one read
   }
   const int kch = (a.c_in + OSB_KC - 1) / OSB_KC;
   const int steps = __popc(all) * kch;
@@ -703,11 +717,12 @@ __global__ void __launch_bounds__(256, 2) osb_kernel(TileArgs a, OsbArgs o) {
   }
   __syncthreads();  // the ring becomes the epilogue staging area
   OsbOut<CB> out;
-  out.init(a, nw, q);
-  half_t *region = (half_t *)lds + wave * (16 * (CB * 16 + 8));
+  out.init(OSB_RB, rows, a, nw, lane);
+  float *region = (float *)lds + wave * (16 * OsbOut<CB>::LD);
 #pragma unroll
   for (int rb = 0; rb < OSB_RB; ++rb) {
-    out.store(acc[rb], rows[rb * 16 + l16], a, nw, region, lane);
+    out.store(acc[rb], rb, rows, a, nw, region, lane);
+    if (rb + OSB_AHEAD < OSB_RB) out.request(rb + OSB_AHEAD, rows, a, nw, lane);
   }
 }
 
@@ -715,15 +730,20 @@ __global__ void __launch_bounds__(256, 2) osb_kernel(TileArgs a, OsbArgs o) {
 // per column group.
 template <int CB>
 __global__ void __launch_bounds__(256) osb_reduce_kernel(TileArgs a, OsbArgs o) {
-  __shared__ __attribute__((aligned(16))) half_t lds[4][16 * (CB * 16 + 8)];
+  __shared__ __attribute__((aligned(16))) float lds[4][16 * OsbOut<CB>::LD];
+  __shared__ int rows[16];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int x = blockIdx.x % PCE_XCDS, c = blockIdx.x / PCE_XCDS / OSB_RB, rb = blockIdx.x / PCE_XCDS % OSB_RB;
   const int *cut = o.plan + (x * OSB_MAX_CUT + c) * 2;
   const int item = cut[0], parts = cut[1];
   if (item < 0) return;
   const int nw = (item % a.slabs) * (4 * CB * 16) + wave * CB * 16;
-  const long long p = (long long)(item / a.slabs) * OSB_ROWS + rb * 16 + (lane & 15);
-  if (p - (lane & 15) >= a.n_rows || nw >= a.c_out) return;
+  const long long p0 = (long long)(item / a.slabs) * OSB_ROWS + rb * 16;
+  if (threadIdx.x < 16) rows[threadIdx.x] = p0 + threadIdx.x < a.n_rows ? o.perm[p0 + threadIdx.x] : -1;
+  __syncthreads();
+  if (p0 >= a.n_rows || nw >= a.c_out) return;
+  OsbOut<CB> out;
+  out.init(1, rows, a, nw, lane);
   f32x4 acc[CB];
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb) acc[cb] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -739,9 +759,7 @@ __global__ void __launch_bounds__(256) osb_reduce_kernel(TileArgs a, OsbArgs o) 
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb) acc[cb] += v[k][cb];
     }
-  OsbOut<CB> out;
-  out.init(a, nw, lane >> 4);
-  out.store(acc, p < a.n_rows ? o.perm[p] : -1, a, nw, lds[wave], lane);
+  out.store(acc, 0, rows, a, nw, lds[wave], lane);
 }
 
 // column blocks of 16 per wavefront (four wavefronts beside one another) and column slabs of a layer
