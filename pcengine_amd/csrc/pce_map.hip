@@ -1707,7 +1707,7 @@ struct Job {
   int kind;
   int pad;
 };
-enum { JOB_CSR_SUBM = 0, JOB_CSR_IN = 1, JOB_CSR_COUNT_OUT = 2, JOB_CSR_OUT = 3, JOB_ORDER_SCATTER = 4 };
+enum { JOB_CSR_SUBM = 0, JOB_CSR_IN = 1, JOB_CSR_COUNT_OUT = 2, JOB_CSR_OUT = 3, JOB_ORDER_SCATTER = 4, JOB_FILL_VIEWS = 5 };
 
 struct FillRegion {
   unsigned *p;
@@ -2432,36 +2432,40 @@ __global__ void __launch_bounds__(1024) kmap_offsets_kernel(const ProbDev *__res
 // Emits the pair lists in (offset, input row) order from ballot ranks, the rank of every pair inside
 // its offset (irank, and orank scattered by output row for strided layers), and the output-major
 // neighbour table: scattered for strided layers, read off the mirrored row for submanifold ones.
-__global__ void __launch_bounds__(256) kmap_fill_kernel(const ProbDev *__restrict__ P, JobList jl) {
-  const Job &job = find_job(jl, blockIdx.x);
-  const ProbDev &q = P[job.prob];
-  if (job.kind == JOB_ORDER_SCATTER) {   // the row order of a symmetric map: masks and bases are complete by now
-    // (a symmetric map: the fill jobs of this launch may be writing nbr_out, so the probe table is read, mirrored,
-    // unless the probe wrote the output-major table itself)
-    if (q.fused)
-      order_scatter_block(q.n_out, q.order, blockIdx.x - job.blk0, q.nbr_out, -1);
-    else
-      order_scatter_block(q.n_out, q.order, blockIdx.x - job.blk0, q.dense, q.g.kv - 1);
-    return;
-  }
+// VIEWS: a symmetric map with a row order, whose masks say at which offsets a row has neighbours: both CSR-coded views are
+// written here.  Their row pointers are the same; the input view's entries of a row follow one another as the row's pairs do,
+// and the output view's entry of the pair (i, o, kp) lies behind those of o at lower offsets, which the mask of o counts.  (A
+// table of the ranks and a launch that reads it back, as for maps without an order, take 55 + 50 us for the five levels of a
+// 100 k-voxel scan and 650 + 290 for 2 M rows of indoor scenes, TODO here.)
+// FULL3: of the fused probe, which leaves 27 offsets and nothing else to write.
+template <bool VIEWS, bool FULL3>
+__device__ __forceinline__ void fill_rows(const ProbDev &q, int block) {
   const long long n_in = q.n_in, n_out = q.n_out, nseg = q.nseg;
-  const int kv = q.g.kv, subm = q.g.subm, sym = q.g.sym, mid = q.g.mid, fused = q.fused;
+  const int kv = FULL3 ? 27 : q.g.kv, subm = FULL3 ? 1 : q.g.subm, sym = FULL3 ? 1 : q.g.sym, mid = FULL3 ? 13 : q.g.mid;
+  const int fused = FULL3 ? 1 : q.fused;
   // (pointers read from the descriptor are cast to the global address space, or the loads are compiled as flat
   // ones; every load of a batch goes out from a valid address and is masked afterwards, or each is compiled to a
   // branch with a wait behind it)
   const PCE_GLOBAL int *table = (const PCE_GLOBAL int *)(fused ? q.nbr_out : q.dense);
   const PCE_GLOBAL int *segoff = (const PCE_GLOBAL int *)q.seg;
-  int *__restrict__ imap = q.imap;
-  int *__restrict__ omap = q.omap;
-  int *__restrict__ irank = q.irank;
-  int *__restrict__ orank = q.orank;
-  int *__restrict__ nbr_out = q.nbr_out;
-  long long i = (long long)(blockIdx.x - job.blk0) * blockDim.x + threadIdx.x;
+  const PCE_GLOBAL int *csr = (const PCE_GLOBAL int *)q.icsr, *masks = (const PCE_GLOBAL int *)(q.order + n_out);
+  PCE_GLOBAL int *imap = (PCE_GLOBAL int *)q.imap, *omap = (PCE_GLOBAL int *)q.omap;
+  PCE_GLOBAL int *icode = (PCE_GLOBAL int *)q.icode, *ocode = (PCE_GLOBAL int *)q.ocode;
+  PCE_GLOBAL int *islot = (PCE_GLOBAL int *)q.islot, *oslot = (PCE_GLOBAL int *)q.oslot;
+  int *__restrict__ irank = FULL3 ? nullptr : q.irank;
+  int *__restrict__ orank = FULL3 ? nullptr : q.orank;
+  int *__restrict__ nbr_out = FULL3 ? nullptr : q.nbr_out;
+  long long i = (long long)block * blockDim.x + threadIdx.x;
   long long seg = i >> 6;
   bool live = i < n_in;
   const bool mirror = !fused && nbr_out && sym;
+  int pi = 0;   // the row's next entry of the input view
+  if (VIEWS) {
+    pi = csr[i <= n_in ? i : 0];
+    if (i <= n_in) q.ocsr[i] = pi;
+  }
   for (int kp0 = 0; kp0 < kv; kp0 += ROW_BATCH) {
-    int vv[ROW_BATCH], mm[ROW_BATCH], base[ROW_BATCH], first[ROW_BATCH];
+    int vv[ROW_BATCH], mm[ROW_BATCH], base[ROW_BATCH], first[ROW_BATCH], om[VIEWS ? ROW_BATCH : 1], op[VIEWS ? ROW_BATCH : 1];
 #pragma unroll
     for (int j = 0; j < ROW_BATCH; ++j) {
       const int kp = kp0 + j;
@@ -2479,6 +2483,14 @@ __global__ void __launch_bounds__(256) kmap_fill_kernel(const ProbDev *__restric
       const int f = segoff[in ? (long long)kp * nseg : 0];
       first[j] = in ? f : 0;
     }
+    if (VIEWS) {
+#pragma unroll
+      for (int j = 0; j < ROW_BATCH; ++j) {
+        const int o = vv[j] >= 0 ? vv[j] : 0;
+        om[j] = masks[o];
+        op[j] = csr[o];
+      }
+    }
 #pragma unroll
     for (int j = 0; j < ROW_BATCH; ++j) {
       int kp = kp0 + j;
@@ -2492,8 +2504,16 @@ __global__ void __launch_bounds__(256) kmap_fill_kernel(const ProbDev *__restric
         omap[p] = v;
         if (nbr_out && !sym) nbr_out[(long long)kp * n_out + v] = (int)i;   // (a fused map is symmetric)
         rank = p - first[j];
-        if (irank && rank >= PCE_CSR_CODE) q.status[2] = 1;
+        if ((VIEWS || irank) && rank >= PCE_CSR_CODE) q.status[2] = 1;
         if (orank) orank[(long long)kp * n_out + v] = rank;
+        if (VIEWS) {
+          const int po = op[j] + __popc((unsigned)om[j] & ((1u << kp) - 1)), code = kp * PCE_CSR_CODE + rank;
+          icode[pi] = code;
+          if (islot) islot[p] = pi;
+          ++pi;
+          ocode[po] = code;
+          if (oslot) oslot[p] = po;
+        }
       }
       if (irank && live) irank[(long long)kp * n_in + i] = rank;
       if (nbr_out && sym && !fused && live)  // nbr_out[kp][o] = input of the pair whose output is o = mirrored probe result
@@ -2503,10 +2523,30 @@ __global__ void __launch_bounds__(256) kmap_fill_kernel(const ProbDev *__restric
   }
 }
 
+__global__ void __launch_bounds__(256) kmap_fill_kernel(const ProbDev *__restrict__ P, JobList jl) {
+  const Job &job = find_job(jl, blockIdx.x);
+  const ProbDev &q = P[job.prob];
+  if (job.kind == JOB_ORDER_SCATTER) {   // the row order of a symmetric map: masks and bases are complete by now
+    // (a symmetric map: the fill jobs of this launch may be writing nbr_out, so the probe table is read, mirrored,
+    // unless the probe wrote the output-major table itself)
+    if (q.fused)
+      order_scatter_block(q.n_out, q.order, blockIdx.x - job.blk0, q.nbr_out, -1);
+    else
+      order_scatter_block(q.n_out, q.order, blockIdx.x - job.blk0, q.dense, q.g.kv - 1);
+    return;
+  }
+  if (job.kind == JOB_FILL_VIEWS && q.fused)
+    fill_rows<true, true>(q, blockIdx.x - job.blk0);
+  else if (job.kind == JOB_FILL_VIEWS)
+    fill_rows<true, false>(q, blockIdx.x - job.blk0);
+  else
+    fill_rows<false, false>(q, blockIdx.x - job.blk0);
+}
+
 // CSR-coded views.  Entries of every row in ascending offset order, code = kp * PCE_CSR_CODE + rank, plus,
 // for every pair (offset kp, rank rk), the slot of its entry: slot_of_pair[kpos[kp] + rk] = position.
 // Jobs of one launch (the kind is uniform over a workgroup):
-//   JOB_CSR_SUBM      symmetric submanifold map (odd kernel sizes), both views in one pass: the input-side entry of row r at offset kp
+//   JOB_CSR_SUBM      symmetric submanifold map (odd kernel sizes) without a row order, both views in one pass: the input-side entry of row r at offset kp
 //                     is the pair (r, dense[kp][r], kp); the output-side entry is the pair
 //                     (dense[kv-1-kp][r], r, kp), whose rank is read from the rank table at its input row.
 //                     Both views have the same row pointers.
@@ -2878,12 +2918,17 @@ extern "C" int pce_kmap_build_batch(const pce_kmap_problem_t *probs, int32_t n_p
     if (!lazy) {
       add_scan(0, q.seg, L.scan_len, scan_tmp);
       if (want_csr) add_scan(0, q.icsr, n_in + 1, scan_tmp + scan_tmp_ints(L.scan_len));
-      add_job(ST_FILL, p, 0, n_in);
+      if (want_csr && q.g.sym && q.order) {
+        add_job(ST_FILL, p, JOB_FILL_VIEWS, n_in + 1);
+        q.irank = nullptr;
+      } else {
+        add_job(ST_FILL, p, 0, n_in);
+      }
     }
     if (q.order && q.g.sym) add_job(ST_FILL, p, JOB_ORDER_SCATTER, n_out);
     // 5. CSR-coded views
     if (want_csr && q.g.sym) {
-      add_job(ST_CSR_A, p, JOB_CSR_SUBM, n_in + 1);
+      if (!q.order) add_job(ST_CSR_A, p, JOB_CSR_SUBM, n_in + 1);   // else the fill has written them
     } else if (want_csr) {
       add_job(ST_CSR_A, p, JOB_CSR_IN, n_in);
       add_job(ST_CSR_A, p, JOB_CSR_COUNT_OUT, n_out + 1);
