@@ -2434,9 +2434,10 @@ __global__ void __launch_bounds__(1024) kmap_offsets_kernel(const ProbDev *__res
 // neighbour table: scattered for strided layers, read off the mirrored row for submanifold ones.
 // VIEWS: a symmetric map with a row order, whose masks say at which offsets a row has neighbours: both CSR-coded views are
 // written here.  Their row pointers are the same; the input view's entries of a row follow one another as the row's pairs do,
-// and the output view's entry of the pair (i, o, kp) lies behind those of o at lower offsets, which the mask of o counts.  (A
-// table of the ranks and a launch that reads it back, as for maps without an order, take 55 + 50 us for the five levels of a
-// 100 k-voxel scan and 650 + 290 for 2 M rows of indoor scenes, TODO here.)
+// and the output view's entry of the pair (i, o, kp) lies behind those of o at lower offsets, which the mask of o counts.  (As a table
+// of the ranks and a launch that reads it back, what maps without an order take, this was 78 + 57 us for the nine maps of a
+// 100 k-voxel scan and 649 + 293 for 2 M rows of indoor scenes; 84 + 20 and 751 + 79 with the strided maps' part left.)  Bound by
+// the scattered 4-byte stores, six a pair.
 // FULL3: of the fused probe, which leaves 27 offsets and nothing else to write.
 template <bool VIEWS, bool FULL3>
 __device__ __forceinline__ void fill_rows(const ProbDev &q, int block) {
