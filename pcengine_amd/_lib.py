@@ -6,12 +6,14 @@ the package fails with that error.  There is no CPU fallback.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from ctypes import c_int32, c_int64, c_void_p, c_char_p, POINTER, Structure
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libpcengine_amd.so")
 MEASURE_LIB_PATH = os.path.join(_HERE, "lib", "libpcengine_amd_measure.so")
+HOST_PATH = os.path.join(_HERE, "lib", "_host.so")
 
 PCE_OK, PCE_EINVAL, PCE_ECAPACITY, PCE_EHIP, PCE_EWORKSPACE, PCE_ECOORD = range(6)
 PCE_F16, PCE_F32, PCE_F64 = 0, 1, 2
@@ -179,6 +181,7 @@ _MEASURE_SIGNATURES = {"pce_set_stage_mask": (None, [ctypes.c_uint32])}
 
 _lib = None
 _measure_lib = None
+_host = None
 
 
 def exported_names():
@@ -211,6 +214,33 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+def host():
+    """The extension module that runs the host side of a layer (csrc/pce_torch.cpp), loaded once."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise PCEError(f"{HOST_PATH} is missing: build it with `python -m pcengine_amd.build`")
+        spec = importlib.util.spec_from_file_location("_host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        for name in _NATIVE:
+            if globals()[name] is _first[name]:
+                globals()[name] = getattr(module, name)
+        _host = module
+    return _host
+
+
+def _loads(name):
+    return lambda *args: getattr(host(), name)(*args)
+
+
+# the host side of the calls a network makes once per layer, on the library in use; None: the general path takes the call
+_NATIVE = ("layer", "bn_forward", "bn_backward", "wgrad")
+_first = {name: _loads(name) for name in _NATIVE}
+layer, bn_forward, bn_backward, wgrad = (_first[name] for name in _NATIVE)
+
+
 class measurement_build:
     """Context manager for benchmarks and A/B tests: inside it every operator of the package runs on
     libpcengine_amd_measure.so (the same kernels, plus ``pce_set_stage_mask``); on exit the mask is reset
@@ -227,10 +257,15 @@ class measurement_build:
             _attach(m, _MEASURE_SIGNATURES)
             _measure_lib = m
         self._product, _lib = _lib, _measure_lib
+        host()
+        for name in _NATIVE:                                # (linked to the product library: the general path runs here)
+            globals()[name] = lambda *args: None
         return _measure_lib
 
     def __exit__(self, *exc) -> None:
         global _lib
+        for name in _NATIVE:
+            globals()[name] = getattr(_host, name)
         _measure_lib.pce_set_stage_mask(0xFFFFFFFF)
         _lib = self._product
 

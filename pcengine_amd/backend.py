@@ -96,6 +96,7 @@ class _Cut:
 
     def __set__(self, obj, value):
         obj.__dict__[self.slot] = value
+        obj.__dict__.pop("_calls", None)      # what was laid out from the array that was here
 
 
 @dataclass
@@ -551,6 +552,14 @@ class ForwardArena:
             return torch.empty(shape, dtype=dtype, device=device)
         return self.buf[start:start + nbytes].view(dtype).view(shape)
 
+    def piece(self, rows: int, cols: int, like: torch.Tensor) -> Optional[torch.Tensor]:
+        """``empty`` for a matrix of like's type on like's device, or None where the arena does not hold it."""
+        start = self.need
+        self.need = start + (rows * cols * _ITEMSIZE[like.dtype] + 255) // 256 * 256
+        if self.buf is None or self.need > self.buf.numel() or like.device != self.device:
+            return None
+        return _lib.host().piece(self.buf, start, rows, cols, like)
+
     def staging(self, numel: int, dtype, device) -> torch.Tensor:
         """The shared staging buffer, at least ``numel`` elements of ``dtype`` (grown when a layer needs more)."""
         nbytes = int(numel) * _ITEMSIZE[dtype]
@@ -586,6 +595,14 @@ class allocate_from:
     def __exit__(self, *exc):
         global _arena
         _arena = self.prev
+
+
+def _place(rows: int, cols: int, like: torch.Tensor) -> Optional[torch.Tensor]:
+    """A [rows, cols] output of like's type in the active arena; None where there is none or it is full (``_lib.layer`` then
+    takes memory from torch)."""
+    if _arena is None:
+        return None
+    return _arena.piece(rows, cols, like)
 
 
 def _new(shape, dtype, device) -> torch.Tensor:
@@ -946,6 +963,9 @@ def prepare_weights(weight: torch.Tensor, dtype: torch.dtype, transpose: bool = 
     return out, packed
 
 
+_ACT_CODES = {None: (_lib.ACT_NONE, 0.0), "relu": (_lib.ACT_RELU, 0.0)}
+
+
 def _act_code(act) -> Tuple[int, float]:
     """``act``: None, 'relu', or ('leaky_relu', negative_slope) -> (PCE_ACT_*, slope)."""
     if act is None:
@@ -1003,6 +1023,11 @@ def dense_forward(feats: torch.Tensor, weight: torch.Tensor, packed: Optional[to
     """act(feats @ weight + bias + residual) for the 1x1 stride-1 layer (script/spconv.py:297-304)."""
     lib = _lib.load()
     _require_cuda(feats, "feats")
+    code = _ACT_CODES.get(act) if act is None or act == "relu" else _act_code(act)
+    done = _lib.layer(_HOST_DENSE, (), feats, weight, packed, bias, residual, _place(feats.shape[0], weight.shape[-1], feats)
+                             if feats.dim() == 2 else None, code[0], code[1], None, _stream(feats.device))
+    if done is not None:
+        return done if type(done) is not int else _lib.check(done)
     feats = feats.contiguous()
     weight = weight.contiguous()
     if feats.shape[1] != weight.shape[0]:
@@ -1012,6 +1037,69 @@ def dense_forward(feats: torch.Tensor, weight: torch.Tensor, packed: Optional[to
     _lib.check(lib.pce_conv_fwd_dense(feats.data_ptr(), weight.data_ptr(), _ptr(packed), out.data_ptr(), _dtype_code(feats),
                                       feats.shape[0], feats.shape[1], weight.shape[1], epi, _stream(feats.device)))
     return out
+
+
+# kinds of layer of _lib.layer (csrc/pce_torch.cpp)
+_HOST_OSO, _HOST_OSB, _HOST_OS, _HOST_FDS, _HOST_DENSE = range(5)
+
+
+def _routes_pairs(km: KernelMap, c_in: int, c_out: int, dtype) -> bool:
+    """Whether a deferred-scatter layer over this map routes its single pairs (``pair_route``)."""
+    return (not km.subm and tuple(km.ks) == tuple(km.stride) and km.M > 0 and dtype == torch.float16 and c_in >= 64 and c_in % 32 == 0
+            and c_out >= 96 and c_out % 8 == 0)
+
+
+def _blocks_can_read(feats, *others) -> bool:
+    """Whether the pointers and rows of a call suit the block kernel: no order is built for one that it cannot take."""
+    return feats.dim() == 2 and feats.data_ptr() % 16 == 0 and feats.shape[0] * max(feats.stride(0), feats.shape[1]) * 2 < _OSB_MAX_BYTES and \
+        all(t is None or t.data_ptr() % 16 == 0 for t in others)
+
+
+def _lay_out(km: KernelMap, dataflow: int, shape, dtype, transposed: bool, split_offsets: bool):
+    """(kind, view, scratch elements, whether they are of the features' type, entry of a kept array) of a layer's native call,
+    or () where the general path has to take it.  The view holds the map's numbers and arrays in the order ``_lib.layer``
+    reads them.  Kept on the map until one of its arrays is replaced, except where an array belongs to a graph capture."""
+    kv, c_in, c_out = shape
+    if kv != km.kv or dtype not in (torch.float16, torch.float32) or transposed and km.subm:
+        return ()
+    lib = _lib.load()
+    n_in, n_out = (km.n_out, km.n_in) if transposed else (km.n_in, km.n_out)
+    mid = _mid(km.ks) if km.subm else -1
+    kept = None
+    if dataflow == DATAFLOW_OSO:
+        if not oso_takes(km, c_in, c_out, dtype, transposed):
+            return ()
+        order = row_order(km)
+        call = (_HOST_OSO, (n_in, n_out, kv, km.nbr_out, order, mid, km.order_heavy, km.order_nonzero, km.order_single), 0, False, None)
+    elif dataflow == DATAFLOW_OS and osb_takes(kv, c_in, c_out, dtype):
+        ensure_nbr(km, transposed)
+        order, kept = block_order(km, transposed), km._blocks.get(transposed)
+        need = lib.pce_conv_osb_scratch_bytes(n_out, km.M, c_in, c_out, kv)
+        call = (_HOST_OSB, (n_in, n_out, kv, km.nbr_in if transposed else km.nbr_out, order, km.M), need, False, kept)
+        if kept is None:
+            return call
+    elif dataflow == DATAFLOW_OS and dataflow is not BLOCKS_LEAD:
+        ensure_nbr(km, transposed)
+        need = lib.pce_conv_os_workspace_bytes(PCE_F32, n_out, c_in, c_out, kv) if split_offsets and dtype == torch.float32 else 0
+        call = (_HOST_OS, (n_in, n_out, kv, km.nbr_in if transposed else km.nbr_out), need, False, None)
+    elif dataflow == DATAFLOW_FDS:
+        ensure_csr(km)
+        single = transposed and tuple(km.ks) == tuple(km.stride) and km.M == n_out and km.M > 0
+        route = None
+        if not single and _routes_pairs(km, c_in, c_out, dtype):
+            route, kept = pair_route(km, transposed), km._routes.get(transposed)
+        imap, omap, ocsr, oslot = (km.omap, km.imap, km.icsr, km.islot) if transposed else (km.imap, km.omap, km.ocsr, km.oslot)
+        if km.kpos_host is None or km.qkpos_host is None:
+            return ()
+        call = (_HOST_FDS, (n_in, n_out, kv, imap, omap, oslot, km.kpos, km.qkpos, ocsr, route, mid, km.M, km.qsum,
+                            _lib.ctypes.addressof(km.kpos_host), _lib.ctypes.addressof(km.qkpos_host)),
+                0 if single else max(km.M * c_out, 1), True, kept)
+        if route is not None and kept is None:
+            return call
+    else:
+        return ()
+    km.__dict__.setdefault("_calls", {})[(int(dataflow), shape, dtype, transposed, split_offsets)] = call
+    return call
 
 
 def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataflow: int, transposed: bool = False,
@@ -1031,8 +1119,36 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
     ``split_offsets``: output-stationary fp32 layers of few rows may add up shares of the offsets.  The layers of a
     training step don't: a last bit there decides which side of a ReLU an activation is on, 0.5 % of a gradient at the
     deep levels of a small scan, and a run that is continued should go on as it began."""
+    if not feats.is_cuda:
+        _require_cuda(feats, "feats")
+    if route_single_pairs and weight.dim() == 3:
+        # the usual call: its map's arrays are laid out once, the rest is native
+        shape, dtype = weight.shape, feats.dtype
+        calls = km.__dict__.get("_calls")
+        call = None if calls is None else calls.get((dataflow, shape, dtype, transposed, split_offsets))
+        if call is None and (dataflow != DATAFLOW_OS or _blocks_can_read(feats, out, bias, residual)):
+            call = _lay_out(km, dataflow, shape, dtype, transposed, split_offsets)
+        if call:
+            kind, view, need, typed, kept = call
+            s = _stream(feats.device)
+            if kept is not None and kept[1] != s:
+                _kept(kept)
+            if not need:
+                scratch = None
+            elif not typed:
+                scratch = _scratch(buffer, need, feats.device)
+            elif buffer is not None and buffer.numel() >= need and buffer.dtype == dtype and buffer.device == feats.device:
+                scratch = buffer
+            else:
+                scratch = _staging(need, dtype, feats.device)
+            code = _ACT_CODES.get(act) if act is None or act == "relu" else _act_code(act)
+            if packed is None and dtype == torch.float16:
+                packed = pack_weights(weight)
+            done = _lib.layer(kind, view, feats, weight, packed, bias, residual, _place(view[1], shape[2], feats) if out is None else out,
+                                     code[0], code[1], scratch, s)
+            if done is not None:
+                return done if type(done) is not int else _lib.check(done)
     lib = _lib.load()
-    _require_cuda(feats, "feats")
     # the deferred-scatter and output-stationary kernels take column slices of wider matrices in place (the halves
     # of a concatenated skip connection); everything else gets dense rows
     strided_ok = dataflow in (DATAFLOW_FDS, DATAFLOW_OS, DATAFLOW_OSO)
@@ -1104,8 +1220,7 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
         # transposed layer over such a map has at most one pair per output row: exactly one unless the voxel's
         # parent was clipped away, and those rows (no pair) are the only ones left to the row sum.
         route = None
-        if (route_single_pairs and not single and not km.subm and tuple(km.ks) == tuple(km.stride)
-                and km.M > 0 and feats.dtype == torch.float16 and c_in >= 64 and c_in % 32 == 0 and c_out >= 96 and c_out % 8 == 0):
+        if route_single_pairs and not single and _routes_pairs(km, c_in, c_out, feats.dtype):
             route = pair_route(km, transposed)
         _lib.check(lib.pce_conv_fwd_fds(feats.data_ptr(), weight.data_ptr(), _ptr(packed), out.data_ptr(), dt, n_in, n_out,
                                         c_in, c_out, kv, mid, imap.data_ptr(), omap.data_ptr(), oslot.data_ptr(), km.kpos.data_ptr(),
@@ -1228,8 +1343,12 @@ def bn_forward(x: torch.Tensor, weight, bias, running_mean, running_var, use_bat
     """``act(batch_norm(x) + residual)`` over the rows of ``x`` [n, c] (fp16 / fp32) in three launches.
     ``momentum`` < 0 leaves the running statistics alone; they must be fp32 and are updated in place
     otherwise.  Returns (y, save_mean, save_rstd)."""
-    lib = _lib.load()
     _require_cuda(x, "x")
+    code, slope = _act_code(act)
+    done = _lib.bn_forward(x, residual, weight, bias, running_mean, running_var, use_batch_stats, momentum, eps, code, slope, _stream(x.device))
+    if done is not None:
+        return done if type(done) is tuple else _lib.check(done)
+    lib = _lib.load()
     x = x.contiguous()
     n, c = x.shape
     for name, t in (("running_mean", running_mean), ("running_var", running_var)):
@@ -1244,7 +1363,6 @@ def bn_forward(x: torch.Tensor, weight, bias, running_mean, running_var, use_bat
     save = torch.empty((2, c), dtype=torch.float32, device=x.device)
     ws_bytes = lib.pce_bn_workspace_bytes(n, c)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-    code, slope = _act_code(act)
     _lib.check(lib.pce_bn_forward(x.data_ptr(), _ptr(residual), y.data_ptr(), _dtype_code(x), n, c, _ptr(w), _ptr(b),
                                   _ptr(running_mean), _ptr(running_var), int(use_batch_stats), float(momentum), float(eps),
                                   save[0].data_ptr(), save[1].data_ptr(), ws.data_ptr(), ws_bytes, code, slope, _stream(x.device)))
@@ -1255,12 +1373,15 @@ def bn_backward(x: torch.Tensor, dy: torch.Tensor, weight, save_mean: torch.Tens
                 use_batch_stats: bool, y_act: Optional[torch.Tensor] = None, act=None):
     """(dx, grad_weight fp32, grad_bias fp32) of ``bn_forward``.  With ``act`` and its output ``y_act`` the
     incoming gradient is taken with respect to the activation's output and masked while it is read."""
+    code, slope = _act_code(act)
+    done = _lib.bn_backward(x, dy, y_act, weight, save_mean, save_rstd, use_batch_stats, code, slope, _stream(x.device))
+    if done is not None:
+        return done if type(done) is tuple else _lib.check(done)
     lib = _lib.load()
     x = x.contiguous()
     dy = dy.to(x.dtype).contiguous()
     n, c = x.shape
     w = _f32(weight)
-    code, slope = _act_code(act)
     if code != _lib.ACT_NONE:
         if y_act is None or y_act.shape != x.shape or y_act.dtype != x.dtype:
             raise ValueError("the gradient of an activation needs its output, shaped and typed like x")
@@ -1283,6 +1404,11 @@ def conv_wgrad(feats: torch.Tensor, grad_out: torch.Tensor, km: KernelMap, trans
     """Gradient of ``conv_forward`` with respect to the kernel: fp32 [kv, c_in, c_out]."""
     lib = _lib.load()
     _require_cuda(feats, "feats")
+    a, b = (km.omap, km.imap) if transposed else (km.imap, km.omap)
+    done = _lib.wgrad(feats, grad_out, a, b, km.kpos, km.qkpos, km.n_out if transposed else km.n_in, km.n_in if transposed else km.n_out,
+                      km.kv, _mid(km.ks) if km.subm else -1, km.qsum, _stream(feats.device))
+    if done is not None:
+        return done if type(done) is not int else _lib.check(done)
     feats, grad_out = feats.contiguous(), grad_out.contiguous()
     if feats.dtype != grad_out.dtype:
         raise TypeError(f"features are {feats.dtype} but the output gradient is {grad_out.dtype}")

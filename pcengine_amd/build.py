@@ -18,6 +18,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libpcengine_amd.so")
 MEASURE_LIB_PATH = os.path.join(LIB_DIR, "libpcengine_amd_measure.so")
+HOST_SOURCE = "pce_torch.cpp"           # the Python extension beside it: host code over torch's tensors (_lib.host)
+HOST_PATH = os.path.join(LIB_DIR, "_host.so")
 SOURCES = ["pce_map.hip", "pce_conv.hip", "pce_osb.hip", "pce_plan.hip"]
 MEASURE_SOURCES = ["pce_conv.hip"]      # the sources that read PCE_MEASURE; the others are shared as objects
 HEADERS = [os.path.join(CSRC, "pce_common.h"), os.path.join(CSRC, "pce_tile.h"), os.path.join(ROOT, "include", "pcengine_amd.h"),
@@ -35,11 +37,24 @@ def _hipcc() -> str:
     return exe
 
 
+def _torch_dir() -> str:
+    import torch
+    return os.path.dirname(torch.__file__)
+
+
+def _torch_includes():
+    import sysconfig
+    import torch
+    return [f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-isystem", os.path.join(_torch_dir(), "include"),
+            "-isystem", os.path.join(_torch_dir(), "include", "torch", "csrc", "api", "include"), "-isystem", sysconfig.get_paths()["include"]]
+
+
 def up_to_date() -> bool:
-    if not os.path.exists(LIB_PATH) or not os.path.exists(MEASURE_LIB_PATH):
+    paths = (LIB_PATH, MEASURE_LIB_PATH, HOST_PATH)
+    if not all(os.path.exists(p) for p in paths):
         return False
-    t = min(os.path.getmtime(LIB_PATH), os.path.getmtime(MEASURE_LIB_PATH))
-    deps = [os.path.join(CSRC, s) for s in SOURCES] + HEADERS
+    t = min(os.path.getmtime(p) for p in paths)
+    deps = [os.path.join(CSRC, s) for s in SOURCES + [HOST_SOURCE]] + HEADERS
     return all(os.path.getmtime(d) <= t for d in deps)
 
 
@@ -62,16 +77,23 @@ def build(force: bool = True, verbose: bool = False) -> str:
             objs.append(obj)
             if src not in MEASURE_SOURCES:
                 measure_objs.append(obj)
+    obj = os.path.join(LIB_DIR, "pce_torch.o")
+    procs.append((HOST_SOURCE, subprocess.Popen(["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", *_torch_includes(), "-I", os.path.join(ROOT, "include"),
+                                                 "-c", os.path.join(CSRC, HOST_SOURCE), "-o", obj],
+                                                stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
     for src, p in procs:
         out, _ = p.communicate()
         # the host pass does not know the device feature flag and says so; nothing else is filtered
         out = "\n".join(l for l in out.splitlines() if "packed-fp32-ops" not in l)
         if p.returncode != 0:
-            raise RuntimeError(f"hipcc failed on {src}:\n{out}")
+            raise RuntimeError(f"{src} does not compile:\n{out}")
         if verbose and out.strip():
             print(out)
     for path, members in ((LIB_PATH, objs), (MEASURE_LIB_PATH, measure_objs)):
         subprocess.run([_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", path, *members], check=True)
+    torch_lib = os.path.join(_torch_dir(), "lib")
+    subprocess.run(["g++", "-shared", "-o", HOST_PATH, obj, "-L", LIB_DIR, "-lpcengine_amd", "-L", torch_lib, "-lc10", "-ltorch_cpu",
+                    "-ltorch_python", "-Wl,-rpath,$ORIGIN"], check=True)
     return LIB_PATH
 
 

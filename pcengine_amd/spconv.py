@@ -129,11 +129,44 @@ class conv3d(nn.Module):
                              tensorcore=self.tensorcore, dataflow=self.dataflow, packed=None, act=act,
                              residual=None if residual is None else residual.feats, out=out)
         w, packed = self._weights_for(input.feats.dtype)
+        bias = self._bias_for(input.feats.dtype)
+        if residual is not None:
+            residual = residual.feats
+        done = self._cached_map_forward(input, w, packed, bias, act, residual, out)
+        if done is not None:
+            return done
         return conv_func(input=input, in_channel=self.in_channels, out_channel=self.out_channels, kernel=w,
                          kernel_size_code=self.kernel_size_code, stride_code=self.stride_code,
-                         padding_code=self.padding_code, bias=self._bias_for(input.feats.dtype),
+                         padding_code=self.padding_code, bias=bias,
                          transposed=self.transposed, tensorcore=self.tensorcore, dataflow=self.dataflow, packed=packed,
-                         act=act, residual=None if residual is None else residual.feats, out=out)
+                         act=act, residual=residual, out=out)
+
+    def _cached_map_forward(self, input: spTensor, w, packed, bias, act, residual, out) -> Optional[spTensor]:
+        """What ``conv_func`` does at inference for a layer whose map is in the cache and whose features have its width, with
+        nothing looked up twice; None for the others."""
+        feats = input.feats
+        if w.dim() != 3 or feats.dim() != 2 or feats.shape[1] != w.shape[1] or layer_log is not None:
+            return None
+        unit = self.stride_code == _UNIT
+        if unit and not self.transposed:
+            stride = input.stride
+            km = input.kmaps.get((self.kernel_size_code, stride, self.stride_code))
+        else:
+            stride = output_stride_compute(self.stride_code, input.stride, self.transposed)
+            km = input.kmaps.get((self.kernel_size_code, stride if self.transposed else input.stride, self.stride_code))
+        if km is None or isinstance(km, backend._MapJob):
+            return None
+        if self.transposed:
+            coords, cmax = input.cbook[stride], input.coords_max
+        else:
+            input.cbook.setdefault(input.stride, input.coords)
+            coords, cmax = km.out_coords, input.coords_max if unit else list(km._cmax)
+        df = _pick_dataflow(km, self.dataflow, w.shape[1], self.out_channels, feats.dtype, self.transposed)
+        y = backend.conv_forward(feats, w, km, df, transposed=self.transposed, buffer=input.buffer, packed=packed, out=out, bias=bias,
+                                 residual=residual, act=act)
+        result = spTensor(y, coords, input.buffer, input.coords_min, cmax, input.batchsize, stride, input.init_tag)
+        result.kmaps, result.cbook = input.kmaps, input.cbook
+        return result
 
 
 def _pick_dataflow(km: backend.KernelMap, requested: str, c_in: int, c_out: int, dtype, transposed: bool) -> int:

@@ -1,6 +1,7 @@
 """Front-end helpers with the reference's names and meaning (script/utils.py)."""
 from __future__ import annotations
 
+from functools import lru_cache
 from itertools import repeat
 from typing import Any, Callable, Dict, List, Tuple, Union
 
@@ -24,6 +25,7 @@ def conv_info_decoder(code: int) -> Tuple[int, int, int]:
     return (x, rest // _B, rest - rest // _B * _B)
 
 
+@lru_cache(maxsize=1024)
 def output_stride_compute(l_stride_code: int, t_stride_code: int, transposed: bool = False) -> int:
     """Tensor stride after a layer: product for a conv, quotient for a transposed conv
     (script/utils.py:116-138)."""
