@@ -11,6 +11,9 @@
 
 #include "pce_tile.h"
 
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
 template <typename T>
 struct Cfg;
 template <>
@@ -554,6 +557,143 @@ __global__ void __launch_bounds__(256, ((TMODE >= 0 && sizeof(T) == 2 && NB <= 2
   }
 }
 
+// ---- fp32 layers and plain products of few rows -------------------------------------------------------------------
+// A wavefront of tile_gemm_kernel adds up its 32 x 32 sums with v_mfma_f32_32x32x2_f32, 32 clocks per input channel one
+// after the other (27 offsets of 256 channels: 92 us), whatever the number of workgroups.  Where the rows leave the chip
+// without work, tiles of 32 x 32 are split over four wavefronts of 16 x 16 sums (v_mfma_f32_16x16x4_f32, 8 clocks per
+// channel).  Both instructions are chains of fused multiply-adds in the order of their channels; the channels are fed in the
+// order that the 32 x 32 form visits them (0 4 1 5 2 6 3 7 of every eight), offsets that none of a tile's 32 rows has are left
+// out as there, and the sums are the same bit for bit.
+// Rows and weights pass through LDS in chunks of 32 channels, requested SMALL_AHEAD chunks ahead.  In LDS the eight values of a
+// lane and chunk lie in two 16-byte pieces, [half][lane group][row or column][4]; the planes are four floats apart in banks.
+#define SMALL_KC 32
+#define SMALL_AHEAD 3
+#define SMALL_PLANE (32 * 4 + 4)
+#define SMALL_MAX_KV 32
+#define SMALL_MISSING 0xF0000000u   // bytes that rows and weights stay below
+__global__ void __launch_bounds__(256) small_f32_kernel(TileArgs a) {
+  __shared__ __attribute__((aligned(16))) float As[SMALL_AHEAD][8 * SMALL_PLANE], Bs[SMALL_AHEAD][8 * SMALL_PLANE];
+  __shared__ int idx[SMALL_MAX_KV][32];
+  __shared__ unsigned present;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4, wr = wave >> 1, wc = wave & 1;
+  long long tile;
+  int slab;
+  if (!xcd_item(a.items, a.slabs, true, &tile, &slab)) return;
+  const int n0 = slab * 32, kv = a.mode == MODE_OS ? a.kv : 1;
+  const float *A = (const float *)a.A, *W = (const float *)a.W + (a.mode == MODE_OS ? 0ll : (long long)a.w_fixed * a.c_in * a.c_out);
+  // input rows of the tile at every offset, and the offsets that some row has
+  if (threadIdx.x == 0) present = 0;
+  __syncthreads();
+  int mine[SMALL_MAX_KV / 8];
+#pragma unroll
+  for (int i = 0; i < SMALL_MAX_KV / 8; ++i) {
+    const int kp = i * 8 + threadIdx.x / 32;
+    const long long row = tile * 32 + (threadIdx.x & 31);
+    const bool ok = kp < kv && row < a.n_rows;
+    mine[i] = -1;
+    if (a.mode == MODE_OS)
+      mine[i] = a.nbr[ok ? (long long)kp * a.n_rows + row : 0];
+    else
+      mine[i] = (int)row;
+    mine[i] = ok ? mine[i] : -1;
+  }
+#pragma unroll
+  for (int i = 0; i < SMALL_MAX_KV / 8; ++i) {
+    const int kp = i * 8 + threadIdx.x / 32;
+    idx[kp][threadIdx.x & 31] = mine[i];
+    const unsigned long long has = __ballot(mine[i] >= 0);
+    if ((threadIdx.x & 31) == 0 && (unsigned)(has >> (threadIdx.x & 32))) atomicOr(&present, 1u << kp);
+  }
+  __syncthreads();
+  unsigned rest = __builtin_amdgcn_readfirstlane(present);
+  float *out = (float *)a.out;
+  if (a.parts > 1) {   // a share of the offsets, its sums to the share's own rows
+    const int p = blockIdx.y, from = kv * p / a.parts, to = kv * (p + 1) / a.parts;   // at most SMALL_MAX_KV, `from` below it
+    rest &= (to < 32 ? (1u << to) - 1 : ~0u) & ~((1u << from) - 1);
+    out += (long long)p * a.n_rows * a.c_out;
+  }
+  const int chunks = (a.c_in + SMALL_KC - 1) / SMALL_KC, steps = __popc(rest) * chunks;
+  // A thread's pieces of a chunk: four channels of a row, four columns of a channel's weights.  Through buffer loads, which
+  // read zeros beyond the range: where a row is missing and behind the last channel and column.  (With selected addresses and
+  // values a step is 110 instructions of 4 clocks for 256 clocks of products: 256 -> 256 on 603 rows 85 us, 60 so.)
+  const auto rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A), 0, SMALL_MISSING, 0x00020000);
+  const auto weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(W), 0, SMALL_MISSING, 0x00020000);
+  const int tr = threadIdx.x / 8, tq = threadIdx.x & 7;
+  const unsigned col_at = n0 + tq * 4 < a.c_out ? (unsigned)((tr * a.c_out + n0 + tq * 4) * 4) : SMALL_MISSING;
+  int w = rest ? __ffs(rest) - 1 : 0, c = 0;     // cursor of the requests
+  auto row_at = [&] {
+    const int row = rest ? idx[w][tr] : -1;
+    return row >= 0 ? (unsigned)row * (unsigned)(a.lda * 4) + tq * 16 : SMALL_MISSING;
+  };
+  unsigned arow = row_at(), col_now = rest ? col_at : SMALL_MISSING;
+  u32x4 ra[SMALL_AHEAD], rb[SMALL_AHEAD];
+  auto request = [&](u32x4 &va, u32x4 &vb) {
+    const int k0 = c * SMALL_KC;
+    const unsigned x = arow + k0 * 4, y = col_now + (unsigned)((w * a.c_in + k0) * a.c_out * 4);
+    va = __builtin_amdgcn_raw_buffer_load_b128(rows, k0 + tq * 4 < a.c_in ? x : SMALL_MISSING, 0, 0);
+    vb = __builtin_amdgcn_raw_buffer_load_b128(weights, k0 + tr < a.c_in ? y : SMALL_MISSING, 0, 0);
+    if (++c == chunks) {
+      c = 0;
+      rest &= rest - 1;
+      w = rest ? __ffs(rest) - 1 : 0;
+      arow = row_at();
+      col_now = rest ? col_at : SMALL_MISSING;
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < SMALL_AHEAD; ++i) request(ra[i], rb[i]);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  // channel 8 s + kk of a chunk: instruction 2 s + (kk & 2) / 2, lane group 2 (kk & 1) + kk / 4
+  const int at_a = ((tq / 4 * 4 + (tq & 1)) * SMALL_PLANE) + tr * 4 + (tq / 2 & 1) * 2;
+  const int kk = tr & 7, at_b = (tr / 16 * 4 + 2 * (kk & 1) + kk / 4) * SMALL_PLANE + tq * 16 + (tr / 8 & 1) * 2 + (kk & 2) / 2;
+  auto put = [&](int i) {   // the pieces requested as the i-th to LDS, and the next request in their place
+    *reinterpret_cast<u32x2 *>(As[i] + at_a) = (u32x2){ra[i][0], ra[i][2]};
+    *reinterpret_cast<u32x2 *>(As[i] + at_a + 2 * SMALL_PLANE) = (u32x2){ra[i][1], ra[i][3]};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) reinterpret_cast<unsigned *>(Bs[i])[at_b + 4 * j] = rb[i][j];
+    request(ra[i], rb[i]);
+  };
+  f32x4 x[2] = {acc, acc}, y[2] = {acc, acc};
+  auto multiply = [&] {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(y[h][j], x[h][j], acc, 0, 0, 0);
+  };
+  // a step reads its chunk from LDS while the one before is multiplied and the one after is written; the steps behind the last
+  // one multiply zeros
+  put(0);
+  for (int t = 0; t < steps; t += SMALL_AHEAD) {
+#pragma unroll
+    for (int i = 0; i < SMALL_AHEAD; ++i) {   // (no test in here: the waits for the requests would be for all of them)
+      lds_barrier();
+      f32x4 nx[2], ny[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        nx[h] = *reinterpret_cast<const f32x4 *>(As[i] + (h * 4 + g) * SMALL_PLANE + (wr * 16 + r16) * 4);
+        ny[h] = *reinterpret_cast<const f32x4 *>(Bs[i] + (h * 4 + g) * SMALL_PLANE + (wc * 16 + r16) * 4);
+      }
+      multiply();
+      put((i + 1) % SMALL_AHEAD);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        x[h] = nx[h];
+        y[h] = ny[h];
+      }
+    }
+  }
+  multiply();
+  // lane: columns 4 g .. of its row
+  const long long row = tile * 32 + wr * 16 + r16;
+  const int col = n0 + wc * 16 + 4 * g;
+  if (row >= a.n_rows || col >= a.c_out) return;
+  if (a.bias) acc += *reinterpret_cast<const f32x4 *>((const float *)a.bias + col);
+  if (a.res) acc += *reinterpret_cast<const f32x4 *>((const float *)a.res + row * a.c_out + col);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) acc[j] = act_apply(acc[j], a.act, a.slope);
+  *reinterpret_cast<f32x4 *>(out + row * a.ldo + col) = acc;
+}
+
 // ---- wavefront-independent form of the pair tiles and of the centre GEMM -------------------------
 // For fp16 rows of at most 64 channels a layer is bound by memory, and a workgroup that stages its
 // weight tile through LDS behind a barrier makes all resident workgroups read, compute and write in
@@ -704,8 +844,6 @@ static bool wave_gemm_ok(const TileArgs &a, int elem_size) {
 // The feature fragments of the pipelined kernel are requested by loads the compiler does not track:
 // it would otherwise wait for every outstanding load (the ones just issued included) before the first
 // use of a fragment inside the loop.  The waits are written by hand instead (pipe_wait_barrier).
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ u32x4 load16_untracked(const void *p) {
   u32x4 v;
@@ -1161,6 +1299,22 @@ static void launch_tile_nb(TileArgs a, long long tiles, hipStream_t s) {
     hipLaunchKernelGGL((tile_gemm_kernel<T, 1, FAST, TMODE, TEPI>), grid, dim3(256), 0, s, a);
 }
 
+// Where small_f32_kernel leads, by its workgroups (32 rows by 32 columns).  Output-stationary layers, tile kernel -> this one:
+// 256 -> 256 on 603 rows (152) 249 us -> 60, on 5 k (1 280) 341 -> 178, on 10 k (2 512) 455 -> 339, 128 -> 128 on 41 k (5 092)
+// 429 -> 342, on 85 k (10 572) 691 -> 703; with a last chunk that is mostly padding 20 -> 40 on 20 k (1 264) 44 -> 30, on 41 k (2 546)
+// 54.1 -> 55.3, 48 -> 96 on 41 k (3 819) 117 -> 140.  Plain products: 128 -> 128 on 603 (76) 7.8 -> 4.9, on 10 k (1 256) 11.1 -> 10.3,
+// on 20 k (2 528) 16.4 -> 17.6; 384 -> 256 on 10 k (2 512) 36 -> 27; 64 -> 64 on 10 k (628) 6.1 -> 6.0, on 20 k (1 264) 8.0 -> 8.1; 32 -> 32
+// 5.1-5.8 -> 4.9-6.0 up to 314, slower beyond.
+static bool small_f32_ok(const TileArgs &a) {
+  if (a.epi != EPI_ROWS || a.act_alone_only || (a.mode != MODE_DENSE && (a.mode != MODE_OS || a.kv > SMALL_MAX_KV))) return false;
+  const long long rows = a.mode == MODE_OS ? a.a_rows : a.n_rows;
+  if (rows <= 0 || rows * a.lda * 4 >= (long long)SMALL_MISSING || (long long)a.kv * a.c_in * a.c_out * 4 >= (1ll << 27)) return false;
+  if (a.parts > 1) return true;
+  const long long wgs = pce_div_up(a.n_rows, 32) * (a.n_pad / 32);
+  if (a.mode == MODE_OS) return wgs <= (8 * pce_div_up(a.c_in, SMALL_KC) * SMALL_KC > 9 * a.c_in ? 1280 : 5120);
+  return a.c_in >= 64 && wgs <= (a.c_in >= 256 ? 2560 : a.c_in >= 96 ? 1280 : 640);
+}
+
 template <typename T>
 static int launch_tile(const TileArgs &a, long long tiles, hipStream_t s) {
   if (tiles <= 0) return PCE_OK;
@@ -1176,6 +1330,13 @@ static int launch_tile(const TileArgs &a, long long tiles, hipStream_t s) {
   if (stage_on(9) && os_pipe_ok(a, sizeof(T)) && tiles * ((a.c_out + 127) / 128) <= 448) return launch_os_pipe(a, tiles, s);
   bool fast = a.a_vec && a.o_vec && (sizeof(T) == 2 ? a.Wp != nullptr : a.w_vec != 0) &&
               (a.epi != EPI_ROWS_CSR || a.b_vec) && aligned16(a.bias) && aligned16(a.res);
+  if (fast && sizeof(T) == 4 && small_f32_ok(a)) {
+    TileArgs b = a;
+    const unsigned grid = xcd_grid(&b, pce_div_up(a.n_rows, 32), a.n_pad / 32);
+    hipLaunchKernelGGL(small_f32_kernel, dim3(grid, a.parts > 1 ? a.parts : 1), dim3(256), 0, s, b);
+    PCE_LAUNCH_CHECK("small_f32");
+    return PCE_OK;
+  }
   if (!fast)
     launch_tile_nb<T, false, -1, -1>(a, tiles, s);
   else if (a.mode == MODE_DENSE && a.epi == EPI_ROWS_CSR)
@@ -2014,30 +2175,28 @@ extern "C" int pce_conv_fwd_fds(const void *in, const void *w, const void *wp, v
 }
 
 template <typename T>
-static int os_impl(const void *in, const void *w, const void *wp, void *out, int64_t n_out, int c_in, int c_out, int kv,
+static int os_impl(const void *in, const void *w, const void *wp, void *out, int64_t n_in, int64_t n_out, int c_in, int c_out, int kv,
                    const int *nbr, const Epi &e, hipStream_t s) {
   TileArgs a = base_args<T>(in, w, wp, kv, c_in, c_out, e.lda);
   set_out<T>(&a, out, false, n_out, e.ldo);
   set_epi(&a, e);
   a.nbr = nbr;
   a.n_rows = n_out;
+  a.a_rows = n_in;
   a.mode = MODE_OS;
   a.epi = EPI_ROWS;
   return launch_tile<T>(a, pce_div_up(n_out, 128), s);
 }
 
-// Output-stationary fp32 layers of few rows: a tile walks its offsets one after the other (10 us each at 256 -> 256
-// channels), so a few tiles take as long as many.  The offsets are shared out among `parts` workgroups per tile and
-// column slab, as many as make two workgroups per compute unit; every share stores its fp32 sums and os_parts_kernel adds
-// them up in the order of the offsets and finishes the rows.  The partial sums are at most 512 tiles of 128 x 32 (8 MB).
-// Where a tile has less to do than about six offsets of 128 channels the second launch costs what the shares give.
-// Layers of a U-Net on a 28 k-voxel surface scan whose tiles make 8 to 88 workgroups: 5.2 ms in 29 launches -> 0.9 ms in 60;
-// a forward of it 4.64 -> 2.32 ms, of the wide one on 8 k voxels 4.64 -> 2.94.
+// Output-stationary fp32 layers of few rows: a tile walks its offsets one after the other (2.2 us each at 256 channels,
+// small_f32_kernel), so a few tiles take as long as many.  The offsets are shared out among `parts` workgroups per tile of 32
+// rows by 32 columns; every share stores its fp32 sums and os_parts_kernel adds them up in the order of the offsets and finishes
+// the rows.  As many shares as make 1536, 768 or 512 workgroups, the fewer the shorter a share is (the partial sums, at most
+// 6 MB, and the second launch then cost more than it gives): 256 -> 256 on 603 rows 60 us -> 36, on 2.2 k 116 -> 97; 64 -> 64 on 603
+// 19.5 -> 13, on 5 k 27 -> 24; 32 -> 32 on 2.2 k 12.4 -> 11.5.  Below six offsets of 128 channels nothing is gained.
 static int os_parts(int dtype, long long n_out, int c_in, int c_out, int kv) {
   if (dtype != PCE_F32 || n_out <= 0 || (long long)kv * c_in < 768) return 1;
-  const long long tiles = pce_div_up(n_out, 128);
-  const int nb = narrow_blocks(tiles, c_out);
-  const long long parts = OS_WORKGROUPS / (tiles * (((c_out + 31) / 32 + nb - 1) / nb));
+  const long long parts = (c_in >= 128 ? 1536 : c_in >= 64 ? 768 : 512) / (pce_div_up(n_out, 32) * ((c_out + 31) / 32));
   return parts < 2 ? 1 : parts < kv ? (int)parts : kv;
 }
 
@@ -2085,6 +2244,7 @@ extern "C" int pce_conv_fwd_os_parts(const void *in, const void *w, void *out, i
   set_out<float>(&a, ws, false);
   a.nbr = nbr;
   a.n_rows = n_out;
+  a.a_rows = n_in;
   a.mode = MODE_OS;
   a.epi = EPI_ROWS;
   a.parts = os_parts(dtype, n_out, c_in, c_out, kv);
@@ -2113,8 +2273,8 @@ extern "C" int pce_conv_fwd_os(const void *in, const void *w, const void *wp, vo
   Epi e;
   if ((rc = read_epilogue("pce_conv_fwd_os", epilogue, out, &e, c_in, c_out))) return rc;
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == PCE_F16) return os_impl<half_t>(in, w, wp, out, n_out, c_in, c_out, kv, nbr, e, s);
-  return os_impl<float>(in, w, wp, out, n_out, c_in, c_out, kv, nbr, e, s);
+  if (dtype == PCE_F16) return os_impl<half_t>(in, w, wp, out, n_in, n_out, c_in, c_out, kv, nbr, e, s);
+  return os_impl<float>(in, w, wp, out, n_in, n_out, c_in, c_out, kv, nbr, e, s);
 }
 
 // ---- output-stationary over rows ordered by their neighbour pattern --------------------------------------------

@@ -56,6 +56,7 @@ struct TileArgs {
   const int *oslot;
   const void *buf;
   long long n_rows;  // MODE_DENSE / MODE_OS: rows of the output
+  long long a_rows;  // MODE_OS: rows of A (0: not stated)
   long long items;   // (tile, column slab) work items of the launch
   int slabs;         // column slabs per tile
   int parts;         // MODE_OS: shares of the offsets, blockIdx.y; the sums of share p at out + p * n_rows * c_out (0, 1: one)
