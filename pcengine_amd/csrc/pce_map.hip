@@ -1707,7 +1707,7 @@ struct Job {
   int kind;
   int pad;
 };
-enum { JOB_CSR_SUBM = 0, JOB_CSR_IN = 1, JOB_CSR_COUNT_OUT = 2, JOB_CSR_OUT = 3, JOB_ORDER_SCATTER = 4, JOB_FILL_VIEWS = 5 };
+enum { JOB_CSR_SUBM = 0, JOB_CSR_IN = 1, JOB_CSR_COUNT_OUT = 2, JOB_CSR_OUT = 3, JOB_ORDER_SCATTER = 4, JOB_FILL_VIEWS = 5, JOB_FILL_FULL3 = 6 };
 
 struct FillRegion {
   unsigned *p;
@@ -2436,14 +2436,12 @@ __global__ void __launch_bounds__(1024) kmap_offsets_kernel(const ProbDev *__res
 // written here.  Their row pointers are the same; the input view's entries of a row follow one another as the row's pairs do,
 // and the output view's entry of the pair (i, o, kp) lies behind those of o at lower offsets, which the mask of o counts.  (As a table
 // of the ranks and a launch that reads it back, what maps without an order take, this was 78 + 57 us for the nine maps of a
-// 100 k-voxel scan and 649 + 293 for 2 M rows of indoor scenes; 84 + 20 and 751 + 79 with the strided maps' part left.)  Bound by
+// 100 k-voxel scan and 649 + 293 for 2 M rows of indoor scenes; 80 + 20 and 707 + 80 with the strided maps' part left.)  Bound by
 // the scattered 4-byte stores, six a pair.
-// FULL3: of the fused probe, which leaves 27 offsets and nothing else to write.
-template <bool VIEWS, bool FULL3>
+template <bool VIEWS>
 __device__ __forceinline__ void fill_rows(const ProbDev &q, int block) {
   const long long n_in = q.n_in, n_out = q.n_out, nseg = q.nseg;
-  const int kv = FULL3 ? 27 : q.g.kv, subm = FULL3 ? 1 : q.g.subm, sym = FULL3 ? 1 : q.g.sym, mid = FULL3 ? 13 : q.g.mid;
-  const int fused = FULL3 ? 1 : q.fused;
+  const int kv = q.g.kv, subm = q.g.subm, sym = q.g.sym, mid = q.g.mid, fused = q.fused;
   // (pointers read from the descriptor are cast to the global address space, or the loads are compiled as flat
   // ones; every load of a batch goes out from a valid address and is masked afterwards, or each is compiled to a
   // branch with a wait behind it)
@@ -2453,9 +2451,9 @@ __device__ __forceinline__ void fill_rows(const ProbDev &q, int block) {
   PCE_GLOBAL int *imap = (PCE_GLOBAL int *)q.imap, *omap = (PCE_GLOBAL int *)q.omap;
   PCE_GLOBAL int *icode = (PCE_GLOBAL int *)q.icode, *ocode = (PCE_GLOBAL int *)q.ocode;
   PCE_GLOBAL int *islot = (PCE_GLOBAL int *)q.islot, *oslot = (PCE_GLOBAL int *)q.oslot;
-  int *__restrict__ irank = FULL3 ? nullptr : q.irank;
-  int *__restrict__ orank = FULL3 ? nullptr : q.orank;
-  int *__restrict__ nbr_out = FULL3 ? nullptr : q.nbr_out;
+  int *__restrict__ irank = q.irank;
+  int *__restrict__ orank = q.orank;
+  int *__restrict__ nbr_out = q.nbr_out;
   long long i = (long long)block * blockDim.x + threadIdx.x;
   long long seg = i >> 6;
   bool live = i < n_in;
@@ -2524,6 +2522,57 @@ __device__ __forceinline__ void fill_rows(const ProbDev &q, int block) {
   }
 }
 
+// The same for the 27 offsets of the fused probe, nine of them to a workgroup of rows: a row's hits at lower offsets are counted
+// by its own mask, so nothing is carried from one offset to the next (the launch 18 -> 10 us on the five levels of a 21 k-voxel
+// scan, 84 -> 80 on those of 100 k voxels, 751 -> 707 on 2 M rows).
+#define FULL3_GROUPS 3
+__device__ __forceinline__ void fill_full3(const ProbDev &q, int block) {
+  constexpr int N = 27 / FULL3_GROUPS;
+  typedef const __attribute__((address_space(4))) int *Uniform;   // read through the scalar cache
+  const int n = (int)q.n_in, nseg = (int)q.nseg, kp0 = block % FULL3_GROUPS * N;
+  const int i = block / FULL3_GROUPS * 256 + threadIdx.x, seg = __builtin_amdgcn_readfirstlane(i >> 6);
+  const bool live = i < n;
+  const PCE_GLOBAL int *table = (const PCE_GLOBAL int *)q.nbr_out, *csr = (const PCE_GLOBAL int *)q.icsr, *masks = (const PCE_GLOBAL int *)(q.order + n);
+  Uniform segoff = (Uniform)q.seg, kpos = (Uniform)q.kpos;
+  PCE_GLOBAL int *imap = (PCE_GLOBAL int *)q.imap, *omap = (PCE_GLOBAL int *)q.omap;
+  PCE_GLOBAL int *icode = (PCE_GLOBAL int *)q.icode, *ocode = (PCE_GLOBAL int *)q.ocode;
+  PCE_GLOBAL int *islot = (PCE_GLOBAL int *)q.islot, *oslot = (PCE_GLOBAL int *)q.oslot;
+  int v[N], om[N], op[N];
+  // (the row of the table at offset 26 - kp holds the pairs of offset kp; its centre row holds the identity and is no pair)
+#pragma unroll
+  for (int j = 0; j < N; ++j) v[j] = table[(26 - kp0 - j) * n + (live ? i : 0)];
+  const int first = csr[i <= n ? i : 0];
+  // the row has a pair at offset kp where its mask has bit 26 - kp
+  const unsigned hits = __brev((unsigned)masks[live ? i : 0] & ~(1u << 13)) >> 5;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    v[j] = live && kp0 + j != 13 ? v[j] : -1;
+    const int o = v[j] >= 0 ? v[j] : 0;
+    om[j] = masks[o];
+    op[j] = csr[o];
+  }
+  if (kp0 == 0 && i <= n) q.ocsr[i] = first;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int kp = kp0 + j;
+    const unsigned long long bal = __ballot(v[j] >= 0);
+    if (bal == 0) continue;
+    const int base = segoff[kp * nseg + seg], start = kpos[kp];
+    if (v[j] >= 0) {
+      const int p = base + __popcll(bal & lanemask_lt()), rank = p - start;
+      const unsigned below = (1u << kp) - 1;
+      const int pi = first + __popc(hits & below), po = op[j] + __popc((unsigned)om[j] & ~(1u << 13) & below), code = kp * PCE_CSR_CODE + rank;
+      imap[p] = i;
+      omap[p] = v[j];
+      icode[pi] = code;
+      ocode[po] = code;
+      if (islot) islot[p] = pi;
+      if (oslot) oslot[p] = po;
+      if (rank >= PCE_CSR_CODE) q.status[2] = 1;
+    }
+  }
+}
+
 __global__ void __launch_bounds__(256) kmap_fill_kernel(const ProbDev *__restrict__ P, JobList jl) {
   const Job &job = find_job(jl, blockIdx.x);
   const ProbDev &q = P[job.prob];
@@ -2536,12 +2585,12 @@ __global__ void __launch_bounds__(256) kmap_fill_kernel(const ProbDev *__restric
       order_scatter_block(q.n_out, q.order, blockIdx.x - job.blk0, q.dense, q.g.kv - 1);
     return;
   }
-  if (job.kind == JOB_FILL_VIEWS && q.fused)
-    fill_rows<true, true>(q, blockIdx.x - job.blk0);
+  if (job.kind == JOB_FILL_FULL3)
+    fill_full3(q, blockIdx.x - job.blk0);
   else if (job.kind == JOB_FILL_VIEWS)
-    fill_rows<true, false>(q, blockIdx.x - job.blk0);
+    fill_rows<true>(q, blockIdx.x - job.blk0);
   else
-    fill_rows<false, false>(q, blockIdx.x - job.blk0);
+    fill_rows<false>(q, blockIdx.x - job.blk0);
 }
 
 // CSR-coded views.  Entries of every row in ascending offset order, code = kp * PCE_CSR_CODE + rank, plus,
@@ -2920,7 +2969,10 @@ extern "C" int pce_kmap_build_batch(const pce_kmap_problem_t *probs, int32_t n_p
       add_scan(0, q.seg, L.scan_len, scan_tmp);
       if (want_csr) add_scan(0, q.icsr, n_in + 1, scan_tmp + scan_tmp_ints(L.scan_len));
       if (want_csr && q.g.sym && q.order) {
-        add_job(ST_FILL, p, JOB_FILL_VIEWS, n_in + 1);
+        if (fused)
+          add_job(ST_FILL, p, JOB_FILL_FULL3, FULL3_GROUPS * pce_align_up(n_in + 1, 256));
+        else
+          add_job(ST_FILL, p, JOB_FILL_VIEWS, n_in + 1);
         q.irank = nullptr;
       } else {
         add_job(ST_FILL, p, 0, n_in);
@@ -2936,7 +2988,7 @@ extern "C" int pce_kmap_build_batch(const pce_kmap_problem_t *probs, int32_t n_p
       add_scan(1, q.ocsr, n_out + 1, scan_tmp + scan_tmp_ints(L.scan_len) + scan_tmp_ints(n_in + 1));
       add_job(ST_CSR_B, p, JOB_CSR_OUT, n_out);
     }
-    total_blocks += pce_div_up(n_in + 1, 256) + pce_div_up(n_out + 1, 256) +
+    total_blocks += FULL3_GROUPS * pce_div_up(n_in + 1, 256) + pce_div_up(n_out + 1, 256) +
                     pce_div_up(use_grid ? box.cells * 2 : L.slots * 4, FILL_WORDS_PER_BLOCK) +
                     3 * pce_div_up((int64_t)q.g.kv * (n_in > n_out ? n_in : n_out), FILL_WORDS_PER_BLOCK);
   }
