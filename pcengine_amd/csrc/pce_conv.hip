@@ -3429,6 +3429,207 @@ __global__ void __launch_bounds__(BLK == 256 ? 512 : 256, BLK == 256 ? 1 : 2) wg
   if (cur >= 0) flush(cur);
 }
 
+// The same 128 x 128 blocks for rows of whole 16-byte pieces, as the rows lie in memory: pairs of both operands are copied
+// global -> LDS, [pair][channel], and the fragments are read with the transposing LDS read (ds_read_b64_tr_b16: of the four rows
+// that sixteen lanes address, 32 bytes each, lane l gets element l of every row), so nothing passes through registers on its
+// way in (wgrad_f16_kernel: 16 permutations and 16 eight-byte stores a thread and stage).  Stages of 32 pairs, a ring of four of
+// them, copied three ahead; every wavefront issues four copies per stage whatever it has to copy, and one of row indices per tile
+// of 128 pairs, so that waiting for all but the youngest eight operations means that its copies of this stage are there.
+// The 16-byte pieces of a row are exchanged by its pair index (piece ^ (pair & 3) * 4): the rows that one read addresses then
+// lie in different banks.
+// Bound by the LDS: a stage writes 16 KB and reads 32 for 256 clocks of matrix products of each wavefront.  wgrad_f16_kernel -> this
+// one: 256 -> 256 on 27 k rows of 19 pairs 222 us -> 117 (627 TFLOP/s), on 66 k of 9 241 -> 127, 384 -> 256 334 -> 182, 128 -> 128 on 66 k
+// 85 -> 65, on 89 k of 3 55 -> 38, 96 -> 96 on 99 k of 0.1 33 -> 25 (the sums' way to memory).
+#define WP_PAIRS 32
+#define WP_ST 4
+#define WP_MAX_BYTES 0xF0000000ll   // of rows that the copies address; offsets of missing pieces lie beyond
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) char lds_char;
+
+// `n` bytes per lane (16 or 4), global -> LDS at dst + n * lane, as the compiler does not track it: the caller waits by hand.  A lane whose
+// offset lies beyond the range writes zero.
+template <int N>
+__device__ __forceinline__ void copy_to_lds(u32x4 rsrc, unsigned off, unsigned dst) {
+  if (N == 16)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(off), "s"(rsrc), "s"(dst) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" : : "v"(off), "s"(rsrc), "s"(dst) : "memory", "m0");
+}
+__device__ __forceinline__ u32x4 byte_range(const void *p, unsigned bytes) {
+  return (u32x4){(unsigned)(uintptr_t)p, (unsigned)((uintptr_t)p >> 32), bytes, 0x00020000u};
+}
+
+__global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__restrict__ in, const half_t *__restrict__ gout, long long n_rows,
+                                                            unsigned in_bytes, unsigned out_bytes, int c_in, int c_out, int kv, int mid,
+                                                            const int *__restrict__ imap, const int *__restrict__ omap,
+                                                            const int *__restrict__ kpos, const int *__restrict__ qkpos,
+                                                            long long pair_tiles, long long tiles, int run, int ci_blocks,
+                                                            int co_blocks, float *__restrict__ gw) {
+  constexpr int OP = WP_PAIRS * 256, STAGE = 2 * OP;   // bytes of one operand's pairs, and of both
+  __shared__ __attribute__((aligned(1024))) char lds[WP_ST * STAGE];
+  __shared__ __attribute__((aligned(16))) int rows[2][2][128];   // input and output rows of a tile, for two tiles
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l32 = lane & 31, l16 = lane & 15, g = lane >> 5, wr = wave >> 1, wc = wave & 1;
+  // (the blocks of one run of tiles go to one XCD, as in wgrad_f16_kernel)
+  const long long slot = blockIdx.x >> 3;
+  const int rest = (int)(slot % (ci_blocks * co_blocks));
+  const long long grp = (slot / (ci_blocks * co_blocks)) * 8 + (blockIdx.x & 7);
+  const int ci0 = (rest / co_blocks) * 128, co0 = (rest % co_blocks) * 128;
+  const long long t_begin = grp * run, t_end = (grp + 1) * run < tiles ? (grp + 1) * run : tiles;
+  if (t_begin >= t_end) return;
+  const int n_tiles = (int)(t_end - t_begin);
+
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  auto flush = [&](int widx) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int co = co0 + wc * 64 + j * 32 + l32;
+      float *dst = gw + ((long long)widx * c_in + ci0 + wr * 64 + g * 4) * c_out + co;
+      if (co < c_out) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; ++e)   // (eight input channels at a time are there or not)
+            if (ci0 + wr * 64 + i * 32 + e / 4 * 8 < c_in) unsafeAtomicAdd(dst + (long long)(i * 32 + e / 4 * 8 + e % 4) * c_out, acc[i][j][e]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  };
+
+  // a tile: its offset (-1: none), its first pair or row, how many, and whether rows pair with themselves
+  struct Tile {
+    int w, first, count, same;
+  };
+  int lw = 0;
+  if (t_begin < pair_tiles)
+    for (int i = 0; i < kv; ++i) lw += ((long long)qkpos[i + 1] <= t_begin * 128) ? 1 : 0;
+  auto describe = [&](int t) {   // called for consecutive tiles
+    Tile d = {-1, 0, 0, 1};
+    const long long tile = t_begin + t;
+    if (t >= n_tiles) return d;
+    if (tile < pair_tiles) {
+      while (lw < kv && (long long)qkpos[lw + 1] <= tile * 128) ++lw;
+      if (lw >= kv) return d;
+      d.w = lw;
+      d.first = (int)(tile * 128 - qkpos[lw]) + kpos[lw];
+      d.count = kpos[lw + 1] - d.first;
+      d.same = 0;
+    } else {
+      d.w = mid;
+      d.first = (int)((tile - pair_tiles) * 128);
+      d.count = (int)(n_rows - d.first);
+    }
+    d.count = d.count < 128 ? (d.count > 0 ? d.count : 0) : 128;
+    // (uniform: in scalar registers from here on)
+    d.w = __builtin_amdgcn_readfirstlane(d.w);
+    d.first = __builtin_amdgcn_readfirstlane(d.first);
+    d.count = __builtin_amdgcn_readfirstlane(d.count);
+    d.same = __builtin_amdgcn_readfirstlane(d.same);
+    lw = __builtin_amdgcn_readfirstlane(lw);
+    return d;
+  };
+  const u32x4 in_rows = byte_range(in, in_bytes), out_rows = byte_range(gout, out_bytes);
+  const unsigned lds0 = (unsigned)(uintptr_t)(lds_char *)lds, rows0 = (unsigned)(uintptr_t)(lds_char *)(char *)rows;
+  // the row indices of a tile of pairs: wavefronts 0 and 1 the input rows, 2 and 3 the output rows, 64 each
+  auto fetch_rows = [&](const Tile &d, int slot_) {
+    const int *list = (wave < 2 ? imap : omap) + d.first;
+    const int part = (wave & 1) * 64;
+    copy_to_lds<4>(byte_range(list, d.same ? 0u : (unsigned)d.count * 4u), (part + lane) * 4,
+                   rows0 + ((slot_ * 2 + (wave >> 1)) * 128 + part) * 4);
+  };
+  // pairs 8 wave .. + 7 of a stage of both operands: this lane's row and its piece of it
+  const int piece = (lane & 15) ^ ((lane >> 4) << 2);
+  const unsigned in_at = (unsigned)(ci0 + piece * 8) * 2u, in_gone = ci0 + piece * 8 < c_in ? 0u : ~0u;
+  const unsigned out_at = (unsigned)(co0 + piece * 8) * 2u, out_gone = co0 + piece * 8 < c_out ? 0u : ~0u;
+  auto issue = [&](const Tile &d, int slot_, int stage, int buf) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int r = wave * 8 + t * 4 + (lane >> 4), pos = stage * WP_PAIRS + r;
+      // (both are formed whatever the tile is: a test would be a branch with a wait)
+      const int li = rows[slot_][0][pos], lo = rows[slot_][1][pos], own = d.first + pos;
+      const unsigned x = (unsigned)(d.same ? own : li) * (unsigned)(c_in * 2) + in_at, y = (unsigned)(d.same ? own : lo) * (unsigned)(c_out * 2) + out_at;
+      const unsigned gone = pos < d.count ? 0u : ~0u;
+      copy_to_lds<16>(in_rows, x | gone | in_gone, lds0 + buf * STAGE + (wave * 8 + t * 4) * 256);
+      copy_to_lds<16>(out_rows, y | gone | out_gone, lds0 + buf * STAGE + OP + (wave * 8 + t * 4) * 256);
+    }
+  };
+  // where the fragments of channels c .. c + 31 start: sixteen lanes address four pairs, 32 bytes each
+  auto frag_at = [&](int c) {
+    const int ch = c + ((lane >> 4) & 1) * 16 + (l16 & 3) * 4, pair = 8 * g + (l16 >> 2);
+    return pair * 256 + (((ch >> 3) ^ ((l16 >> 2) << 2)) * 16) + (ch & 4) * 2;
+  };
+  int a_at[2], b_at[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    a_at[i] = frag_at(wr * 64 + i * 32);
+    b_at[i] = OP + frag_at(wc * 64 + i * 32);
+  }
+  auto frag = [&](int at) -> half8 {
+    typedef __attribute__((address_space(3))) v4s lds_v4s;
+    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)((lds_char *)lds + at));
+    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)((lds_char *)lds + at + 4 * 256));
+    typedef short v8s __attribute__((ext_vector_type(8)));
+    return __builtin_bit_cast(half8, (v8s)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  auto multiply = [&](int buf) {
+#pragma unroll
+    for (int k = 0; k < WP_PAIRS; k += 16) {
+      half8 av[2], bv[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        av[i] = frag(buf * STAGE + k * 256 + a_at[i]);
+        bv[i] = frag(buf * STAGE + k * 256 + b_at[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[i], bv[j], acc[i][j], 0, 0, 0);
+    }
+  };
+#define WP_LANDED() asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory")
+  Tile d = describe(0), next = describe(1);
+  fetch_rows(d, 0);
+  fetch_rows(next, 1);
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  for (int st = 0; st < 3; ++st) issue(d, 0, st, st);
+  int cur = -1;
+  for (int t = 0; t < n_tiles; ++t) {
+    WP_LANDED();
+    issue(d, t & 1, 3, 3);
+    if (d.w != cur) {
+      if (cur >= 0) flush(cur);
+      cur = d.w;
+    }
+    multiply(0);
+    WP_LANDED();   // (every wavefront has issued this tile's last copies: its row indices are not read any more)
+    d = next;
+    issue(d, (t + 1) & 1, 0, 0);
+    multiply(1);
+    WP_LANDED();
+    issue(d, (t + 1) & 1, 1, 1);
+    next = describe(t + 2);
+    fetch_rows(next, t & 1);
+    multiply(2);
+    WP_LANDED();
+    issue(d, (t + 1) & 1, 2, 2);
+    multiply(3);
+  }
+#undef WP_LANDED
+  if (cur >= 0) flush(cur);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the copies behind the last stage end before the LDS is given back
+}
+
 template <typename T, int BLK>
 __global__ void __launch_bounds__(256) wgrad_kernel(const T *__restrict__ in, const T *__restrict__ gout, long long n_rows,
                                                     int c_in, int c_out, int kv, int mid, const int *__restrict__ imap,
@@ -3566,6 +3767,15 @@ extern "C" int pce_conv_wgrad(const void *in, const void *gout, int32_t dtype, i
   if (blk == 128 && ci_blocks * co_blocks >= 4) target_wgs = 1024;
   if (blk == 64 && tile_blocks >= 2048) target_wgs = 512;
   long long run = tile_blocks / target_wgs;
+  const int64_t in_bytes = n_in * c_in * 2, out_bytes = n_out * c_out * 2;
+  const bool pipe = dtype == PCE_F16 && blk == 128 && c_in % 8 == 0 && c_out % 8 == 0 && aligned16(in) && aligned16(gout) &&
+                    in_bytes < WP_MAX_BYTES && out_bytes < WP_MAX_BYTES;
+  if (pipe) {
+    // one workgroup per compute unit, as many runs on every XCD (256 -> 256 on 27 k rows of 19 pairs 117 us with 256 workgroups,
+    // 122 with 512, 149 with 2048; 96 -> 96 on 97 k rows of 0.8 25 with 256, 39 with 512)
+    const long long runs = 256 / (ci_blocks * co_blocks) / 8 * 8;
+    run = pce_div_up(tiles, runs < 8 ? 8 : runs);
+  }
   run = run < 1 ? 1 : (run > 256 ? 256 : run);
   long long blocks = pce_div_up(pce_div_up(tiles, run), 8) * 8 * ci_blocks * co_blocks;
   if (blocks >= (1ll << 31)) PCE_FAIL(PCE_ECAPACITY, "pce_conv_wgrad: %lld workgroups exceed the grid limit", blocks);
@@ -3577,7 +3787,11 @@ extern "C" int pce_conv_wgrad(const void *in, const void *gout, int32_t dtype, i
   hipLaunchKernelGGL((wgrad_f16_kernel<BLK_>), dim3((unsigned)blocks), dim3(256), 0, s, (const half_t *)in,            \
                      (const half_t *)gout, (long long)n_out, c_in, c_out, kv, mid, imap, omap, kpos, qkpos, pair_tiles, \
                      tiles, (int)run, ci_blocks, co_blocks, gw)
-  if (dtype == PCE_F16 && blk == 128)
+  if (pipe)
+    hipLaunchKernelGGL(wgrad_pipe_kernel, dim3((unsigned)blocks), dim3(256), 0, s, (const half_t *)in, (const half_t *)gout, (long long)n_out,
+                       (unsigned)in_bytes, (unsigned)out_bytes, c_in, c_out, kv, mid, imap, omap, kpos, qkpos, pair_tiles, tiles, (int)run,
+                       ci_blocks, co_blocks, gw);
+  else if (dtype == PCE_F16 && blk == 128)
     PCE_WGRAD16(128);
   else if (dtype == PCE_F16)
     PCE_WGRAD16(64);
