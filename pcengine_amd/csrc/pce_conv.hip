@@ -2435,6 +2435,129 @@ __global__ void __launch_bounds__(256, 4) wave_os_kernel(TileArgs a, const int *
   store_rows_via_lds<half_t, NB>(V, Pl[wave], (half_t *)a.out, orow, a, 0, lane, l32, g, a.stream);
 }
 
+// The same layers on large clouds where many rows have neighbours: 128 rows of the order per workgroup, 32 per wavefront, and
+// all four wavefronts walk the offsets of the workgroup's rows together, the centre as one of them.
+// What bounds wave_os_kernel there is the weights and its waits: a workgroup fetches an offset's fragments (8 KB at 64 -> 64)
+// for 32 rows, 2 GB from the L2s on 680 k rows with 5.2 neighbours, and a wavefront waits for rows and weights of one offset
+// after the other.  Here an offset's fragments come once for 128 rows, through LDS (two slots; the next offset's are in
+// registers meanwhile), the neighbour indices of a wavefront in one trip (a table in LDS), and the rows of three offsets
+// are in flight.  The loads are unconditional -- buffer loads, which read zero for a row without a neighbour at the
+// offset -- so that every wait is counted; a wavefront whose rows lack an offset leaves its products out.  Ascending
+// offsets: the sums of a row do not depend on the rows beside it.
+// 64 -> 64 with bias, residual and ReLU, wave_os_kernel / this one: 221 / 161 us on 680 k rows of indoor scenes with 5.2
+// neighbours, 198 / 160 on 954 k with 1.9, 103 / 87 on 276 k with 8.7; random clouds 326 / 217 on 815 k with 4.7, 87 / 72 on
+// 221 k with 5.6, 32 / 27 on 66 k with 5.6.  What is left is the gathers: the order visits a cloud once for every
+// pair of lowest offsets, so neighbour rows and table entries come from beyond the L2s (groups of 16 tiles on one XCD: no
+// change).  To 32 columns the two are equal (16 -> 16 on 680 k rows 79 / 80 us), so those stay with wave_os_kernel.
+#define WOSD_KV 27
+#define WOSD_MISSING 0xF0000000u
+template <int NB, int KS>
+__global__ void __launch_bounds__(256, 4) wave_osd_kernel(TileArgs a, const int *__restrict__ perm,
+                                                          const unsigned *__restrict__ rmask, int mid, int kv) {
+  constexpr int FR = KS * 2 * NB * 32;          // weight fragments of an offset: [k8][column]
+  constexpr int FRT = (FR + 255) / 256;
+  constexpr int IDX = WOSD_KV * 32;             // a wavefront's neighbour indices: [offset][row]
+  constexpr int WORK = 2 * FR + 4 * IDX / 4, OUT = 4 * WaveLds<NB>::PIECES;
+  __shared__ __attribute__((aligned(16))) half8 lds[WORK > OUT ? WORK : OUT];
+  __shared__ unsigned unions[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int l32 = lane & 31, g = lane >> 5;
+  half8 *const Wl = lds;
+  int *const idx = reinterpret_cast<int *>(lds + 2 * FR) + wave * IDX;
+  // the last tiles first: they hold the rows with the most offsets
+  const long long j = ((long long)gridDim.x - 1 - blockIdx.x) * 128 + wave * 32 + l32;
+  const int orow = j < a.n_rows ? perm[j] : -1;
+  const unsigned m = orow >= 0 ? rmask[orow] | 1u << mid : 0u;
+  unsigned u = m;
+#pragma unroll
+  for (int d = 1; d < 32; d <<= 1) u |= (unsigned)__shfl_xor((int)u, d, PCE_WAVE);
+  u = (unsigned)__builtin_amdgcn_readfirstlane((int)u);
+  if (lane == 0) unions[wave] = u;
+  {
+    const auto table = __builtin_amdgcn_make_buffer_rsrc(const_cast<int *>(a.nbr), 0, WOSD_MISSING, 0x00020000);
+    int v[(WOSD_KV + 1) / 2];
+#pragma unroll
+    for (int i = 0; i < (WOSD_KV + 1) / 2; ++i) {
+      const int k = 2 * i + g;
+      const bool have = k < kv && k != mid && ((m >> k) & 1u);
+      v[i] = __builtin_amdgcn_raw_buffer_load_b32(table, have ? (unsigned)((k * a.n_rows + orow) * 4) : WOSD_MISSING, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < (WOSD_KV + 1) / 2; ++i) {
+      const int k = 2 * i + g;
+      if (k < WOSD_KV) idx[k * 32 + l32] = k == mid ? orow : ((m >> k) & 1u) ? v[i] : -1;
+    }
+  }
+  __syncthreads();
+  unsigned rem = (unsigned)__builtin_amdgcn_readfirstlane((int)(unions[0] | unions[1] | unions[2] | unions[3]));
+  const int steps = __popc(rem);
+  const half_t *Wp = (const half_t *)a.Wp;
+  const long long wstep = (long long)a.k8_total * a.n_pad * 8;
+  const auto rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>((const void *)a.A), 0, WOSD_MISSING, 0x00020000);
+  const unsigned row_bytes = (unsigned)a.lda * 2;
+  typedef unsigned u4 __attribute__((ext_vector_type(4)));
+  u4 af[3][KS];
+  half8 wr[FRT];
+  int kk[3];
+  // offset of the next step (none left: 31, which no row has), its weights and its rows
+#define PCE_WOSD_ISSUE(J_)                                                                                             \
+  {                                                                                                                    \
+    const bool more_ = rem != 0;                                                                                       \
+    const int k_ = more_ ? __ffs((int)rem) - 1 : mid;                                                                  \
+    kk[J_] = more_ ? k_ : 31;                                                                                          \
+    rem &= rem - 1u;                                                                                                   \
+    _Pragma("unroll") for (int i = 0; i < FRT; ++i) {                                                                  \
+      const int f_ = i * 256 + (int)threadIdx.x;                                                                       \
+      wr[i] = *reinterpret_cast<const half8 *>(Wp + k_ * wstep + (f_ < FR ? f_ : FR - 1) * 8);                         \
+    }                                                                                                                  \
+    const int r_ = idx[k_ * 32 + l32];                                                                                 \
+    const unsigned at_ = more_ && r_ >= 0 ? (unsigned)r_ * row_bytes + (unsigned)g * 16u : WOSD_MISSING;               \
+    _Pragma("unroll") for (int s = 0; s < KS; ++s)                                                                     \
+      af[J_][s] = __builtin_amdgcn_raw_buffer_load_b128(rows, at_ + s * 32u, 0, 0);                                    \
+  }
+#define PCE_WOSD_PUT(SLOT_)                                                                                            \
+  _Pragma("unroll") for (int i = 0; i < FRT; ++i)                                                                      \
+    if (i * 256 + wave * 64 < FR) Wl[(SLOT_) * FR + i * 256 + threadIdx.x] = wr[i];
+  f32x16 acc[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[nb][i] = 0.f;
+  PCE_WOSD_ISSUE(0)
+  PCE_WOSD_PUT(0)
+  PCE_WOSD_ISSUE(1)
+  int slot = 0;
+  // a step: the next offset's weights into the slot that everyone has read, the loads of the offset after it, then the
+  // products of its own.  Whole rounds of three steps: the ones past the last offset have no rows.
+#define PCE_WOSD_STEP(J_)                                                                                              \
+  {                                                                                                                    \
+    __syncthreads();                                                                                                   \
+    PCE_WOSD_PUT(slot ^ 1)                                                                                             \
+    PCE_WOSD_ISSUE((J_ + 2) % 3)                                                                                       \
+    if ((u >> kk[J_]) & 1u) {                                                                                          \
+      _Pragma("unroll") for (int s = 0; s < KS; ++s)                                                                   \
+        _Pragma("unroll") for (int nb = 0; nb < NB; ++nb)                                                              \
+          acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Wl[slot * FR + (2 * s + g) * (NB * 32) + nb * 32 + l32],    \
+                                                           __builtin_bit_cast(half8, af[J_][s]), acc[nb], 0, 0, 0);    \
+    }                                                                                                                  \
+    slot ^= 1;                                                                                                         \
+  }
+  for (int t = 0; t < steps; t += 3) {
+    PCE_WOSD_STEP(0)
+    PCE_WOSD_STEP(1)
+    PCE_WOSD_STEP(2)
+  }
+#undef PCE_WOSD_STEP
+#undef PCE_WOSD_PUT
+#undef PCE_WOSD_ISSUE
+  __syncthreads();   // weights and indices have been read: the space becomes the output staging area
+  half8 *const region = lds + wave * WaveLds<NB>::PIECES;
+  float V[NB][2][8];
+  gather_row_pieces<NB>(acc, V, g);
+  if (a.bias || a.res || a.act) epilogue_row_pieces<half_t, NB, true>(V, a, orow, 0, g, a.act != PCE_ACT_NONE);
+  store_rows_via_lds<half_t, NB>(V, region, (half_t *)a.out, orow, a, 0, lane, l32, g, a.stream);
+}
+
 // A chunk of 32 rows with two neighbours or more, NBW column blocks of it from column n0 on, by one workgroup.
 // The four wavefronts split the INPUT CHANNELS, 16 each (one K step of the MFMA), and all walk the offsets of the
 // chunk's union: a step then holds 16 bytes of a neighbour row and 16 bytes of weights per column block in a lane
@@ -3176,6 +3299,23 @@ extern "C" int pce_conv_fwd_oso(const void *in, const void *w, const void *wp, v
       n_nonzero - n_single <= PCE_ORDER_SREC_ROWS(n_out) && 8 * (n_nonzero - n_single) <= n_out &&
       os2_workgroups(n_out, n_nonzero, n_single, n_heavy, nb) <= 4ll * cu_count() && stage_on(12))
     return launch_wave_os2(a, order, (int)mid, n_out, n_nonzero, n_single, n_heavy, nb, ks, s);
+  // More than 32 columns, more than two rounds of that kernel's shared workgroups (four per compute unit at a time, 32 rows
+  // each) and at least a third of the rows in them: the kernel whose wavefronts share the weights.  Times against the other
+  // kernel's at 16 -> 48, 32 -> 64, 48 -> 48, 64 -> 64: 1980 to 2030 shared workgroups with 0.96 of the rows 1.05,
+  // 0.92, 0.87, 0.87, with 0.44 of them 0.99, 0.95, 1.01, 1.02; 2110 with 0.71 1.05, 1.01, 1.00, 1.00; 3340 with
+  // 0.44 0.92, 0.88, 0.91, 0.90; 5490 with 0.36 0.92, 0.89, 0.95, 0.92; 1390 with 0.50 (64 -> 64) 1.03, 1510 with 0.04 1.13.
+  if (mid >= 0 && kv <= WOSD_KV && nb == 2 && heavy_wgs > 8ll * cu_count() && 3 * n_split >= n_out &&
+      n_in * (int64_t)a.lda * 2 < (int64_t)WOSD_MISSING - 256 && n_out * kv * 4 < (int64_t)WOSD_MISSING) {
+    const unsigned tiles = (unsigned)pce_div_up(n_out, 128);
+#define PCE_WOSD_CASE(NB_, KS_)                                                                                        \
+  if (nb == NB_ && ks == KS_) {                                                                                        \
+    hipLaunchKernelGGL((wave_osd_kernel<NB_, KS_>), dim3(tiles), dim3(256), 0, s, a, perm, rmask, (int)mid, (int)kv);  \
+    PCE_LAUNCH_CHECK("wave_osd");                                                                                      \
+    return PCE_OK;                                                                                                     \
+  }
+    PCE_WOSD_CASE(2, 1) PCE_WOSD_CASE(2, 2) PCE_WOSD_CASE(2, 3) PCE_WOSD_CASE(2, 4)
+#undef PCE_WOSD_CASE
+  }
 #define PCE_WOS_CASE(NB_, KS_)                                                                              \
   if (nb == NB_ && ks == KS_) {                                                                              \
     hipLaunchKernelGGL((wave_os_kernel<NB_, KS_>), dim3(grid), dim3(256), 0, s, a, perm, rmask, (int)mid, n_main,   \

@@ -1,0 +1,53 @@
+"""fp16 layers of 33 to 64 columns on large clouds with many neighbours: four wavefronts that share an offset's weights."""
+import pytest
+import torch
+
+import pcengine_amd as pe
+from pcengine_amd import backend, synth
+from pcengine_amd.spconv import prebuild_maps
+from tests.util import DEV
+
+pytestmark = pytest.mark.gpu
+
+
+def _map(n, density, seed):
+    coords = torch.as_tensor(synth.random_cloud(seed=seed, n=n, extent=max(2, round((n / density) ** (1 / 3)))), device=DEV).int()
+    x = pe.spTensor(torch.zeros((len(coords), 1), device=DEV), coords, None, [0, 0, 0], coords[:, 1:].max(0).values.tolist(), batchsize=1)
+    prebuild_maps(x, [(3, 1, 0)])
+    return next(iter(x.kmaps.values()))
+
+
+# rows just beyond the line of the selection (more than 2048 groups of 32 rows with two neighbours), in mixed tiles of 128,
+# and of a cloud whose rows with none or one are more than half
+@pytest.mark.parametrize("n,density", [(78001, 0.25), (110011, 0.9), (250003, 0.06)])
+@pytest.mark.parametrize("c_in,c_out,slices", [(16, 40, False), (32, 64, True), (48, 48, False), (64, 64, False), (64, 56, True)])
+def test_sums_of_rows_that_share_weights(n, density, c_in, c_out, slices):
+    km = _map(n, density, seed=11)
+    backend.row_order(km)
+    rows, split = km.n_out, km.order_nonzero - km.order_single
+    assert split > 2048 * 32 and 3 * split >= rows
+    gen = torch.Generator(device=DEV).manual_seed(c_in * 100 + c_out)
+    wide = torch.randn((rows, c_in + (8 if slices else 0)), generator=gen, device=DEV).half()
+    x = wide[:, :c_in]
+    w = (torch.randn((27, c_in, c_out), generator=gen, device=DEV) * 0.1).half()
+    bias = torch.randn(c_out, generator=gen, device=DEV).half()
+    residual = torch.randn((rows, c_out), generator=gen, device=DEV).half()
+    out = torch.full((rows, c_out + (8 if slices else 0)), 7.0, dtype=torch.float16, device=DEV)
+    backend.conv_forward(x, w, km, backend.DATAFLOW_OSO, bias=bias, residual=residual, act="relu", out=out[:, :c_out])
+    nbr = km.nbr_out.view(27, rows).long()
+    nbr[13] = torch.arange(rows, device=DEV)
+    want = torch.zeros((rows, c_out), dtype=torch.float64, device=DEV)
+    size = torch.zeros((rows, c_out), dtype=torch.float64, device=DEV)
+    for k in range(27):
+        at = torch.nonzero(nbr[k] >= 0)[:, 0]
+        f = x[nbr[k][at]].double()
+        want[at] += f @ w[k].double()
+        size[at] += f.abs() @ w[k].double().abs()
+    want = want + bias.double() + residual.double()
+    size = size + bias.double().abs() + residual.double().abs()
+    # one rounding to fp16 of the result, and of every fp32 addition at most half a unit of what is summed
+    bound = 2.0 ** -11 * want.abs() + (27 * c_in + 2) * 2.0 ** -24 * size + 2.0 ** -24
+    got = out[:, :c_out].double()
+    assert ((got - want.clamp(min=0)).abs() <= bound).all()
+    if slices:
+        assert (out[:, c_out:] == 7.0).all()
