@@ -51,3 +51,12 @@ def test_sums_of_rows_that_share_weights(n, density, c_in, c_out, slices):
     assert ((got - want.clamp(min=0)).abs() <= bound).all()
     if slices:
         assert (out[:, c_out:] == 7.0).all()
+
+
+@pytest.mark.parametrize("rows,pairs,c_out,ordered", [(65535, 12.0, 32, True), (65536, 12.0, 32, False), (65536, 12.0, 40, True),
+                                                      ((1 << 18) - 1, 12.0, 64, True), (1 << 18, 12.0, 64, False),
+                                                      (100000, 12.1, 64, False), (1 << 18, 6.0, 64, True)])
+def test_selection_by_rows_pairs_and_columns(rows, pairs, c_out, ordered):
+    n_pairs = int(rows * pairs)
+    got = backend._lib.load().pce_select_dataflow(rows, rows, n_pairs, 48, c_out, 27, 13, 0, backend.PCE_F16)
+    assert got == (backend.DATAFLOW_OSO if ordered else backend.DATAFLOW_OS)
