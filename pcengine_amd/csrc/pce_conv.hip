@@ -2446,9 +2446,9 @@ __global__ void __launch_bounds__(256, 4) wave_os_kernel(TileArgs a, const int *
 // offsets: the sums of a row do not depend on the rows beside it.
 // 64 -> 64 with bias, residual and ReLU, wave_os_kernel / this one: 221 / 161 us on 680 k rows of indoor scenes with 5.2
 // neighbours, 198 / 160 on 954 k with 1.9, 103 / 87 on 276 k with 8.7; random clouds 326 / 217 on 815 k with 4.7, 87 / 72 on
-// 221 k with 5.6, 32 / 27 on 66 k with 5.6.  What is left is the gathers: the order visits a cloud once for every
-// pair of lowest offsets, so neighbour rows and table entries come from beyond the L2s (groups of 16 tiles on one XCD: no
-// change).  To 32 columns the two are equal (16 -> 16 on 680 k rows 79 / 80 us), so those stay with wave_os_kernel.
+// 221 k with 5.6, 32 / 27 on 66 k with 5.6.  What is left is memory: the 680 k rows fetch 744 MB
+// and write 87 MB, 5.2 TB/s, where the tensors hold 261 MB; the order visits a cloud once for every pair of lowest offsets,
+// so 41 % of the L2 requests for neighbour rows and table entries miss (groups of 16 tiles on one XCD: no change).  To 32 columns the two are equal (16 -> 16 on 680 k rows 79 / 80 us), so those stay with wave_os_kernel.
 #define WOSD_KV 27
 #define WOSD_MISSING 0xF0000000u
 template <int NB, int KS>

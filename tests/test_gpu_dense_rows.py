@@ -60,3 +60,23 @@ def test_selection_by_rows_pairs_and_columns(rows, pairs, c_out, ordered):
     n_pairs = int(rows * pairs)
     got = backend._lib.load().pce_select_dataflow(rows, rows, n_pairs, 48, c_out, 27, 13, 0, backend.PCE_F16)
     assert got == (backend.DATAFLOW_OSO if ordered else backend.DATAFLOW_OS)
+
+
+def test_pointers_the_ordered_rows_refuse():
+    """A layer of the selector's ordered range with an odd pointer takes the dense tiles."""
+    km = _map(110003, 0.46, seed=3)
+    rows = km.n_out
+    assert rows >= 1 << 16 and 6 < km.M / rows <= 12
+    df = backend.select_dataflow(km, 48, 40, torch.float16)
+    assert df == backend.DATAFLOW_OSO and df is backend.ROWS_LEAD
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn((rows, 48), generator=gen, device=DEV).half()
+    w = (torch.randn((27, 48, 40), generator=gen, device=DEV) * 0.1).half()
+    bias = torch.randn(40, generator=gen, device=DEV).half()
+    want = backend.conv_forward(x, w, km, backend.DATAFLOW_OS, bias=bias)
+
+    def odd(t):
+        return torch.empty(t.numel() + 4, dtype=t.dtype, device=DEV)[4:].view(t.shape).copy_(t)
+
+    for feats, b, out in ((odd(x), bias, None), (x, odd(bias), None), (x, bias, odd(want))):
+        assert torch.equal(backend.conv_forward(feats, w, km, df, bias=b, out=out), want)
