@@ -159,8 +159,9 @@ int pce_outcoords_chain_planned(const int32_t *in_coords_dev, int64_t n_in, int6
  * on the host: voxel = floor(point / voxel_size) in double precision; the unique voxels in
  * ascending (x,y,z) order (the order of the ravelled code); for every voxel the first point that
  * falls into it (numpy.unique return_index); for every point its voxel (return_inverse).
- * points_dev[n_points,3] are PCE_F32 or PCE_F64.  pce_voxelize synchronises the stream twice
- * (coordinate bounds, then the voxel count) and returns the count and the bounds of the integer
+ * points_dev[n_points,3] are PCE_F32 or PCE_F64.  pce_voxelize synchronises the stream once, behind
+ * the coordinate bounds and the voxel count (twice where the box is too empty for a bitmap of its
+ * occupied blocks and the points are sorted), and returns the count and the bounds of the integer
  * coordinates on the host; pce_voxelize_emit (same workspace, untouched since; the bounds handed
  * back) writes coords_out[n_voxels,4] = (batch_index, x, y, z), index_out[n_voxels] and
  * inverse_out[n_points]; any of the three may be NULL.  Negative coordinates are kept, as in the
