@@ -4447,12 +4447,13 @@ extern "C" int pce_select_dataflow(int64_t n_in, int64_t n_out, int64_t n_pairs,
   if (oso && subm && dtype == PCE_F32 && rho <= (c_in <= 16 ? 6.0 : 2.0)) return PCE_DATAFLOW_OSO;
   // (a cloud of fewer than two 128-row tiles per compute unit -- 256 of them -- leaves the dense tiles' launch short
   // of workgroups: 24 k rows at 9.2 pairs per row, 48 -> 48 channels: ordered rows 17 us, deferred scatter 21, tiles 28)
-  // (more than 32 columns, which the ordered rows then take 128 at a time with shared weights: to twelve pairs per row on up to
-  // 0.26 M rows 0.62-0.97 of the faster of the other two -- 16 -> 40 .. 64 -> 64 at 6.5, 9.3 and 11.7 on random clouds of 78 k
-  // to 214 k rows, at 8.7 to 9.9 on levels of scans and rooms of 66 k to 276 k; on random clouds of 0.6 M rows at 7 to 12
+  // (more than 32 columns, which the ordered rows take 128 at a time with shared weights from eight groups of 32 rows with two
+  // neighbours per compute unit on -- nearly all rows have two at these densities, hence the ninth: to twelve pairs per row on
+  // up to 0.26 M rows 0.62-0.97 of the faster of the other two -- 16 -> 40 .. 64 -> 64 at 6.5, 9.3 and 11.7 on random
+  // clouds of 78 k to 214 k rows, at 8.7 on a level of rooms of 276 k; on random clouds of 0.6 M rows at 7 to 12
   // 0.80-1.34, most of it above 1; at 14 on 0.2 M 0.85-1.06)
-  if (oso && subm && dtype == PCE_F16 && os_widths(c_in, c_out) &&
-      rho <= (n_out < 2 * 256 * 128 || (c_out > 32 && n_out < (1 << 18)) ? 12.0 : 6.0))
+  const bool shared = c_out > 32 && n_out >= 9 * 256 * 32 && n_out < (1 << 18);
+  if (oso && subm && dtype == PCE_F16 && os_widths(c_in, c_out) && rho <= (n_out < 2 * 256 * 128 || shared ? 12.0 : 6.0))
     return PCE_DATAFLOW_OSO;
   // the K-stepped form of the same kernel (wave_osw_kernel): a wavefront walks c_in / 16 K steps per offset of its
   // rows' union, so the density up to which it leads falls with the input width.  Measured on the levels of a

@@ -53,7 +53,8 @@ def test_sums_of_rows_that_share_weights(n, density, c_in, c_out, slices):
         assert (out[:, c_out:] == 7.0).all()
 
 
-@pytest.mark.parametrize("rows,pairs,c_out,ordered", [(65535, 12.0, 32, True), (65536, 12.0, 32, False), (65536, 12.0, 40, True),
+@pytest.mark.parametrize("rows,pairs,c_out,ordered", [(65535, 12.0, 32, True), (65536, 12.0, 40, False), (73727, 12.0, 40, False),
+                                                      (73728, 12.0, 32, False), (73728, 12.0, 40, True),
                                                       ((1 << 18) - 1, 12.0, 64, True), (1 << 18, 12.0, 64, False),
                                                       (100000, 12.1, 64, False), (1 << 18, 6.0, 64, True)])
 def test_selection_by_rows_pairs_and_columns(rows, pairs, c_out, ordered):
@@ -66,7 +67,7 @@ def test_pointers_the_ordered_rows_refuse():
     """A layer of the selector's ordered range with an odd pointer takes the dense tiles."""
     km = _map(110003, 0.46, seed=3)
     rows = km.n_out
-    assert rows >= 1 << 16 and 6 < km.M / rows <= 12
+    assert rows >= 73728 and 6 < km.M / rows <= 12
     df = backend.select_dataflow(km, 48, 40, torch.float16)
     assert df == backend.DATAFLOW_OSO and df is backend.ROWS_LEAD
     gen = torch.Generator(device=DEV).manual_seed(1)
