@@ -35,6 +35,9 @@ __device__ constexpr int osb_key_bit27(int kp) {
 // entries behind the last row of the cloud, which share their key with a pattern of offset 0 alone, stay behind every row.
 // Bound by the ballots and the LDS counters, not by memory: with the plan 36 us for 72 k rows of a random cloud as for
 // 100 k of a scan (ranked by LDS atomics, whose lanes met at few counters: 36 and 43).
+// SHORT: a cloud of one window that is not full, where a thread has per = rows / 1024 entries instead of eight (with the plan
+// 31 -> 15 us on 700 rows, 21 on 3 k, 29 on 6 k; in a full window the conditions would cost 1 us of 33).
+template <bool SHORT>
 __global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(const int *__restrict__ nbr, const unsigned *__restrict__ known,
                                                                       unsigned centre, int kv, int n, int *__restrict__ perm,
                                                                       unsigned *__restrict__ bmask) {
@@ -46,6 +49,7 @@ __global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(const int 
   __shared__ unsigned wave_sum[WAVES];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int r0 = blockIdx.x * OSB_WINDOW, cnt = n - r0 < OSB_WINDOW ? n - r0 : OSB_WINDOW;
+  const int per = SHORT ? (cnt + OSB_ORDER_THREADS - 1) / OSB_ORDER_THREADS : PER;
   unsigned m[PER];
   if (known) {
 #pragma unroll
@@ -69,6 +73,7 @@ __global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(const int 
   }
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
+    if (SHORT && i >= per) break;
     const int li = i * OSB_ORDER_THREADS + t;
     const bool ok = li < cnt;
     const unsigned pat = m[i] | centre;
@@ -99,12 +104,13 @@ __global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(const int 
     // before (a counter per (digit, wavefront), updated by the first lane of a digit)
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int at = (wave * PER + i) * 64 + lane;
+      const int at = (wave * per + (!SHORT || i < per ? i : 0)) * 64 + lane;
       key[i] = keys[at];
       rw[i] = rows[at];
     }
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
+      if (SHORT && i >= per) break;
       const unsigned d = (key[i] >> shift) & (BINS - 1);
       unsigned long long peers = ~0ull;
 #pragma unroll
@@ -144,6 +150,7 @@ __global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(const int 
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
+      if (SHORT && i >= per) break;
       const unsigned d = (key[i] >> shift) & (BINS - 1);
       const unsigned p = hist[counter(d, wave)] + pos[i];
       keys[p] = key[i];
@@ -151,7 +158,7 @@ __global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(const int 
     }
     __syncthreads();
   }
-  for (int i = 0; i < PER; ++i) {
+  for (int i = 0; i < per; ++i) {
     const int p = i * OSB_ORDER_THREADS + t;
     const int li = rows[p];
     unsigned m = p < cnt ? masks[li] : 0u;
@@ -302,8 +309,12 @@ extern "C" int pce_osb_order(const int32_t *nbr, const int32_t *mask, int32_t mi
     PCE_FAIL(PCE_EWORKSPACE, "pce_osb_order: order holds %lld elements, needs %lld", (long long)order_elems, (long long)pce_osb_order_elems(n));
   hipStream_t s = (hipStream_t)stream;
   unsigned *bmask = (unsigned *)order + osb_mask_offset(n);
-  hipLaunchKernelGGL(osb_order_kernel, dim3((unsigned)pce_div_up(n, OSB_WINDOW)), dim3(OSB_ORDER_THREADS), 0, s, nbr, (const unsigned *)mask,
-                     mid >= 0 ? 1u << mid : 0u, kv, (int)n, order, bmask);
+  if (n <= OSB_WINDOW - OSB_ORDER_THREADS)
+    hipLaunchKernelGGL(osb_order_kernel<true>, dim3(1), dim3(OSB_ORDER_THREADS), 0, s, nbr, (const unsigned *)mask, mid >= 0 ? 1u << mid : 0u, kv,
+                       (int)n, order, bmask);
+  else
+    hipLaunchKernelGGL(osb_order_kernel<false>, dim3((unsigned)pce_div_up(n, OSB_WINDOW)), dim3(OSB_ORDER_THREADS), 0, s, nbr,
+                       (const unsigned *)mask, mid >= 0 ? 1u << mid : 0u, kv, (int)n, order, bmask);
   PCE_LAUNCH_CHECK("osb_order");
   hipLaunchKernelGGL(osb_plan_kernel, dim3(8, OSB_MAX_SLABS), dim3(1024), 0, s, bmask, (int)n, (int)pce_div_up(n, OSB_ROWS),
                      order + osb_plans_offset(n));
