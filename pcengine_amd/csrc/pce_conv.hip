@@ -2436,26 +2436,36 @@ __global__ void __launch_bounds__(256, 4) wave_os_kernel(TileArgs a, const int *
 }
 
 // The same layers on large clouds where many rows have neighbours: 128 rows of the order per workgroup, 32 per wavefront, and
-// all four wavefronts walk the offsets of the workgroup's rows together, the centre as one of them.
+// all four wavefronts walk the offsets of the workgroup's rows together, the centre first.
 // What bounds wave_os_kernel there is the weights and its waits: a workgroup fetches an offset's fragments (8 KB at 64 -> 64)
 // for 32 rows, 2 GB from the L2s on 680 k rows with 5.2 neighbours, and a wavefront waits for rows and weights of one offset
 // after the other.  Here an offset's fragments come once for 128 rows, through LDS (two slots; the next offset's are in
-// registers meanwhile), the neighbour indices of a wavefront in one trip (a table in LDS), and the rows of three offsets
-// are in flight.  The loads are unconditional -- buffer loads, which read zero for a row without a neighbour at the
-// offset -- so that every wait is counted; a wavefront whose rows lack an offset leaves its products out.  Ascending
-// offsets: the sums of a row do not depend on the rows beside it.
-// 64 -> 64 with bias, residual and ReLU, wave_os_kernel / this one: 221 / 161 us on 680 k rows of indoor scenes with 5.2
-// neighbours, 198 / 160 on 954 k with 1.9, 103 / 87 on 276 k with 8.7; random clouds 326 / 217 on 815 k with 4.7, 87 / 72 on
-// 221 k with 5.6, 32 / 27 on 66 k with 5.6.  What is left is memory: the 680 k rows fetch 744 MB
-// and write 87 MB, 5.2 TB/s, where the tensors hold 261 MB; the order visits a cloud once for every pair of lowest offsets,
-// so 41 % of the L2 requests for neighbour rows and table entries miss (groups of 16 tiles on one XCD: no change).  To 32 columns the two are equal (16 -> 16 on 680 k rows 79 / 80 us), so those stay with wave_os_kernel.
+// registers meanwhile), the neighbour indices of a wavefront in one trip (a table in LDS), and the rows of two or three
+// offsets are in flight.  The loads are unconditional -- buffer loads, which read zero for a row without a neighbour at the
+// offset -- so that every wait is counted; a wavefront whose rows lack an offset leaves its products out.
+// The sums are wave_os_kernel's bit for bit.  Rows with two neighbours or more and the others have workgroups of their
+// own, as there.  The former walk the offsets share by share (the centre and the offsets whose number is a multiple of four,
+// then those of remainder 1, 2, 3), each share's sum starts from zero, and the shares are added in this order; the
+// others add centre and offsets up in one chain.
+// With the shares' sum beside the share's the rows of three offsets fit four wavefronts to a SIMD at 32 input channels; from 48
+// on two are kept in flight and a step's are requested behind its products (three of them, three wavefronts: 64 -> 64 on
+// 954 k rows of indoor scenes 173 us, 162 so; on 0.13 M rows of a random cloud, whose second round then is nearly empty, 54 and 47).
+// With bias, residual and ReLU, wave_os_kernel / this one: 64 -> 64 on 680 k rows of indoor scenes with 5.2 neighbours
+// 223 / 170 us, on 954 k with 1.9 201 / 162, on 276 k with 8.7 103 / 95; on random clouds 325 / 223 on 815 k with 4.7, 88 / 78 on
+// 223 k with 5.7; 32 -> 64 on the same five 148 / 124, 152 / 133, 64 / 57, 214 / 187, 62 / 62.
+// What is left is memory: 64 -> 64 on the 680 k rows fetches 744 MB and writes 87 MB where the tensors hold 261 MB; the order
+// visits a cloud once for every pair of lowest offsets, so 41 % of the L2 requests for neighbour rows and table entries miss.
+// To 32 columns and from 16 input channels there is nothing to share (16 -> 16 on 680 k rows 79 / 80 us, 16 -> 64 on 73 k 20.6 / 24.5):
+// those stay with wave_os_kernel.
 #define WOSD_KV 27
 #define WOSD_MISSING 0xF0000000u
 template <int NB, int KS>
 __global__ void __launch_bounds__(256, 4) wave_osd_kernel(TileArgs a, const int *__restrict__ perm,
-                                                          const unsigned *__restrict__ rmask, int mid, int kv) {
+                                                                       const unsigned *__restrict__ rmask, int mid, int kv,
+                                                                       long long n_main, int heavy_wgs) {
   constexpr int FR = KS * 2 * NB * 32;          // weight fragments of an offset: [k8][column]
   constexpr int FRT = (FR + 255) / 256;
+  constexpr int RING = KS > 2 ? 2 : 3;          // offsets whose rows are in flight
   constexpr int IDX = WOSD_KV * 32;             // a wavefront's neighbour indices: [offset][row]
   constexpr int WORK = 2 * FR + 4 * IDX / 4, OUT = 4 * WaveLds<NB>::PIECES;
   __shared__ __attribute__((aligned(16))) half8 lds[WORK > OUT ? WORK : OUT];
@@ -2465,8 +2475,10 @@ __global__ void __launch_bounds__(256, 4) wave_osd_kernel(TileArgs a, const int 
   half8 *const Wl = lds;
   int *const idx = reinterpret_cast<int *>(lds + 2 * FR) + wave * IDX;
   // the last tiles first: they hold the rows with the most offsets
-  const long long j = ((long long)gridDim.x - 1 - blockIdx.x) * 128 + wave * 32 + l32;
-  const int orow = j < a.n_rows ? perm[j] : -1;
+  const bool heavy = (int)blockIdx.x < heavy_wgs;
+  const long long tile = (heavy ? heavy_wgs : (int)gridDim.x) - 1 - (int)blockIdx.x;   // of its part of the rows
+  const long long j = (heavy ? n_main : 0) + tile * 128 + wave * 32 + l32;
+  const int orow = j < (heavy ? a.n_rows : n_main) ? perm[j] : -1;
   const unsigned m = orow >= 0 ? rmask[orow] | 1u << mid : 0u;
   unsigned u = m;
 #pragma unroll
@@ -2491,21 +2503,29 @@ __global__ void __launch_bounds__(256, 4) wave_osd_kernel(TileArgs a, const int 
   __syncthreads();
   unsigned rem = (unsigned)__builtin_amdgcn_readfirstlane((int)(unions[0] | unions[1] | unions[2] | unions[3]));
   const int steps = __popc(rem);
+  rem &= ~(1u << mid);
+  const unsigned share = heavy ? 0x11111111u : ~0u;
+  int first = 1, cls = 0;   // the centre comes first; share of the next offset
   const half_t *Wp = (const half_t *)a.Wp;
   const long long wstep = (long long)a.k8_total * a.n_pad * 8;
   const auto rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>((const void *)a.A), 0, WOSD_MISSING, 0x00020000);
   const unsigned row_bytes = (unsigned)a.lda * 2;
   typedef unsigned u4 __attribute__((ext_vector_type(4)));
-  u4 af[3][KS];
+  u4 af[RING][KS];
   half8 wr[FRT];
-  int kk[3];
-  // offset of the next step (none left: 31, which no row has), its weights and its rows
+  int kk[RING], kc[RING];
+  // offset of the next step (none left: 31, which no row has) and its share, its weights and its rows
 #define PCE_WOSD_ISSUE(J_)                                                                                             \
   {                                                                                                                    \
-    const bool more_ = rem != 0;                                                                                       \
-    const int k_ = more_ ? __ffs((int)rem) - 1 : mid;                                                                  \
+    if (!first)                                                                                                        \
+      for (int c_ = 0; c_ < 3; ++c_) cls += cls < 3 && !(rem & (share << cls)) ? 1 : 0;                                \
+    const unsigned left_ = rem & (share << cls);                                                                       \
+    const bool more_ = first || left_ != 0;                                                                            \
+    const int k_ = first || !left_ ? mid : __ffs((int)left_) - 1;                                                      \
     kk[J_] = more_ ? k_ : 31;                                                                                          \
-    rem &= rem - 1u;                                                                                                   \
+    kc[J_] = cls;                                                                                                      \
+    rem &= first ? ~0u : ~(left_ & (0u - left_));                                                                      \
+    first = 0;                                                                                                         \
     _Pragma("unroll") for (int i = 0; i < FRT; ++i) {                                                                  \
       const int f_ = i * 256 + (int)threadIdx.x;                                                                       \
       wr[i] = *reinterpret_cast<const half8 *>(Wp + k_ * wstep + (f_ < FR ? f_ : FR - 1) * 8);                         \
@@ -2518,38 +2538,50 @@ __global__ void __launch_bounds__(256, 4) wave_osd_kernel(TileArgs a, const int 
 #define PCE_WOSD_PUT(SLOT_)                                                                                            \
   _Pragma("unroll") for (int i = 0; i < FRT; ++i)                                                                      \
     if (i * 256 + wave * 64 < FR) Wl[(SLOT_) * FR + i * 256 + threadIdx.x] = wr[i];
-  f32x16 acc[NB];
+  f32x16 acc[NB], sum[NB];   // of the share, and of the shares before it
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[nb][i] = 0.f;
+    for (int i = 0; i < 16; ++i) acc[nb][i] = sum[nb][i] = 0.f;
   PCE_WOSD_ISSUE(0)
   PCE_WOSD_PUT(0)
   PCE_WOSD_ISSUE(1)
-  int slot = 0;
-  // a step: the next offset's weights into the slot that everyone has read, the loads of the offset after it, then the
-  // products of its own.  Whole rounds of three steps: the ones past the last offset have no rows.
+  int slot = 0, now = 0;
+  // a step: the next offset's weights into the slot that everyone has read, the loads of the offset after it, and the
+  // products of its own.  Whole rounds of RING steps: the ones past the last offset have no rows.
 #define PCE_WOSD_STEP(J_)                                                                                              \
   {                                                                                                                    \
     __syncthreads();                                                                                                   \
     PCE_WOSD_PUT(slot ^ 1)                                                                                             \
-    PCE_WOSD_ISSUE((J_ + 2) % 3)                                                                                       \
+    if constexpr (RING == 3) PCE_WOSD_ISSUE((J_ + 2) % RING)                                                           \
+    if (kc[J_] != now) {                                                                                               \
+      _Pragma("unroll") for (int nb = 0; nb < NB; ++nb) _Pragma("unroll") for (int i = 0; i < 16; ++i) {               \
+        sum[nb][i] += acc[nb][i];                                                                                      \
+        acc[nb][i] = 0.f;                                                                                              \
+      }                                                                                                                \
+      now = kc[J_];                                                                                                    \
+    }                                                                                                                  \
     if ((u >> kk[J_]) & 1u) {                                                                                          \
       _Pragma("unroll") for (int s = 0; s < KS; ++s)                                                                   \
         _Pragma("unroll") for (int nb = 0; nb < NB; ++nb)                                                              \
           acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(Wl[slot * FR + (2 * s + g) * (NB * 32) + nb * 32 + l32],    \
                                                            __builtin_bit_cast(half8, af[J_][s]), acc[nb], 0, 0, 0);    \
     }                                                                                                                  \
+    if constexpr (RING == 2) PCE_WOSD_ISSUE(J_)                                                                        \
     slot ^= 1;                                                                                                         \
   }
-  for (int t = 0; t < steps; t += 3) {
+  for (int t = 0; t < steps; t += RING) {
     PCE_WOSD_STEP(0)
     PCE_WOSD_STEP(1)
-    PCE_WOSD_STEP(2)
+    if constexpr (RING == 3) PCE_WOSD_STEP(2 % RING)
   }
 #undef PCE_WOSD_STEP
 #undef PCE_WOSD_PUT
 #undef PCE_WOSD_ISSUE
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[nb][i] += sum[nb][i];
   __syncthreads();   // weights and indices have been read: the space becomes the output staging area
   half8 *const region = lds + wave * WaveLds<NB>::PIECES;
   float V[NB][2][8];
@@ -3299,21 +3331,25 @@ extern "C" int pce_conv_fwd_oso(const void *in, const void *w, const void *wp, v
       n_nonzero - n_single <= PCE_ORDER_SREC_ROWS(n_out) && 8 * (n_nonzero - n_single) <= n_out &&
       os2_workgroups(n_out, n_nonzero, n_single, n_heavy, nb) <= 4ll * cu_count() && stage_on(12))
     return launch_wave_os2(a, order, (int)mid, n_out, n_nonzero, n_single, n_heavy, nb, ks, s);
-  // More than 32 columns, more than two rounds of that kernel's shared workgroups (four per compute unit at a time, 32 rows
-  // each) and at least a third of the rows in them: the kernel whose wavefronts share the weights.  Times against the other
-  // kernel's at 16 -> 48, 32 -> 64, 48 -> 48, 64 -> 64: 1980 to 2030 shared workgroups with 0.96 of the rows 1.05,
-  // 0.92, 0.87, 0.87, with 0.44 of them 0.99, 0.95, 1.01, 1.02; 2110 with 0.71 1.05, 1.01, 1.00, 1.00; 3340 with
-  // 0.44 0.92, 0.88, 0.91, 0.90; 5490 with 0.36 0.92, 0.89, 0.95, 0.92; 1390 with 0.50 (64 -> 64) 1.03, 1510 with 0.04 1.13.
-  if (mid >= 0 && kv <= WOSD_KV && nb == 2 && heavy_wgs > 8ll * cu_count() && 3 * n_split >= n_out &&
+  // More than 32 columns from 32 channels or more, at least three rounds of that kernel's shared workgroups (four per compute
+  // unit at a time, 32 rows each) and a third of the rows in them: the kernel whose wavefronts share the weights.  Its time in
+  // the other kernel's at 32 -> 64, 48 -> 48, 64 -> 64, by shared workgroups (their share of the rows): 2100 (0.45) 1.05, 1.11,
+  // 1.08; 2110 (0.71) 1.12, 1.21, 1.18; 2440 (0.98) 1.04, 1.08, 1.01; 2620 (0.71) 1.03, 1.10, 1.03; 3190 (0.72) 0.93, 0.99, 0.93;
+  // 3260 (0.98) 0.97, 1.00, 0.93; 3790 (0.45) 0.97, 0.94, 0.92; 4080 (0.98) 0.90, 0.91, 0.83; 6060 (0.44) 0.94, 0.93, 0.87; 6850 (0.98)
+  // 1.00, 1.00, 0.88; 24 400 (0.96) 0.87, 0.83, 0.69.  Its second round of workgroups should not be nearly empty where a step is
+  // short: 4885 (0.98; 1245 tiles of 128 rows) 1.05, 1.07, 0.97.
+  const long long heavy_tiles = pce_div_up(n_split, 128), tiles = heavy_tiles + pce_div_up(n_main, 128);
+  if (mid >= 0 && kv <= WOSD_KV && nb == 2 && ks >= 2 && heavy_wgs > 12ll * cu_count() && 3 * n_split >= n_out &&
+      (ks > 3 || tiles <= 4ll * cu_count() || tiles > 6ll * cu_count()) &&
       n_in * (int64_t)a.lda * 2 < (int64_t)WOSD_MISSING - 256 && n_out * kv * 4 < (int64_t)WOSD_MISSING) {
-    const unsigned tiles = (unsigned)pce_div_up(n_out, 128);
 #define PCE_WOSD_CASE(NB_, KS_)                                                                                        \
   if (nb == NB_ && ks == KS_) {                                                                                        \
-    hipLaunchKernelGGL((wave_osd_kernel<NB_, KS_>), dim3(tiles), dim3(256), 0, s, a, perm, rmask, (int)mid, (int)kv);  \
+    hipLaunchKernelGGL((wave_osd_kernel<NB_, KS_>), dim3((unsigned)tiles), dim3(256), 0, s, a, perm, rmask, (int)mid, (int)kv,   \
+                       n_main, (int)heavy_tiles);                                                                      \
     PCE_LAUNCH_CHECK("wave_osd");                                                                                      \
     return PCE_OK;                                                                                                     \
   }
-    PCE_WOSD_CASE(2, 1) PCE_WOSD_CASE(2, 2) PCE_WOSD_CASE(2, 3) PCE_WOSD_CASE(2, 4)
+    PCE_WOSD_CASE(2, 2) PCE_WOSD_CASE(2, 3) PCE_WOSD_CASE(2, 4)
 #undef PCE_WOSD_CASE
   }
 #define PCE_WOS_CASE(NB_, KS_)                                                                              \
