@@ -904,14 +904,6 @@ class _BlocksLead(int):
 BLOCKS_LEAD = _BlocksLead(DATAFLOW_OS)
 
 
-class _RowsLead(int):
-    """``DATAFLOW_OSO`` as the selector's answer for a layer that the dense tiles can take as well: ``conv_forward`` takes
-    those where a pointer is not 16-byte aligned, which the ordered rows refuse."""
-
-
-ROWS_LEAD = _RowsLead(DATAFLOW_OSO)
-
-
 def select_dataflow(km: KernelMap, c_in: int, c_out: int, dtype: torch.dtype, transposed: bool = False, blocks: bool = True) -> int:
     lib = _lib.load()
     n_in, n_out = (km.n_out, km.n_in) if transposed else (km.n_in, km.n_out)
@@ -920,8 +912,6 @@ def select_dataflow(km: KernelMap, c_in: int, c_out: int, dtype: torch.dtype, tr
                 PCE_F16 if dtype == torch.float16 else PCE_F32)
     if df == DATAFLOW_OSB:
         return BLOCKS_LEAD
-    if df == DATAFLOW_OSO and dtype == torch.float16 and km.subm and c_out > 32 and n_out >= 1 << 16 and km.M > 6 * n_out:
-        return ROWS_LEAD
     if not km.has_pairs and df not in (DATAFLOW_OSO, DATAFLOW_OS):
         # a map built without pair lists (its layers were expected to read the neighbour table only): rather than
         # build them now, the layer takes the table-reading dataflow that is closest (a band of densities where the
@@ -1131,8 +1121,6 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
     deep levels of a small scan, and a run that is continued should go on as it began."""
     if not feats.is_cuda:
         _require_cuda(feats, "feats")
-    if dataflow is ROWS_LEAD and any(t is not None and t.data_ptr() % 16 for t in (feats, out, bias, residual)):
-        dataflow = DATAFLOW_OS
     if route_single_pairs and weight.dim() == 3:
         # the usual call: its map's arrays are laid out once, the rest is native
         shape, dtype = weight.shape, feats.dtype

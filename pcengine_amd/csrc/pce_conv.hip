@@ -4483,14 +4483,10 @@ extern "C" int pce_select_dataflow(int64_t n_in, int64_t n_out, int64_t n_pairs,
   if (oso && subm && dtype == PCE_F32 && rho <= (c_in <= 16 ? 6.0 : 2.0)) return PCE_DATAFLOW_OSO;
   // (a cloud of fewer than two 128-row tiles per compute unit -- 256 of them -- leaves the dense tiles' launch short
   // of workgroups: 24 k rows at 9.2 pairs per row, 48 -> 48 channels: ordered rows 17 us, deferred scatter 21, tiles 28)
-  // (more than 32 columns, which the ordered rows take 128 at a time with shared weights from eight groups of 32 rows with two
-  // neighbours per compute unit on -- nearly all rows have two at these densities, hence the ninth: to twelve pairs per row on
-  // up to 0.26 M rows 0.62-0.97 of the faster of the other two -- 16 -> 40 .. 64 -> 64 at 6.5, 9.3 and 11.7 on random
-  // clouds of 78 k to 214 k rows, at 8.7 on a level of rooms of 276 k; on random clouds of 0.6 M rows at 7 to 12
-  // 0.80-1.34, most of it above 1; at 14 on 0.2 M 0.85-1.06)
-  const bool shared = c_out > 32 && n_out >= 9 * 256 * 32 && n_out < (1 << 18);
-  if (oso && subm && dtype == PCE_F16 && os_widths(c_in, c_out) && rho <= (n_out < 2 * 256 * 128 || shared ? 12.0 : 6.0))
-    return PCE_DATAFLOW_OSO;
+  // (beyond those rows the tiles lead on random clouds of 100 to 150 k rows and of 0.2 M and more: 48 -> 48 on 105 k of 7.7 pairs
+  // 41 us and 43 ordered, on 146 k of 9.9 46 and 59, on 211 k of 10.1 76 and 87; between, where the tiles' second round begins, the
+  // ordered rows do: on 172 k of 10.0 71 and 67; on 276 k of indoor scenes at 8.7 78 and 64)
+  if (oso && subm && dtype == PCE_F16 && os_widths(c_in, c_out) && rho <= (n_out < 2 * 256 * 128 ? 12.0 : 6.0)) return PCE_DATAFLOW_OSO;
   // the K-stepped form of the same kernel (wave_osw_kernel): a wavefront walks c_in / 16 K steps per offset of its
   // rows' union, so the density up to which it leads falls with the input width.  Measured on the levels of a
   // 100 k-voxel LiDAR pyramid against the faster of deferred scatter and the dense tiles: 64 -> 96, 96 -> 96, 64 -> 128

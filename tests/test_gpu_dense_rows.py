@@ -98,28 +98,18 @@ def test_kernels_of_fewer_offsets(ks, density):
     assert ((out.double() - want).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("rows,pairs,c_out,ordered", [(65535, 12.0, 32, True), (65536, 12.0, 40, False), (73727, 12.0, 40, False),
-                                                      (73728, 12.0, 32, False), (73728, 12.0, 40, True),
-                                                      ((1 << 18) - 1, 12.0, 64, True), (1 << 18, 12.0, 64, False),
-                                                      (100000, 12.1, 64, False), (1 << 18, 6.0, 64, True)])
-def test_selection_by_rows_pairs_and_columns(rows, pairs, c_out, ordered):
-    n_pairs = int(rows * pairs)
-    got = backend._lib.load().pce_select_dataflow(rows, rows, n_pairs, 48, c_out, 27, 13, 0, backend.PCE_F16)
-    assert got == (backend.DATAFLOW_OSO if ordered else backend.DATAFLOW_OS)
-
-
-def test_pointers_the_ordered_rows_refuse():
-    """A layer of the selector's ordered range with an odd pointer takes the dense tiles."""
-    km = _map(110003, 0.46, seed=3)
+def test_odd_pointers_of_a_selected_layer():
+    """110 k rows at seven pairs or more: the selector's answer takes features, bias and output on any boundary."""
+    km = gpu_map(synth.random_cloud(seed=3, n=110003, extent=62), (3, 3, 3), batchsize=1)
     rows = km.n_out
-    assert rows >= 73728 and 6 < km.M / rows <= 12
-    df = backend.select_dataflow(km, 48, 40, torch.float16)
-    assert df == backend.DATAFLOW_OSO and df is backend.ROWS_LEAD
+    assert rows > 73728 and 6 < km.M / rows <= 12
+    df = backend._lib.load().pce_select_dataflow(rows, rows, km.M, 48, 40, 27, 13, 0, backend.PCE_F16)
+    assert df == backend.select_dataflow(km, 48, 40, torch.float16) == backend.DATAFLOW_OS
     gen = torch.Generator(device=DEV).manual_seed(1)
     x = torch.randn((rows, 48), generator=gen, device=DEV).half()
     w = (torch.randn((27, 48, 40), generator=gen, device=DEV) * 0.1).half()
     bias = torch.randn(40, generator=gen, device=DEV).half()
-    want = backend.conv_forward(x, w, km, backend.DATAFLOW_OS, bias=bias)
+    want = backend.conv_forward(x, w, km, df, bias=bias)
 
     def odd(t):
         return torch.empty(t.numel() + 4, dtype=t.dtype, device=DEV)[4:].view(t.shape).copy_(t)

@@ -109,6 +109,9 @@ def test_selector_on_measured_layers():
         (65807, 65807, 586656, 64, 128, 27, OSO),      # 56 vs 63 us for the dense tiles
         (25916, 25916, 506646, 64, 128, 27, OS),       # rho = 19.5: 33 vs 37 us
     ]
+    # random clouds beyond six pairs per row: the tiles, whose second round begins at 131 k rows, are ahead of the ordered rows
+    cases += [(n, n, int(n * rho), ci, co, 27, OS) for n, rho in ((104643, 7.7), (125524, 10.1), (146087, 9.9), (211474, 10.1))
+              for ci, co in ((48, 48), (48, 64), (64, 64))]
     mid_of = lambda kv: kv // 2 if kv == 27 else -1
     for n_in, n_out, pairs, ci, co, kv, want in cases:
         assert lib.pce_select_dataflow(n_in, n_out, pairs, ci, co, kv, mid_of(kv), 0, _lib.PCE_F16) == want, (n_in, n_out, ci, co, kv)
