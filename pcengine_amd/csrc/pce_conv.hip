@@ -3613,6 +3613,9 @@ __global__ void __launch_bounds__(BLK == 256 ? 512 : 256, BLK == 256 ? 1 : 2) wg
 // of 128 pairs, so that waiting for all but the youngest eight operations means that its copies of this stage are there.
 // The 16-byte pieces of a row are exchanged by its pair index (piece ^ (pair & 3) * 4): the rows that one read addresses then
 // lie in different banks.
+// Sums are added up in chains of at most `fold` tiles, then to the sums of the chains before them: one workgroup per CU walks up
+// to four times the tiles that a workgroup of wgrad_f16_kernel walks, and as one chain (FP32 additions of 128 pairs a tile) its relative
+// error was twice as large (256 -> 256 on 61 k rows of 7 pairs 5.3e-7 of the result where wgrad_f16_kernel has 2.8e-7; 2.1e-7 this way, for 1 % of the time).
 // Bound by the LDS: a stage writes 16 KB and reads 32 for 256 clocks of matrix products of each wavefront.  wgrad_f16_kernel -> this
 // one: 256 -> 256 on 27 k rows of 19 pairs 222 us -> 117 (627 TFLOP/s), on 66 k of 9 241 -> 127, 384 -> 256 334 -> 182, 128 -> 128 on 66 k
 // 85 -> 65, on 89 k of 3 55 -> 38, 96 -> 96 on 99 k of 0.1 33 -> 25 (the sums' way to memory).
@@ -3639,7 +3642,7 @@ __global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__rest
                                                             unsigned in_bytes, unsigned out_bytes, int c_in, int c_out, int kv, int mid,
                                                             const int *__restrict__ imap, const int *__restrict__ omap,
                                                             const int *__restrict__ kpos, const int *__restrict__ qkpos,
-                                                            long long pair_tiles, long long tiles, int run, int ci_blocks,
+                                                            long long pair_tiles, long long tiles, int run, int fold, int ci_blocks,
                                                             int co_blocks, float *__restrict__ gw) {
   constexpr int OP = WP_PAIRS * 256, STAGE = 2 * OP;   // bytes of one operand's pairs, and of both
   __shared__ __attribute__((aligned(1024))) char lds[WP_ST * STAGE];
@@ -3655,13 +3658,24 @@ __global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__rest
   if (t_begin >= t_end) return;
   const int n_tiles = (int)(t_end - t_begin);
 
-  f32x16 acc[2][2];
+  f32x16 acc[2][2], sum[2][2];   // of the chain, and of the chains of this offset before it
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = sum[i][j][e] = 0.f;
+  auto end_chain = [&] {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          sum[i][j][e] += acc[i][j][e];
+          acc[i][j][e] = 0.f;
+        }
+  };
   auto flush = [&](int widx) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -3672,7 +3686,7 @@ __global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__rest
         for (int i = 0; i < 2; ++i)
 #pragma unroll
           for (int e = 0; e < 16; ++e)   // (eight input channels at a time are there or not)
-            if (ci0 + wr * 64 + i * 32 + e / 4 * 8 < c_in) unsafeAtomicAdd(dst + (long long)(i * 32 + e / 4 * 8 + e % 4) * c_out, acc[i][j][e]);
+            if (ci0 + wr * 64 + i * 32 + e / 4 * 8 < c_in) unsafeAtomicAdd(dst + (long long)(i * 32 + e / 4 * 8 + e % 4) * c_out, sum[i][j][e]);
       }
     }
 #pragma unroll
@@ -3680,7 +3694,7 @@ __global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__rest
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+        for (int e = 0; e < 16; ++e) sum[i][j][e] = 0.f;
   };
 
   // a tile: its offset (-1: none), its first pair or row, how many, and whether rows pair with themselves
@@ -3779,14 +3793,19 @@ __global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__rest
   fetch_rows(next, 1);
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
   for (int st = 0; st < 3; ++st) issue(d, 0, st, st);
-  int cur = -1;
+  int cur = -1, chain = 0;
   for (int t = 0; t < n_tiles; ++t) {
     WP_LANDED();
     issue(d, t & 1, 3, 3);
-    if (d.w != cur) {
-      if (cur >= 0) flush(cur);
-      cur = d.w;
+    if (d.w != cur || chain == fold) {
+      end_chain();
+      chain = 0;
+      if (d.w != cur) {
+        if (cur >= 0) flush(cur);
+        cur = d.w;
+      }
     }
+    ++chain;
     multiply(0);
     WP_LANDED();   // (every wavefront has issued this tile's last copies: its row indices are not read any more)
     d = next;
@@ -3802,6 +3821,7 @@ __global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__rest
     multiply(3);
   }
 #undef WP_LANDED
+  end_chain();
   if (cur >= 0) flush(cur);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the copies behind the last stage end before the LDS is given back
 }
@@ -3946,6 +3966,7 @@ extern "C" int pce_conv_wgrad(const void *in, const void *gout, int32_t dtype, i
   const int64_t in_bytes = n_in * c_in * 2, out_bytes = n_out * c_out * 2;
   const bool pipe = dtype == PCE_F16 && blk == 128 && c_in % 8 == 0 && c_out % 8 == 0 && aligned16(in) && aligned16(gout) &&
                     in_bytes < WP_MAX_BYTES && out_bytes < WP_MAX_BYTES;
+  const int fold = (int)(run < 1 ? 1 : (run > 8 ? 8 : run));   // wgrad_pipe_kernel: chains no longer than that run, nor than eight tiles
   if (pipe) {
     // one workgroup per compute unit, as many runs on every XCD (256 -> 256 on 27 k rows of 19 pairs 117 us with 256 workgroups,
     // 122 with 512, 149 with 2048; 96 -> 96 on 97 k rows of 0.8 25 with 256, 39 with 512)
@@ -3966,7 +3987,7 @@ extern "C" int pce_conv_wgrad(const void *in, const void *gout, int32_t dtype, i
   if (pipe)
     hipLaunchKernelGGL(wgrad_pipe_kernel, dim3((unsigned)blocks), dim3(256), 0, s, (const half_t *)in, (const half_t *)gout, (long long)n_out,
                        (unsigned)in_bytes, (unsigned)out_bytes, c_in, c_out, kv, mid, imap, omap, kpos, qkpos, pair_tiles, tiles, (int)run,
-                       ci_blocks, co_blocks, gw);
+                       fold, ci_blocks, co_blocks, gw);
   else if (dtype == PCE_F16 && blk == 128)
     PCE_WGRAD16(128);
   else if (dtype == PCE_F16)

@@ -34,3 +34,19 @@ def test_kernel_gradient(n, extent, ks, stride, transposed, c_in, c_out):
     assert ((got - want).norm() / want.norm()).item() <= tol
     empty = want.abs().sum(dim=(1, 2)) == 0
     assert bool((got[empty] == 0).all())
+
+
+@pytest.mark.parametrize("n,extent,c_in,c_out", [(30000, 35, 256, 256), (72000, 59, 256, 256), (72000, 59, 384, 256), (72000, 59, 136, 136)])
+def test_long_runs_are_added_up_in_chains(n, extent, c_in, c_out):
+    km = gpu_map(synth.random_cloud(seed=7, n=n, extent=extent), (3, 3, 3))
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn((km.n_in, c_in), generator=gen, device=DEV).half()
+    g = torch.randn((km.n_out, c_out), generator=gen, device=DEV).half()
+    got = backend.conv_wgrad(x, g, km).double()
+    kpos = km.kpos.cpu().tolist()
+    want = torch.stack([x.double().t() @ g.double() if k == 13 else
+                        x[km.imap[kpos[k]:kpos[k + 1]].long()].double().t() @ g[km.omap[kpos[k]:kpos[k + 1]].long()].double() for k in range(27)])
+    # T additions in a row, each off by up to half a unit of a partial sum whose variance grows evenly: 2^-24 sqrt(T / 6) of the
+    # result.  Chains of 8 tiles of 128 pairs, two roundings for 16 of them; then at most 32 chains a run, 8 runs an offset
+    tol = 2 ** -24 * np.sqrt((8 * 128 / 8 + 32 + 8) / 6)
+    assert ((got - want).norm() / want.norm()).item() <= tol
