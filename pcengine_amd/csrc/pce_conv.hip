@@ -571,6 +571,9 @@ __global__ void __launch_bounds__(256, ((TMODE >= 0 && sizeof(T) == 2 && NB <= 2
 #define SMALL_PLANE (32 * 4 + 4)
 #define SMALL_MAX_KV 32
 #define SMALL_MISSING 0xF0000000u   // bytes that rows and weights stay below
+// GROUPS: the sums of every group of offsets (a.groups of them, as even as the shares are) are added up from zero, and the groups'
+// sums in their order; for layers whose offsets may be shared out (os_groups).
+template <bool GROUPS>
 __global__ void __launch_bounds__(256) small_f32_kernel(TileArgs a) {
   __shared__ __attribute__((aligned(16))) float As[SMALL_AHEAD][8 * SMALL_PLANE], Bs[SMALL_AHEAD][8 * SMALL_PLANE];
   __shared__ int idx[SMALL_MAX_KV][32];
@@ -613,6 +616,11 @@ __global__ void __launch_bounds__(256) small_f32_kernel(TileArgs a) {
     out += (long long)p * a.n_rows * a.c_out;
   }
   const int chunks = (a.c_in + SMALL_KC - 1) / SMALL_KC, steps = __popc(rest) * chunks;
+  // the step that is multiplied: its chunk, the offsets from its own on, and those that begin a group
+  int mc = -2;   // (the first product is of zeros, the one behind it the first step's)
+  unsigned mrest = rest, begins = 0;
+  if (GROUPS)
+    for (int p = 0; p < a.groups; ++p) begins |= 1u << (kv * p / a.groups);
   // A thread's pieces of a chunk: four channels of a row, four columns of a channel's weights.  Through buffer loads, which
   // read zeros beyond the range: where a row is missing and behind the last channel and column.  (With selected addresses and
   // values a step is 110 instructions of 4 clocks for 256 clocks of products: 256 -> 256 on 603 rows 85 us, 60 so.)
@@ -642,7 +650,7 @@ __global__ void __launch_bounds__(256) small_f32_kernel(TileArgs a) {
   };
 #pragma unroll
   for (int i = 0; i < SMALL_AHEAD; ++i) request(ra[i], rb[i]);
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f}, sum = acc;
   // channel 8 s + kk of a chunk: instruction 2 s + (kk & 2) / 2, lane group 2 (kk & 1) + kk / 4
   const int at_a = ((tq / 4 * 4 + (tq & 1)) * SMALL_PLANE) + tr * 4 + (tq / 2 & 1) * 2;
   const int kk = tr & 7, at_b = (tr / 16 * 4 + 2 * (kk & 1) + kk / 4) * SMALL_PLANE + tq * 16 + (tr / 8 & 1) * 2 + (kk & 2) / 2;
@@ -660,6 +668,17 @@ __global__ void __launch_bounds__(256) small_f32_kernel(TileArgs a) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(y[h][j], x[h][j], acc, 0, 0, 0);
   };
+  auto next_step = [&] {   // ends the group where the step's offset begins another one
+    if (!GROUPS || ++mc < chunks) return;
+    mc = 0;
+    const unsigned was = mrest & (0u - mrest);
+    mrest &= mrest - 1;
+    const unsigned is = mrest & (0u - mrest);   // (0 behind the last one)
+    if (begins & (is - 1 | is) & ~(was - 1 | was)) {
+      sum += acc;
+      acc = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+  };
   // a step reads its chunk from LDS while the one before is multiplied and the one after is written; the steps behind the last
   // one multiply zeros
   put(0);
@@ -673,6 +692,7 @@ __global__ void __launch_bounds__(256) small_f32_kernel(TileArgs a) {
         nx[h] = *reinterpret_cast<const f32x4 *>(As[i] + (h * 4 + g) * SMALL_PLANE + (wr * 16 + r16) * 4);
         ny[h] = *reinterpret_cast<const f32x4 *>(Bs[i] + (h * 4 + g) * SMALL_PLANE + (wc * 16 + r16) * 4);
       }
+      next_step();
       multiply();
       put((i + 1) % SMALL_AHEAD);
 #pragma unroll
@@ -682,7 +702,9 @@ __global__ void __launch_bounds__(256) small_f32_kernel(TileArgs a) {
       }
     }
   }
+  next_step();
   multiply();
+  if (GROUPS) acc += sum;
   // lane: columns 4 g .. of its row
   const long long row = tile * 32 + wr * 16 + r16;
   const int col = n0 + wc * 16 + 4 * g;
@@ -1309,10 +1331,16 @@ static bool small_f32_ok(const TileArgs &a) {
   if (a.epi != EPI_ROWS || a.act_alone_only || (a.mode != MODE_DENSE && (a.mode != MODE_OS || a.kv > SMALL_MAX_KV))) return false;
   const long long rows = a.mode == MODE_OS ? a.a_rows : a.n_rows;
   if (rows <= 0 || rows * a.lda * 4 >= (long long)SMALL_MISSING || (long long)a.kv * a.c_in * a.c_out * 4 >= (1ll << 27)) return false;
-  if (a.parts > 1) return true;
+  if (a.parts > 1 || a.groups > 1) return a.groups > 1;   // (os_parts)
   const long long wgs = pce_div_up(a.n_rows, 32) * (a.n_pad / 32);
   if (a.mode == MODE_OS) return wgs <= (8 * pce_div_up(a.c_in, SMALL_KC) * SMALL_KC > 9 * a.c_in ? 1280 : 5120);
   return a.c_in >= 64 && wgs <= (a.c_in >= 256 ? 2560 : a.c_in >= 96 ? 1280 : 640);
+}
+
+template <typename T>
+static bool fast_ok(const TileArgs &a) {   // 16-byte accesses to everything, packed weights in fp16
+  return a.a_vec && a.o_vec && (sizeof(T) == 2 ? a.Wp != nullptr : a.w_vec != 0) && (a.epi != EPI_ROWS_CSR || a.b_vec) && aligned16(a.bias) &&
+         aligned16(a.res);
 }
 
 template <typename T>
@@ -1328,12 +1356,15 @@ static int launch_tile(const TileArgs &a, long long tiles, hipStream_t s) {
   // measured: 154 instead of 177 us and 88 instead of 96 us on 406 (tile, slab) items (26 k rows, 256 output
   // channels), 66 instead of 62 us and 113 instead of 111 us on 515 (66 k rows, 128 output channels)
   if (stage_on(9) && os_pipe_ok(a, sizeof(T)) && tiles * ((a.c_out + 127) / 128) <= 448) return launch_os_pipe(a, tiles, s);
-  bool fast = a.a_vec && a.o_vec && (sizeof(T) == 2 ? a.Wp != nullptr : a.w_vec != 0) &&
-              (a.epi != EPI_ROWS_CSR || a.b_vec) && aligned16(a.bias) && aligned16(a.res);
+  const bool fast = fast_ok<T>(a);
   if (fast && sizeof(T) == 4 && small_f32_ok(a)) {
     TileArgs b = a;
     const unsigned grid = xcd_grid(&b, pce_div_up(a.n_rows, 32), a.n_pad / 32);
-    hipLaunchKernelGGL(small_f32_kernel, dim3(grid, a.parts > 1 ? a.parts : 1), dim3(256), 0, s, b);
+    const dim3 wgs(grid, a.parts > 1 ? a.parts : 1);
+    if (a.groups > 1 && a.groups != a.parts)
+      hipLaunchKernelGGL(small_f32_kernel<true>, wgs, dim3(256), 0, s, b);
+    else
+      hipLaunchKernelGGL(small_f32_kernel<false>, wgs, dim3(256), 0, s, b);
     PCE_LAUNCH_CHECK("small_f32");
     return PCE_OK;
   }
@@ -2189,15 +2220,32 @@ static int os_impl(const void *in, const void *w, const void *wp, void *out, int
 }
 
 // Output-stationary fp32 layers of few rows: a tile walks its offsets one after the other (2.2 us each at 256 channels,
-// small_f32_kernel), so a few tiles take as long as many.  The offsets are shared out among `parts` workgroups per tile of 32
-// rows by 32 columns; every share stores its fp32 sums and os_parts_kernel adds them up in the order of the offsets and finishes
-// the rows.  As many shares as make 1536, 768 or 512 workgroups, the fewer the shorter a share is (the partial sums, at most
-// 6 MB, and the second launch then cost more than it gives): 256 -> 256 on 603 rows 60 us -> 36, on 2.2 k 116 -> 97; 64 -> 64 on 603
-// 19.5 -> 13, on 5 k 27 -> 24; 32 -> 32 on 2.2 k 12.4 -> 11.5.  Below six offsets of 128 channels nothing is gained.
-static int os_parts(int dtype, long long n_out, int c_in, int c_out, int kv) {
+// small_f32_kernel; 10 us, tile_gemm_kernel), so a few tiles take as long as many.  The offsets are shared out among
+// workgroups; every share stores its fp32 sums and os_parts_kernel adds them up in the order of the offsets and finishes the
+// rows.  Below six offsets of 128 channels nothing is gained.
+// The groups of offsets whose sums are added up from zero: as many as make two workgroups of tile_gemm_kernel per compute unit,
+// whose shares they are.  They decide the sums' error, and the workspace holds one sum of each (at most 512 tiles of 128 x 32, 8 MB).
+static int os_groups(int dtype, long long n_out, int c_in, int c_out, int kv) {
   if (dtype != PCE_F32 || n_out <= 0 || (long long)kv * c_in < 768) return 1;
-  const long long parts = (c_in >= 128 ? 1536 : c_in >= 64 ? 768 : 512) / (pce_div_up(n_out, 32) * ((c_out + 31) / 32));
-  return parts < 2 ? 1 : parts < kv ? (int)parts : kv;
+  const long long tiles = pce_div_up(n_out, 128);
+  const int nb = narrow_blocks(tiles, c_out);
+  const long long groups = OS_WORKGROUPS / (tiles * (((c_out + 31) / 32 + nb - 1) / nb));
+  return groups < 2 ? 1 : groups < kv ? (int)groups : kv;
+}
+
+// The shares of small_f32_kernel, 0 where tile_gemm_kernel with a share per group is faster.  Up to five groups and 64 channels it
+// takes several groups one behind the other: as many shares as make 768 or 512 workgroups, the fewer the shorter a share is
+// (the partial sums and the second launch then cost more than it gives).  That kernel -> this one: 64 -> 64 on 12.1 k rows (2 groups)
+// 51 us -> 38, on 8.2 k (4) 33 -> 30, on 6.1 k (5) 29 -> 27, 32 -> 64 on 12.1 k (2) 34 -> 23, on 6.1 k (5) 21 -> 19; but 64 -> 64 on 4.4 k
+// (7) 24 -> 26, 32 -> 32 on 1.9 k (27) 12.2 -> 13.7.  Wider ones with a share per group: 96 -> 96 on 8.2 k (2) 70 -> 53, on 4.4 k (5) 44 -> 35,
+// on 3.1 k (7) 29 -> 30, 80 -> 80 on 6.1 k (3) 44 -> 43, 128 -> 128 on 1.9 k (8) 32 -> 35, 256 -> 256 on 600 rows (12) 43 -> 35, 256 -> 96 (27)
+// 21 -> 21.  Where the last of two chunks is mostly padding: 40 -> 40 on 14.6 k (2) 41 -> 46, on 8.2 k (4) 25 -> 30.
+static int os_parts(int groups, long long n_out, int c_in, int c_out) {
+  if (groups > 5) return c_in >= 256 ? groups : 0;
+  if (c_in > 64) return groups;
+  if (c_in % SMALL_KC) return 0;
+  const long long parts = (c_in >= 64 ? 768 : 512) / (pce_div_up(n_out, 32) * ((c_out + 31) / 32));
+  return parts < 2 ? 1 : parts < groups ? (int)parts : groups;
 }
 
 template <int VEC>
@@ -2223,8 +2271,8 @@ __global__ void __launch_bounds__(256) os_parts_kernel(const float *__restrict__
 }
 
 extern "C" int64_t pce_conv_os_workspace_bytes(int32_t dtype, int64_t n_out, int32_t c_in, int32_t c_out, int32_t kv) {
-  const int parts = c_in > 0 && c_out > 0 && kv > 0 ? os_parts(dtype, n_out, c_in, c_out, kv) : 1;
-  return parts > 1 ? (int64_t)parts * n_out * c_out * 4 : 0;
+  const int groups = c_in > 0 && c_out > 0 && kv > 0 ? os_groups(dtype, n_out, c_in, c_out, kv) : 1;
+  return groups > 1 ? (int64_t)groups * n_out * c_out * 4 : 0;
 }
 
 extern "C" int pce_conv_fwd_os_parts(const void *in, const void *w, void *out, int32_t dtype, int64_t n_in, int64_t n_out,
@@ -2241,13 +2289,29 @@ extern "C" int pce_conv_fwd_os_parts(const void *in, const void *w, void *out, i
   if ((rc = read_epilogue("pce_conv_fwd_os_parts", epilogue, out, &e, c_in, c_out))) return rc;
   hipStream_t s = (hipStream_t)stream;
   TileArgs a = base_args<float>(in, w, nullptr, kv, c_in, c_out, e.lda);
-  set_out<float>(&a, ws, false);
   a.nbr = nbr;
   a.n_rows = n_out;
   a.a_rows = n_in;
   a.mode = MODE_OS;
   a.epi = EPI_ROWS;
-  a.parts = os_parts(dtype, n_out, c_in, c_out, kv);
+  const int groups = os_groups(dtype, n_out, c_in, c_out, kv), shares = os_parts(groups, n_out, c_in, c_out);
+  if (shares == 1) {   // all groups by one workgroup, which finishes the rows
+    TileArgs whole = a;
+    whole.groups = groups;
+    set_out<float>(&whole, out, false, n_out, e.ldo);
+    set_epi(&whole, e);
+    if (fast_ok<float>(whole) && small_f32_ok(whole)) return launch_tile<float>(whole, pce_div_up(n_out, 128), s);
+  }
+  set_out<float>(&a, ws, false);
+  a.parts = groups;
+  if (shares > 1) {
+    a.parts = shares;
+    a.groups = groups;
+    if (!fast_ok<float>(a) || !small_f32_ok(a)) {
+      a.parts = groups;
+      a.groups = 0;
+    }
+  }
   if ((rc = launch_tile<float>(a, pce_div_up(n_out, 128), s))) return rc;
   const int ldo = e.ldo > 0 ? e.ldo : c_out;
   const bool vec = c_out % 4 == 0 && ldo % 4 == 0 && aligned16(out) && aligned16(e.bias) && aligned16(e.res);

@@ -59,6 +59,7 @@ struct TileArgs {
   long long a_rows;  // MODE_OS: rows of A (0: not stated)
   long long items;   // (tile, column slab) work items of the launch
   int slabs;         // column slabs per tile
+  int groups;        // MODE_OS, small_f32_kernel (not tile_gemm_kernel): groups of offsets whose sums are added up from zero (0, 1: one)
   int parts;         // MODE_OS: shares of the offsets, blockIdx.y; the sums of share p at out + p * n_rows * c_out (0, 1: one)
   int kv, c_in, c_out;
   int lda, ldo;      // elements between consecutive rows of A and of `out` (rows of buf, res and out_alt are dense)

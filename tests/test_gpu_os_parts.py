@@ -86,3 +86,22 @@ def test_entry_point_checks_its_workspace():
     assert need == 27 * 100 * 256 * 4
     for ws, size in ((None, need), (8, need), (16, need - 1)):
         assert lib.pce_conv_fwd_os_parts(16, 16, 16, _lib.PCE_F32, 100, 100, 256, 256, 27, 16, ws, size, None, None) == _lib.PCE_EINVAL
+
+
+@pytest.mark.parametrize("side,c_in,c_out,groups", [(12, 64, 128, 9), (16, 32, 64, 8), (16, 64, 64, 8), (16, 96, 96, 5), (16, 256, 96, 5), (20, 32, 32, 8),
+                                                    (20, 40, 72, 2), (23, 64, 64, 2), (18, 64, 64, 5)])
+def test_error_of_groups_of_offsets(side, c_in, c_out, groups):
+    """However few workgroups the offsets are shared out to, they are added up in as many groups as the workspace holds sums."""
+    coords = np.stack([0 * np.arange(side ** 3), *np.unravel_index(np.arange(side ** 3), (side,) * 3)], axis=1).astype(np.int32)
+    km = gpu_map(coords, (3, 3, 3), batchsize=1)
+    n = km.n_out
+    assert _lib.load().pce_conv_os_workspace_bytes(_lib.PCE_F32, n, c_in, c_out, 27) == groups * n * c_out * 4
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    f = torch.randn((n, c_in), generator=gen, device=DEV)
+    w = torch.randn((27, c_in, c_out), generator=gen, device=DEV) * 0.1
+    want = reference(f, w, km, False)
+    # T additions in a row, each off by up to half a unit of a partial sum whose variance grows evenly: 2^-24 sqrt(T / 6)
+    tol = 2.0 ** -24 * ((-(-27 // groups) * c_in + groups) / 6) ** 0.5
+    for kw in (dict(), dict(bias=torch.zeros(c_out + 1, device=DEV)[1:])):      # (odd pointers: the shares' sums)
+        got = backend.conv_forward(f, w, km, DATAFLOW_OS, **kw)
+        assert ((got.double() - want).norm() / want.norm()).item() <= tol
