@@ -1091,8 +1091,8 @@ def _lay_out(km: KernelMap, dataflow: int, shape, dtype, transposed: bool, split
         imap, omap, ocsr, oslot = (km.omap, km.imap, km.icsr, km.islot) if transposed else (km.imap, km.omap, km.ocsr, km.oslot)
         if km.kpos_host is None or km.qkpos_host is None:
             return ()
-        call = (_HOST_FDS, (n_in, n_out, kv, imap, omap, oslot, km.kpos, km.qkpos, ocsr, route, mid, km.M, km.qsum,
-                            _lib.ctypes.addressof(km.kpos_host), _lib.ctypes.addressof(km.qkpos_host)),
+        call = (_HOST_FDS, (n_in, n_out, kv, imap, omap, oslot, km.kpos, km.qkpos, ocsr, route, mid, km.M, km.qsum, km.kpos_host,
+                            km.qkpos_host),
                 0 if single else max(km.M * c_out, 1), True, kept)
         if route is not None and kept is None:
             return call

@@ -51,6 +51,23 @@ struct View {   // the integers and arrays of a map, as the caller laid them out
   }
 };
 
+// the kv + 1 offsets that a map mirrors on the host, as the array the view holds: read at the call, never kept as an address
+struct HostPos {
+  Py_buffer buffer;
+  bool held = false;
+  const int32_t *read(PyObject *o, int64_t kv) {
+    if (PyObject_GetBuffer(o, &buffer, PyBUF_SIMPLE)) {
+      PyErr_Clear();
+      return nullptr;
+    }
+    held = true;
+    return buffer.len >= (Py_ssize_t)((kv + 1) * sizeof(int32_t)) ? (const int32_t *)buffer.buf : nullptr;
+  }
+  ~HostPos() {
+    if (held) PyBuffer_Release(&buffer);
+  }
+};
+
 // layer(kind, view, feats, weight, packed, bias, residual, out, act, slope, scratch, stream)
 //   -> the output, or None where the general path has to take the call; an int is the library's error code
 PyObject *layer(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
@@ -112,6 +129,10 @@ PyObject *layer(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   const int arrays = kind == KIND_OSO || kind == KIND_OSB ? 2 : kind == KIND_OS ? 1 : kind == KIND_FDS ? 7 : 0;
   for (int i = 0; i < arrays; ++i) m[i] = v.array(3 + i, dev);
   if (v.bad) Py_RETURN_NONE;
+  HostPos kpos, qkpos;
+  const int32_t *kpos_h = nullptr, *qkpos_h = nullptr;
+  if (kind == KIND_FDS && (!(kpos_h = kpos.read(PyTuple_GET_ITEM(args[1], 13), kv)) || !(qkpos_h = qkpos.read(PyTuple_GET_ITEM(args[1], 14), kv))))
+    Py_RETURN_NONE;
   void *stream = PyLong_AsVoidPtr(args[11]);
   if (PyErr_Occurred()) return nullptr;
   const void *x = feats->data_ptr(), *w = weight->data_ptr(), *wp = dt == PCE_F16 ? packed->data_ptr() : nullptr;
@@ -138,10 +159,10 @@ PyObject *layer(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   } else if (kind == KIND_OS) {    // nbr
     rc = ws ? pce_conv_fwd_os_parts(x, w, y, dt, n_in, n_out, ci, co, k, m[0], ws, ws_bytes, e, stream)
             : pce_conv_fwd_os(x, w, wp, y, dt, n_in, n_out, ci, co, k, m[0], e, stream);
-  } else if (kind == KIND_FDS) {   // imap, omap, oslot, kpos, qkpos, ocsr, route | mid, pairs, qsum, addresses of kpos and qkpos on the host
+  } else if (kind == KIND_FDS) {   // imap, omap, oslot, kpos, qkpos, ocsr, route | mid, pairs, qsum, kpos and qkpos on the host
     const int64_t es = dt == PCE_F16 ? 2 : 4;
-    rc = pce_conv_fwd_fds(x, w, wp, y, dt, n_in, n_out, ci, co, k, (int)v.num(10), m[0], m[1], m[2], m[3], m[4], (const int32_t *)v.num(13),
-                          (const int32_t *)v.num(14), m[5], m[6], v.num(11), v.num(12), ws, ws ? ws_bytes / es : 0, e, stream);
+    rc = pce_conv_fwd_fds(x, w, wp, y, dt, n_in, n_out, ci, co, k, (int)v.num(10), m[0], m[1], m[2], m[3], m[4], kpos_h, qkpos_h,
+                          m[5], m[6], v.num(11), v.num(12), ws, ws ? ws_bytes / es : 0, e, stream);
   } else if (dense) {
     rc = pce_conv_fwd_dense(x, w, wp, y, dt, n_in, ci, co, e, stream);
   }
