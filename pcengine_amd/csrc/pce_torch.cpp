@@ -17,6 +17,14 @@ namespace {
 
 enum Kind { KIND_OSO = 0, KIND_OSB = 1, KIND_OS = 2, KIND_FDS = 3, KIND_DENSE = 4 };
 
+// Other Python threads run while a call allocates or launches (both may wait for the device), as they do around a ctypes call.
+struct Unlocked {
+  PyThreadState *state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+  Unlocked(const Unlocked &) = delete;
+  Unlocked() = default;
+};
+
 // a plain tensor on a GPU: not one that stands for another (functorch, fake tensors and other modes)
 const at::Tensor *plain(PyObject *o) {
   if (!THPVariable_CheckExact(o)) return nullptr;
@@ -140,33 +148,37 @@ PyObject *layer(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     const uintptr_t all = (uintptr_t)x | (uintptr_t)wp | (uintptr_t)epi.bias | (uintptr_t)epi.residual | (out ? (uintptr_t)out->data_ptr() : 0);
     if (dt != PCE_F16 || all % 16 || n_in * (epi.ld_in ? epi.ld_in : c_in) * 2 >= 0xF0000000ll) Py_RETURN_NONE;
   }
-  if (!out) {
-    made = at::empty({n_out, c_out}, feats->options());
-    out = &made;
-  }
-  void *y = out->data_ptr();
-  const bool plain_call = !epi.bias && !epi.residual && epi.act == PCE_ACT_NONE && !epi.ld_in && !epi.ld_out;
-  const pce_epilogue_t *e = plain_call ? nullptr : &epi;
+  int64_t num[10] = {};   // the numbers behind n_in, n_out, kv and the arrays
+  for (Py_ssize_t i = 3 + arrays; i < PyTuple_GET_SIZE(args[1]) && i < 3 + arrays + (kind == KIND_FDS ? 3 : 10); ++i) num[i - 3 - arrays] = v.num(i);
+  if (PyErr_Occurred()) return nullptr;
   void *ws = scratch ? scratch->data_ptr() : nullptr;
   const int64_t ws_bytes = scratch ? (int64_t)scratch->nbytes() : 0;
   int rc = PCE_EINVAL;
   const int ci = (int)c_in, co = (int)c_out, k = (int)kv;
-  if (kind == KIND_OSO) {          // nbr, order | mid, heavy, nonzero, single
-    const int64_t counts[3] = {v.num(6), v.num(7), v.num(8)};
-    rc = pce_conv_fwd_oso(x, w, wp, y, dt, n_in, n_out, ci, co, k, (int)v.num(5), m[0], m[1], counts, e, stream);
-  } else if (kind == KIND_OSB) {   // nbr, order | pairs
-    rc = pce_conv_fwd_osb(x, wp, y, dt, n_in, n_out, v.num(5), ci, co, k, m[0], m[1], ws, ws_bytes, e, stream);
-  } else if (kind == KIND_OS) {    // nbr
-    rc = ws ? pce_conv_fwd_os_parts(x, w, y, dt, n_in, n_out, ci, co, k, m[0], ws, ws_bytes, e, stream)
-            : pce_conv_fwd_os(x, w, wp, y, dt, n_in, n_out, ci, co, k, m[0], e, stream);
-  } else if (kind == KIND_FDS) {   // imap, omap, oslot, kpos, qkpos, ocsr, route | mid, pairs, qsum, kpos and qkpos on the host
-    const int64_t es = dt == PCE_F16 ? 2 : 4;
-    rc = pce_conv_fwd_fds(x, w, wp, y, dt, n_in, n_out, ci, co, k, (int)v.num(10), m[0], m[1], m[2], m[3], m[4], kpos_h, qkpos_h,
-                          m[5], m[6], v.num(11), v.num(12), ws, ws ? ws_bytes / es : 0, e, stream);
-  } else if (dense) {
-    rc = pce_conv_fwd_dense(x, w, wp, y, dt, n_in, ci, co, e, stream);
+  {
+    Unlocked unlocked;
+    if (!out) {
+      made = at::empty({n_out, c_out}, feats->options());
+      out = &made;
+    }
+    void *y = out->data_ptr();
+    const bool plain_call = !epi.bias && !epi.residual && epi.act == PCE_ACT_NONE && !epi.ld_in && !epi.ld_out;
+    const pce_epilogue_t *e = plain_call ? nullptr : &epi;
+    if (kind == KIND_OSO) {          // nbr, order | mid, heavy, nonzero, single
+      rc = pce_conv_fwd_oso(x, w, wp, y, dt, n_in, n_out, ci, co, k, (int)num[0], m[0], m[1], num + 1, e, stream);
+    } else if (kind == KIND_OSB) {   // nbr, order | pairs
+      rc = pce_conv_fwd_osb(x, wp, y, dt, n_in, n_out, num[0], ci, co, k, m[0], m[1], ws, ws_bytes, e, stream);
+    } else if (kind == KIND_OS) {    // nbr
+      rc = ws ? pce_conv_fwd_os_parts(x, w, y, dt, n_in, n_out, ci, co, k, m[0], ws, ws_bytes, e, stream)
+              : pce_conv_fwd_os(x, w, wp, y, dt, n_in, n_out, ci, co, k, m[0], e, stream);
+    } else if (kind == KIND_FDS) {   // imap, omap, oslot, kpos, qkpos, ocsr, route | mid, pairs, qsum, kpos and qkpos on the host
+      const int64_t es = dt == PCE_F16 ? 2 : 4;
+      rc = pce_conv_fwd_fds(x, w, wp, y, dt, n_in, n_out, ci, co, k, (int)num[0], m[0], m[1], m[2], m[3], m[4], kpos_h, qkpos_h, m[5], m[6],
+                            num[1], num[2], ws, ws ? ws_bytes / es : 0, e, stream);
+    } else if (dense) {
+      rc = pce_conv_fwd_dense(x, w, wp, y, dt, n_in, ci, co, e, stream);
+    }
   }
-  if (PyErr_Occurred()) return nullptr;
   if (rc != PCE_OK) return PyLong_FromLong(rc);
   if (made.defined()) return THPVariable_Wrap(std::move(made));
   Py_INCREF(args[7]);
@@ -236,12 +248,18 @@ PyObject *bn_forward(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   const float momentum = (float)PyFloat_AsDouble(args[7]), eps = (float)PyFloat_AsDouble(args[8]), slope = (float)PyFloat_AsDouble(args[10]);
   void *stream = PyLong_AsVoidPtr(args[11]);
   if (PyErr_Occurred()) return nullptr;
-  const int64_t ws_bytes = pce_bn_workspace_bytes(n, (int32_t)c);
-  at::Tensor y = at::empty({n, c}, x->options()), save = at::empty({2 * c}, x->options().dtype(at::kFloat)),
-             ws = at::empty({ws_bytes}, x->options().dtype(at::kByte));
-  float *s = save.data_ptr<float>();
-  const int rc = pce_bn_forward(x->data_ptr(), res, y.data_ptr(), dt, n, (int32_t)c, w, b, const_cast<float *>(mean), const_cast<float *>(var),
-                                batch, momentum, eps, s, s + c, ws.data_ptr(), ws_bytes, act, slope, stream);
+  at::Tensor y, save, ws;
+  int rc;
+  {
+    Unlocked unlocked;
+    const int64_t ws_bytes = pce_bn_workspace_bytes(n, (int32_t)c);
+    y = at::empty({n, c}, x->options());
+    save = at::empty({2 * c}, x->options().dtype(at::kFloat));
+    ws = at::empty({ws_bytes}, x->options().dtype(at::kByte));
+    float *s = save.data_ptr<float>();
+    rc = pce_bn_forward(x->data_ptr(), res, y.data_ptr(), dt, n, (int32_t)c, w, b, const_cast<float *>(mean), const_cast<float *>(var), batch,
+                        momentum, eps, s, s + c, ws.data_ptr(), ws_bytes, act, slope, stream);
+  }
   if (rc != PCE_OK) return PyLong_FromLong(rc);
   return three(std::move(y), part(save, 0, c), part(save, c, c));
   END_HANDLE_TH_ERRORS
@@ -267,12 +285,18 @@ PyObject *bn_backward(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   void *stream = PyLong_AsVoidPtr(args[9]);
   if (PyErr_Occurred()) return nullptr;
   if (act != PCE_ACT_NONE && (!y || (act == PCE_ACT_LEAKY_RELU && !(slope > 0)))) Py_RETURN_NONE;
-  const int64_t ws_bytes = pce_bn_workspace_bytes(n, (int32_t)c);
-  at::Tensor dx = at::empty({n, c}, x->options()), grads = at::empty({2 * c}, x->options().dtype(at::kFloat)),
-             ws = at::empty({ws_bytes}, x->options().dtype(at::kByte));
-  float *g = grads.data_ptr<float>();
-  const int rc = pce_bn_backward(x->data_ptr(), dy, act == PCE_ACT_NONE ? nullptr : y, act, slope, dx.data_ptr(), dt, n, (int32_t)c, w, mean, rstd,
-                                 batch, g, g + c, ws.data_ptr(), ws_bytes, stream);
+  at::Tensor dx, grads, ws;
+  int rc;
+  {
+    Unlocked unlocked;
+    const int64_t ws_bytes = pce_bn_workspace_bytes(n, (int32_t)c);
+    dx = at::empty({n, c}, x->options());
+    grads = at::empty({2 * c}, x->options().dtype(at::kFloat));
+    ws = at::empty({ws_bytes}, x->options().dtype(at::kByte));
+    float *g = grads.data_ptr<float>();
+    rc = pce_bn_backward(x->data_ptr(), dy, act == PCE_ACT_NONE ? nullptr : y, act, slope, dx.data_ptr(), dt, n, (int32_t)c, w, mean, rstd, batch, g,
+                         g + c, ws.data_ptr(), ws_bytes, stream);
+  }
   if (rc != PCE_OK) return PyLong_FromLong(rc);
   return three(std::move(dx), part(grads, 0, c), part(grads, c, c));
   END_HANDLE_TH_ERRORS
@@ -300,9 +324,14 @@ PyObject *wgrad(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   Py_DECREF(tuple);   // (the caller holds the tensors)
   if (v.bad || num[2] <= 0) Py_RETURN_NONE;
   const int64_t c_in = x->size(1), c_out = g->size(1);
-  at::Tensor gw = at::empty({num[2], c_in, c_out}, x->options().dtype(at::kFloat));
-  const int rc = pce_conv_wgrad(x->data_ptr(), g->data_ptr(), x->scalar_type() == at::kHalf ? PCE_F16 : PCE_F32, num[0], num[1], (int32_t)c_in,
-                                (int32_t)c_out, (int32_t)num[2], (int32_t)num[3], m[0], m[1], m[2], m[3], num[4], gw.data_ptr<float>(), stream);
+  at::Tensor gw;
+  int rc;
+  {
+    Unlocked unlocked;
+    gw = at::empty({num[2], c_in, c_out}, x->options().dtype(at::kFloat));
+    rc = pce_conv_wgrad(x->data_ptr(), g->data_ptr(), x->scalar_type() == at::kHalf ? PCE_F16 : PCE_F32, num[0], num[1], (int32_t)c_in, (int32_t)c_out,
+                        (int32_t)num[2], (int32_t)num[3], m[0], m[1], m[2], m[3], num[4], gw.data_ptr<float>(), stream);
+  }
   if (rc != PCE_OK) return PyLong_FromLong(rc);
   return THPVariable_Wrap(std::move(gw));
   END_HANDLE_TH_ERRORS

@@ -121,6 +121,16 @@ other = copy.deepcopy(km, {id(t): t for t in km.__dict__.values() if torch.is_te
 other.kpos_host[KV], other.qkpos_host[KV] = 7, 8
 run(other)
 assert (seen("kpos_last"), seen("qkpos_last")) == (7, 8), (seen("kpos_last"), seen("qkpos_last"))
+
+# other Python threads may run while the library is called
+held, calls = seen("held_lock"), seen("calls")
+x = f32(4, 48)
+assert torch.is_tensor(backend.dense_forward(x, f32(48, 40)))
+y = backend.bn_forward(x, None, None, None, None, True, 0.1, 1e-5)
+assert len(backend.bn_backward(x, x, None, y[1], y[2], True)) == 3
+assert backend.conv_wgrad(f32(4, 32), f32(3, 48), km).shape == (KV, 32, 48)
+assert seen("calls") == calls + 4, "a call did not run natively"
+assert seen("held_lock") == 0, f"{seen('held_lock')} of {seen('calls')} calls held the interpreter's lock"
 """
 
 
