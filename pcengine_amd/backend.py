@@ -1142,8 +1142,8 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
             else:
                 scratch = _staging(need, dtype, feats.device)
             code = _ACT_CODES.get(act) if act is None or act == "relu" else _act_code(act)
-            if packed is None and dtype == torch.float16:
-                packed = pack_weights(weight)
+            if packed is None and dtype == torch.float16 and (kind == _HOST_OSO or kind == _HOST_OSB):
+                packed = pack_weights(weight)     # (the others read the kernel as it is where no packed copy is passed)
             done = _lib.layer(kind, view, feats, weight, packed, bias, residual, _place(view[1], shape[2], feats) if out is None else out,
                                      code[0], code[1], scratch, s)
             if done is not None:

@@ -94,3 +94,22 @@ def test_dense_norm_and_kernel_gradient(monkeypatch, dtype, layout):
         backend.conv_wgrad(f[:-1], g, km)
     with pytest.raises(ValueError):
         backend.bn_forward(x, weight, bias, torch.zeros(c + 1, device=DEV), None, True, 0.1, 1e-5)
+
+
+@pytest.mark.parametrize("df,c_in,c_out,ks,stride,transposed", [
+    (DATAFLOW_FDS, 64, 96, (2, 2, 2), (2, 2, 2), False), (DATAFLOW_FDS, 32, 48, (3, 3, 3), (1, 1, 1), False),
+    (DATAFLOW_OS, 32, 48, (3, 3, 3), (1, 1, 1), False), (DATAFLOW_OS, 64, 40, (2, 2, 2), (2, 2, 2), True)])
+def test_no_memory_is_taken_without_packed_weights(monkeypatch, df, c_in, c_out, ks, stride, transposed):
+    """fp16 layers that were given an output and a buffer, but no packed kernel: nothing is packed for them."""
+    km = gpu_map(synth.random_cloud(seed=3, n=1500, extent=14), ks, stride, want_nbr_in=transposed)
+    n_in, n_out = (km.n_out, km.n_in) if transposed else (km.n_in, km.n_out)
+    x, out = matrix(n_in, c_in, torch.float16, "dense", 1), torch.empty((n_out, c_out), dtype=torch.float16, device=DEV)
+    w = matrix(km.kv * c_in, c_out, torch.float16, "dense", 2).view(km.kv, c_in, c_out) * 0.1
+    buffer = torch.empty(km.M * c_out, dtype=torch.float16, device=DEV)
+    run = lambda: backend.conv_forward(x, w, km, df, transposed=transposed, out=out, buffer=buffer)
+    run()
+    taken = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+    before = taken()
+    got = run()
+    assert taken() == before
+    assert torch.equal(got.clone(), general(monkeypatch, run))
