@@ -597,14 +597,6 @@ class allocate_from:
         _arena = self.prev
 
 
-def _place(rows: int, cols: int, like: torch.Tensor) -> Optional[torch.Tensor]:
-    """A [rows, cols] output of like's type in the active arena; None where there is none or it is full (``_lib.layer`` then
-    takes memory from torch)."""
-    if _arena is None:
-        return None
-    return _arena.piece(rows, cols, like)
-
-
 def _new(shape, dtype, device) -> torch.Tensor:
     """Uninitialised device memory for an operator's output: from the active arena, else from torch."""
     if _arena is not None:
@@ -1024,10 +1016,10 @@ def dense_forward(feats: torch.Tensor, weight: torch.Tensor, packed: Optional[to
     lib = _lib.load()
     _require_cuda(feats, "feats")
     code = _ACT_CODES.get(act) if act is None or act == "relu" else _act_code(act)
-    done = _lib.layer(_HOST_DENSE, (), feats, weight, packed, bias, residual, _place(feats.shape[0], weight.shape[-1], feats)
-                             if feats.dim() == 2 else None, code[0], code[1], None, _stream(feats.device))
+    done = _native_layer(_HOST_DENSE, (), feats, weight, packed, bias, residual, None, (feats.shape[0], weight.shape[-1]), code, None,
+                         _stream(feats.device))
     if done is not None:
-        return done if type(done) is not int else _lib.check(done)
+        return done
     feats = feats.contiguous()
     weight = weight.contiguous()
     if feats.shape[1] != weight.shape[0]:
@@ -1037,6 +1029,21 @@ def dense_forward(feats: torch.Tensor, weight: torch.Tensor, packed: Optional[to
     _lib.check(lib.pce_conv_fwd_dense(feats.data_ptr(), weight.data_ptr(), _ptr(packed), out.data_ptr(), _dtype_code(feats),
                                       feats.shape[0], feats.shape[1], weight.shape[1], epi, _stream(feats.device)))
     return out
+
+
+def _native_layer(kind: int, view: tuple, feats, weight, packed, bias, residual, out, shape, code, scratch, stream):
+    """``_lib.layer`` with its output of `shape` in the active arena where none is passed, or None where the general path has to
+    take the call: the arena is then left as it was, and the place goes to that path's output."""
+    mark = None
+    if out is None and _arena is not None:
+        mark = _arena.need
+        out = _arena.piece(shape[0], shape[1], feats)
+    done = _lib.layer(kind, view, feats, weight, packed, bias, residual, out, code[0], code[1], scratch, stream)
+    if done is None:
+        if mark is not None:
+            _arena.need = mark
+        return None
+    return done if type(done) is not int else _lib.check(done)
 
 
 # kinds of layer of _lib.layer (csrc/pce_torch.cpp)
@@ -1144,10 +1151,9 @@ def conv_forward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, dataf
             code = _ACT_CODES.get(act) if act is None or act == "relu" else _act_code(act)
             if packed is None and dtype == torch.float16 and (kind == _HOST_OSO or kind == _HOST_OSB):
                 packed = pack_weights(weight)     # (the others read the kernel as it is where no packed copy is passed)
-            done = _lib.layer(kind, view, feats, weight, packed, bias, residual, _place(view[1], shape[2], feats) if out is None else out,
-                                     code[0], code[1], scratch, s)
+            done = _native_layer(kind, view, feats, weight, packed, bias, residual, out, (view[1], shape[2]), code, scratch, s)
             if done is not None:
-                return done if type(done) is not int else _lib.check(done)
+                return done
     lib = _lib.load()
     # the deferred-scatter and output-stationary kernels take column slices of wider matrices in place (the halves
     # of a concatenated skip connection); everything else gets dense rows

@@ -113,3 +113,24 @@ def test_no_memory_is_taken_without_packed_weights(monkeypatch, df, c_in, c_out,
     got = run()
     assert taken() == before
     assert torch.equal(got.clone(), general(monkeypatch, run))
+
+
+def test_a_declined_call_leaves_the_arena_as_it_was(monkeypatch):
+    """Layers that the general path takes in the end ask the forward's arena for one output, as without the native call."""
+    km = gpu_map(synth.random_cloud(seed=3, n=1500, extent=14), (3, 3, 3))
+    x, wide = matrix(km.n_in, 64, torch.float16, "dense", 1), matrix(km.n_in, 64, torch.float16, "slice", 1)
+    w, w1 = matrix(27 * 64, 48, torch.float16, "dense", 2).view(27, 64, 48), matrix(64, 48, torch.float16, "dense", 3)
+    residual = matrix(km.n_out, 48, torch.float16, "slice", 4)
+    arena = backend.ForwardArena(DEV)
+
+    def run():
+        p, p1 = backend.pack_weights(w), backend.pack_weights(w1)
+        with backend.allocate_from(arena):
+            outs = [backend.conv_forward(x, w, km, DATAFLOW_OSO, packed=p, residual=residual), backend.dense_forward(wide, w1, p1),
+                    backend.conv_forward(x, w, km, DATAFLOW_OSO, packed=p)]
+        return arena.need, outs
+
+    run()
+    for _ in range(2):
+        (need, outs), (plain, same) = run(), general(monkeypatch, run)
+        assert need == plain == 3 * (-(-km.n_out * 48 * 2 // 256) * 256)
