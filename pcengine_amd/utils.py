@@ -25,14 +25,22 @@ def conv_info_decoder(code: int) -> Tuple[int, int, int]:
     return (x, rest // _B, rest - rest // _B * _B)
 
 
-@lru_cache(maxsize=1024)
 def output_stride_compute(l_stride_code: int, t_stride_code: int, transposed: bool = False) -> int:
     """Tensor stride after a layer: product for a conv, quotient for a transposed conv
     (script/utils.py:116-138)."""
+    if type(l_stride_code) is int and type(t_stride_code) is int:
+        return _output_stride_of_codes(l_stride_code, t_stride_code, bool(transposed))
+    return _output_stride(l_stride_code, t_stride_code, transposed)
+
+
+def _output_stride(l_stride_code, t_stride_code, transposed):
     ls, ts = conv_info_decoder(l_stride_code), conv_info_decoder(t_stride_code)
     if transposed:
         return conv_info_encoder([t // l for t, l in zip(ts, ls)])
     return conv_info_encoder([t * l for t, l in zip(ts, ls)])
+
+
+_output_stride_of_codes = lru_cache(maxsize=1024)(_output_stride)     # (plain numbers: a layer asks for the same few)
 
 
 def load_file(file_name):

@@ -401,3 +401,17 @@ def test_every_global_to_lds_copy_is_followed_by_a_hand_written_wait():
             assert wait.search(body) or any(re.search(r"\b" + h + r"\b", body) for h in waiting_helpers), \
                 f"{name} copies global -> LDS through {called} and never waits by hand"
     assert sites >= 6
+
+
+def test_output_stride_of_numbers_and_arrays():
+    """Codes of any integer type: arrays give arrays, and a tensor that changes gives its new value."""
+    import numpy as np
+    import torch
+    from pcengine_amd.utils import conv_info_encoder, output_stride_compute
+    one, two, four = (conv_info_encoder((k, k, k)) for k in (1, 2, 4))
+    assert output_stride_compute(two, two) == four and output_stride_compute(two, four, True) == two
+    assert np.array_equal(output_stride_compute(np.array([two, one]), np.array([two, four])), [four, four])
+    code = torch.tensor(one)
+    assert int(output_stride_compute(two, code)) == two
+    code.fill_(two)
+    assert int(output_stride_compute(two, code)) == four
