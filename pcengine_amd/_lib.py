@@ -214,6 +214,19 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+def host_stamp() -> bytes:
+    """What the extension module has to have been built for: the bytes that the build leaves in it."""
+    import sys
+    import torch
+    return f"pcengine_amd host calls for torch {torch.__version__}, Python {sys.version_info[0]}.{sys.version_info[1]};".encode()
+
+
+def host_is_current(path: str) -> bool:
+    """Whether the extension module at `path` was built for this torch and this Python (it knows the layout of torch's objects)."""
+    with open(path, "rb") as f:
+        return host_stamp() in f.read()
+
+
 def host():
     """The extension module that runs the host side of a layer (csrc/pce_torch.cpp), loaded once."""
     global _host
@@ -221,6 +234,8 @@ def host():
         load()
         if not os.path.exists(HOST_PATH):
             raise PCEError(f"{HOST_PATH} is missing: build it with `python -m pcengine_amd.build`")
+        if not host_is_current(HOST_PATH):
+            raise PCEError(f"{HOST_PATH} was built for another torch or Python: rebuild it with `python -m pcengine_amd.build`")
         spec = importlib.util.spec_from_file_location("_host", HOST_PATH)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)

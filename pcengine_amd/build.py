@@ -14,6 +14,10 @@ import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
+if ROOT not in sys.path:                # (run as a file)
+    sys.path.append(ROOT)
+from pcengine_amd import _lib            # noqa: E402
+
 CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libpcengine_amd.so")
@@ -55,7 +59,7 @@ def up_to_date() -> bool:
         return False
     t = min(os.path.getmtime(p) for p in paths)
     deps = [os.path.join(CSRC, s) for s in SOURCES + [HOST_SOURCE]] + HEADERS
-    return all(os.path.getmtime(d) <= t for d in deps)
+    return all(os.path.getmtime(d) <= t for d in deps) and _lib.host_is_current(HOST_PATH)
 
 
 def build(force: bool = True, verbose: bool = False) -> str:
@@ -78,7 +82,8 @@ def build(force: bool = True, verbose: bool = False) -> str:
             if src not in MEASURE_SOURCES:
                 measure_objs.append(obj)
     obj = os.path.join(LIB_DIR, "pce_torch.o")
-    procs.append((HOST_SOURCE, subprocess.Popen(["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", *_torch_includes(), "-I", os.path.join(ROOT, "include"),
+    procs.append((HOST_SOURCE, subprocess.Popen(["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", *_torch_includes(),
+                                                 f'-DPCE_HOST_STAMP="{_lib.host_stamp().decode()}"', "-I", os.path.join(ROOT, "include"),
                                                  "-c", os.path.join(CSRC, HOST_SOURCE), "-o", obj],
                                                 stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
     for src, p in procs:

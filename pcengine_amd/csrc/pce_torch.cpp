@@ -369,4 +369,7 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Host side of a forward la
 
 }  // namespace
 
+// the torch and the Python this was compiled against; the front end looks for it before it loads the file (_lib.host_is_current)
+extern "C" __attribute__((used, visibility("default"))) const char pce_host_stamp[] = PCE_HOST_STAMP;
+
 PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&module); }

@@ -142,3 +142,19 @@ def test_calls_of_the_extension(tmp_path):
     subprocess.run(["gcc", "-D_GNU_SOURCE", "-shared", "-fPIC", "-w", "-o", str(tmp_path / "libpcengine_amd.so"), str(tmp_path / "stub.c"), "-ldl"], check=True)
     child = subprocess.run([sys.executable, "-c", CHILD, str(tmp_path)], cwd=build.ROOT, capture_output=True, text=True, timeout=300)
     assert child.returncode == 0, child.stderr[-3000:]
+
+
+def test_an_extension_of_another_torch_is_refused(tmp_path, monkeypatch):
+    if not os.path.exists(build.HOST_PATH):
+        build.build(force=True)
+    with open(build.HOST_PATH, "rb") as f:
+        built = f.read()
+    version = torch.__version__.encode()
+    other = tmp_path / "_host.so"
+    other.write_bytes(built.replace(b"for torch " + version, b"for torch " + b"9" * len(version)))
+    for module in (_lib, build):
+        monkeypatch.setattr(module, "HOST_PATH", str(other))
+    monkeypatch.setattr(_lib, "_host", None)
+    assert not build.up_to_date()
+    with pytest.raises(_lib.PCEError, match="another torch"):
+        _lib.host()
