@@ -1031,7 +1031,7 @@ extern "C" int pce_outcoords_chain_planned(const int32_t *in_coords, int64_t n_i
 // of them: its blocks are numbered as they lie.  The box is worked out on the device, so all of this is queued before the
 // host waits, once, for the box and the number of voxels: 60 us of kernels for 172 k points of a 64-ring scan in 238 M cells
 // (one bit per cell of the whole box: 45, and as much as the sort in 1.9 G cells; sorted: 150, and two waits).
-// Boxes too empty even for a bit per block: keys code << idx_bits | point index are sorted; the sort is stable, so only the
+// Boxes too empty even for a bit per block, and of more than VOX_POINTS_MAX points those of 2^31 cells or more: keys code << idx_bits | point index are sorted; the sort is stable, so only the
 // code's bits are passed over.
 #define VOX_LIMIT (1 << 30)
 #define VOX_SUB 16           // words per counted block of a bitmap: a line of 64 bytes
@@ -1039,7 +1039,7 @@ extern "C" int pce_outcoords_chain_planned(const int32_t *in_coords, int64_t n_i
 #define VOX_TILE 4096        // words a workgroup counts at a time: 256 blocks
 #define VOX_WORDS_PER_POINT 16   // words of the box's map per point, what the sort's arrays are too
 #define VOX_WORDS_MAX (1ll << 26)
-#define VOX_POINTS_MAX (1ll << 26)   // more points are sorted: the blocks' cells take 64 bytes a point, the sort 24
+#define VOX_POINTS_MAX (VOX_WORDS_MAX / VOX_SUB)   // points whose blocks' cells fit that many words; of more, boxes of blocks as they lie
 #define VOX_BLOCKS 512       // workgroups that read the points; each leaves its bounds in a line of its own
 
 struct VoxLayout {
@@ -1052,6 +1052,9 @@ __host__ __device__ static inline int64_t vox_words_cap(int64_t n) {
   int64_t words = VOX_WORDS_PER_POINT * n + 65536;
   return words < VOX_WORDS_MAX ? words : VOX_WORDS_MAX;
 }
+
+// words of the blocks' cells: of a block per point, or of every block of a box
+__host__ __device__ static inline int64_t vox_cells_cap(int64_t n) { return n < VOX_POINTS_MAX ? VOX_SUB * n : VOX_WORDS_MAX; }
 
 // the words that are cleared and counted
 __host__ __device__ static inline int64_t vox_padded(int64_t words) { return (words + VOX_TILE - 1) / VOX_TILE * VOX_TILE; }
@@ -1076,7 +1079,7 @@ struct VoxBox {
 static void vox_layout(int64_t n, VoxLayout *L) {
   int64_t nblocks = pce_div_up(n, SORT_KEYS_PER_BLOCK);
   L->words[0] = vox_padded(vox_words_cap(n));
-  L->words[1] = L->words[0] ? vox_padded(VOX_SUB * n) : 0;
+  L->words[1] = vox_padded(vox_cells_cap(n));
   int64_t o = 0;
   L->off_q = o;
   o += pce_align_up(n * 16, 256);
@@ -1171,8 +1174,8 @@ __host__ __device__ static inline int vox_box(int64_t n, const int *lo, const in
   *code_bits = 1;
   while (*code_bits < 64 && cells > (double)(1ull << *code_bits)) ++*code_bits;
   *words = 0;
-  if (!(cells < 32.0 * VOX_CELLS * (double)(vox_words_cap(n) - 1))) return VOX_SORT;
-  const bool all = cells < (double)VOX_CELLS * (double)(n - 1);
+  const bool all = cells < 32.0 * (double)(vox_cells_cap(n) - VOX_SUB);
+  if (!all && !(cells < 32.0 * VOX_CELLS * (double)(vox_words_cap(n) - 1))) return VOX_SORT;
   *words = (int64_t)(cells / (all ? 32.0 : 32.0 * VOX_CELLS)) + 1;
   return all ? VOX_BLOCKS_ALL : VOX_BLOCKS_MAPPED;
 }
@@ -1435,25 +1438,24 @@ extern "C" int pce_voxelize(const void *points, int32_t dtype, int64_t n_points,
   int *tiles[2] = {(int *)(w + L.off_tiles[0]), (int *)(w + L.off_tiles[1])};
   hipLaunchKernelGGL(vox_clear_kernel, dim3(1024), dim3(256), 0, s, (const int *)bounds, (int)readers, (long long)n_points, box, bits[0], bits[1]);
   PCE_LAUNCH_CHECK("vox_clear");
-  if (L.words[0]) {
-    hipLaunchKernelGGL(vox_mark_kernel, dim3(blocks), dim3(256), 0, s, (const int4 *)q, (long long)n_points, (const VoxBox *)box, (unsigned *)bits[0]);
-    PCE_LAUNCH_CHECK("vox_mark");
-    for (int k = 0; k < 2; ++k) {
-      if (k == 1) {
-        hipLaunchKernelGGL(vox_cells_kernel, dim3(blocks), dim3(256), 0, s, q, (long long)n_points, (const VoxBox *)box, (const uint4 *)bits[0],
-                           (const int *)count[0], (const int *)tiles[0], (unsigned *)bits[1], (int *)(w + L.off_first));
-        PCE_LAUNCH_CHECK("vox_cells");
-      }
-      const int64_t most = L.words[k] / VOX_TILE;
-      hipLaunchKernelGGL(vox_count_kernel, dim3((unsigned)(most < 1024 ? most : 1024)), dim3(256), 0, s, (const uint4 *)bits[k],
-                         (const long long *)&box->words[k], count[k], tiles[k]);
-      PCE_LAUNCH_CHECK("vox_count");
-      if (k == 0)
-        hipLaunchKernelGGL(vox_total_kernel<0>, dim3(1), dim3(1024), 0, s, box, (int4 *)tiles[k]);
-      else
-        hipLaunchKernelGGL(vox_total_kernel<1>, dim3(1), dim3(1024), 0, s, box, (int4 *)tiles[k]);
-      PCE_LAUNCH_CHECK("vox_total");
+  for (int k = L.words[0] ? 0 : 1; k < 2; ++k) {
+    if (k == 0) {
+      hipLaunchKernelGGL(vox_mark_kernel, dim3(blocks), dim3(256), 0, s, (const int4 *)q, (long long)n_points, (const VoxBox *)box, (unsigned *)bits[0]);
+      PCE_LAUNCH_CHECK("vox_mark");
+    } else {
+      hipLaunchKernelGGL(vox_cells_kernel, dim3(blocks), dim3(256), 0, s, q, (long long)n_points, (const VoxBox *)box, (const uint4 *)bits[0],
+                         (const int *)count[0], (const int *)tiles[0], (unsigned *)bits[1], (int *)(w + L.off_first));
+      PCE_LAUNCH_CHECK("vox_cells");
     }
+    const int64_t most = L.words[k] / VOX_TILE;
+    hipLaunchKernelGGL(vox_count_kernel, dim3((unsigned)(most < 1024 ? most : 1024)), dim3(256), 0, s, (const uint4 *)bits[k],
+                       (const long long *)&box->words[k], count[k], tiles[k]);
+    PCE_LAUNCH_CHECK("vox_count");
+    if (k == 0)
+      hipLaunchKernelGGL(vox_total_kernel<0>, dim3(1), dim3(1024), 0, s, box, (int4 *)tiles[k]);
+    else
+      hipLaunchKernelGGL(vox_total_kernel<1>, dim3(1), dim3(1024), 0, s, box, (int4 *)tiles[k]);
+    PCE_LAUNCH_CHECK("vox_total");
   }
   VoxBox host;
   PCE_HIP(hipMemcpyAsync(&host, box, sizeof(host), hipMemcpyDeviceToHost, s));

@@ -53,6 +53,16 @@ def test_voxelize_large_boxes(n, side):
     assert np.array_equal(index.cpu().numpy(), first) and np.array_equal(inv.cpu().numpy(), inverse)
 
 
+# the most points whose blocks have bitmaps of their own and more than those, in boxes on both sides of 2^31 cells
+@pytest.mark.parametrize("n,side", [(1 << 22, 1200), (1 << 22, 1300), ((1 << 22) + 1, 1290), ((1 << 22) + 1, 1291), (4300001, 200)])
+def test_voxelize_many_points(n, side):
+    pts = _points(n, side, np.float32, side)
+    want, first, inverse = orc.sparse_quantize(pts, (0.5, 0.5, 0.5))
+    coords, index, inv = utils.sparse_quantize(torch.as_tensor(pts, device=DEV), 0.5, return_index=True, return_inverse=True)
+    assert np.array_equal(coords.cpu().numpy(), want)
+    assert np.array_equal(index.cpu().numpy(), first) and np.array_equal(inv.cpu().numpy(), inverse)
+
+
 @pytest.mark.parametrize("rows", [[1], [3, 0, 5], [256, 257, 1], [70000, 1, 12345], [7] * 64, [7] * 65])
 def test_collate(rows):
     rng = np.random.default_rng(len(rows))

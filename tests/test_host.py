@@ -415,3 +415,9 @@ def test_output_stride_of_numbers_and_arrays():
     assert int(output_stride_compute(two, code)) == two
     code.fill_(two)
     assert int(output_stride_compute(two, code)) == four
+
+
+def test_voxel_workspace_is_the_sorts_and_two_bitmaps():
+    """Beyond the points whose blocks' cells fit the largest bitmap the workspace grows by what a sorted point takes."""
+    for n in (1, 1000, 1 << 20, 1 << 22, (1 << 22) + 1, 10 ** 7, 1 << 25, 1 << 26, (1 << 26) + 1, 1 << 28):
+        assert _lib.load().pce_voxelize_workspace_bytes(n) <= 48 * n + (2 << 28) + (64 << 20), n
