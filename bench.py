@@ -174,6 +174,9 @@ def main() -> int:
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--no-net", action="store_true", help="skip the MinkUNet-style forward (configuration 4)")
     ap.add_argument("--no-layers", action="store_true", help="skip the per-layer record of the configuration-4 network")
+    ap.add_argument("--layer-records", default=None, metavar="FILE",
+                    help="write the per-layer records of the configuration-4 and -5 networks to FILE (JSON, 25 KB): the printed "
+                         "line holds their summary only, so that whoever keeps the end of the output has all of it")
     ap.add_argument("--no-other-configs", action="store_true",
                     help="skip configurations 1 (fp32 C16 layer), 3 (k2s2 down + transposed up) and 5 (8-scene indoor "
                          "batch, widened network), whose timings go to extra.cfg1 / cfg3 / cfg5")
@@ -491,6 +494,7 @@ def main() -> int:
                                 if "device_copy_ms" in floors else {})}},
     }
 
+    layers = {}
     # ---- configuration 4: MinkUNet-style forward, ~100k voxels, fp16, BN folded --------------------
     if not args.no_net:
         import pcengine_amd as pe
@@ -561,7 +565,7 @@ def main() -> int:
         if not args.no_layers:
             y0 = forward()
             recs4 = layer_records(lambda: forward(y0), graph_ms)
-            result["extra"]["cfg4_minkunet"]["layers"] = recs4
+            layers["cfg4_minkunet"] = recs4
             result["extra"].setdefault("selector_regret", {})["cfg4"] = regret_summary(recs4)
         # the same network in training mode (BatchNorm on batch statistics, cross-entropy on random labels):
         # forward + backward with kernel maps built every step, fp16 features and fp32 parameters
@@ -654,7 +658,7 @@ def main() -> int:
                                    "forward_ms_cached_maps": round(ev_ms(lambda: forward5(y5), 10, 2), 3)}
         if not args.no_layers:
             recs5 = layer_records(lambda: forward5(y5), graph_ms)
-            result["extra"]["cfg5"]["layers"] = recs5
+            layers["cfg5"] = recs5
             result["extra"].setdefault("selector_regret", {})["cfg5"] = regret_summary(recs5)
         del model5, y5, f5, c5d
 
@@ -676,6 +680,9 @@ def main() -> int:
         result["extra"]["rel_l2_vs_cpu"] = float(orc.rel_l2(gpu_out, cpu_out))
         if not result["extra"]["rel_l2_vs_cpu"] <= 1e-3:
             raise RuntimeError(f"the timed layer is {result['extra']['rel_l2_vs_cpu']:.3e} (rel-L2) away from the CPU path: bar 1e-3")
+    if args.layer_records:
+        with open(args.layer_records, "w") as f:
+            json.dump(layers, f)
     print(json.dumps(result))
     return 0
 
