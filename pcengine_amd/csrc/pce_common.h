@@ -101,6 +101,7 @@ __host__ __device__ static inline unsigned long long pce_home_slot(unsigned long
 #define ORDER_N_SINGLE 8187   // rows with exactly one neighbour
 #define ORDER_N_NONZERO 8188  // rows with any neighbour
 #define ORDER_N_HEAVY 8189    // rows with ORDER_HEAVY_POPC neighbours or more
-#define ORDER_PLAIN_CURSOR 8191
+#define ORDER_PLAIN 6144       // rows without neighbours of each workgroup of the sort
+#define ORDER_PLAIN_COUNTS 2040
 #define ORDER_HEAVY_POPC 3
 

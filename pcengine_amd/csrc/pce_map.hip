@@ -1707,7 +1707,7 @@ struct Job {
   unsigned blk0;
   int prob;
   int kind;
-  int pad;
+  int per;   // row order: rows per workgroup, in 256s
 };
 enum { JOB_CSR_SUBM = 0, JOB_CSR_IN = 1, JOB_CSR_COUNT_OUT = 2, JOB_CSR_OUT = 3, JOB_ORDER_SCATTER = 4, JOB_FILL_VIEWS = 5, JOB_FILL_FULL3 = 6 };
 
@@ -2016,7 +2016,7 @@ __global__ void __launch_bounds__(256) grid_query_kernel(const ProbDev *__restri
 
 // ---- row order of the ordered output-stationary dataflow -----------------------------------------------------
 // Output rows of a map in an order that puts equal neighbour patterns side by side: rows without neighbours
-// first (block by block, each block's rows in their own order), then the rows with one or two neighbours sorted
+// first (in their own order), then the rows with one or two neighbours sorted
 // by the (lowest, second-lowest) offset they have one at, then the rows with ORDER_HEAVY_POPC or more, sorted
 // likewise.  A counting sort: masks and a histogram of the keys, one block that turns the histogram into
 // bases, a scatter pass with one cursor per key.  The kernels exist twice: over the job lists of a batched map
@@ -2032,26 +2032,61 @@ __device__ __forceinline__ int order_key(unsigned m) {   // m != 0
   return (__popc(m) >= ORDER_HEAVY_POPC ? 1024 : 0) + 32 + first * 32 + second;
 }
 
-// mask[row] = offsets (other than the centre) at which the row has a neighbour; hist[key] += the block's count.
-// The keys of a block of 256 rows are counted in LDS first: on a dense cloud nearly every row has a key and a few
-// keys hold most rows, and one global atomic per row on those few addresses costs milliseconds.
-__device__ __forceinline__ void order_mask_block(const int *__restrict__ nbr, int kv, long long n_rows, int mid,
-                                                 int *__restrict__ order, unsigned blk) {
-  __shared__ int cnt[ORDER_KEYS];
+// Workgroups of the sort take order_per() times 256 rows.  The sort is bound by its global atomics: every key that a workgroup
+// holds costs one in the histogram and one in the scatter, on 64 lines that all workgroups share (about 30 ns each on a line), and
+// 256 rows of an indoor scene hold some 200 keys.  So as few workgroups as still give every compute unit one, and no more than
+// the tail has places for their counts.  The scatter of the five submanifold maps of eight indoor scenes (2.0 M rows) 337 us with
+// 256 rows a workgroup, 84 / 60 / 62 / 65 us with 1024 / 256 / 128 / 64 workgroups a map; of a 100 k-voxel scan (0.38 M rows) 32,
+// then 24 / 17 / 19 / 22.
+#define ORDER_WORKGROUPS 256
+#define ORDER_PER 16
+static int order_per(int64_t n_rows) {
+  const int64_t per = pce_div_up(n_rows, 256 * ORDER_WORKGROUPS), least = pce_div_up(n_rows, 256 * ORDER_PLAIN_COUNTS);
+  return (int)(least > ORDER_PER ? least : per < ORDER_PER ? per : ORDER_PER);
+}
+// first row of a wavefront of such a workgroup; its rows follow one another
+__device__ __forceinline__ long long order_row0(unsigned blk, int per) { return ((long long)blk * 4 + (threadIdx.x >> 6)) * per * 64; }
+
+// hist[key] += the rows of the workgroup with that key, and the workgroup's rows without neighbours.  The keys are
+// counted in LDS first: on a dense cloud nearly every row has a key and a few keys hold most rows, and one global atomic per row
+// on those few addresses costs milliseconds.  `mask_of(row)`: the offsets at which the row has a neighbour.
+template <typename F>
+__device__ __forceinline__ void order_count_block(long long n_rows, int *__restrict__ tail, unsigned blk, int per, int *cnt, F mask_of) {
+  __shared__ int plain[4];
   for (int i = threadIdx.x; i < ORDER_KEYS; i += 256) cnt[i] = 0;
   __syncthreads();
-  const long long row = (long long)blk * 256 + threadIdx.x;
-  if (row < n_rows) {
-    unsigned m = 0;
-    for (int k = 0; k < kv; ++k)
-      if (k != mid && nbr[(long long)k * n_rows + row] >= 0) m |= 1u << k;
-    order[n_rows + row] = (int)m;
-    if (m) atomicAdd(&cnt[order_key(m)], 1);   // rows without neighbours are placed by the scatter pass
+  const int lane = threadIdx.x & 63;
+  const long long row0 = order_row0(blk, per) + lane;
+  int without = 0;
+  for (int t = 0; t < per; ++t) {
+    const long long row = row0 + t * 64;
+    const unsigned m = row < n_rows ? mask_of(row) : 0u;
+    if (m) atomicAdd(&cnt[order_key(m)], 1);
+    without += __popcll(__ballot(row < n_rows && m == 0));
   }
+  if (lane == 0) plain[threadIdx.x >> 6] = without;
   __syncthreads();
-  int *hist = order + 2 * n_rows + ORDER_HIST;
+  if (threadIdx.x == 0) tail[ORDER_PLAIN + blk] = plain[0] + plain[1] + plain[2] + plain[3];
   for (int i = threadIdx.x; i < ORDER_KEYS; i += 256)
-    if (cnt[i]) atomicAdd(&hist[i], cnt[i]);
+    if (cnt[i]) atomicAdd(&tail[ORDER_HIST + i], cnt[i]);
+}
+
+// the same, and mask[row] = offsets (other than the centre) at which the row has a neighbour, from the output-major table
+__device__ __forceinline__ void order_mask_block(const int *__restrict__ nbr, int kv, long long n_rows, int mid,
+                                                 int *__restrict__ order, unsigned blk, int per) {
+  __shared__ int cnt[ORDER_KEYS];
+  order_count_block(n_rows, order + 2 * n_rows, blk, per, cnt, [&](long long row) {
+    unsigned m = 0;
+    for (int k0 = 0; k0 < kv; k0 += 8) {   // eight entries out together, from addresses valid for every k
+      int v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = nbr[(long long)(k0 + j < kv ? k0 + j : 0) * n_rows + row];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) m |= k0 + j < kv && k0 + j != mid && v[j] >= 0 ? 1u << (k0 + j) : 0u;
+    }
+    order[n_rows + row] = (int)m;
+    return m;
+  });
 }
 
 // base[key] = first position of the key's rows behind the rows without neighbours (one block of 1024); the counts
@@ -2089,66 +2124,107 @@ __device__ __forceinline__ void order_scan_block(int *tail, int *n_heavy_out) {
   }
 }
 
-// perm: the rows of one block of 256 (block `blk` of the map), placed as described above.  A block takes one range
-// per key it holds (one global atomic per key and block); its rows of a key keep the ranks LDS atomics gave them.
+// perm: the rows of one workgroup, placed as described above.  A workgroup takes one range per key it holds (one global atomic per
+// key), and its rows a place each in those through LDS atomics.  Rows without neighbours keep their order (64 -> 64 channels on
+// 1.2 M rows of eight scans read theirs in 97.4 us; 101.1 where workgroups took their ranges as they came).
 // `nbr` is the output-major neighbour table, or (mirror >= 0) the probe table of a symmetric map, whose row
 // mirror - k is the output-major row k: the table the same launch may still be writing is never read.
-__device__ __forceinline__ void order_scatter_block(long long n_rows, int *__restrict__ order, unsigned blk,
+#define ORDER_BATCH 4   // rows of a thread whose loads are out together
+__device__ __forceinline__ void order_scatter_block(long long n_rows, int *__restrict__ order, unsigned blk, int per,
                                                     const int *__restrict__ nbr, int mirror) {
-  __shared__ int cnt[ORDER_KEYS], gbase[ORDER_KEYS];
-  __shared__ int wcount[4], wbase;
+  __shared__ int cnt[ORDER_KEYS];    // rows of the key, then the key's next place
+  __shared__ int plain[2][4];        // of every wavefront: its own rows without neighbours, and a share of those in front of the workgroup
+  const unsigned none = 0xFFFFFFFFu; // mask of a row behind the last one
   int *perm = order, *tail = order + 2 * n_rows;
+  const int *masks = order + n_rows;
   for (int i = threadIdx.x; i < ORDER_KEYS; i += 256) cnt[i] = 0;
-  const long long n_plain = n_rows - tail[ORDER_N_NONZERO];
-  long long row = (long long)blk * 256 + threadIdx.x;
-  const bool live = row < n_rows;
-  const unsigned m = live ? (unsigned)order[n_rows + row] : 1u;
-  const bool plain = live && m == 0;
-  const unsigned long long b = __ballot(plain);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) wcount[wave] = __popcll(b);
+  int before = 0;
+  for (int i = threadIdx.x; i < (int)blk; i += 256) before += tail[ORDER_PLAIN + i];
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) before += __shfl_xor(before, d, PCE_WAVE);
   __syncthreads();
-  if (threadIdx.x == 0) wbase = atomicAdd(&tail[ORDER_PLAIN_CURSOR], wcount[0] + wcount[1] + wcount[2] + wcount[3]);
-  const int key = (live && !plain) ? order_key(m) : -1;
-  int rank = 0;
-  if (key >= 0) rank = atomicAdd(&cnt[key], 1);
+  const long long n_nonzero = tail[ORDER_N_NONZERO], n_plain = n_rows - n_nonzero, n_single = tail[ORDER_N_SINGLE];
+  const bool shared_records = n_nonzero - n_single <= PCE_ORDER_SREC_ROWS(n_rows);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long long row0 = order_row0(blk, per) + lane;
+  int without = 0;
+  for (int t0 = 0; t0 < per; t0 += ORDER_BATCH) {
+    unsigned m[ORDER_BATCH];
+#pragma unroll
+    for (int j = 0; j < ORDER_BATCH; ++j) {
+      const long long row = row0 + (t0 + j) * 64;
+      const bool in = t0 + j < per && row < n_rows;
+      const unsigned v = (unsigned)masks[in ? row : 0];
+      m[j] = in ? v : none;
+    }
+#pragma unroll
+    for (int j = 0; j < ORDER_BATCH; ++j) {
+      without += __popcll(__ballot(m[j] == 0));
+      if (m[j] != 0 && m[j] != none) atomicAdd(&cnt[order_key(m[j])], 1);
+    }
+  }
+  if (lane == 0) {
+    plain[0][wave] = without;
+    plain[1][wave] = before;
+  }
   __syncthreads();
   for (int i = threadIdx.x; i < ORDER_KEYS; i += 256)
-    if (cnt[i]) gbase[i] = tail[ORDER_BASE + i] + atomicAdd(&tail[ORDER_CURSOR + i], cnt[i]);
+    if (cnt[i]) cnt[i] = tail[ORDER_BASE + i] + atomicAdd(&tail[ORDER_CURSOR + i], cnt[i]);
+  long long plain_at = plain[1][0] + plain[1][1] + plain[1][2] + plain[1][3];
+  for (int w = 0; w < wave; ++w) plain_at += plain[0][w];
   __syncthreads();
-  if (plain) {
-    int before = __popcll(b & ((1ull << lane) - 1ull));
-    for (int w2 = 0; w2 < wave; ++w2) before += wcount[w2];
-    perm[wbase + before] = (int)row;
-  } else if (key >= 0) {
-    const long long p = n_plain + gbase[key] + rank;
-    perm[p] = (int)row;
-    // the record of the row: what a wavefront of the ordered dataflow reads of it in one load
-    const int k1 = __ffs((int)m) - 1;
-    const unsigned rest = m & (m - 1u);
-    const int k2 = rest ? __ffs((int)rest) - 1 : -1;
-    int4 r;
-    r.x = (int)row;
-    r.y = (int)m;
-    r.z = nbr[(long long)(mirror >= 0 ? mirror - k1 : k1) * n_rows + row];
-    r.w = k2 >= 0 ? nbr[(long long)(mirror >= 0 ? mirror - k2 : k2) * n_rows + row] : -1;
-    reinterpret_cast<int4 *>(order + PCE_ORDER_REC_OFFSET(n_rows))[p] = r;
-    // rows with two neighbours or more: the 128-byte record with the neighbour at every offset
-    const long long n_single = tail[ORDER_N_SINGLE];
-    const long long si = (long long)gbase[key] + rank - n_single;
-    if (key >= 32 && (long long)tail[ORDER_N_NONZERO] - n_single <= PCE_ORDER_SREC_ROWS(n_rows)) {
-      int v[32];
-      v[0] = (int)row;
-      v[1] = (int)m;
+  for (int t0 = 0; t0 < per; t0 += ORDER_BATCH) {
+    unsigned m[ORDER_BATCH];
+    int near[ORDER_BATCH][2];
 #pragma unroll
-      for (int k = 0; k < PCE_ORDER_SREC_KV; ++k) {   // (loads from an address valid for every k, selected afterwards)
-        const bool has = (m >> k) & 1u;
-        const int x = nbr[(long long)(has ? (mirror >= 0 ? mirror - k : k) : 0) * n_rows + row];
-        v[2 + k] = has ? x : -1;
+    for (int j = 0; j < ORDER_BATCH; ++j) {
+      const long long row = row0 + (t0 + j) * 64;
+      const bool in = t0 + j < per && row < n_rows;
+      const unsigned v = (unsigned)masks[in ? row : 0];
+      m[j] = in ? v : none;
+    }
+    // the neighbours at the two lowest offsets, from addresses valid for every lane
+#pragma unroll
+    for (int j = 0; j < ORDER_BATCH; ++j) {
+      const long long row = row0 + (t0 + j) * 64;
+      const bool has = m[j] != 0 && m[j] != none;
+      const unsigned rest = has ? m[j] & (m[j] - 1u) : 0u;
+      const int k1 = has ? __ffs((int)m[j]) - 1 : 0, k2 = rest ? __ffs((int)rest) - 1 : 0;
+      const int a = nbr[(long long)(has ? (mirror >= 0 ? mirror - k1 : k1) : 0) * n_rows + (has ? row : 0)];
+      const int b = nbr[(long long)(rest ? (mirror >= 0 ? mirror - k2 : k2) : 0) * n_rows + (has ? row : 0)];
+      near[j][0] = a;
+      near[j][1] = rest ? b : -1;
+    }
+#pragma unroll
+    for (int j = 0; j < ORDER_BATCH; ++j) {
+      const long long row = row0 + (t0 + j) * 64;
+      const unsigned long long b = __ballot(m[j] == 0);
+      if (m[j] == 0) {
+        perm[plain_at + __popcll(b & ((1ull << lane) - 1ull))] = (int)row;
+      } else if (m[j] != none) {
+        const int key = order_key(m[j]);
+        const long long at = atomicAdd(&cnt[key], 1), p = n_plain + at;
+        perm[p] = (int)row;
+        // the record of the row: what a wavefront of the ordered dataflow reads of it in one load
+        reinterpret_cast<int4 *>(order + PCE_ORDER_REC_OFFSET(n_rows))[p] = make_int4((int)row, (int)m[j], near[j][0], near[j][1]);
+        // rows with two neighbours or more: the 128-byte record with the neighbour at every offset
+        const long long si = at - n_single;
+        if (key >= 32 && shared_records) {
+          int v[32];
+          v[0] = (int)row;
+          v[1] = (int)m[j];
+#pragma unroll
+          for (int k = 0; k < PCE_ORDER_SREC_KV; ++k) {   // (loads from an address valid for every k, selected afterwards)
+            const bool has = (m[j] >> k) & 1u;
+            const int x = nbr[(long long)(has ? (mirror >= 0 ? mirror - k : k) : 0) * n_rows + row];
+            v[2 + k] = has ? x : -1;
+          }
+          pce_v4i *dst = reinterpret_cast<pce_v4i *>(order + PCE_ORDER_SREC_OFFSET(n_rows) + si * 32);
+#pragma unroll
+          for (int q = 0; q < 8; ++q) dst[q] = pce_v4i{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+        }
       }
-      pce_v4i *dst = reinterpret_cast<pce_v4i *>(order + PCE_ORDER_SREC_OFFSET(n_rows) + si * 32);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) dst[q] = pce_v4i{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+      plain_at += __popcll(b);
     }
   }
 }
@@ -2157,7 +2233,7 @@ __device__ __forceinline__ void order_scatter_block(long long n_rows, int *__res
 // its own row (nine cells; a probe of half the offsets with mirrored writes, as above, leaves a row's results
 // scattered over the lanes of other rows) and so holds everything about the row at once -- it writes the
 // output-major table nbr_out[k][o] = row at coords[o] + d(k) (coalesced, the centre row the identity), the row's
-// offset mask and the key histogram of the row order, and what the pair lists need: by the symmetry of such a map
+// offset mask, and what the pair lists need: by the symmetry of such a map
 // row o is the INPUT of a pair at offset k exactly when it has a neighbour at 26 - k, so the wave ballots are the
 // (offset, 64-row segment) counts of the pair lists and the popcount of the mask is the row's CSR length.  No
 // probe table, no counting pass, no -1 prefill.  lazy: no pair lists are wanted; the counts per offset go to knnz
@@ -2184,10 +2260,7 @@ __global__ void __launch_bounds__(256) grid_query_full3_kernel(const ProbDev *__
     q.status[0] = 1;
     live = false;
   }
-  __shared__ int keycnt[ORDER_KEYS];
   __shared__ int offcnt[32];
-  if (order)
-    for (int t = threadIdx.x; t < ORDER_KEYS; t += 256) keycnt[t] = 0;
   if (threadIdx.x < 32) offcnt[threadIdx.x] = 0;
   __syncthreads();
   int2 se[9];
@@ -2276,16 +2349,8 @@ __global__ void __launch_bounds__(256) grid_query_full3_kernel(const ProbDev *__
     if (want_csr && i <= n) q.icsr[i] = live ? __popc(m) : 0;   // icsr[n] = 0 receives the total after the scan
     if (i == 0) q.seg[27 * nseg] = 0;
   }
-  if (order && live) {
-    q.order[n + i] = (int)m;
-    if (m) atomicAdd(&keycnt[order_key(m)], 1);   // rows without neighbours are placed by the scatter pass
-  }
+  if (order && i < n) q.order[n + i] = (int)m;   // (0 for a coordinate out of range)
   __syncthreads();
-  if (order) {
-    int *hist = q.order + 2 * n + ORDER_HIST;
-    for (int t = threadIdx.x; t < ORDER_KEYS; t += 256)
-      if (keycnt[t]) atomicAdd(&hist[t], keycnt[t]);
-  }
   if (lazy && threadIdx.x < 27 && offcnt[threadIdx.x]) atomicAdd(&q.knnz[threadIdx.x], offcnt[threadIdx.x]);
 }
 
@@ -2306,13 +2371,8 @@ __global__ void __launch_bounds__(256) kmap_count_kernel(const ProbDev *__restri
   long long seg = i >> 6;
   bool live = i < n_in;
   // A symmetric map's output-major table is its probe table mirrored (nbr_out[kp] = dense[kv-1-kp]), so the offset
-  // masks and the key histogram of its row order come out of this pass (order_mask_block does the same from nbr_out).
+  // masks of its row order come out of this pass (order_mask_block forms them from nbr_out).
   const bool masks = q.order && q.g.sym;      // the same for the whole workgroup
-  __shared__ int keycnt[ORDER_KEYS];
-  if (masks) {
-    for (int t = threadIdx.x; t < ORDER_KEYS; t += 256) keycnt[t] = 0;
-    __syncthreads();
-  }
   unsigned m = 0;
   int c = 0;
   for (int kp0 = 0; kp0 < kv; kp0 += ROW_BATCH) {
@@ -2331,21 +2391,23 @@ __global__ void __launch_bounds__(256) kmap_count_kernel(const ProbDev *__restri
   }
   if (rowcnt && i <= n_in) rowcnt[i] = live ? c : 0;  // rowcnt[n_in] = 0 receives the total after the scan
   if (i == 0) segcnt[(long long)kv * nseg] = 0;
-  if (masks) {
-    if (live) {
-      q.order[n_in + i] = (int)m;
-      if (m) atomicAdd(&keycnt[order_key(m)], 1);
-    }
-    __syncthreads();
-    int *hist = q.order + 2 * n_in + ORDER_HIST;
-    for (int t = threadIdx.x; t < ORDER_KEYS; t += 256)
-      if (keycnt[t]) atomicAdd(&hist[t], keycnt[t]);
-  }
+  if (masks && live) q.order[n_in + i] = (int)m;
 }
 
 // Exclusive scans of several arrays in two launches: every workgroup scans its SCAN_TILE items in place
 // and records its total; then every workgroup adds the totals of the workgroups before it in its array.
-__global__ void __launch_bounds__(256) multi_scan_local_kernel(const ScanArr *__restrict__ arrs, int n_arrs) {
+// Workgroups behind the `scan_blocks` of the scans count the keys of the symmetric maps' row orders from their masks.
+__global__ void __launch_bounds__(256) multi_scan_local_kernel(const ScanArr *__restrict__ arrs, int n_arrs, unsigned scan_blocks,
+                                                               const ProbDev *__restrict__ P, JobList order) {
+  if (blockIdx.x >= scan_blocks) {
+    __shared__ int cnt[ORDER_KEYS];
+    const Job &job = find_job(order, blockIdx.x - scan_blocks);
+    const ProbDev &q = P[job.prob];
+    const long long n = q.n_out;
+    const PCE_GLOBAL int *masks = (const PCE_GLOBAL int *)(q.order + n);
+    order_count_block(n, q.order + 2 * n, blockIdx.x - scan_blocks - job.blk0, job.per, cnt, [&](long long row) { return (unsigned)masks[row]; });
+    return;
+  }
   int a = 0;
   while (a + 1 < n_arrs && blockIdx.x >= arrs[a + 1].blk0) ++a;
   const ScanArr arr = arrs[a];
@@ -2387,7 +2449,7 @@ __global__ void __launch_bounds__(256) multi_scan_add_kernel(const ScanArr *__re
 // kpos[kp] = first pair of offset kp; then the scan of counts rounded up to the tile height
 // (backend/hash.cuh:478-497).  One workgroup per problem.
 // Workgroups [n_probs, 2 n_probs): the bases of the row order's counting sort for the maps whose key histogram the
-// counting pass has filled (symmetric maps).
+// launch of the scans has filled (symmetric maps).
 __global__ void __launch_bounds__(1024) kmap_offsets_kernel(const ProbDev *__restrict__ P, int n_probs) {
   if ((int)blockIdx.x >= n_probs) {
     const ProbDev &o = P[blockIdx.x - n_probs];
@@ -2525,13 +2587,22 @@ __device__ __forceinline__ void fill_rows(const ProbDev &q, int block) {
 }
 
 // The same for the 27 offsets of the fused probe, nine of them to a workgroup of rows: a row's hits at lower offsets are counted
-// by its own mask, so nothing is carried from one offset to the next (the launch 18 -> 10 us on the five levels of a 21 k-voxel
-// scan, 84 -> 80 on those of 100 k voxels, 751 -> 707 on 2 M rows).
+// by its own mask, so nothing is carried from one offset to the next (with the row order's scatter, the launch 18 -> 10 us on the
+// five levels of a 21 k-voxel scan, 84 -> 80 on those of 100 k voxels).  The groups of the same rows, and neighbouring rows, run on one
+// XCD: the lines of the views that several workgroups write a part of meet in its L2 (these workgroups alone: 179 -> 161 us on the
+// five levels of eight indoor scenes, 2.0 M rows; 36 -> 35 on 0.38 M of a scan).
 #define FULL3_GROUPS 3
+// workgroup -> item: workgroups are dealt to the eight XCDs round robin, and each XCD gets one contiguous range of the items
+__device__ __forceinline__ int xcd_contiguous(int block, int blocks) {
+  const int x = block & 7, per = blocks >> 3, more = blocks & 7;
+  return x * per + (x < more ? x : more) + (block >> 3);
+}
 __device__ __forceinline__ void fill_full3(const ProbDev &q, int block) {
   constexpr int N = 27 / FULL3_GROUPS;
   typedef const __attribute__((address_space(4))) int *Uniform;   // read through the scalar cache
-  const int n = (int)q.n_in, nseg = (int)q.nseg, kp0 = block % FULL3_GROUPS * N;
+  const int n = (int)q.n_in, nseg = (int)q.nseg;
+  block = xcd_contiguous(block, FULL3_GROUPS * (n / 256 + 1));
+  const int kp0 = block % FULL3_GROUPS * N;
   const int i = block / FULL3_GROUPS * 256 + threadIdx.x, seg = __builtin_amdgcn_readfirstlane(i >> 6);
   const bool live = i < n;
   const PCE_GLOBAL int *table = (const PCE_GLOBAL int *)q.nbr_out, *csr = (const PCE_GLOBAL int *)q.icsr, *masks = (const PCE_GLOBAL int *)(q.order + n);
@@ -2582,9 +2653,9 @@ __global__ void __launch_bounds__(256) kmap_fill_kernel(const ProbDev *__restric
     // (a symmetric map: the fill jobs of this launch may be writing nbr_out, so the probe table is read, mirrored,
     // unless the probe wrote the output-major table itself)
     if (q.fused)
-      order_scatter_block(q.n_out, q.order, blockIdx.x - job.blk0, q.nbr_out, -1);
+      order_scatter_block(q.n_out, q.order, blockIdx.x - job.blk0, job.per, q.nbr_out, -1);
     else
-      order_scatter_block(q.n_out, q.order, blockIdx.x - job.blk0, q.dense, q.g.kv - 1);
+      order_scatter_block(q.n_out, q.order, blockIdx.x - job.blk0, job.per, q.dense, q.g.kv - 1);
     return;
   }
   if (job.kind == JOB_FILL_FULL3)
@@ -2721,20 +2792,20 @@ __global__ void order_clear_kernel(int *tail) {
   for (int i = threadIdx.x; i < PCE_ORDER_TAIL; i += blockDim.x) tail[i] = 0;
 }
 __global__ void __launch_bounds__(256) order_mask_kernel(const int *__restrict__ nbr, int kv, long long n_rows, int mid,
-                                                         int *__restrict__ order) {
-  order_mask_block(nbr, kv, n_rows, mid, order, blockIdx.x);
+                                                         int *__restrict__ order, int per) {
+  order_mask_block(nbr, kv, n_rows, mid, order, blockIdx.x, per);
 }
 __global__ void __launch_bounds__(1024) order_scan_kernel(int *tail) { order_scan_block(tail, nullptr); }
 __global__ void __launch_bounds__(256) order_scatter_kernel(long long n_rows, int *__restrict__ order,
-                                                            const int *__restrict__ nbr) {
-  order_scatter_block(n_rows, order, blockIdx.x, nbr, -1);
+                                                            const int *__restrict__ nbr, int per) {
+  order_scatter_block(n_rows, order, blockIdx.x, per, nbr, -1);
 }
 
 // the same over the problems of a batched build; status[4] of a problem receives its number of heavy rows
 __global__ void __launch_bounds__(256) order_mask_batch_kernel(const ProbDev *__restrict__ P, JobList jl) {
   const Job &job = find_job(jl, blockIdx.x);
   const ProbDev &q = P[job.prob];
-  order_mask_block(q.nbr_out, q.g.kv, q.n_out, q.g.subm ? q.g.mid : -1, q.order, blockIdx.x - job.blk0);
+  order_mask_block(q.nbr_out, q.g.kv, q.n_out, q.g.subm ? q.g.mid : -1, q.order, blockIdx.x - job.blk0, job.per);
 }
 __global__ void __launch_bounds__(1024) order_scan_batch_kernel(const ProbDev *__restrict__ P) {
   const ProbDev &q = P[blockIdx.x];
@@ -2744,7 +2815,7 @@ __global__ void __launch_bounds__(1024) order_scan_batch_kernel(const ProbDev *_
 __global__ void __launch_bounds__(256) order_scatter_batch_kernel(const ProbDev *__restrict__ P, JobList jl) {
   const Job &job = find_job(jl, blockIdx.x);
   const ProbDev &q = P[job.prob];
-  order_scatter_block(q.n_out, q.order, blockIdx.x - job.blk0, q.nbr_out, -1);
+  order_scatter_block(q.n_out, q.order, blockIdx.x - job.blk0, job.per, q.nbr_out, -1);
 }
 
 extern "C" int64_t pce_row_order_elems(int64_t n_rows) { return n_rows < 0 ? 0 : PCE_ORDER_ELEMS(n_rows); }
@@ -2760,14 +2831,15 @@ extern "C" int pce_row_order(const int32_t *nbr, int32_t kv, int64_t n_rows, int
     PCE_FAIL(PCE_EWORKSPACE, "pce_row_order: order holds %lld elements, needs %lld", (long long)order_elems, (long long)pce_row_order_elems(n_rows));
   hipStream_t s = (hipStream_t)stream;
   int *tail = order + 2 * n_rows;
-  const unsigned blocks = (unsigned)pce_div_up(n_rows, 256);
+  const int per = order_per(n_rows);
+  const unsigned blocks = (unsigned)pce_div_up(n_rows, 256 * per);
   hipLaunchKernelGGL(order_clear_kernel, dim3(1), dim3(1024), 0, s, tail);
   PCE_LAUNCH_CHECK("order_clear");
-  hipLaunchKernelGGL(order_mask_kernel, dim3(blocks), dim3(256), 0, s, nbr, (int)kv, (long long)n_rows, (int)mid, order);
+  hipLaunchKernelGGL(order_mask_kernel, dim3(blocks), dim3(256), 0, s, nbr, (int)kv, (long long)n_rows, (int)mid, order, per);
   PCE_LAUNCH_CHECK("order_mask");
   hipLaunchKernelGGL(order_scan_kernel, dim3(1), dim3(1024), 0, s, tail);
   PCE_LAUNCH_CHECK("order_scan");
-  hipLaunchKernelGGL(order_scatter_kernel, dim3(blocks), dim3(256), 0, s, (long long)n_rows, order, (const int *)nbr);
+  hipLaunchKernelGGL(order_scatter_kernel, dim3(blocks), dim3(256), 0, s, (long long)n_rows, order, (const int *)nbr, per);
   PCE_LAUNCH_CHECK("order_scatter");
   static_assert(ORDER_N_HEAVY == ORDER_N_NONZERO + 1 && ORDER_N_NONZERO == ORDER_N_SINGLE + 1, "the counts are read back in one copy");
   int counts[3] = {0, 0, 0};
@@ -2780,7 +2852,7 @@ extern "C" int pce_row_order(const int32_t *nbr, int32_t kv, int64_t n_rows, int
 }
 
 enum { ST_INSERT = 0, ST_QUERY, ST_COUNT, ST_FILL, ST_CSR_A, ST_CSR_B, ST_GRID_BUILD, ST_GRID_QUERY, ST_GRID_QUERY3, ST_GRID_FULL3,
-       ST_ORDER_MASK, ST_ORDER_SCATTER, ST_COUNT_ };
+       ST_ORDER_COUNT, ST_ORDER_MASK, ST_ORDER_SCATTER, ST_COUNT_ };
 
 // host-side image of everything the kernels of one batch read
 struct BatchImage {
@@ -2838,12 +2910,13 @@ extern "C" int pce_kmap_build_batch(const pce_kmap_problem_t *probs, int32_t n_p
   unsigned blk[ST_COUNT_] = {};
   unsigned fill_blk = 0, scan_blk[2] = {0, 0};
   int n_fill = 0, n_scan[2] = {0, 0};
-  auto add_job = [&](int stage, int prob, int kind, long long items) {
+  auto add_job = [&](int stage, int prob, int kind, long long items, int per = 1) {
     Job &j = img.jobs[stage][img.n_jobs[stage]++];
     j.blk0 = blk[stage];
     j.prob = prob;
     j.kind = kind;
-    blk[stage] += (unsigned)pce_div_up(items, 256);
+    j.per = per;
+    blk[stage] += (unsigned)pce_div_up(items, 256 * per);
   };
   auto add_fill = [&](void *p, long long words, unsigned zero = 0) {
     if (words <= 0) return;
@@ -2930,9 +3003,13 @@ extern "C" int pce_kmap_build_batch(const pce_kmap_problem_t *probs, int32_t n_p
       if (n_out >= (1ll << 30)) PCE_FAIL(PCE_ECAPACITY, "pce_kmap_build: too many rows for a row order");
       q.order = u.order;
       add_fill(u.order + 2 * n_out, PCE_ORDER_TAIL, 1);
-      if (!q.g.sym) {   // a symmetric map's order rides on the counting, offset and fill launches (see there)
-        add_job(ST_ORDER_MASK, p, 0, n_out);
-        add_job(ST_ORDER_SCATTER, p, 0, n_out);
+      const int per = order_per(n_out);
+      if (q.g.sym) {   // masks from the probe or the counting pass, counted and sorted beside the scans and the pair lists
+        add_job(ST_ORDER_COUNT, p, 0, n_out, per);
+        add_job(ST_FILL, p, JOB_ORDER_SCATTER, n_out, per);
+      } else {
+        add_job(ST_ORDER_MASK, p, 0, n_out, per);
+        add_job(ST_ORDER_SCATTER, p, 0, n_out, per);
       }
     }
     q.want_csr = want_csr;
@@ -2980,7 +3057,6 @@ extern "C" int pce_kmap_build_batch(const pce_kmap_problem_t *probs, int32_t n_p
         add_job(ST_FILL, p, 0, n_in);
       }
     }
-    if (q.order && q.g.sym) add_job(ST_FILL, p, JOB_ORDER_SCATTER, n_out);
     // 5. CSR-coded views
     if (want_csr && q.g.sym) {
       if (!q.order) add_job(ST_CSR_A, p, JOB_CSR_SUBM, n_in + 1);   // else the fill has written them
@@ -3039,9 +3115,12 @@ extern "C" int pce_kmap_build_batch(const pce_kmap_problem_t *probs, int32_t n_p
     hipLaunchKernelGGL(kmap_count_kernel, dim3(blk[ST_COUNT]), dim3(256), 0, s, P, jl(ST_COUNT));
     PCE_LAUNCH_CHECK("kmap_count");
   }
-  if (scan_blk[0]) {
-    hipLaunchKernelGGL(multi_scan_local_kernel, dim3(scan_blk[0]), dim3(256), 0, s, (const ScanArr *)D->scans[0], n_scan[0]);
+  if (scan_blk[0] + blk[ST_ORDER_COUNT]) {
+    hipLaunchKernelGGL(multi_scan_local_kernel, dim3(scan_blk[0] + blk[ST_ORDER_COUNT]), dim3(256), 0, s, (const ScanArr *)D->scans[0],
+                       n_scan[0], scan_blk[0], P, jl(ST_ORDER_COUNT));
     PCE_LAUNCH_CHECK("scan_local");
+  }
+  if (scan_blk[0]) {
     hipLaunchKernelGGL(multi_scan_add_kernel, dim3(scan_blk[0]), dim3(256), 0, s, (const ScanArr *)D->scans[0], n_scan[0]);
     PCE_LAUNCH_CHECK("scan_add");
   }
@@ -3056,7 +3135,8 @@ extern "C" int pce_kmap_build_batch(const pce_kmap_problem_t *probs, int32_t n_p
     PCE_LAUNCH_CHECK("csr_stage_a");
   }
   if (blk[ST_CSR_B]) {
-    hipLaunchKernelGGL(multi_scan_local_kernel, dim3(scan_blk[1]), dim3(256), 0, s, (const ScanArr *)D->scans[1], n_scan[1]);
+    hipLaunchKernelGGL(multi_scan_local_kernel, dim3(scan_blk[1]), dim3(256), 0, s, (const ScanArr *)D->scans[1], n_scan[1],
+                       scan_blk[1], P, JobList{nullptr, 0});
     PCE_LAUNCH_CHECK("scan_local");
     hipLaunchKernelGGL(multi_scan_add_kernel, dim3(scan_blk[1]), dim3(256), 0, s, (const ScanArr *)D->scans[1], n_scan[1]);
     PCE_LAUNCH_CHECK("scan_add");
