@@ -569,8 +569,8 @@ int pce_col_sums(const void *a_dev, const void *b_dev, int32_t dtype, int64_t n,
 int pce_col_affine(const void *x_dev, const void *d_dev, void *y_dev, int32_t dtype, int64_t n, int32_t c,
                    const float *kx_dev, const float *kd_dev, const float *k0_dev, int32_t act, float slope,
                    pce_stream_t stream);
-/* The whole pass in one call (three launches: partial sums, one wavefront per channel for the statistics
- * and coefficients, the affine map).  weight, bias (fp32 [c], NULL: 1 and 0), running_mean / running_var
+/* The whole pass in one call (one launch for few rows; else three: partial sums, the statistics and
+ * coefficients of the channels, the affine map).  weight, bias (fp32 [c], NULL: 1 and 0), running_mean / running_var
  * (fp32 [c]; updated in place with `momentum` and the unbiased variance when use_batch_stats and
  * momentum >= 0; read when !use_batch_stats) follow torch.nn.BatchNorm1d.  save_mean / save_rstd (fp32 [c])
  * receive what pce_bn_backward needs.  grad_weight / grad_bias (fp32 [c]) may be NULL.  ws: device,
@@ -580,14 +580,26 @@ int pce_col_affine(const void *x_dev, const void *d_dev, void *y_dev, int32_t dt
  * passes: forward y = act(bn(x) + residual) (residual_dev [n,c] of the same dtype, or NULL); backward takes
  * dy with respect to y together with y itself (y_act_dev) and the activation, multiplies dy by the
  * activation's derivative (y > 0 ? 1 : 0 or slope) while it reads it, and returns the gradient with respect
- * to x; the gradient with respect to the residual is that masked dy, which the caller forms itself when it
- * needs it (then it passes the masked dy and PCE_ACT_NONE).  LeakyReLU needs slope > 0. */
+ * to x; the gradient with respect to the residual is that masked dy: pce_bn_backward_masked writes it to dy_masked_dev ([n,c] of
+ * the same dtype, no memory of the other operands; dy where y > 0, else 0 or dy * slope rounded to the dtype, and for ReLU dy where y
+ * is NaN) and takes the norm's gradients from it, or the caller forms it itself and passes it with PCE_ACT_NONE.  LeakyReLU needs
+ * slope > 0.  pce_bn_forward_counted adds one to *batches_dev (int64, NULL: none), torch's num_batches_tracked. */
 int64_t pce_bn_workspace_bytes(int64_t n, int32_t c);
 int pce_bn_forward(const void *x_dev, const void *residual_dev, void *y_dev, int32_t dtype, int64_t n, int32_t c,
                    const float *weight_dev, const float *bias_dev, float *running_mean_dev, float *running_var_dev,
                    int32_t use_batch_stats, float momentum, float eps, float *save_mean_dev,
                    float *save_rstd_dev, void *ws_dev, int64_t ws_bytes, int32_t act, float slope,
                    pce_stream_t stream);
+int pce_bn_forward_counted(const void *x_dev, const void *residual_dev, void *y_dev, int32_t dtype, int64_t n, int32_t c,
+                           const float *weight_dev, const float *bias_dev, float *running_mean_dev, float *running_var_dev,
+                           int64_t *batches_dev, int32_t use_batch_stats, float momentum, float eps, float *save_mean_dev,
+                           float *save_rstd_dev, void *ws_dev, int64_t ws_bytes, int32_t act, float slope,
+                           pce_stream_t stream);
+int pce_bn_backward_masked(const void *x_dev, const void *dy_dev, const void *y_act_dev, int32_t act, float slope,
+                           void *dy_masked_dev, void *dx_dev, int32_t dtype, int64_t n, int32_t c, const float *weight_dev,
+                           const float *save_mean_dev, const float *save_rstd_dev, int32_t use_batch_stats,
+                           float *grad_weight_dev, float *grad_bias_dev, void *ws_dev, int64_t ws_bytes,
+                           pce_stream_t stream);
 int pce_bn_backward(const void *x_dev, const void *dy_dev, const void *y_act_dev, int32_t act, float slope,
                     void *dx_dev, int32_t dtype, int64_t n, int32_t c, const float *weight_dev,
                     const float *save_mean_dev, const float *save_rstd_dev, int32_t use_batch_stats,

@@ -1345,13 +1345,14 @@ def _f32(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
 
 
 def bn_forward(x: torch.Tensor, weight, bias, running_mean, running_var, use_batch_stats: bool, momentum: float, eps: float,
-               act=None, residual: Optional[torch.Tensor] = None):
-    """``act(batch_norm(x) + residual)`` over the rows of ``x`` [n, c] (fp16 / fp32) in three launches.
+               act=None, residual: Optional[torch.Tensor] = None, batches: Optional[torch.Tensor] = None):
+    """``act(batch_norm(x) + residual)`` over the rows of ``x`` [n, c] (fp16 / fp32) in one to three launches.
     ``momentum`` < 0 leaves the running statistics alone; they must be fp32 and are updated in place
-    otherwise.  Returns (y, save_mean, save_rstd)."""
+    otherwise.  ``batches``: an int64 tensor of one element that is counted up.  Returns (y, save_mean, save_rstd)."""
     _require_cuda(x, "x")
     code, slope = _act_code(act)
-    done = _lib.bn_forward(x, residual, weight, bias, running_mean, running_var, use_batch_stats, momentum, eps, code, slope, _stream(x.device))
+    done = _lib.bn_forward(x, residual, weight, bias, running_mean, running_var, use_batch_stats, momentum, eps, code, slope, _stream(x.device),
+                           batches)
     if done is not None:
         return done if type(done) is tuple else _lib.check(done)
     lib = _lib.load()
@@ -1364,23 +1365,29 @@ def bn_forward(x: torch.Tensor, weight, bias, running_mean, running_var, use_bat
         if residual.shape != x.shape or residual.dtype != x.dtype or residual.device != x.device:
             raise ValueError("the residual must match the normalised tensor in shape, dtype and device")
         residual = residual.contiguous()
+    if batches is not None and (batches.dtype != torch.int64 or batches.numel() != 1 or batches.device != x.device):
+        raise ValueError("the count of batches must be an int64 tensor of one element")
     w, b = _f32(weight), _f32(bias)
     y = torch.empty_like(x)
     save = torch.empty((2, c), dtype=torch.float32, device=x.device)
     ws_bytes = lib.pce_bn_workspace_bytes(n, c)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-    _lib.check(lib.pce_bn_forward(x.data_ptr(), _ptr(residual), y.data_ptr(), _dtype_code(x), n, c, _ptr(w), _ptr(b),
-                                  _ptr(running_mean), _ptr(running_var), int(use_batch_stats), float(momentum), float(eps),
-                                  save[0].data_ptr(), save[1].data_ptr(), ws.data_ptr(), ws_bytes, code, slope, _stream(x.device)))
+    _lib.check(lib.pce_bn_forward_counted(x.data_ptr(), _ptr(residual), y.data_ptr(), _dtype_code(x), n, c, _ptr(w), _ptr(b),
+                                          _ptr(running_mean), _ptr(running_var), _ptr(batches), int(use_batch_stats), float(momentum),
+                                          float(eps), save[0].data_ptr(), save[1].data_ptr(), ws.data_ptr(), ws_bytes, code, slope,
+                                          _stream(x.device)))
     return y, save[0], save[1]
 
 
 def bn_backward(x: torch.Tensor, dy: torch.Tensor, weight, save_mean: torch.Tensor, save_rstd: torch.Tensor,
-                use_batch_stats: bool, y_act: Optional[torch.Tensor] = None, act=None):
+                use_batch_stats: bool, y_act: Optional[torch.Tensor] = None, act=None, masked: bool = False):
     """(dx, grad_weight fp32, grad_bias fp32) of ``bn_forward``.  With ``act`` and its output ``y_act`` the
-    incoming gradient is taken with respect to the activation's output and masked while it is read."""
+    incoming gradient is taken with respect to the activation's output and masked while it is read; ``masked``: that gradient,
+    the residual's, is the fourth result."""
     code, slope = _act_code(act)
-    done = _lib.bn_backward(x, dy, y_act, weight, save_mean, save_rstd, use_batch_stats, code, slope, _stream(x.device))
+    if masked and code == _lib.ACT_NONE:
+        raise ValueError("a masked gradient needs an activation")
+    done = _lib.bn_backward(x, dy, y_act, weight, save_mean, save_rstd, use_batch_stats, code, slope, _stream(x.device), masked)
     if done is not None:
         return done if type(done) is tuple else _lib.check(done)
     lib = _lib.load()
@@ -1400,10 +1407,11 @@ def bn_backward(x: torch.Tensor, dy: torch.Tensor, weight, save_mean: torch.Tens
     grads = torch.empty((2, c), dtype=torch.float32, device=x.device)
     ws_bytes = lib.pce_bn_workspace_bytes(n, c)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-    _lib.check(lib.pce_bn_backward(x.data_ptr(), dy.data_ptr(), _ptr(y_act), code, slope, dx.data_ptr(), _dtype_code(x), n, c,
-                                   _ptr(w), save_mean.data_ptr(), save_rstd.data_ptr(), int(use_batch_stats),
-                                   grads[0].data_ptr(), grads[1].data_ptr(), ws.data_ptr(), ws_bytes, _stream(x.device)))
-    return dx, grads[0], grads[1]
+    dm = torch.empty_like(x) if masked else None
+    _lib.check(lib.pce_bn_backward_masked(x.data_ptr(), dy.data_ptr(), _ptr(y_act), code, slope, _ptr(dm), dx.data_ptr(), _dtype_code(x), n, c,
+                                          _ptr(w), save_mean.data_ptr(), save_rstd.data_ptr(), int(use_batch_stats),
+                                          grads[0].data_ptr(), grads[1].data_ptr(), ws.data_ptr(), ws_bytes, _stream(x.device)))
+    return (dx, grads[0], grads[1]) + ((dm,) if masked else ())
 
 
 def conv_wgrad(feats: torch.Tensor, grad_out: torch.Tensor, km: KernelMap, transposed: bool = False) -> torch.Tensor:

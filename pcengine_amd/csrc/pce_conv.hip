@@ -4067,17 +4067,17 @@ extern "C" int pce_conv_wgrad(const void *in, const void *gout, int32_t dtype, i
 }
 
 // ---- batch normalisation over the rows of a feature matrix (script/batchnorm.py:7-10) -----------------
-// Two kernels carry the forward and the backward pass of nn.BatchNorm1d on [n, c]:
+// Two kinds of pass carry the forward and the backward pass of nn.BatchNorm1d on [n, c]:
 //   column sums:   out[j] = sum_r a[r][j],  out[c + j] = sum_r a[r][j] * b[r][j]   (b = a when b is null)
 //     forward statistics from (x, x): sum and sum of squares; backward from (dy, x): sum dy, sum dy*x
 //   column affine: y[r][j] = act(x[r][j] * kx[j] + d[r][j] * kd[j] + k0[j])         (d may be null)
 //     forward: y = x * (w*rstd) + (b - mean*w*rstd); backward: dx = dy*k1 + x*k2 + k3
-// The per-channel coefficients between them are c-element vector arithmetic left to the caller.
-// A thread owns VEC adjacent columns (one 16-byte vector when the layout allows) and walks down the rows in
-// steps of the grid, 8 rows requested at a time; sums are accumulated in fp32 over those 8 rows, then in fp64:
-// per workgroup through LDS, across workgroups by a second kernel over the per-workgroup partial sums (no
-// atomics: same bits every run).  At most BN_MAX_ROW_BLOCKS workgroups share the rows: three per CU, what the
-// vector forms keep resident, so that no second, partial round of workgroups follows the first.
+// Few rows: one kernel does both (bn_small_kernel).  Otherwise three: partial sums, coefficients, affine map.  A thread owns
+// VEC adjacent columns (one 16-byte vector when the layout allows) and walks down the rows, several requested at a time.  Sums are
+// accumulated in fp32 over at most 8 rows, always the same ones (bn_groups), then in fp64: per workgroup through LDS, across
+// workgroups by a second kernel over the per-workgroup partial sums (no atomics).  So whatever the split, the sums differ by roundings
+// in fp64 alone, and what is rounded to fp32 from them hardly ever: a statistic that differs in its last bit decides signs at ReLU
+// boundaries.
 #define BN_ROWS_IN_FLIGHT 8
 #define BN_MAX_ROW_BLOCKS 768
 template <typename T, int VEC>
@@ -4088,66 +4088,122 @@ __device__ __forceinline__ float vec_get(const typename VecOf<T, VEC>::type &v, 
     return (float)v[j];
 }
 template <typename T, int VEC>
+__device__ __forceinline__ void vec_set(typename VecOf<T, VEC>::type &v, int j, float x) {
+  if constexpr (VEC == 1)
+    v = (T)x;
+  else
+    v[j] = (T)x;
+}
+template <typename T, int VEC>
 __device__ __forceinline__ typename VecOf<T, VEC>::type vec_zero() {
   typename VecOf<T, VEC>::type v;
-  if constexpr (VEC == 1) {
-    v = (T)0;
-  } else {
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) v[j] = (T)0;
-  }
+  for (int j = 0; j < VEC; ++j) vec_set<T, VEC>(v, j, 0.f);
   return v;
 }
-// GATED: a third operand (the gate) is read, and half as many rows are requested per step
-template <typename T, int VEC, bool GATED>
-__global__ void __launch_bounds__(256) col_sums_partial_kernel(const T *__restrict__ a, const T *__restrict__ b,
-                                                               const T *__restrict__ gate, int gate_act, float gate_slope,
-                                                               long long n, int c, int cols_per_block,
-                                                               double *__restrict__ partial) {
+
+// What a gradient goes through before it enters the norm's backward pass: GATE_SLOPE multiplies it by the derivative of an
+// activation whose output is the gate, GATE_MASK forms the gradient of a residual sum's two terms from that of its activation (the
+// values torch's threshold_backward and where give, rounded to T), which is written out as well.
+enum Gate { GATE_NONE = 0, GATE_SLOPE = 1, GATE_MASK = 2 };
+struct GateArgs {
+  const void *gate;   // the activation's output
+  void *out;          // GATE_MASK
+  int act;
+  float slope;
+};
+template <typename T, int GATE>
+__device__ __forceinline__ float gated(float x, float gate, const GateArgs &g) {
+  if (GATE == GATE_SLOPE) return x * act_slope_at(gate, g.act, g.slope);
+  if (GATE == GATE_MASK) return g.act == PCE_ACT_RELU ? (gate <= 0.f ? 0.f : x) : (gate > 0.f ? x : (float)(T)(x * g.slope));
+  return x;
+}
+
+// Threads -> (vector column, row lane): cpb vector columns side by side, then the next row; what does not make a whole row of the
+// 256 threads is idle.
+struct ColSplit {
+  int cpb, lanes;
+};
+static ColSplit col_split(int vcols) {
+  ColSplit p;
+  p.cpb = vcols < 256 ? vcols : 256;
+  p.lanes = 256 / p.cpb;
+  return p;
+}
+
+// The rows whose terms are added up in fp32: g, g + groups, g + 2 groups ... (BN_ROWS_IN_FLIGHT of them, half as many of three
+// operands; then the next so many), for g below `groups`.
+static int bn_columns(int vcols) {
+  int cols = 1;
+  while (cols < vcols && cols < 256) cols <<= 1;
+  return cols;
+}
+static int64_t bn_groups(int64_t n, int vcols) {
+  const int64_t lanes = 256 / bn_columns(vcols), blocks = pce_div_up(n, lanes * BN_ROWS_IN_FLIGHT);
+  return lanes * (blocks < BN_MAX_ROW_BLOCKS ? blocks : BN_MAX_ROW_BLOCKS);
+}
+template <int GATE>
+struct BnRows {
+  static constexpr int N = GATE ? BN_ROWS_IN_FLIGHT / 2 : BN_ROWS_IN_FLIGHT;
+};
+// the terms of one such group, from row r0 on
+template <typename T, int VEC, int GATE>
+__device__ __forceinline__ void bn_group(const T *__restrict__ a, const T *__restrict__ b, const GateArgs &g, long long r0, long long groups,
+                                         long long n, int c, int col0, bool write, double (&s1)[VEC], double (&s2)[VEC]) {
   typedef typename VecOf<T, VEC>::type V;
-  constexpr int ROWS = GATED ? BN_ROWS_IN_FLIGHT / 2 : BN_ROWS_IN_FLIGHT;
-  // thread -> (vector column, row lane): a workgroup covers cols_per_block vector columns (a power of two up to
-  // 256) with 256 / cols_per_block row lanes; blockIdx.y walks over the column blocks
-  const int tc = threadIdx.x % cols_per_block;
-  const int col0 = (blockIdx.y * cols_per_block + tc) * VEC;
-  const int lanes = 256 / cols_per_block, rl = threadIdx.x / cols_per_block;
+  constexpr int ROWS = BnRows<GATE>::N;
+  // all loads are requested before the first is used
+  V xs[ROWS], ys[ROWS], gs[GATE ? ROWS : 1];
+  const V zero = vec_zero<T, VEC>();
+#pragma unroll
+  for (int k = 0; k < ROWS; ++k) {
+    const long long r = r0 + k * groups;
+    xs[k] = r < n ? *reinterpret_cast<const V *>(a + r * c + col0) : zero;
+    ys[k] = b ? (r < n ? *reinterpret_cast<const V *>(b + r * c + col0) : zero) : xs[k];
+    if (GATE) gs[k] = r < n ? *reinterpret_cast<const V *>((const T *)g.gate + r * c + col0) : zero;
+  }
+  float f1[VEC], f2[VEC];
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) f1[j] = f2[j] = 0.f;
+#pragma unroll
+  for (int k = 0; k < ROWS; ++k) {
+    V masked = xs[k];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      float x = vec_get<T, VEC>(xs[k], j);
+      const float y = vec_get<T, VEC>(ys[k], j);
+      if (GATE) x = gated<T, GATE>(x, vec_get<T, VEC>(gs[k], j), g);
+      if (GATE == GATE_MASK) vec_set<T, VEC>(masked, j, x);
+      f1[j] += x;
+      f2[j] = fmaf(x, y, f2[j]);   // (spelled out: one kernel had it, another multiplied first)
+    }
+    const long long r = r0 + k * groups;
+    if (GATE == GATE_MASK && write && r < n) *reinterpret_cast<V *>((T *)g.out + r * c + col0) = masked;
+  }
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) {
+    s1[j] += (double)f1[j];
+    s2[j] += (double)f2[j];
+  }
+}
+
+// Bound by the bytes of its operands where they are many, by one trip to memory, the LDS sum and the launch where they are few.
+// cpb: vector columns of a workgroup, a power of two up to 256 (with as many as a row has, the lanes left over put to use, a
+// workgroup's sums over the lanes cost what that gained).
+template <typename T, int VEC, int GATE>
+__global__ void __launch_bounds__(256) col_sums_partial_kernel(const T *__restrict__ a, const T *__restrict__ b, GateArgs g, long long n, int c,
+                                                               int cpb, double *__restrict__ partial) {
+  const int tc = threadIdx.x % cpb, lanes = 256 / cpb, rl = threadIdx.x / cpb;
+  const int col0 = (blockIdx.y * cpb + tc) * VEC;
   double s1[VEC], s2[VEC];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) s1[j] = s2[j] = 0.0;
   if (col0 < c) {
-    const long long stride = (long long)gridDim.x * lanes;
-    for (long long r0 = (long long)blockIdx.x * lanes + rl; r0 < n; r0 += stride * ROWS) {
-      // all loads of a step are requested before the first is used
-      V xs[ROWS], ys[ROWS], gs[GATED ? ROWS : 1];
-      const V zero = vec_zero<T, VEC>();
-#pragma unroll
-      for (int k = 0; k < ROWS; ++k) {
-        const long long r = r0 + k * stride;
-        xs[k] = r < n ? *reinterpret_cast<const V *>(a + r * c + col0) : zero;
-        ys[k] = b ? (r < n ? *reinterpret_cast<const V *>(b + r * c + col0) : zero) : xs[k];
-        if (GATED) gs[k] = r < n ? *reinterpret_cast<const V *>(gate + r * c + col0) : zero;
-      }
-      float f1[VEC], f2[VEC];
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) f1[j] = f2[j] = 0.f;
-#pragma unroll
-      for (int k = 0; k < ROWS; ++k)
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) {
-          float x = vec_get<T, VEC>(xs[k], j);
-          const float y = vec_get<T, VEC>(ys[k], j);
-          if (GATED) x *= act_slope_at(vec_get<T, VEC>(gs[k], j), gate_act, gate_slope);
-          f1[j] += x;
-          f2[j] += x * y;
-        }
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) {
-        s1[j] += (double)f1[j];
-        s2[j] += (double)f2[j];
-      }
-    }
+    const long long groups = (long long)gridDim.x * lanes;   // bn_groups()
+    for (long long r0 = (long long)blockIdx.x * lanes + rl; r0 < n; r0 += groups * BnRows<GATE>::N)
+      bn_group<T, VEC, GATE>(a, b, g, r0, groups, n, c, col0, true, s1, s2);
   }
-  // the row lanes of a column are cols_per_block threads apart: halving tree over them, both sums at once
+  // the row lanes of a column are cpb threads apart: halving tree over them, both sums at once
   __shared__ double red[2 * VEC * 256];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
@@ -4160,7 +4216,7 @@ __global__ void __launch_bounds__(256) col_sums_partial_kernel(const T *__restri
     if (rl < off) {
       double other[2 * VEC];
 #pragma unroll
-      for (int q = 0; q < 2 * VEC; ++q) other[q] = red[q * 256 + threadIdx.x + off * cols_per_block];
+      for (int q = 0; q < 2 * VEC; ++q) other[q] = red[q * 256 + threadIdx.x + off * cpb];
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
         s1[j] += other[j];
@@ -4237,33 +4293,33 @@ extern "C" int64_t pce_col_sums_workspace_bytes(int64_t n, int32_t c) {
 }
 
 // launches the partial-sum kernel; *blocks_out = row blocks written (partial[block][2][c])
-static int bn_partial(const void *a, const void *b, const void *gate, int gate_act, float gate_slope, int32_t dtype, int64_t n,
-                      int32_t c, double *partial, int64_t *blocks_out, hipStream_t s) {
+static int bn_partial(const void *a, const void *b, int gate, const GateArgs &g, int32_t dtype, int64_t n, int32_t c, double *partial,
+                      int64_t *blocks_out, hipStream_t s) {
   const int full = dtype == PCE_F16 ? 8 : 4;
-  const int vec = (c % full == 0 && aligned16(a) && aligned16(b) && aligned16(gate)) ? full : 1;
-  const int vcols = c / vec;
-  int cpb = 1;   // vector columns per workgroup: the power of two >= vcols, at most 256
-  while (cpb < vcols && cpb < 256) cpb <<= 1;
-  const int lanes = 256 / cpb;
-  int64_t blocks = pce_div_up(n, (int64_t)lanes * BN_ROWS_IN_FLIGHT);
-  if (blocks > BN_MAX_ROW_BLOCKS) blocks = BN_MAX_ROW_BLOCKS;
+  const int vec = (c % full == 0 && aligned16(a) && aligned16(b) && aligned16(g.gate) && aligned16(g.out)) ? full : 1;
+  const int vcols = c / vec, cpb = bn_columns(vcols);
+  const int64_t blocks = bn_groups(n, vcols) / (256 / cpb);
   dim3 grid((unsigned)blocks, (unsigned)pce_div_up(vcols, cpb));
-#define PCE_COLSUMS(T_, V_)                                                                                                   \
-  if (gate)                                                                                                                  \
-    hipLaunchKernelGGL((col_sums_partial_kernel<T_, V_, true>), grid, dim3(256), 0, s, (const T_ *)a,       \
-                       (const T_ *)b, (const T_ *)gate, gate_act, gate_slope, (long long)n, c, cpb, partial);                \
-  else                                                                                                                       \
-    hipLaunchKernelGGL((col_sums_partial_kernel<T_, V_, false>), grid, dim3(256), 0, s, (const T_ *)a,                       \
-                       (const T_ *)b, (const T_ *)gate, gate_act, gate_slope, (long long)n, c, cpb, partial)
-  if (dtype == PCE_F16 && vec == 8)
+#define PCE_COLSUMS_(T_, V_, G_)                                                                                             \
+  hipLaunchKernelGGL((col_sums_partial_kernel<T_, V_, G_>), grid, dim3(256), 0, s, (const T_ *)a, (const T_ *)b, g, (long long)n, c, cpb, partial)
+#define PCE_COLSUMS(T_, V_)               \
+  if (gate == GATE_MASK)                  \
+    PCE_COLSUMS_(T_, V_, GATE_MASK);      \
+  else if (gate == GATE_SLOPE)            \
+    PCE_COLSUMS_(T_, V_, GATE_SLOPE);     \
+  else                                    \
+    PCE_COLSUMS_(T_, V_, GATE_NONE)
+  if (dtype == PCE_F16 && vec == 8) {
     PCE_COLSUMS(half_t, 8);
-  else if (dtype == PCE_F16)
+  } else if (dtype == PCE_F16) {
     PCE_COLSUMS(half_t, 1);
-  else if (vec == 4)
+  } else if (vec == 4) {
     PCE_COLSUMS(float, 4);
-  else
+  } else {
     PCE_COLSUMS(float, 1);
+  }
 #undef PCE_COLSUMS
+#undef PCE_COLSUMS_
   PCE_LAUNCH_CHECK("col_sums_partial");
   *blocks_out = blocks;
   return PCE_OK;
@@ -4278,7 +4334,7 @@ extern "C" int pce_col_sums(const void *a, const void *b, int32_t dtype, int64_t
   if (!ws || ws_bytes < need) PCE_FAIL(PCE_EWORKSPACE, "pce_col_sums: workspace %lld < %lld", (long long)ws_bytes, (long long)need);
   hipStream_t s = (hipStream_t)stream;
   int64_t blocks = 0;
-  int rc = bn_partial(a, b, nullptr, PCE_ACT_NONE, 0.f, dtype, n, c, (double *)ws, &blocks, s);
+  int rc = bn_partial(a, b, GATE_NONE, GateArgs{}, dtype, n, c, (double *)ws, &blocks, s);
   if (rc) return rc;
   hipLaunchKernelGGL(col_sums_final_kernel, dim3((unsigned)c), dim3(64), 0, s, (const double *)ws,
                      (long long)blocks, c, out);
@@ -4286,147 +4342,355 @@ extern "C" int pce_col_sums(const void *a, const void *b, int32_t dtype, int64_t
   return PCE_OK;
 }
 
-// One wavefront per channel: adds up the per-workgroup partial sums and turns them into what the affine pass
-// needs.  Forward (sums of x and x*x): mean, biased variance, rstd; coefficients kx = w*rstd,
-// k0 = b - mean*kx; running statistics updated with the unbiased variance (torch.nn.BatchNorm1d).
-__global__ void __launch_bounds__(64) bn_finish_forward_kernel(const double *__restrict__ partial, long long blocks,
-                                                                long long n, int c, const float *__restrict__ weight,
-                                                                const float *__restrict__ bias, float *running_mean,
-                                                                float *running_var, int use_batch_stats, float momentum,
-                                                                float eps, float *__restrict__ save_mean,
-                                                                float *__restrict__ save_rstd, float *__restrict__ kx,
-                                                                float *__restrict__ k0, float *__restrict__ ones) {
-  const int j = blockIdx.x;   // one wavefront per channel
+// What a channel's sums become.  Forward (sums of x and x*x): mean, biased variance, rstd; coefficients kx = w*rstd,
+// k0 = b - mean*kx; running statistics updated with the unbiased variance (torch.nn.BatchNorm1d), and the count of batches.
+struct BnForward {
+  const float *weight, *bias;
+  float *running_mean, *running_var;
+  long long *batches;    // counted up by the first channel, or null
+  int use_batch_stats;
+  float momentum, eps;
+  float *save_mean, *save_rstd;
+  long long n;
+  int c;
+};
+__device__ __forceinline__ void bn_forward_channel(const BnForward &f, int j, double s1, double s2, bool keep, float *kx, float *k0) {
   double mean, var;
-  if (use_batch_stats) {
-    double s1 = 0.0, s2 = 0.0;
-    wave_sum_partials(partial, blocks, c, j, &s1, &s2);
-    if (threadIdx.x != 0) return;
-    mean = s1 / (double)n;
-    var = s2 / (double)n - mean * mean;
+  if (f.use_batch_stats) {
+    mean = s1 / (double)f.n;
+    var = s2 / (double)f.n - mean * mean;
     if (var < 0.0) var = 0.0;
-    if (momentum >= 0.f && running_mean && running_var) {
-      double unbiased = n > 1 ? var * ((double)n / (double)(n - 1)) : var;
-      running_mean[j] = (float)((1.0 - momentum) * running_mean[j] + momentum * mean);
-      running_var[j] = (float)((1.0 - momentum) * running_var[j] + momentum * unbiased);
+    if (keep && f.momentum >= 0.f && f.running_mean && f.running_var) {
+      double unbiased = f.n > 1 ? var * ((double)f.n / (double)(f.n - 1)) : var;
+      f.running_mean[j] = (float)((1.0 - f.momentum) * f.running_mean[j] + f.momentum * mean);
+      f.running_var[j] = (float)((1.0 - f.momentum) * f.running_var[j] + f.momentum * unbiased);
     }
   } else {
-    if (threadIdx.x != 0) return;
-    mean = running_mean[j];
-    var = running_var[j];
+    mean = f.running_mean[j];
+    var = f.running_var[j];
   }
-  double rstd = 1.0 / sqrt(var + (double)eps);
-  double w = weight ? (double)weight[j] : 1.0, b = bias ? (double)bias[j] : 0.0;
-  save_mean[j] = (float)mean;
-  save_rstd[j] = (float)rstd;
-  kx[j] = (float)(w * rstd);
-  k0[j] = (float)(b - mean * w * rstd);
-  if (ones) ones[j] = 1.f;   // coefficient of the residual term of the affine map
+  double rstd = 1.0 / sqrt(var + (double)f.eps);
+  double w = f.weight ? (double)f.weight[j] : 1.0, b = f.bias ? (double)f.bias[j] : 0.0;
+  if (keep) {
+    f.save_mean[j] = (float)mean;
+    f.save_rstd[j] = (float)rstd;
+    if (j == 0 && f.batches) *f.batches += 1;
+  }
+  *kx = (float)(w * rstd);
+  *k0 = (float)(b - mean * w * rstd);
 }
 
 // Backward (sums of dy and dy*x): grad_bias = sum dy, grad_weight = S = sum dy*xhat,
 // dx = dy*k1 + x*kd + k0 with k1 = w*rstd, kd = -k1*rstd*S/n, k0 = -k1*sum(dy)/n - kd*mean
 // (statistics of the batch), or dx = dy*k1 (fixed statistics).
-__global__ void __launch_bounds__(64) bn_finish_backward_kernel(const double *__restrict__ partial, long long blocks,
-                                                                 long long n, int c, const float *__restrict__ weight,
-                                                                 const float *__restrict__ save_mean,
-                                                                 const float *__restrict__ save_rstd, int use_batch_stats,
-                                                                 float *__restrict__ grad_weight, float *__restrict__ grad_bias,
-                                                                 float *__restrict__ k1, float *__restrict__ kd,
-                                                                 float *__restrict__ k0) {
-  const int j = blockIdx.x;   // one wavefront per channel
-  double s1 = 0.0, s2 = 0.0;
-  wave_sum_partials(partial, blocks, c, j, &s1, &s2);
-  if (threadIdx.x != 0) return;
-  const double mean = save_mean[j], rstd = save_rstd[j], w = weight ? (double)weight[j] : 1.0;
+struct BnBackward {
+  const float *weight, *save_mean, *save_rstd;
+  int use_batch_stats;
+  float *grad_weight, *grad_bias;
+  long long n;
+  int c;
+};
+__device__ __forceinline__ void bn_backward_channel(const BnBackward &f, int j, double s1, double s2, bool keep, float *k1, float *kd, float *k0) {
+  const double mean = f.save_mean[j], rstd = f.save_rstd[j], w = f.weight ? (double)f.weight[j] : 1.0;
   const double S = rstd * (s2 - mean * s1);
-  if (grad_weight) grad_weight[j] = (float)S;
-  if (grad_bias) grad_bias[j] = (float)s1;
+  if (keep && f.grad_weight) f.grad_weight[j] = (float)S;
+  if (keep && f.grad_bias) f.grad_bias[j] = (float)s1;
   const double a = w * rstd;
-  k1[j] = (float)a;
-  if (use_batch_stats) {
-    const double d = -a * rstd * S / (double)n;
-    kd[j] = (float)d;
-    k0[j] = (float)(-a * s1 / (double)n - d * mean);
+  *k1 = (float)a;
+  if (f.use_batch_stats) {
+    const double d = -a * rstd * S / (double)f.n;
+    *kd = (float)d;
+    *k0 = (float)(-a * s1 / (double)f.n - d * mean);
   } else {
-    kd[j] = 0.f;
-    k0[j] = 0.f;
+    *kd = 0.f;
+    *k0 = 0.f;
   }
 }
 
-template <typename T, int VEC>
-__global__ void __launch_bounds__(256) col_affine_kernel(const T *__restrict__ x, const T *__restrict__ d, T *__restrict__ y,
-                                                         long long n, int c, const float *__restrict__ kx,
-                                                         const float *__restrict__ kd, const float *__restrict__ k0, int act,
-                                                         float slope, const T *__restrict__ gate, int gate_act,
-                                                         float gate_slope) {
-  typedef typename VecOf<T, VEC>::type V;
-  const int row_vecs = c / VEC;
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n * row_vecs) return;
-  const int v = (int)(i - (i / row_vecs) * row_vecs);
-  V xv = *reinterpret_cast<const V *>(x + i * VEC);
-  V dv = xv, gv = xv;
-  if (d) dv = *reinterpret_cast<const V *>(d + i * VEC);
-  if (gate) gv = *reinterpret_cast<const V *>(gate + i * VEC);
-  V out;
-  // the thread's VEC coefficients are contiguous: 16-byte loads when VEC is a multiple of four
-  float cx[VEC], c0[VEC], cd[VEC];
-  if (VEC % 4 == 0) {
-#pragma unroll
-    for (int q = 0; q < VEC / 4; ++q) {
-      f32x4 a = *reinterpret_cast<const f32x4 *>(kx + v * VEC + q * 4);
-      f32x4 b = *reinterpret_cast<const f32x4 *>(k0 + v * VEC + q * 4);
-      f32x4 e = a;
-      if (d) e = *reinterpret_cast<const f32x4 *>(kd + v * VEC + q * 4);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        cx[q * 4 + j] = a[j];
-        c0[q * 4 + j] = b[j];
-        cd[q * 4 + j] = e[j];
-      }
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) {
-      cx[j] = kx[v * VEC + j];
-      c0[j] = k0[v * VEC + j];
-      cd[j] = d ? kd[v * VEC + j] : 0.f;
-    }
-  }
+// one wavefront per channel
+__global__ void __launch_bounds__(64) bn_finish_forward_kernel(const double *__restrict__ partial, long long blocks, BnForward f,
+                                                                float *__restrict__ kx, float *__restrict__ k0) {
+  const int j = blockIdx.x;
+  double s1 = 0.0, s2 = 0.0;
+  if (f.use_batch_stats) wave_sum_partials(partial, blocks, f.c, j, &s1, &s2);
+  if (threadIdx.x == 0) bn_forward_channel(f, j, s1, s2, true, kx + j, k0 + j);
+}
+
+__global__ void __launch_bounds__(64) bn_finish_backward_kernel(const double *__restrict__ partial, long long blocks, BnBackward f,
+                                                                 float *__restrict__ k1, float *__restrict__ kd, float *__restrict__ k0) {
+  const int j = blockIdx.x;
+  double s1 = 0.0, s2 = 0.0;
+  wave_sum_partials(partial, blocks, f.c, j, &s1, &s2);
+  if (threadIdx.x == 0) bn_backward_channel(f, j, s1, s2, true, k1 + j, kd + j, k0 + j);
+}
+
+// y = act(x' * kx + d * kd + k0) of VEC columns of a row; x' is x gated
+template <typename T, int VEC, int GATE>
+__device__ __forceinline__ typename VecOf<T, VEC>::type affine_vec(const typename VecOf<T, VEC>::type &x, bool has_d,
+                                                                   const typename VecOf<T, VEC>::type &d,
+                                                                   const typename VecOf<T, VEC>::type &gate, const float (&cx)[VEC],
+                                                                   const float (&cd)[VEC], const float (&c0)[VEC], int act, float slope,
+                                                                   const GateArgs &g) {
+  typename VecOf<T, VEC>::type out;
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
-    float xj = (float)(reinterpret_cast<const T *>(&xv)[j]);
-    if (gate) xj *= act_slope_at((float)(reinterpret_cast<const T *>(&gv)[j]), gate_act, gate_slope);
+    float xj = vec_get<T, VEC>(x, j);
+    if (GATE) xj = gated<T, GATE>(xj, vec_get<T, VEC>(gate, j), g);
     float r = xj * cx[j] + c0[j];
-    if (d) r += (float)(reinterpret_cast<const T *>(&dv)[j]) * cd[j];
-    reinterpret_cast<T *>(&out)[j] = (T)act_apply(r, act, slope);
+    if (has_d) r += vec_get<T, VEC>(d, j) * cd[j];
+    vec_set<T, VEC>(out, j, act_apply(r, act, slope));
   }
-  *reinterpret_cast<V *>(y + i * VEC) = out;
+  return out;
 }
 
-// y = act(x' * kx + d * kd + k0), x' = x times the derivative of another activation where its output was `gate`
-static int col_affine_launch(const char *who, const void *x, const void *d, const void *gate, void *y, int32_t dtype, int64_t n,
-                             int32_t c, const float *kx, const float *kd, const float *k0, int32_t act, float slope,
-                             int32_t gate_act, float gate_slope, hipStream_t s) {
-  const int vec = dtype == PCE_F16 ? 8 : 4;
-  const bool aligned = aligned16(x) && aligned16(y) && aligned16(d) && aligned16(gate) && c % vec == 0;
-  const long long items = aligned ? n * (c / vec) : n * c;
-  if (pce_div_up(items, 256) >= (1ll << 31)) PCE_FAIL(PCE_ECAPACITY, "%s: tensor too large for one launch", who);
-  dim3 grid((unsigned)pce_div_up(items, 256));
-#define PCE_AFFINE(T_, V_)                                                                                               \
-  hipLaunchKernelGGL((col_affine_kernel<T_, V_>), grid, dim3(256), 0, s, (const T_ *)x, (const T_ *)d, (T_ *)y, (long long)n, c, \
-                     kx, kd, k0, act, slope, (const T_ *)gate, gate_act, gate_slope)
-  if (dtype == PCE_F16 && aligned)
+// VEC consecutive coefficients, in 16-byte loads when VEC is a multiple of four
+template <int VEC>
+__device__ __forceinline__ void load_columns(const float *__restrict__ from, float (&to)[VEC]) {
+  if constexpr (VEC % 4 == 0) {
+#pragma unroll
+    for (int q = 0; q < VEC / 4; ++q) {
+      const f32x4 v = *reinterpret_cast<const f32x4 *>(from + q * 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) to[q * 4 + j] = v[j];
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) to[j] = from[j];
+  }
+}
+
+// Bound by its bytes.  A thread keeps its columns' coefficients for ROWS rows, whose loads are out together (with one
+// row a thread the whole forward pass over 100 k x 256 in fp16 took 48.2 us, 45.1 so; 100 k x 96 27.7 and 25.8).  kd null: 1.
+#define AFFINE_ROWS 4
+template <typename T, int VEC, int GATE, int ROWS>
+__global__ void __launch_bounds__(256) col_affine_kernel(const T *__restrict__ x, const T *__restrict__ d, T *__restrict__ y, long long n,
+                                                         int c, ColSplit p, const float *__restrict__ kx, const float *__restrict__ kd,
+                                                         const float *__restrict__ k0, int act, float slope, GateArgs g) {
+  typedef typename VecOf<T, VEC>::type V;
+  const int tc = threadIdx.x % p.cpb, rl = threadIdx.x / p.cpb;
+  const int col0 = (blockIdx.y * p.cpb + tc) * VEC;
+  if (rl >= p.lanes || col0 >= c) return;
+  const long long r0 = (long long)blockIdx.x * p.lanes * ROWS + rl;
+  V xs[ROWS], ds[ROWS], gs[ROWS];
+#pragma unroll
+  for (int k = 0; k < ROWS; ++k) {
+    const long long r = r0 + k * p.lanes, at = (r < n ? r : n - 1) * c + col0;
+    xs[k] = *reinterpret_cast<const V *>(x + at);
+    if (d) ds[k] = *reinterpret_cast<const V *>(d + at);
+    if (GATE) gs[k] = *reinterpret_cast<const V *>((const T *)g.gate + at);
+  }
+  float cx[VEC], c0[VEC], cd[VEC];
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) cd[j] = 1.f;
+  load_columns<VEC>(kx + col0, cx);
+  load_columns<VEC>(k0 + col0, c0);
+  if (d && kd) load_columns<VEC>(kd + col0, cd);
+#pragma unroll
+  for (int k = 0; k < ROWS; ++k) {
+    const long long r = r0 + k * p.lanes;
+    if (r < n)
+      *reinterpret_cast<V *>(y + r * c + col0) = affine_vec<T, VEC, GATE>(xs[k], d != nullptr, ds[k], gs[k], cx, cd, c0, act, slope, g);
+  }
+}
+
+// y = act(x' * kx + d * kd + k0), x' = x times the derivative of another activation where its output was the gate
+static int col_affine_launch(const char *who, const void *x, const void *d, void *y, int32_t dtype, int64_t n, int32_t c, const float *kx,
+                             const float *kd, const float *k0, int32_t act, float slope, const GateArgs &g, hipStream_t s) {
+  const int full = dtype == PCE_F16 ? 8 : 4;
+  const int vec = aligned16(x) && aligned16(y) && aligned16(d) && aligned16(g.gate) && c % full == 0 ? full : 1;
+  const int vcols = c / vec;
+  const ColSplit p = col_split(vcols);
+  // one row a thread until that is eight workgroups a compute unit: below, the chain of a thread's rows is what takes the time (4096
+  // rows of 96 columns: 10.3 us for the whole backward pass, 11.1 with four)
+  const bool many = pce_div_up(n, (int64_t)p.lanes) * pce_div_up(vcols, p.cpb) >= 2048;
+  const int64_t blocks = pce_div_up(n, (int64_t)p.lanes * (many ? AFFINE_ROWS : 1));
+  if (blocks >= (1ll << 31)) PCE_FAIL(PCE_ECAPACITY, "%s: tensor too large for one launch", who);
+  dim3 grid((unsigned)blocks, (unsigned)pce_div_up(vcols, p.cpb));
+#define PCE_AFFINE_(T_, V_, G_, R_)                                                                                                      \
+  hipLaunchKernelGGL((col_affine_kernel<T_, V_, G_, R_>), grid, dim3(256), 0, s, (const T_ *)x, (const T_ *)d, (T_ *)y, (long long)n, c, \
+                     p, kx, kd, k0, act, slope, g)
+#define PCE_AFFINE(T_, V_)                           \
+  if (g.gate && many)                                \
+    PCE_AFFINE_(T_, V_, GATE_SLOPE, AFFINE_ROWS);    \
+  else if (g.gate)                                   \
+    PCE_AFFINE_(T_, V_, GATE_SLOPE, 1);              \
+  else if (many)                                     \
+    PCE_AFFINE_(T_, V_, GATE_NONE, AFFINE_ROWS);     \
+  else                                               \
+    PCE_AFFINE_(T_, V_, GATE_NONE, 1)
+  if (dtype == PCE_F16 && vec == 8) {
     PCE_AFFINE(half_t, 8);
-  else if (dtype == PCE_F16)
+  } else if (dtype == PCE_F16) {
     PCE_AFFINE(half_t, 1);
-  else if (aligned)
+  } else if (vec == 4) {
     PCE_AFFINE(float, 4);
-  else
+  } else {
     PCE_AFFINE(float, 1);
+  }
 #undef PCE_AFFINE
+#undef PCE_AFFINE_
   PCE_LAUNCH_CHECK("col_affine");
+  return PCE_OK;
+}
+
+// The whole pass over few rows in one launch.  A workgroup forms the sums of BN_SMALL_COLS vector columns over all rows
+// (32 bytes of a row, two threads beside one another), its coefficients, and writes its share of the rows: blockIdx.y of gridDim.y
+// workgroups do so for the same columns, each for itself, so that nothing is handed from one to another.  Bound by the launch, the
+// trips to memory and the instructions of a compute unit's eight wavefronts (1024 threads, and 8 rows requested whether there are
+// so many or not, took 16 us on 512 rows in fp16; 5.7 so).
+#define BN_SMALL_THREADS 512
+#define BN_SMALL_COLS 2
+#define BN_SMALL_LANES (BN_SMALL_THREADS / BN_SMALL_COLS)
+#define BN_SMALL_WORKGROUPS 128
+// both sums of every column over the row lanes, in red[0], red[1]; the wavefronts halve their lanes' values and lanes together
+template <int VEC>
+__device__ __forceinline__ void bn_small_sums(double (&v)[2 * VEC], double (*red)[BN_SMALL_COLS * VEC]) {
+  constexpr int N = 2 * VEC, WAVES = BN_SMALL_THREADS / 64;
+  __shared__ double part[WAVES][N][BN_SMALL_COLS];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int which = 0;
+#pragma unroll
+  for (int half = N / 2, bit = 32; bit >= BN_SMALL_COLS; half >>= 1, bit >>= 1) {
+    const bool up = (lane & bit) != 0;
+    if (half >= 1) {
+#pragma unroll
+      for (int j = 0; j < (half >= 1 ? half : 1); ++j) {
+        const double send = up ? v[j] : v[j + half], keep = up ? v[j + half] : v[j];
+        v[j] = keep + __shfl_xor(send, bit, 64);
+      }
+      which += up ? half : 0;
+    } else {
+      v[0] += __shfl_xor(v[0], bit, 64);
+    }
+  }
+  part[wave][which][lane % BN_SMALL_COLS] = v[0];   // (lanes that hold the same sum write the same value)
+  __syncthreads();
+  if (threadIdx.x < N * BN_SMALL_COLS) {
+    const int q = threadIdx.x / BN_SMALL_COLS, t = threadIdx.x % BN_SMALL_COLS;
+    double sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) sum += part[w][q][t];
+    red[q / VEC][t * VEC + q % VEC] = sum;
+  }
+  __syncthreads();
+}
+
+// FORWARD: x, b = residual or null, y.  Backward: x = dy, b = the norm's input, y = dx.
+template <typename T, bool FORWARD, int GATE>
+__global__ void __launch_bounds__(BN_SMALL_THREADS) bn_small_kernel(const T *__restrict__ x, const T *__restrict__ b, T *__restrict__ y,
+                                                                    int groups, int n, int c, BnForward f, BnBackward w, int act, float slope,
+                                                                    GateArgs g) {
+  constexpr int VEC = 16 / sizeof(T);
+  typedef typename VecOf<T, VEC>::type V;
+  __shared__ double red[2][BN_SMALL_COLS * VEC];
+  __shared__ float coef[3][BN_SMALL_COLS * VEC];
+  const int tc = threadIdx.x % BN_SMALL_COLS, rl = threadIdx.x / BN_SMALL_COLS;
+  const int first = blockIdx.x * BN_SMALL_COLS * VEC, col0 = first + tc * VEC;
+  const bool live = col0 < c;
+  const int lo = (int)((long long)n * blockIdx.y / gridDim.y), hi = (int)((long long)n * (blockIdx.y + 1) / gridDim.y);
+  double v[2 * VEC];
+  {
+    double s1[VEC], s2[VEC];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) s1[j] = s2[j] = 0.0;
+    if (live)
+      for (int g0 = rl; g0 < groups; g0 += BN_SMALL_LANES)
+        for (int r0 = g0; r0 < n; r0 += groups * BnRows<GATE>::N)
+          bn_group<T, VEC, GATE>(x, FORWARD ? nullptr : b, g, r0, groups, n, c, col0, false, s1, s2);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      v[j] = s1[j];
+      v[VEC + j] = s2[j];
+    }
+  }
+  bn_small_sums<VEC>(v, red);
+  if (threadIdx.x < BN_SMALL_COLS * VEC && first + (int)threadIdx.x < c) {
+    const int t = threadIdx.x;
+    if (FORWARD)
+      bn_forward_channel(f, first + t, red[0][t], red[1][t], blockIdx.y == 0, &coef[0][t], &coef[2][t]);
+    else
+      bn_backward_channel(w, first + t, red[0][t], red[1][t], blockIdx.y == 0, &coef[0][t], &coef[1][t], &coef[2][t]);
+  }
+  __syncthreads();
+  if (!live) return;
+  float cx[VEC], cd[VEC], c0[VEC];
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) {
+    cx[j] = coef[0][tc * VEC + j];
+    cd[j] = FORWARD ? 1.f : coef[1][tc * VEC + j];
+    c0[j] = coef[2][tc * VEC + j];
+  }
+  for (int r0 = lo + rl; r0 < hi; r0 += BN_SMALL_LANES * AFFINE_ROWS) {
+    V xs[AFFINE_ROWS], ds[AFFINE_ROWS], gs[AFFINE_ROWS];
+#pragma unroll
+    for (int k = 0; k < AFFINE_ROWS; ++k) {
+      const int r = r0 + k * BN_SMALL_LANES;
+      const long long at = (long long)(r < hi ? r : hi - 1) * c + col0;
+      xs[k] = *reinterpret_cast<const V *>(x + at);
+      if (b) ds[k] = *reinterpret_cast<const V *>(b + at);
+      if (GATE) gs[k] = *reinterpret_cast<const V *>((const T *)g.gate + at);
+    }
+#pragma unroll
+    for (int k = 0; k < AFFINE_ROWS; ++k) {
+      const int r = r0 + k * BN_SMALL_LANES;
+      const long long at = (long long)r * c + col0;
+      V in = xs[k];
+      if (GATE == GATE_MASK) {   // (what is written is what enters the map)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) vec_set<T, VEC>(in, j, gated<T, GATE>(vec_get<T, VEC>(xs[k], j), vec_get<T, VEC>(gs[k], j), g));
+        if (r < hi) *reinterpret_cast<V *>((T *)g.out + at) = in;
+      }
+      const V out = affine_vec<T, VEC, GATE == GATE_SLOPE ? GATE_SLOPE : GATE_NONE>(in, b != nullptr, ds[k], gs[k], cx, cd, c0, act, slope, g);
+      if (r < hi) *reinterpret_cast<V *>(y + at) = out;
+    }
+  }
+}
+
+// Where the one launch leads: to 4096 rows forward and 2048 backward, fewer of rows wider than 512 and 768 bytes (their 32-byte
+// pieces lie in few of a cache's channels).  Against three launches, us, replayed from a graph: forward, fp16, 4096 rows of 32 / 96 / 256
+// columns 8.2 / 8.5 / 9.4 against 10.8 / 10.6 / 11.2, of 384 13.3 against 12.9; fp32, 4096 of 96 8.3 against 9.9, 2048 and 4096 of
+// 256 7.6 against 11.2 and 16.9 against 11.5; backward through an activation, fp16, 2048 of 96 9.2 against 11.6, 4096 13.0 against 11.7;
+// fp32, 1536 of 256 9.1 against 11.0, of 384 14.2 against 11.4.  (200 rows: 5.5 against 10.)
+static bool bn_small_rows(bool forward, int64_t n, int64_t row_bytes) {
+  return forward ? n <= 4096 && n * row_bytes <= (2 << 20) : n <= 2048 && n * row_bytes <= (3 << 19);
+}
+
+// whether the n x c matrices at p and q (either may be null) share memory
+static bool overlap(const void *p, const void *q, int64_t bytes) {
+  const uintptr_t a = (uintptr_t)p, b = (uintptr_t)q;
+  return p && q && a < b + (uintptr_t)bytes && b < a + (uintptr_t)bytes;
+}
+
+// `outs` must not share memory with `ins`: a workgroup reads rows that another one writes
+static bool bn_small_takes(bool forward, int32_t dtype, int64_t n, int32_t c, const void *const *ins, int n_ins, const void *const *outs, int n_outs) {
+  const int vec = dtype == PCE_F16 ? 8 : 4;
+  if (c % vec) return false;
+  const int64_t row_bytes = (int64_t)c * (dtype == PCE_F16 ? 2 : 4), bytes = n * row_bytes;
+  if (!bn_small_rows(forward, n, row_bytes)) return false;
+  for (int i = 0; i < n_ins; ++i)
+    if (!aligned16(ins[i])) return false;
+  for (int o = 0; o < n_outs; ++o) {
+    if (!aligned16(outs[o])) return false;
+    for (int i = 0; i < n_ins; ++i)
+      if (overlap(ins[i], outs[o], bytes)) return false;
+    for (int q = 0; q < o; ++q)
+      if (overlap(outs[q], outs[o], bytes)) return false;
+  }
+  return true;
+}
+
+template <typename T, bool FORWARD, int GATE>
+static int bn_small_launch(const void *x, const void *b, void *y, int64_t n, int32_t c, const BnForward &f, const BnBackward &w, int act,
+                           float slope, const GateArgs &g, hipStream_t s) {
+  const int cols = (int)pce_div_up(c, BN_SMALL_COLS * (16 / (int)sizeof(T)));
+  int shares = BN_SMALL_WORKGROUPS / cols;
+  const int most = (int)pce_div_up(n, BN_SMALL_LANES);
+  shares = shares < 1 ? 1 : shares > 8 ? 8 : shares;
+  if (shares > most) shares = most;
+  hipLaunchKernelGGL((bn_small_kernel<T, FORWARD, GATE>), dim3(cols, shares), dim3(BN_SMALL_THREADS), 0, s, (const T *)x, (const T *)b, (T *)y,
+                     (int)bn_groups(n, c / (16 / (int)sizeof(T))), (int)n, c,
+                     f, w, act, slope, g);
+  PCE_LAUNCH_CHECK("bn_small");
   return PCE_OK;
 }
 
@@ -4438,8 +4702,7 @@ extern "C" int pce_col_affine(const void *x, const void *d, void *y, int32_t dty
   if (dtype != PCE_F16 && dtype != PCE_F32) PCE_FAIL(PCE_EINVAL, "pce_col_affine: dtype %d", (int)dtype);
   if (n <= 0 || c <= 0) PCE_FAIL(PCE_EINVAL, "pce_col_affine: n=%lld c=%d", (long long)n, (int)c);
   if (!act_known(act)) PCE_FAIL(PCE_EINVAL, "pce_col_affine: activation %d", (int)act);
-  return col_affine_launch("pce_col_affine", x, d, nullptr, y, dtype, n, c, kx, kd, k0, act, slope, PCE_ACT_NONE, 0.f,
-                           (hipStream_t)stream);
+  return col_affine_launch("pce_col_affine", x, d, y, dtype, n, c, kx, kd, k0, act, slope, GateArgs{}, (hipStream_t)stream);
 }
 
 // workspace of the fused entry points: the partial sums, then 3*c floats of coefficients
@@ -4448,10 +4711,10 @@ extern "C" int64_t pce_bn_workspace_bytes(int64_t n, int32_t c) {
   return pce_align_up(pce_col_sums_workspace_bytes(n, c), 256) + 3 * (int64_t)c * (int64_t)sizeof(float);
 }
 
-extern "C" int pce_bn_forward(const void *x, const void *residual, void *y, int32_t dtype, int64_t n, int32_t c, const float *weight,
-                              const float *bias, float *running_mean, float *running_var, int32_t use_batch_stats,
-                              float momentum, float eps, float *save_mean, float *save_rstd, void *ws, int64_t ws_bytes,
-                              int32_t act, float slope, pce_stream_t stream) {
+extern "C" int pce_bn_forward_counted(const void *x, const void *residual, void *y, int32_t dtype, int64_t n, int32_t c, const float *weight,
+                                      const float *bias, float *running_mean, float *running_var, int64_t *batches, int32_t use_batch_stats,
+                                      float momentum, float eps, float *save_mean, float *save_rstd, void *ws, int64_t ws_bytes,
+                                      int32_t act, float slope, pce_stream_t stream) {
   if (!x || !y || !save_mean || !save_rstd) PCE_FAIL(PCE_EINVAL, "pce_bn_forward: null pointer");
   if (dtype != PCE_F16 && dtype != PCE_F32) PCE_FAIL(PCE_EINVAL, "pce_bn_forward: dtype %d", (int)dtype);
   if (n <= 0 || c <= 0) PCE_FAIL(PCE_EINVAL, "pce_bn_forward: n=%lld c=%d", (long long)n, (int)c);
@@ -4459,42 +4722,77 @@ extern "C" int pce_bn_forward(const void *x, const void *residual, void *y, int3
   if (!act_known(act)) PCE_FAIL(PCE_EINVAL, "pce_bn_forward: activation %d", (int)act);
   if (!ws || ws_bytes < pce_bn_workspace_bytes(n, c)) PCE_FAIL(PCE_EWORKSPACE, "pce_bn_forward: workspace %lld < %lld", (long long)ws_bytes, (long long)pce_bn_workspace_bytes(n, c));
   hipStream_t s = (hipStream_t)stream;
+  const BnForward f = {weight, bias, running_mean, running_var, (long long *)batches, use_batch_stats, momentum, eps, save_mean, save_rstd, (long long)n, c};
+  const void *ins[2] = {x, residual}, *outs[1] = {y};
+  if (use_batch_stats && bn_small_takes(true, dtype, n, c, ins, 2, outs, 1))
+    return dtype == PCE_F16 ? bn_small_launch<half_t, true, GATE_NONE>(x, residual, y, n, c, f, BnBackward{}, act, slope, GateArgs{}, s)
+                            : bn_small_launch<float, true, GATE_NONE>(x, residual, y, n, c, f, BnBackward{}, act, slope, GateArgs{}, s);
   double *partial = (double *)ws;
   float *coef = (float *)((char *)ws + pce_align_up(pce_col_sums_workspace_bytes(n, c), 256));
   int64_t blocks = 0;
   int rc;
-  if (use_batch_stats && (rc = bn_partial(x, nullptr, nullptr, PCE_ACT_NONE, 0.f, dtype, n, c, partial, &blocks, s))) return rc;
+  if (use_batch_stats && (rc = bn_partial(x, nullptr, GATE_NONE, GateArgs{}, dtype, n, c, partial, &blocks, s))) return rc;
   hipLaunchKernelGGL(bn_finish_forward_kernel, dim3((unsigned)c), dim3(64), 0, s, (const double *)partial,
-                     (long long)blocks, (long long)n, c, weight, bias, running_mean, running_var, use_batch_stats, momentum, eps,
-                     save_mean, save_rstd, coef, coef + c, residual ? coef + 2 * c : nullptr);
+                     (long long)blocks, f, coef, coef + c);
   PCE_LAUNCH_CHECK("bn_finish_forward");
-  return col_affine_launch("pce_bn_forward", x, residual, nullptr, y, dtype, n, c, coef, residual ? coef + 2 * c : nullptr, coef + c,
-                           act, slope, PCE_ACT_NONE, 0.f, s);
+  return col_affine_launch("pce_bn_forward", x, residual, y, dtype, n, c, coef, nullptr, coef + c, act, slope, GateArgs{}, s);
+}
+
+extern "C" int pce_bn_forward(const void *x, const void *residual, void *y, int32_t dtype, int64_t n, int32_t c, const float *weight,
+                              const float *bias, float *running_mean, float *running_var, int32_t use_batch_stats,
+                              float momentum, float eps, float *save_mean, float *save_rstd, void *ws, int64_t ws_bytes,
+                              int32_t act, float slope, pce_stream_t stream) {
+  return pce_bn_forward_counted(x, residual, y, dtype, n, c, weight, bias, running_mean, running_var, nullptr, use_batch_stats, momentum, eps,
+                                save_mean, save_rstd, ws, ws_bytes, act, slope, stream);
+}
+
+extern "C" int pce_bn_backward_masked(const void *x, const void *dy, const void *y_act, int32_t act, float slope, void *dy_masked, void *dx,
+                                      int32_t dtype, int64_t n, int32_t c, const float *weight, const float *save_mean,
+                                      const float *save_rstd, int32_t use_batch_stats, float *grad_weight, float *grad_bias, void *ws,
+                                      int64_t ws_bytes, pce_stream_t stream) {
+  if (!x || !dy || !dx || !save_mean || !save_rstd) PCE_FAIL(PCE_EINVAL, "pce_bn_backward: null pointer");
+  if (!act_known(act)) PCE_FAIL(PCE_EINVAL, "pce_bn_backward: activation %d", (int)act);
+  if (act != PCE_ACT_NONE && !y_act) PCE_FAIL(PCE_EINVAL, "pce_bn_backward: the gradient of an activation needs its output");
+  if (act == PCE_ACT_NONE) y_act = nullptr;
+  if (dy_masked && !y_act) PCE_FAIL(PCE_EINVAL, "pce_bn_backward: a masked gradient needs an activation");
+  if (dtype != PCE_F16 && dtype != PCE_F32) PCE_FAIL(PCE_EINVAL, "pce_bn_backward: dtype %d", (int)dtype);
+  if (n <= 0 || c <= 0) PCE_FAIL(PCE_EINVAL, "pce_bn_backward: n=%lld c=%d", (long long)n, (int)c);
+  if (!ws || ws_bytes < pce_bn_workspace_bytes(n, c)) PCE_FAIL(PCE_EWORKSPACE, "pce_bn_backward: workspace %lld < %lld", (long long)ws_bytes, (long long)pce_bn_workspace_bytes(n, c));
+  hipStream_t s = (hipStream_t)stream;
+  const int gate = dy_masked ? GATE_MASK : y_act ? GATE_SLOPE : GATE_NONE;
+  GateArgs g = {y_act, dy_masked, act, slope};
+  const BnBackward w = {weight, save_mean, save_rstd, use_batch_stats, grad_weight, grad_bias, (long long)n, c};
+  const void *ins[3] = {dy, x, y_act}, *outs[2] = {dx, dy_masked};
+  if (bn_small_takes(false, dtype, n, c, ins, 3, outs, 2)) {
+#define PCE_BN_SMALL(G_)                                                                                                                   \
+  return dtype == PCE_F16 ? bn_small_launch<half_t, false, G_>(dy, x, dx, n, c, BnForward{}, w, PCE_ACT_NONE, 0.f, g, s)                     \
+                          : bn_small_launch<float, false, G_>(dy, x, dx, n, c, BnForward{}, w, PCE_ACT_NONE, 0.f, g, s)
+    if (gate == GATE_MASK) PCE_BN_SMALL(GATE_MASK);
+    if (gate == GATE_SLOPE) PCE_BN_SMALL(GATE_SLOPE);
+    PCE_BN_SMALL(GATE_NONE);
+#undef PCE_BN_SMALL
+  }
+  double *partial = (double *)ws;
+  float *coef = (float *)((char *)ws + pce_align_up(pce_col_sums_workspace_bytes(n, c), 256));
+  int64_t blocks = 0;
+  int rc = bn_partial(dy, x, gate, g, dtype, n, c, partial, &blocks, s);
+  if (rc) return rc;
+  hipLaunchKernelGGL(bn_finish_backward_kernel, dim3((unsigned)c), dim3(64), 0, s, (const double *)partial,
+                     (long long)blocks, w, coef, coef + c, coef + 2 * c);
+  PCE_LAUNCH_CHECK("bn_finish_backward");
+  if (dy_masked) {   // the sums have written it
+    dy = dy_masked;
+    g = GateArgs{};
+  }
+  return col_affine_launch("pce_bn_backward", dy, x, dx, dtype, n, c, coef, coef + c, coef + 2 * c, PCE_ACT_NONE, 0.f, g, s);
 }
 
 extern "C" int pce_bn_backward(const void *x, const void *dy, const void *y_act, int32_t act, float slope, void *dx,
                                int32_t dtype, int64_t n, int32_t c, const float *weight, const float *save_mean,
                                const float *save_rstd, int32_t use_batch_stats, float *grad_weight, float *grad_bias, void *ws,
                                int64_t ws_bytes, pce_stream_t stream) {
-  if (!x || !dy || !dx || !save_mean || !save_rstd) PCE_FAIL(PCE_EINVAL, "pce_bn_backward: null pointer");
-  if (!act_known(act)) PCE_FAIL(PCE_EINVAL, "pce_bn_backward: activation %d", (int)act);
-  if (act != PCE_ACT_NONE && !y_act) PCE_FAIL(PCE_EINVAL, "pce_bn_backward: the gradient of an activation needs its output");
-  if (act == PCE_ACT_NONE) y_act = nullptr;
-  if (dtype != PCE_F16 && dtype != PCE_F32) PCE_FAIL(PCE_EINVAL, "pce_bn_backward: dtype %d", (int)dtype);
-  if (n <= 0 || c <= 0) PCE_FAIL(PCE_EINVAL, "pce_bn_backward: n=%lld c=%d", (long long)n, (int)c);
-  if (!ws || ws_bytes < pce_bn_workspace_bytes(n, c)) PCE_FAIL(PCE_EWORKSPACE, "pce_bn_backward: workspace %lld < %lld", (long long)ws_bytes, (long long)pce_bn_workspace_bytes(n, c));
-  hipStream_t s = (hipStream_t)stream;
-  double *partial = (double *)ws;
-  float *coef = (float *)((char *)ws + pce_align_up(pce_col_sums_workspace_bytes(n, c), 256));
-  int64_t blocks = 0;
-  int rc = bn_partial(dy, x, y_act, act, slope, dtype, n, c, partial, &blocks, s);
-  if (rc) return rc;
-  hipLaunchKernelGGL(bn_finish_backward_kernel, dim3((unsigned)c), dim3(64), 0, s, (const double *)partial,
-                     (long long)blocks, (long long)n, c, weight, save_mean, save_rstd, use_batch_stats, grad_weight, grad_bias, coef,
-                     coef + c, coef + 2 * c);
-  PCE_LAUNCH_CHECK("bn_finish_backward");
-  return col_affine_launch("pce_bn_backward", dy, x, y_act, dx, dtype, n, c, coef, coef + c, coef + 2 * c, PCE_ACT_NONE, 0.f, act,
-                           slope, s);
+  return pce_bn_backward_masked(x, dy, y_act, act, slope, nullptr, dx, dtype, n, c, weight, save_mean, save_rstd, use_batch_stats, grad_weight,
+                                grad_bias, ws, ws_bytes, stream);
 }
 
 // ---- channel concatenation of two feature matrices on the same rows (script/utils.py:152-164) ---------

@@ -13,6 +13,10 @@
 
 #include "pcengine_amd.h"
 
+// entry points that a library beside this extension may be without: the calls that need them are then declined
+#pragma weak pce_bn_forward_counted
+#pragma weak pce_bn_backward_masked
+
 namespace {
 
 enum Kind { KIND_OSO = 0, KIND_OSB = 1, KIND_OS = 2, KIND_FDS = 3, KIND_DENSE = 4 };
@@ -228,12 +232,12 @@ PyObject *three(at::Tensor a, at::Tensor b, at::Tensor c) {
   return t;
 }
 
-// bn_forward(x, residual, weight, bias, running mean, running variance, batch statistics, momentum, eps, act, slope, stream)
+// bn_forward(x, residual, weight, bias, running mean, running variance, batch statistics, momentum, eps, act, slope, stream, batch count)
 //   -> (y, mean, rstd), None or an error code
 PyObject *bn_forward(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  if (n_args != 12) {
-    PyErr_SetString(PyExc_TypeError, "bn_forward: twelve arguments");
+  if (n_args != 13) {
+    PyErr_SetString(PyExc_TypeError, "bn_forward: thirteen arguments");
     return nullptr;
   }
   const at::Tensor *x = rows_of(args[0]);
@@ -244,6 +248,12 @@ PyObject *bn_forward(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   if (!like(args[1], *x, &res) || !floats(args[2], x->device(), c, &w) || !floats(args[3], x->device(), c, &b) ||
       !floats(args[4], x->device(), c, &mean) || !floats(args[5], x->device(), c, &var))
     Py_RETURN_NONE;
+  int64_t *batches = nullptr;
+  if (args[12] != Py_None) {
+    const at::Tensor *t = plain(args[12]);
+    if (!t || t->scalar_type() != at::kLong || t->device() != x->device() || t->numel() != 1 || !pce_bn_forward_counted) Py_RETURN_NONE;
+    batches = t->data_ptr<int64_t>();
+  }
   const int batch = PyObject_IsTrue(args[6]), act = (int)PyLong_AsLong(args[9]), dt = x->scalar_type() == at::kHalf ? PCE_F16 : PCE_F32;
   const float momentum = (float)PyFloat_AsDouble(args[7]), eps = (float)PyFloat_AsDouble(args[8]), slope = (float)PyFloat_AsDouble(args[10]);
   void *stream = PyLong_AsVoidPtr(args[11]);
@@ -257,19 +267,23 @@ PyObject *bn_forward(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     save = at::empty({2 * c}, x->options().dtype(at::kFloat));
     ws = at::empty({ws_bytes}, x->options().dtype(at::kByte));
     float *s = save.data_ptr<float>();
-    rc = pce_bn_forward(x->data_ptr(), res, y.data_ptr(), dt, n, (int32_t)c, w, b, const_cast<float *>(mean), const_cast<float *>(var), batch,
-                        momentum, eps, s, s + c, ws.data_ptr(), ws_bytes, act, slope, stream);
+    float *m = const_cast<float *>(mean), *v = const_cast<float *>(var);
+    rc = batches ? pce_bn_forward_counted(x->data_ptr(), res, y.data_ptr(), dt, n, (int32_t)c, w, b, m, v, batches, batch, momentum, eps, s, s + c,
+                                          ws.data_ptr(), ws_bytes, act, slope, stream)
+                 : pce_bn_forward(x->data_ptr(), res, y.data_ptr(), dt, n, (int32_t)c, w, b, m, v, batch, momentum, eps, s, s + c, ws.data_ptr(),
+                                  ws_bytes, act, slope, stream);
   }
   if (rc != PCE_OK) return PyLong_FromLong(rc);
   return three(std::move(y), part(save, 0, c), part(save, c, c));
   END_HANDLE_TH_ERRORS
 }
 
-// bn_backward(x, dy, y, weight, mean, rstd, batch statistics, act, slope, stream) -> (dx, grad of weight, grad of bias), None or an error code
+// bn_backward(x, dy, y, weight, mean, rstd, batch statistics, act, slope, stream, masked)
+//   -> (dx, grad of weight, grad of bias[, masked dy]), None or an error code
 PyObject *bn_backward(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  if (n_args != 10) {
-    PyErr_SetString(PyExc_TypeError, "bn_backward: ten arguments");
+  if (n_args != 11) {
+    PyErr_SetString(PyExc_TypeError, "bn_backward: eleven arguments");
     return nullptr;
   }
   const at::Tensor *x = rows_of(args[0]);
@@ -283,9 +297,11 @@ PyObject *bn_backward(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   const int batch = PyObject_IsTrue(args[6]), act = (int)PyLong_AsLong(args[7]), dt = x->scalar_type() == at::kHalf ? PCE_F16 : PCE_F32;
   const float slope = (float)PyFloat_AsDouble(args[8]);
   void *stream = PyLong_AsVoidPtr(args[9]);
+  const int mask = PyObject_IsTrue(args[10]);
   if (PyErr_Occurred()) return nullptr;
+  if (mask && (act == PCE_ACT_NONE || !pce_bn_backward_masked)) Py_RETURN_NONE;
   if (act != PCE_ACT_NONE && (!y || (act == PCE_ACT_LEAKY_RELU && !(slope > 0)))) Py_RETURN_NONE;
-  at::Tensor dx, grads, ws;
+  at::Tensor dx, grads, ws, masked;
   int rc;
   {
     Unlocked unlocked;
@@ -294,11 +310,17 @@ PyObject *bn_backward(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
     grads = at::empty({2 * c}, x->options().dtype(at::kFloat));
     ws = at::empty({ws_bytes}, x->options().dtype(at::kByte));
     float *g = grads.data_ptr<float>();
-    rc = pce_bn_backward(x->data_ptr(), dy, act == PCE_ACT_NONE ? nullptr : y, act, slope, dx.data_ptr(), dt, n, (int32_t)c, w, mean, rstd, batch, g,
-                         g + c, ws.data_ptr(), ws_bytes, stream);
+    if (mask) masked = at::empty({n, c}, x->options());
+    const void *out = act == PCE_ACT_NONE ? nullptr : y;
+    rc = mask ? pce_bn_backward_masked(x->data_ptr(), dy, out, act, slope, masked.data_ptr(), dx.data_ptr(), dt, n, (int32_t)c, w, mean, rstd, batch,
+                                       g, g + c, ws.data_ptr(), ws_bytes, stream)
+              : pce_bn_backward(x->data_ptr(), dy, out, act, slope, dx.data_ptr(), dt, n, (int32_t)c, w, mean, rstd, batch, g, g + c, ws.data_ptr(),
+                                ws_bytes, stream);
   }
   if (rc != PCE_OK) return PyLong_FromLong(rc);
-  return three(std::move(dx), part(grads, 0, c), part(grads, c, c));
+  PyObject *t = three(std::move(dx), part(grads, 0, c), part(grads, c, c));
+  if (t && mask && _PyTuple_Resize(&t, 4) == 0) PyTuple_SET_ITEM(t, 3, THPVariable_Wrap(std::move(masked)));
+  return t;
   END_HANDLE_TH_ERRORS
 }
 
