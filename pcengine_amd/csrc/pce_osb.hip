@@ -516,10 +516,10 @@ __global__ void __launch_bounds__(256, 2) osb_kernel(TileArgs a, OsbArgs o) {
   constexpr int COLS = 4 * CB * 16;
   constexpr int W_LOADS = 2 * CB;
   constexpr int NW = CB == 2 ? 4 : CB == 3 ? 3 : 2;   // steps whose weights are held or on their way: what the registers allow
-  // at the start of a step at most this many younger operations may be out: the copies two steps ahead, and the weights
-  constexpr int IN_FLIGHT = (NW - 1) * (OSB_A_LOADS + W_LOADS) < 2 * OSB_A_LOADS + 3 * W_LOADS ? (NW - 1) * (OSB_A_LOADS + W_LOADS)
-                                                                                              : 2 * OSB_A_LOADS + 3 * W_LOADS;
-  static_assert(IN_FLIGHT <= 63, "vmcnt is a 6-bit counter");
+  // younger operations that may be out where a step's weights must have landed (those of the NW - 1 steps behind it, with the copies
+  // between) and where the next step's rows must have (the copies of one step, and the weights issued around them)
+  constexpr int OUT_W = (NW - 1) * (OSB_A_LOADS + W_LOADS), OUT_A = OSB_A_LOADS + 2 * W_LOADS;
+  static_assert(OUT_W <= 63 && OUT_A <= 63, "vmcnt is a 6-bit counter");
   __shared__ __attribute__((aligned(128))) half8 lds[OSB_ST * OSB_STAGE];
   // byte offset of the neighbour row at every offset; the four rows whose pieces a lane gathers lie side by side
   __shared__ __attribute__((aligned(16))) unsigned src[OSB_MAX_KV + 1][OSB_ROWS];
@@ -607,7 +607,7 @@ __global__ void __launch_bounds__(256, 2) osb_kernel(TileArgs a, OsbArgs o) {
   int chunk = 0;
 #define OSB_NEXT(K_, C_)               /* the cursor's step, and on; behind the last one a row table without rows */     \
   {                                                                                                                     \
-    K_ = chunk < kch ? __ffs(rest) - 1 : OSB_MAX_KV;                                                                    \
+    K_ = chunk < kch ? __builtin_ctz(rest) : OSB_MAX_KV;                                                                \
     C_ = chunk;                                                                                                         \
     rest &= rest - 1;                                                                                                   \
     if (rest == 0) {                                                                                                    \
@@ -629,12 +629,14 @@ __global__ void __launch_bounds__(256, 2) osb_kernel(TileArgs a, OsbArgs o) {
     _Pragma("unroll") for (int cb = 0; cb < CB; ++cb) load16_raw(wf[B_][cb], woff[cb], wb);                             \
     _Pragma("unroll") for (int cb = 0; cb < CB; ++cb) load16_raw(wf[B_][CB + cb], woff[cb], wb1);                       \
   }
-  // this step's feature rows and weights have landed, and every wavefront is done with the stage that is filled next
-#define OSB_LANDED(B_, N_)                                                                                              \
+  // at most N_ operations are out: this step's weights have landed
+#define OSB_WEIGHTS(B_, N_)                                                                                             \
   {                                                                                                                     \
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(N_) : "memory");                                            \
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N_) : "memory");                                                         \
     _Pragma("unroll") for (int i = 0; i < W_LOADS; ++i) asm volatile("" : "+v"(wf[B_][i]) : : "memory");                \
   }
+  // the next step's rows have landed in every wavefront, and every wavefront is done with the stage that is filled next
+#define OSB_ROWS_LANDED(N_) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(N_) : "memory");
 #define OSB_BLOCK(F_, RB_, B_)                                                                                          \
   if ((own[RB_] >> k0) & 1u) {                                                                                          \
     _Pragma("unroll") for (int cb = 0; cb < CB; ++cb)                                                                   \
@@ -644,26 +646,32 @@ __global__ void __launch_bounds__(256, 2) osb_kernel(TileArgs a, OsbArgs o) {
           acc[RB_][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, wf[B_][CB + cb]), __builtin_bit_cast(half8, F_[1]), acc[RB_][cb], 0, 0, 0); \
     }                                                                                                                   \
   }
+  // A step begins with its first four blocks' fragments on their way; in its middle the next step's rows are there, and their first
+  // blocks are requested between the last four blocks' products.  (With all of it at the head of a step, the
+  // products waited from the barrier to the first fragments: 256 -> 256 on 72 k rows 179.4 us, 176.9 so; the layers of the eight indoor
+  // scenes' network 9.2 ms, 9.0.)
 #define OSB_STEP(B_, N_)                                                                                                \
   {                                                                                                                     \
-    OSB_LANDED(B_, N_)                                                                                                   \
+    OSB_WEIGHTS(B_, OUT_W)                                                                                              \
+    const unsigned ra0 = row_addr + (t & (OSB_ST - 1)) * (OSB_STAGE * 16), ra1 = ra0 ^ 64;                              \
+    const bool half_step = TAIL && c0 + 1 == kch;                                                                       \
+    OSB_WAIT(f0, 6); OSB_BLOCK(f0, 0, B_) OSB_READ(f0, 4);                                                              \
+    OSB_WAIT(f1, 6); OSB_BLOCK(f1, 1, B_) OSB_READ(f1, 5);                                                              \
+    OSB_WAIT(f2, 6); OSB_BLOCK(f2, 2, B_) OSB_READ(f2, 6);                                                              \
+    OSB_WAIT(f3, 6); OSB_BLOCK(f3, 3, B_) OSB_READ(f3, 7);                                                              \
+    asm volatile("" : "+v"(as) : : "memory");                                                                           \
+    OSB_ROWS_LANDED(N_)                                                                                                 \
     OSB_ISSUE_A((t + 3) & (OSB_ST - 1), c3)                                                                             \
     int k4, c4;                                                                                                         \
     OSB_NEXT(k4, c4)                                                                                                    \
     OSB_SRC(k4);                                                                                                        \
-    const unsigned ra0 = row_addr + (t & (OSB_ST - 1)) * (OSB_STAGE * 16), ra1 = ra0 ^ 64;                              \
-    const bool half_step = TAIL && c0 + 1 == kch;                                                                     \
-    u32x4 f0[2], f1[2], f2[2], f3[2];                                                                                   \
-    OSB_READ(f0, 0); OSB_READ(f1, 1); OSB_READ(f2, 2); OSB_READ(f3, 3);                                                 \
-    asm volatile("s_waitcnt lgkmcnt(6)" : "+v"(f0[0]), "+v"(f0[1]), "+v"(as) : : "memory");                             \
-    OSB_BLOCK(f0, 0, B_) OSB_READ(f0, 4);                                                                               \
-    OSB_WAIT(f1, 6); OSB_BLOCK(f1, 1, B_) OSB_READ(f1, 5);                                                              \
-    OSB_WAIT(f2, 6); OSB_BLOCK(f2, 2, B_) OSB_READ(f2, 6);                                                              \
-    OSB_WAIT(f3, 6); OSB_BLOCK(f3, 3, B_) OSB_READ(f3, 7);                                                              \
-    OSB_WAIT(f0, 6); OSB_BLOCK(f0, 4, B_)                                                                               \
-    OSB_WAIT(f1, 4); OSB_BLOCK(f1, 5, B_)                                                                               \
-    OSB_WAIT(f2, 2); OSB_BLOCK(f2, 6, B_)                                                                               \
-    OSB_WAIT(f3, 0); OSB_BLOCK(f3, 7, B_)                                                                               \
+    {                                                                                                                   \
+      const unsigned ra0 = row_addr + ((t + 1) & (OSB_ST - 1)) * (OSB_STAGE * 16), ra1 = ra0 ^ 64;                      \
+      OSB_WAIT(f0, 7); OSB_BLOCK(f0, 4, B_) OSB_READ(f0, 0);                                                            \
+      OSB_WAIT(f1, 7); OSB_BLOCK(f1, 5, B_) OSB_READ(f1, 1);                                                            \
+      OSB_WAIT(f2, 7); OSB_BLOCK(f2, 6, B_) OSB_READ(f2, 2);                                                            \
+      OSB_WAIT(f3, 7); OSB_BLOCK(f3, 7, B_) OSB_READ(f3, 3);                                                            \
+    }                                                                                                                   \
     __builtin_amdgcn_sched_barrier(0);                                                                                  \
     if (NW == 2) OSB_ISSUE_W(B_, k2, c2)                                                                                \
     if (NW == 3) OSB_ISSUE_W(B_, k3, c3)                                                                                \
@@ -692,17 +700,26 @@ __global__ void __launch_bounds__(256, 2) osb_kernel(TileArgs a, OsbArgs o) {
     OSB_ISSUE_A(2, c2)
     OSB_SRC(k3);
     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(as) : : "memory");
-    // the first steps wait for all but the copies of two stages, which is what may be out before the third
-    int t = 0;
-    OSB_STEP(0, 2 * OSB_A_LOADS)
-    if (++t < steps) OSB_STEP(1, 2 * OSB_A_LOADS)
-    if (++t < steps) OSB_STEP(2 % NW, 2 * OSB_A_LOADS)
-    for (++t; t < steps; ++t) {
-      OSB_STEP(3 % NW, IN_FLIGHT)
-      if (++t < steps) OSB_STEP(4 % NW, IN_FLIGHT)
-      if (NW > 2 && ++t < steps) OSB_STEP(5 % NW, IN_FLIGHT)
-      if (NW > 3 && ++t < steps) OSB_STEP(6 % NW, IN_FLIGHT)
+    // the first step's rows and the weights of the first NW are there once two steps' copies are out
+    OSB_ROWS_LANDED(2 * OSB_A_LOADS)
+    u32x4 f0[2], f1[2], f2[2], f3[2];
+    {
+      const unsigned ra0 = row_addr, ra1 = ra0 ^ 64;
+      OSB_READ(f0, 0); OSB_READ(f1, 1); OSB_READ(f2, 2); OSB_READ(f3, 3);
     }
+    int t = 0;
+    OSB_STEP(0, OSB_A_LOADS)
+    if (++t < steps) OSB_STEP(1, OSB_A_LOADS + W_LOADS)
+    if (++t < steps) OSB_STEP(2 % NW, OUT_A)
+    for (++t; t < steps; ++t) {
+      OSB_STEP(3 % NW, OUT_A)
+      if (++t < steps) OSB_STEP(4 % NW, OUT_A)
+      if (NW > 2 && ++t < steps) OSB_STEP(5 % NW, OUT_A)
+      if (NW > 3 && ++t < steps) OSB_STEP(6 % NW, OUT_A)
+    }
+    // the reads behind the last step
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f0[0]), "+v"(f0[1]), "+v"(f1[0]), "+v"(f1[1]), "+v"(f2[0]), "+v"(f2[1]), "+v"(f3[0]), "+v"(f3[1]),
+                 "+v"(as) : : "memory");
   }
   // the copies and loads behind the last step end before their destinations are used for anything else
 #pragma unroll
@@ -711,7 +728,8 @@ __global__ void __launch_bounds__(256, 2) osb_kernel(TileArgs a, OsbArgs o) {
     for (int i = 0; i < W_LOADS; ++i) asm volatile("s_waitcnt vmcnt(0)" : "+v"(wf[b][i]) : : "memory");
 #undef OSB_STEP
 #undef OSB_BLOCK
-#undef OSB_LANDED
+#undef OSB_ROWS_LANDED
+#undef OSB_WEIGHTS
 #undef OSB_ISSUE_W
 #undef OSB_ISSUE_A
 #undef OSB_SRC
