@@ -492,6 +492,16 @@ int pce_conv_fwd_os_parts(const void *in_feats, const void *weight, void *out_fe
 int64_t pce_osb_order_elems(int64_t n_rows);
 int pce_osb_order(const int32_t *nbr_dev, const int32_t *mask_dev, int32_t mid, int32_t kv, int64_t n_rows, int32_t *order_dev,
                   int64_t order_elems, pce_stream_t stream);
+/* The orders of several tables in the same two launches (the arguments of pce_osb_order, a table each). */
+#define PCE_OSB_ORDER_MAX 8
+typedef struct {
+  const int32_t *nbr_dev, *mask_dev;
+  int32_t mid, kv;
+  int64_t n_rows;
+  int32_t *order_dev;
+  int64_t order_elems;
+} pce_osb_order_problem_t;
+int pce_osb_order_batch(const pce_osb_order_problem_t *problems, int32_t count, pce_stream_t stream);
 int pce_conv_osb_takes(int32_t dtype, int32_t c_in, int32_t c_out, int32_t kv);
 int64_t pce_conv_osb_workspace_bytes(int64_t n_out, int32_t c_out);
 int64_t pce_conv_osb_scratch_bytes(int64_t n_out, int64_t n_pairs, int32_t c_in, int32_t c_out, int32_t kv);

@@ -79,6 +79,15 @@ class PyrPlan(Structure):
                 ("req", PyrRequest * PYR_MAX_MAPS), ("map", PyrMap * PYR_MAX_MAPS)]
 
 
+OSB_ORDER_MAX = 8
+
+
+class OsbOrderProblem(Structure):
+    """pce_osb_order_problem_t."""
+    _fields_ = [("nbr", c_void_p), ("mask", c_void_p), ("mid", c_int32), ("kv", c_int32), ("n_rows", c_int64), ("order", c_void_p),
+                ("order_elems", c_int64)]
+
+
 class Epilogue(Structure):
     """pce_epilogue_t: out = act(conv + bias + residual)."""
     _fields_ = [("bias", c_void_p), ("residual", c_void_p), ("act", c_int32), ("slope", ctypes.c_float),
@@ -162,6 +171,7 @@ _SIGNATURES = {
                                    c_void_p, c_void_p, POINTER(c_int64), POINTER(Epilogue), c_void_p]),
     "pce_osb_order_elems": (c_int64, [c_int64]),
     "pce_osb_order": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int64, c_void_p, c_int64, c_void_p]),
+    "pce_osb_order_batch": (c_int32, [POINTER(OsbOrderProblem), c_int32, c_void_p]),
     "pce_conv_osb_takes": (c_int32, [c_int32, c_int32, c_int32, c_int32]),
     "pce_conv_osb_leads": (c_int32, [c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, c_int32]),
     "pce_conv_osb_workspace_bytes": (c_int64, [c_int64, c_int32]),

@@ -2,6 +2,7 @@
 // offsets and stored once.  Rows are visited in an order that puts equal neighbour patterns side by side inside
 // windows of the storage order (pce_osb_order), so that a 16-row block can leave out the offsets none of its rows has.
 #include <math.h>
+#include <string.h>
 
 #include "pce_tile.h"
 
@@ -28,6 +29,23 @@ __device__ constexpr int osb_key_bit27(int kp) {
   return 26 - pos;
 }
 
+// The orders of several tables are one launch: they are wanted together (a network's levels), and each alone leaves most of the
+// machine idle, a workgroup a window: with the plans four levels of a 100 k-voxel scan 38 us, 140 one after the other, six of eight
+// indoor scenes 70 and 278.
+struct OsbOrderJob {
+  const int *nbr;
+  const unsigned *known;
+  unsigned centre;
+  int kv, n, window0;   // its first workgroup
+  int *perm;
+  unsigned *bmask;
+  int *plans;
+};
+struct OsbOrderJobs {
+  OsbOrderJob job[PCE_OSB_ORDER_MAX];
+  int count;
+};
+
 // One workgroup per window: the rows' patterns (known, or 27 table reads per row), then a radix sort of (key, row) in LDS,
 // three passes of 9 bits.  The key is the rank of the pattern in the reflected Gray code, in which
 // consecutive patterns differ in one bit.  The sort is stable by construction: a wavefront ranks its entries of a digit by
@@ -38,17 +56,23 @@ __device__ constexpr int osb_key_bit27(int kp) {
 // SHORT: a cloud of one window that is not full, where a thread has per = rows / 1024 entries instead of eight (with the plan
 // 31 -> 15 us on 700 rows, 21 on 3 k, 29 on 6 k; in a full window the conditions would cost 1 us of 33).
 template <bool SHORT>
-__global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(const int *__restrict__ nbr, const unsigned *__restrict__ known,
-                                                                      unsigned centre, int kv, int n, int *__restrict__ perm,
-                                                                      unsigned *__restrict__ bmask) {
+__global__ void __launch_bounds__(OSB_ORDER_THREADS) osb_order_kernel(OsbOrderJobs jobs) {
   constexpr int PER = OSB_WINDOW / OSB_ORDER_THREADS, WAVES = OSB_ORDER_THREADS / 64, BITS = 9, BINS = 1 << BITS;
   __shared__ unsigned keys[OSB_WINDOW];
   __shared__ unsigned masks[OSB_WINDOW];
   __shared__ unsigned short rows[OSB_WINDOW];
   __shared__ unsigned hist[BINS * WAVES];
   __shared__ unsigned wave_sum[WAVES];
+  int which = 0;
+  while (which + 1 < jobs.count && (int)blockIdx.x >= jobs.job[which + 1].window0) ++which;
+  const int *__restrict__ nbr = jobs.job[which].nbr;
+  const unsigned *__restrict__ known = jobs.job[which].known;
+  int *__restrict__ perm = jobs.job[which].perm;
+  unsigned *__restrict__ bmask = jobs.job[which].bmask;
+  const unsigned centre = jobs.job[which].centre;
+  const int kv = jobs.job[which].kv, n = jobs.job[which].n;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int r0 = blockIdx.x * OSB_WINDOW, cnt = n - r0 < OSB_WINDOW ? n - r0 : OSB_WINDOW;
+  const int r0 = ((int)blockIdx.x - jobs.job[which].window0) * OSB_WINDOW, cnt = n - r0 < OSB_WINDOW ? n - r0 : OSB_WINDOW;
   const int per = SHORT ? (cnt + OSB_ORDER_THREADS - 1) / OSB_ORDER_THREADS : PER;
   unsigned m[PER];
   if (known) {
@@ -197,8 +221,11 @@ __host__ __device__ static inline long long osb_plan_offset(long long tiles, int
   return at;
 }
 
-// One workgroup per XCD and column slab count.
-__global__ void __launch_bounds__(1024) osb_plan_kernel(const unsigned *__restrict__ bmask, int n, int tiles, int *__restrict__ plans) {
+// One workgroup per XCD and column slab count of an order.
+__global__ void __launch_bounds__(1024) osb_plan_kernel(OsbOrderJobs jobs) {
+  const unsigned *__restrict__ bmask = jobs.job[blockIdx.z].bmask;
+  int *__restrict__ plans = jobs.job[blockIdx.z].plans;
+  const int n = jobs.job[blockIdx.z].n, tiles = (n + OSB_ROWS - 1) / OSB_ROWS;
   __shared__ unsigned sums[16];
   __shared__ int bound[2];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, x = blockIdx.x;
@@ -300,26 +327,51 @@ extern "C" int64_t pce_osb_order_elems(int64_t n) {
   return n <= 0 ? 0 : osb_plans_offset(n) + osb_plan_offset(pce_div_up(n, OSB_ROWS), OSB_MAX_SLABS + 1);
 }
 
-extern "C" int pce_osb_order(const int32_t *nbr, const int32_t *mask, int32_t mid, int32_t kv, int64_t n, int32_t *order,
-                             int64_t order_elems, pce_stream_t stream) {
-  if (!nbr || !order) PCE_FAIL(PCE_EINVAL, "pce_osb_order: null pointer");
-  if (kv <= 0 || kv > OSB_MAX_KV || mid >= kv) PCE_FAIL(PCE_EINVAL, "pce_osb_order: kv=%d outside [1, %d] or mid=%d", kv, OSB_MAX_KV, mid);
-  if (n <= 0 || n >= (1ll << 31) / OSB_MAX_SLABS - OSB_WINDOW) PCE_FAIL(PCE_ECAPACITY, "pce_osb_order: n=%lld", (long long)n);
-  if (order_elems < pce_osb_order_elems(n))
-    PCE_FAIL(PCE_EWORKSPACE, "pce_osb_order: order holds %lld elements, needs %lld", (long long)order_elems, (long long)pce_osb_order_elems(n));
+extern "C" int pce_osb_order_batch(const pce_osb_order_problem_t *problems, int32_t count, pce_stream_t stream) {
+  if (!problems || count < 1 || count > PCE_OSB_ORDER_MAX) PCE_FAIL(PCE_EINVAL, "pce_osb_order: 1..%d tables per call", PCE_OSB_ORDER_MAX);
+  OsbOrderJobs jobs;
+  memset(&jobs, 0, sizeof(jobs));
+  jobs.count = count;
+  int64_t windows = 0;
+  bool whole = false;   // a window is full, or there are several of one table
+  for (int i = 0; i < count; ++i) {
+    const pce_osb_order_problem_t &p = problems[i];
+    const int64_t n = p.n_rows;
+    if (!p.nbr_dev || !p.order_dev) PCE_FAIL(PCE_EINVAL, "pce_osb_order: null pointer");
+    if (p.kv <= 0 || p.kv > OSB_MAX_KV || p.mid >= p.kv)
+      PCE_FAIL(PCE_EINVAL, "pce_osb_order: kv=%d outside [1, %d] or mid=%d", (int)p.kv, OSB_MAX_KV, (int)p.mid);
+    if (n <= 0 || n >= (1ll << 31) / OSB_MAX_SLABS - OSB_WINDOW) PCE_FAIL(PCE_ECAPACITY, "pce_osb_order: n=%lld", (long long)n);
+    if (p.order_elems < pce_osb_order_elems(n))
+      PCE_FAIL(PCE_EWORKSPACE, "pce_osb_order: order holds %lld elements, needs %lld", (long long)p.order_elems, (long long)pce_osb_order_elems(n));
+    OsbOrderJob &q = jobs.job[i];
+    q.nbr = p.nbr_dev;
+    q.known = (const unsigned *)p.mask_dev;
+    q.centre = p.mid >= 0 ? 1u << p.mid : 0u;
+    q.kv = p.kv;
+    q.n = (int)n;
+    q.window0 = (int)windows;
+    q.perm = p.order_dev;
+    q.bmask = (unsigned *)p.order_dev + osb_mask_offset(n);
+    q.plans = p.order_dev + osb_plans_offset(n);
+    windows += pce_div_up(n, OSB_WINDOW);
+    whole |= n > OSB_WINDOW - OSB_ORDER_THREADS;
+  }
+  if (windows >= (1ll << 31)) PCE_FAIL(PCE_ECAPACITY, "pce_osb_order: too many rows");
   hipStream_t s = (hipStream_t)stream;
-  unsigned *bmask = (unsigned *)order + osb_mask_offset(n);
-  if (n <= OSB_WINDOW - OSB_ORDER_THREADS)
-    hipLaunchKernelGGL(osb_order_kernel<true>, dim3(1), dim3(OSB_ORDER_THREADS), 0, s, nbr, (const unsigned *)mask, mid >= 0 ? 1u << mid : 0u, kv,
-                       (int)n, order, bmask);
+  if (whole)
+    hipLaunchKernelGGL(osb_order_kernel<false>, dim3((unsigned)windows), dim3(OSB_ORDER_THREADS), 0, s, jobs);
   else
-    hipLaunchKernelGGL(osb_order_kernel<false>, dim3((unsigned)pce_div_up(n, OSB_WINDOW)), dim3(OSB_ORDER_THREADS), 0, s, nbr,
-                       (const unsigned *)mask, mid >= 0 ? 1u << mid : 0u, kv, (int)n, order, bmask);
+    hipLaunchKernelGGL(osb_order_kernel<true>, dim3((unsigned)windows), dim3(OSB_ORDER_THREADS), 0, s, jobs);
   PCE_LAUNCH_CHECK("osb_order");
-  hipLaunchKernelGGL(osb_plan_kernel, dim3(8, OSB_MAX_SLABS), dim3(1024), 0, s, bmask, (int)n, (int)pce_div_up(n, OSB_ROWS),
-                     order + osb_plans_offset(n));
+  hipLaunchKernelGGL(osb_plan_kernel, dim3(8, OSB_MAX_SLABS, (unsigned)count), dim3(1024), 0, s, jobs);
   PCE_LAUNCH_CHECK("osb_plan");
   return PCE_OK;
+}
+
+extern "C" int pce_osb_order(const int32_t *nbr, const int32_t *mask, int32_t mid, int32_t kv, int64_t n, int32_t *order,
+                             int64_t order_elems, pce_stream_t stream) {
+  const pce_osb_order_problem_t p = {nbr, mask, mid, kv, n, order, order_elems};
+  return pce_osb_order_batch(&p, 1, stream);
 }
 
 // ---- the convolution -----------------------------------------------------------------------------------------------

@@ -17,9 +17,12 @@ from torch import nn
 from . import backend
 from .activation import ReLU
 from .batchnorm import BatchNorm
-from .spconv import conv3d, prebuild_maps
+from .spconv import _pick_dataflow, conv3d, prebuild_maps
 from .sptensor import spTensor
-from .utils import cat
+from .utils import cat, conv_info_encoder, output_stride_compute
+
+
+_TWO = conv_info_encoder([2, 2, 2])
 
 
 class ConvBN(nn.Module):
@@ -101,6 +104,7 @@ class SparseResUNet(nn.Module):
             if isinstance(m, ConvBN):
                 m.fuse()
         self._in_place_ok = None
+        self._block_layers = None
         return self
 
     def use_planner(self, on: bool = True) -> "SparseResUNet":
@@ -160,6 +164,7 @@ class SparseResUNet(nn.Module):
         # laid out and built by the library in one allocation
         inference = not (torch.is_grad_enabled() and (x.feats.requires_grad or any(p.requires_grad for p in self.parameters())))
         prebuild_maps(x, self.map_plan(x.feats.dtype if inference else None), planner)
+        self._prebuild_block_orders(x)
         if self._skips_in_place(x):
             return self._forward_skips_in_place(x)
         x = self.stem(x)
@@ -172,6 +177,31 @@ class SparseResUNet(nn.Module):
             x = up(x)
             x = dec(cat([x, feats.pop()]))
         return self.head(x)
+
+    def _prebuild_block_orders(self, x: spTensor) -> None:
+        """The block orders that the network's layers will ask for, together and before the first layer: the GPU has little to do
+        while the host queues the narrow layers of the first level.  What is missed here is built when its layer asks for it."""
+        dtype = x.feats.dtype
+        if dtype != torch.float16 or not x.feats.is_cuda:
+            return
+        layers = getattr(self, "_block_layers", None)
+        if layers is None:      # the different wide layers of every level; what the modules' widths say, looked up once
+            layers, depth = {}, len(self.down)
+            for level, module in [(l + 1, m) for l, m in enumerate(self.enc)] + [(l, m) for l, m in enumerate(self.down)] + \
+                    [(depth - 1 - i, m) for ms in (self.up, self.dec) for i, m in enumerate(ms)]:
+                for m in module.modules():
+                    if isinstance(m, conv3d) and m.kernel_volume > 1 and backend.osb_takes(m.kernel_volume, m.in_channels, m.out_channels, dtype):
+                        layers[(level, m.kernel_size_code, m.stride_code, m.in_channels, m.out_channels, m.dataflow, m.transposed)] = None
+            layers = self._block_layers = list(layers)
+        strides, wanted = [x.stride], {}
+        for _ in self.down:
+            strides.append(output_stride_compute(_TWO, strides[-1], False))
+        for level, size, stride, c_in, c_out, dataflow, transposed in layers:
+            km = x.kmaps.get((size, strides[level], stride))
+            if isinstance(km, backend.KernelMap) and (id(km), transposed) not in wanted and \
+                    _pick_dataflow(km, dataflow, c_in, c_out, dtype, transposed) == backend.DATAFLOW_OS:
+                wanted[(id(km), transposed)] = (km, transposed)
+        backend.block_orders(list(wanted.values()))
 
     def _skips_in_place(self, x: spTensor) -> bool:
         """Inference with every norm folded, on the GPU, all widths multiples of 8 channels: the two producers of
