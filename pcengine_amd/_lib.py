@@ -33,10 +33,8 @@ class Geom(Structure):
     @classmethod
     def make(cls, ks, stride, pad, cmin, cmax, subm):
         g = cls()
-        for name, v in (("ks", ks), ("stride", stride), ("pad", pad), ("cmin", cmin), ("cmax", cmax)):
-            arr = getattr(g, name)
-            for a in range(3):
-                arr[a] = int(v[a])
+        for arr, v in ((g.ks, ks), (g.stride, stride), (g.pad, pad), (g.cmin, cmin), (g.cmax, cmax)):
+            arr[:] = int(v[0]), int(v[1]), int(v[2])
         g.subm = int(bool(subm))
         return g
 
@@ -186,6 +184,8 @@ _SIGNATURES = {
     "pce_pyramid_plan_sizeof": (c_int64, []),
     "pce_pyramid_plan": (c_int32, [c_int64, c_int32, POINTER(Geom), c_int32, POINTER(PyrRequest), c_int32, POINTER(PyrPlan)]),
     "pce_pyramid_build": (c_int32, [POINTER(PyrPlan), c_void_p, c_int64, c_void_p, c_int64, c_void_p]),
+    "pce_pyramid_plan_levels": (c_int32, [POINTER(c_int64), c_int32, c_int32, POINTER(PyrRequest), c_int32, POINTER(PyrPlan)]),
+    "pce_pyramid_maps": (c_int32, [POINTER(PyrPlan), POINTER(c_void_p), c_void_p, c_int64, c_void_p]),
     "pce_select_dataflow": (c_int32, [c_int64, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32]),
     "pce_select_layer": (c_int32, [c_int64, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32]),
     "pce_conv_oso_takes": (c_int32, [c_int32, c_int32, c_int32, c_int32, c_int32]),

@@ -17,35 +17,14 @@ static int64_t meta_ints(int kv) { return 3 * (int64_t)kv + 2 + META_STATUS; }
 
 extern "C" int64_t pce_pyramid_plan_sizeof(void) { return (int64_t)sizeof(pce_pyr_plan_t); }
 
-extern "C" int pce_pyramid_plan(int64_t n_cap, int32_t n_levels, const pce_geom_t *strided, int32_t n_batch,
-                                const pce_pyr_request_t *requests, int32_t n_requests, pce_pyr_plan_t *plan) {
-  if (!plan || !requests || (n_levels > 0 && !strided)) PCE_FAIL(PCE_EINVAL, "pce_pyramid_plan: null pointer");
-  if (n_cap <= 0 || n_levels < 0 || n_levels > PCE_PYR_MAX_LEVELS || n_requests < 1 || n_requests > PCE_PYR_MAX_MAPS || n_batch <= 0)
-    PCE_FAIL(PCE_EINVAL, "pce_pyramid_plan: %lld rows, %d levels (at most %d), %d maps (1..%d), %d batches", (long long)n_cap,
-             (int)n_levels, PCE_PYR_MAX_LEVELS, (int)n_requests, PCE_PYR_MAX_MAPS, (int)n_batch);
-  memset(plan, 0, sizeof(*plan));
-  plan->n_levels = n_levels;
-  plan->n_maps = n_requests;
-  plan->n_batch = n_batch;
-  plan->level_cap[0] = n_cap;
-  int64_t off = 0;
+// the arrays of every requested map behind `off` bytes, for the rows that level_cap says
+static int lay_out_maps(pce_pyr_plan_t *plan, const pce_pyr_request_t *requests, int64_t off) {
+  const int32_t n_levels = plan->n_levels, n_requests = plan->n_maps, n_batch = plan->n_batch;
   auto take = [&](int64_t bytes) {
     const int64_t at = off;
     off += pce_align_up(bytes > 0 ? bytes : 1, 256);
     return at;
   };
-  if (n_levels > 0) {
-    int64_t ws[PCE_PYR_MAX_LEVELS], cap[PCE_PYR_MAX_LEVELS];
-    const int rc = pce_outcoords_chain_plan(n_cap, n_levels, strided, n_batch, ws, cap);
-    if (rc) return rc;   // PCE_CHAIN_NOT_APPLICABLE: the caller builds level by level
-    for (int l = 0; l < n_levels; ++l) {
-      plan->strided[l] = strided[l];
-      plan->chain_ws_bytes[l] = ws[l];
-      plan->off_chain_ws[l] = take(ws[l]);
-      plan->level_cap[l + 1] = cap[l];
-      plan->off_coords[l + 1] = take(16 * cap[l]);
-    }
-  }
   // the counts and status words of all maps sit together: one copy reads them back
   plan->off_meta = off;
   for (int i = 0; i < n_requests; ++i) {
@@ -93,38 +72,57 @@ extern "C" int pce_pyramid_plan(int64_t n_cap, int32_t n_levels, const pce_geom_
   return PCE_OK;
 }
 
-extern "C" int pce_pyramid_build(pce_pyr_plan_t *plan, const int32_t *in_coords, int64_t n_in, void *arena, int64_t arena_bytes,
-                                 pce_stream_t stream) {
-  if (!plan || !in_coords || !arena) PCE_FAIL(PCE_EINVAL, "pce_pyramid_build: null pointer");
-  if (n_in <= 0 || n_in > plan->level_cap[0])
-    PCE_FAIL(PCE_ECAPACITY, "pce_pyramid_build: %lld rows, the plan holds %lld", (long long)n_in, (long long)plan->level_cap[0]);
-  if (arena_bytes < plan->arena_bytes || ((uintptr_t)arena & 255))
-    PCE_FAIL(PCE_EWORKSPACE, "pce_pyramid_build: the arena holds %lld bytes, the plan needs %lld (256-byte aligned)",
-             (long long)arena_bytes, (long long)plan->arena_bytes);
-  hipStream_t s = (hipStream_t)stream;
-  char *base = (char *)arena;
-  const int32_t *coords[PCE_PYR_MAX_LEVELS + 1];
-  coords[0] = in_coords;
-  plan->level_n[0] = n_in;
-  if (plan->n_levels > 0) {
-    void *ws[PCE_PYR_MAX_LEVELS];
-    int32_t *outs[PCE_PYR_MAX_LEVELS];
-    int64_t n_out[PCE_PYR_MAX_LEVELS];
-    for (int l = 0; l < plan->n_levels; ++l) {
-      ws[l] = base + plan->off_chain_ws[l];
-      outs[l] = (int32_t *)(base + plan->off_coords[l + 1]);
-      coords[l + 1] = outs[l];
-    }
-    // (the chain's own plan was made for the capacity: a smaller cloud fits its workspaces and buffers)
-    const int rc = pce_outcoords_chain_planned(in_coords, n_in, plan->level_cap[0], plan->n_levels, plan->strided, plan->n_batch, ws,
-                                               plan->chain_ws_bytes, outs, n_out, stream);
-    if (rc) return rc;
-    for (int l = 0; l < plan->n_levels; ++l) {
-      if (n_out[l] > plan->level_cap[l + 1])
-        PCE_FAIL(PCE_ECAPACITY, "pce_pyramid_build: level %d holds %lld rows, planned for %lld", l + 1, (long long)n_out[l], (long long)plan->level_cap[l + 1]);
-      plan->level_n[l + 1] = n_out[l];
+extern "C" int pce_pyramid_plan(int64_t n_cap, int32_t n_levels, const pce_geom_t *strided, int32_t n_batch,
+                                const pce_pyr_request_t *requests, int32_t n_requests, pce_pyr_plan_t *plan) {
+  if (!plan || !requests || (n_levels > 0 && !strided)) PCE_FAIL(PCE_EINVAL, "pce_pyramid_plan: null pointer");
+  if (n_cap <= 0 || n_levels < 0 || n_levels > PCE_PYR_MAX_LEVELS || n_requests < 1 || n_requests > PCE_PYR_MAX_MAPS || n_batch <= 0)
+    PCE_FAIL(PCE_EINVAL, "pce_pyramid_plan: %lld rows, %d levels (at most %d), %d maps (1..%d), %d batches", (long long)n_cap,
+             (int)n_levels, PCE_PYR_MAX_LEVELS, (int)n_requests, PCE_PYR_MAX_MAPS, (int)n_batch);
+  memset(plan, 0, sizeof(*plan));
+  plan->n_levels = n_levels;
+  plan->n_maps = n_requests;
+  plan->n_batch = n_batch;
+  plan->level_cap[0] = n_cap;
+  int64_t off = 0;
+  auto take = [&](int64_t bytes) {
+    const int64_t at = off;
+    off += pce_align_up(bytes > 0 ? bytes : 1, 256);
+    return at;
+  };
+  if (n_levels > 0) {
+    int64_t ws[PCE_PYR_MAX_LEVELS], cap[PCE_PYR_MAX_LEVELS];
+    const int rc = pce_outcoords_chain_plan(n_cap, n_levels, strided, n_batch, ws, cap);
+    if (rc) return rc;   // PCE_CHAIN_NOT_APPLICABLE: the caller builds level by level
+    for (int l = 0; l < n_levels; ++l) {
+      plan->strided[l] = strided[l];
+      plan->chain_ws_bytes[l] = ws[l];
+      plan->off_chain_ws[l] = take(ws[l]);
+      plan->level_cap[l + 1] = cap[l];
+      plan->off_coords[l + 1] = take(16 * cap[l]);
     }
   }
+  return lay_out_maps(plan, requests, off);
+}
+
+extern "C" int pce_pyramid_plan_levels(const int64_t *level_n, int32_t n_levels, int32_t n_batch, const pce_pyr_request_t *requests,
+                                       int32_t n_requests, pce_pyr_plan_t *plan) {
+  if (!plan || !requests || !level_n) PCE_FAIL(PCE_EINVAL, "pce_pyramid_plan_levels: null pointer");
+  if (n_levels < 0 || n_levels > PCE_PYR_MAX_LEVELS || n_requests < 1 || n_requests > PCE_PYR_MAX_MAPS || n_batch <= 0)
+    PCE_FAIL(PCE_EINVAL, "pce_pyramid_plan_levels: %d levels (at most %d), %d maps (1..%d), %d batches", (int)n_levels, PCE_PYR_MAX_LEVELS,
+             (int)n_requests, PCE_PYR_MAX_MAPS, (int)n_batch);
+  memset(plan, 0, sizeof(*plan));
+  plan->n_levels = n_levels;
+  plan->n_maps = n_requests;
+  plan->n_batch = n_batch;
+  for (int l = 0; l <= n_levels; ++l) {
+    if (level_n[l] <= 0) PCE_FAIL(PCE_EINVAL, "pce_pyramid_plan_levels: level %d without rows", l);
+    plan->level_cap[l] = plan->level_n[l] = level_n[l];
+  }
+  return lay_out_maps(plan, requests, 0);
+}
+
+// every map of the plan, from the coordinates of its levels; one wait, for the counts
+static int build_maps(pce_pyr_plan_t *plan, const int32_t *const *coords, char *base, hipStream_t s) {
   PCE_HIP(hipMemsetAsync(base + plan->off_meta, 0, (size_t)plan->meta_bytes, s));
   pce_kmap_problem_t probs[PCE_PYR_MAX_MAPS];
   memset(probs, 0, sizeof(probs));
@@ -162,7 +160,7 @@ extern "C" int pce_pyramid_build(pce_pyr_plan_t *plan, const int32_t *in_coords,
     u.n_batch = plan->n_batch;
     u.flags = r.table_only ? PCE_KMAP_TABLE_ONLY : 0;
   }
-  const int rc = pce_kmap_build_batch(probs, plan->n_maps, stream);
+  const int rc = pce_kmap_build_batch(probs, plan->n_maps, (pce_stream_t)s);
   if (rc) return rc;
   int32_t host[PCE_PYR_MAX_MAPS * (3 * 31 + 2 + META_STATUS)];
   PCE_HIP(hipMemcpyAsync(host, base + plan->off_meta, (size_t)plan->meta_bytes, hipMemcpyDeviceToHost, s));
@@ -181,4 +179,49 @@ extern "C" int pce_pyramid_build(pce_pyr_plan_t *plan, const int32_t *in_coords,
     m.qsum = h[3 * m.kv + 1];
   }
   return fallback ? PCE_PYR_UNSORTED : PCE_OK;
+}
+
+extern "C" int pce_pyramid_build(pce_pyr_plan_t *plan, const int32_t *in_coords, int64_t n_in, void *arena, int64_t arena_bytes,
+                                 pce_stream_t stream) {
+  if (!plan || !in_coords || !arena) PCE_FAIL(PCE_EINVAL, "pce_pyramid_build: null pointer");
+  if (n_in <= 0 || n_in > plan->level_cap[0])
+    PCE_FAIL(PCE_ECAPACITY, "pce_pyramid_build: %lld rows, the plan holds %lld", (long long)n_in, (long long)plan->level_cap[0]);
+  if (arena_bytes < plan->arena_bytes || ((uintptr_t)arena & 255))
+    PCE_FAIL(PCE_EWORKSPACE, "pce_pyramid_build: the arena holds %lld bytes, the plan needs %lld (256-byte aligned)",
+             (long long)arena_bytes, (long long)plan->arena_bytes);
+  hipStream_t s = (hipStream_t)stream;
+  char *base = (char *)arena;
+  const int32_t *coords[PCE_PYR_MAX_LEVELS + 1];
+  coords[0] = in_coords;
+  plan->level_n[0] = n_in;
+  if (plan->n_levels > 0) {
+    void *ws[PCE_PYR_MAX_LEVELS];
+    int32_t *outs[PCE_PYR_MAX_LEVELS];
+    int64_t n_out[PCE_PYR_MAX_LEVELS];
+    for (int l = 0; l < plan->n_levels; ++l) {
+      ws[l] = base + plan->off_chain_ws[l];
+      outs[l] = (int32_t *)(base + plan->off_coords[l + 1]);
+      coords[l + 1] = outs[l];
+    }
+    // (the chain's own plan was made for the capacity: a smaller cloud fits its workspaces and buffers)
+    const int rc = pce_outcoords_chain_planned(in_coords, n_in, plan->level_cap[0], plan->n_levels, plan->strided, plan->n_batch, ws,
+                                               plan->chain_ws_bytes, outs, n_out, stream);
+    if (rc) return rc;
+    for (int l = 0; l < plan->n_levels; ++l) {
+      if (n_out[l] > plan->level_cap[l + 1])
+        PCE_FAIL(PCE_ECAPACITY, "pce_pyramid_build: level %d holds %lld rows, planned for %lld", l + 1, (long long)n_out[l], (long long)plan->level_cap[l + 1]);
+      plan->level_n[l + 1] = n_out[l];
+    }
+  }
+  return build_maps(plan, coords, base, s);
+}
+
+extern "C" int pce_pyramid_maps(pce_pyr_plan_t *plan, const int32_t *const *level_coords, void *arena, int64_t arena_bytes, pce_stream_t stream) {
+  if (!plan || !level_coords || !arena) PCE_FAIL(PCE_EINVAL, "pce_pyramid_maps: null pointer");
+  for (int l = 0; l <= plan->n_levels; ++l)
+    if (!level_coords[l]) PCE_FAIL(PCE_EINVAL, "pce_pyramid_maps: no coordinates of level %d", l);
+  if (arena_bytes < plan->arena_bytes || ((uintptr_t)arena & 255))
+    PCE_FAIL(PCE_EWORKSPACE, "pce_pyramid_maps: the arena holds %lld bytes, the plan needs %lld (256-byte aligned)", (long long)arena_bytes,
+             (long long)plan->arena_bytes);
+  return build_maps(plan, level_coords, (char *)arena, (hipStream_t)stream);
 }

@@ -399,8 +399,9 @@ class MapPlanner:
         return plan
 
 
-def _prebuild_planned(input: spTensor, layers, planner: MapPlanner):
-    """The maps `layers` asks for through the native planner, or None where it does not apply (a map already cached,
+def _prebuild_planned(input: spTensor, layers, planner: Optional[MapPlanner]):
+    """The maps `layers` asks for in one library call, in the allocation of a plan that `planner` keeps or (None) in one of their own,
+    or None where that does not apply (a map already cached,
     reference tags, no batch count, a strided layer whose kernel differs from its stride or that is padded, a cloud
     that is not sorted): the caller then builds them map by map.  Same maps, same cache entries."""
     if not input.coords.is_cuda or not input.batchsize or input.batchsize <= 0:
@@ -440,6 +441,12 @@ def _prebuild_planned(input: spTensor, layers, planner: MapPlanner):
         return None
     coords = input.coords if input.coords.is_contiguous() else input.coords.contiguous()
     n = coords.shape[0]
+    if planner is None:
+        try:
+            level_coords, maps = backend.build_pyramid(coords, strided, requests, input.batchsize)
+        except backend.PlanNotApplicable:
+            return None
+        return _pyramid_store(input, entries, level_coords, maps)
     pkey = (tuple(map(tuple, ((r[0], r[1], r[10]) + tuple(r[2]) + tuple(r[6]) for r in requests))), tuple(input.coords_min[:3]),
             int(input.batchsize), coords.device)
     try:
@@ -447,6 +454,10 @@ def _prebuild_planned(input: spTensor, layers, planner: MapPlanner):
         level_coords, maps = plan.build(coords)
     except backend.PlanNotApplicable:
         return None
+    return _pyramid_store(input, entries, level_coords, maps)
+
+
+def _pyramid_store(input: spTensor, entries, level_coords, maps):
     level_stride = {0: input.stride}
     for (key, out_stride, lin, lout), km in zip(entries, maps):
         km.tag = 'auto'
@@ -462,10 +473,9 @@ def _prebuild(input: spTensor, layers, planner: Optional[MapPlanner] = None):
     """Builds the maps `layers` asks for, starting at `input`.  Returns (the tensor at the coordinates the last
     entry leaves, the maps that were built now)."""
     layers = list(layers)
-    if planner is not None:
-        built = _prebuild_planned(input, layers, planner)
-        if built is not None:
-            return input, built
+    built = _prebuild_planned(input, layers, planner)
+    if built is not None:
+        return input, built
     x = input
     pending, done = [], []
     chained = _chain_out_coords(input, layers)
@@ -512,8 +522,8 @@ def prebuild_maps(input: spTensor, layers, planner: Optional[MapPlanner] = None)
     The output coordinates of the strided layers are computed first, level by level (their number has
     to reach the host); then all maps are built together, every stage of the build as one launch over
     all layers, and their pair counts are read back in one copy.  The layers that follow find every
-    map in the cache.  With a ``planner`` the whole pyramid is laid out and built by the library in one allocation
-    (``MapPlanner``); where that does not apply the maps are built as described."""
+    map in the cache.  The whole pyramid is laid out and built by the library in one allocation, with a ``planner`` in one that is
+    kept from cloud to cloud (``MapPlanner``); where that does not apply the maps are built one by one."""
     _prebuild(input, layers, planner)
 
 

@@ -1,0 +1,99 @@
+"""The maps of a cloud built in one library call (``backend.build_pyramid``) against the general path, map by map: the same arrays,
+the same cache entries, the same refusals."""
+import numpy as np
+import pytest
+import torch
+
+import pcengine_amd as pe
+from pcengine_amd import backend, spconv, synth
+from tests.util import DEV, dev_coords
+
+pytestmark = pytest.mark.gpu
+
+UNET = [(3, 1, 0)] + [(2, 2, 0), (3, 1, 0)] * 4
+LISTS = {"unet": UNET, "lean": [(3, 1, 0, True), (2, 2, 0), (3, 1, 0, True), (3, 1, 0)], "one": [(3, 1, 0)], "down": [(2, 2, 0)],
+         "threes": [(3, 3, 0), (3, 1, 0), (2, 2, 0)], "padded": [(3, 1, 0), (3, 2, 1), (3, 1, 0)]}
+CLOUDS = {"lidar": lambda: synth.lidar_cloud(seed=2, azimuths=700, n_ground=7000, voxel=0.1),
+          "rooms": lambda: synth.indoor_batch(scenes=2, n_room=6000, n_box=125),
+          "tiny": lambda: synth.random_cloud(seed=1, n=200, extent=24)}
+
+
+def tensor(c):
+    c = c[np.lexsort(c.T[::-1])] if len(c) else c
+    return pe.spTensor(torch.zeros((len(c), 1), device=DEV), dev_coords(c), None, [0, 0, 0], c[:, 1:].max(0).tolist(),
+                       batchsize=int(c[:, 0].max()) + 1)
+
+
+def general(monkeypatch):
+    def never(*a):
+        raise backend.PlanNotApplicable()
+    monkeypatch.setattr(backend, "build_pyramid", never)
+
+
+@pytest.mark.parametrize("cloud", sorted(CLOUDS))
+@pytest.mark.parametrize("layers", sorted(LISTS))
+def test_same_maps(cloud, layers, monkeypatch):
+    c = CLOUDS[cloud]()
+    a, b = tensor(c), tensor(c)
+    spconv.prebuild_maps(a, LISTS[layers])
+    assert any(km.__dict__.get("_arena") is not None for km in a.kmaps.values()) == (layers != "padded")
+    general(monkeypatch)
+    spconv.prebuild_maps(b, LISTS[layers])
+    assert list(a.kmaps) == list(b.kmaps) and set(a.cbook) == set(b.cbook)
+    for s in a.cbook:
+        assert torch.equal(a.cbook[s], b.cbook[s])
+    for key in a.kmaps:
+        p, q = a.kmaps[key], b.kmaps[key]
+        for name in ("ks", "stride", "pad", "subm", "n_in", "n_out", "kv", "M", "qsum", "order_heavy", "order_nonzero", "order_single", "tag",
+                     "has_pairs", "batchsize", "_cmin", "_cmax"):
+            assert getattr(p, name) == getattr(q, name), name
+        assert list(p.knnz_host) == list(q.knnz_host) and list(p.kpos_host) == list(q.kpos_host) and list(p.qkpos_host) == list(q.qkpos_host)
+        assert (p.order is None) == (q.order is None)
+        for name in ("knnz", "kpos", "qkpos", "out_coords", "nbr_out", "nbr_in", "icsr", "ocsr", "icode", "ocode", "islot", "oslot", "imap", "omap"):
+            x, y = getattr(p, name), getattr(q, name)
+            assert (x is None) == (y is None), name
+            assert x is None or torch.equal(x.reshape(-1), y.reshape(-1)), name
+        assert [torch.equal(u, v) for u, v in zip(p._as_list()[:4], q._as_list()[:4])] == [True] * 4
+        assert all(torch.is_tensor(p[i]) and torch.equal(p[i], q[i]) for i in range(4)) and p[4] == q[4] and p[5] == q[5] and p[-1] == q[-1]
+        if p.order is not None:
+            n = p.n_out
+            assert torch.equal(p.order[n:2 * n], q.order[n:2 * n])                     # patterns
+            assert torch.equal(p.order[:n].sort().values, q.order[:n].sort().values)   # (rows of one pattern lie as they came)
+
+
+@pytest.mark.parametrize("kind", ["unsorted", "far", "outside the box"])
+def test_what_it_does_not_take(kind, monkeypatch):
+    c = CLOUDS["lidar"]()
+    x = tensor(c)
+    if kind == "unsorted":
+        x.coords = x.coords[torch.randperm(len(c), device=DEV)].contiguous()
+    elif kind == "far":
+        x.coords[-1, 1] = 40000
+    else:
+        x.coords_max = [v // 2 for v in x.coords_max]
+    def outcome():
+        y = pe.spTensor(x.feats, x.coords.clone(), None, [0, 0, 0], list(x.coords_max), batchsize=1)
+        try:
+            spconv.prebuild_maps(y, UNET)
+        except Exception as e:
+            return type(e), str(e)
+        return [(k, m.M, m.imap.clone(), m.omap.clone()) for k, m in y.kmaps.items()]
+    got = outcome()
+    general(monkeypatch)
+    want = outcome()
+    assert type(got) is type(want)
+    if isinstance(got, tuple):
+        assert got == want
+    else:
+        for (k, m, i, o), (k2, m2, i2, o2) in zip(got, want):
+            assert k == k2 and m == m2 and torch.equal(i, i2) and torch.equal(o, o2)
+
+
+def test_memory_of_maps_built_on_another_stream_is_told():
+    x = tensor(CLOUDS["lidar"]())
+    spconv.prebuild_maps(x, UNET)
+    for km in x.kmaps.values():
+        spans = [(t.untyped_storage().data_ptr(), t.untyped_storage().nbytes()) for t in km.device_tensors()]
+        for name in ("imap", "nbr_out", "order", "out_coords", "kpos"):
+            at = getattr(km, name).data_ptr()
+            assert any(lo <= at < lo + n for lo, n in spans), name
