@@ -368,6 +368,9 @@ int pce_pack_weights(const void *weight, int32_t dtype, int32_t kv, int32_t c_in
  * packed copy of `out` (pce_packed_weight_bytes of its shape, 16-byte aligned; NULL for fp32).  out must not overlap w. */
 int pce_prepare_weights(const void *w, int32_t dtype_w, int32_t dtype, int32_t kv, int32_t c_in, int32_t c_out,
                         int32_t transpose, int32_t flip, void *out, void *packed_dev, pce_stream_t stream);
+/* The same, and clears zero_dev[kv][c_in][c_out] (NULL: nothing) in the launch: what pce_conv_wgrad_add adds to. */
+int pce_prepare_weights_zero(const void *w, int32_t dtype_w, int32_t dtype, int32_t kv, int32_t c_in, int32_t c_out,
+                             int32_t transpose, int32_t flip, void *out, void *packed_dev, float *zero_dev, pce_stream_t stream);
 
 /* Fetch-on-demand: pairs (imap, omap, kpos, qkpos) and qsum = qkpos[kv] on the host.
  * fp16 needs an fp32 accumulation scratch of pce_conv_fod_workspace_bytes(); fp32 needs none. */
@@ -653,6 +656,11 @@ int pce_conv_wgrad(const void *in_feats, const void *grad_out, int32_t dtype, in
                    int64_t n_out, int32_t c_in, int32_t c_out, int32_t kv, int32_t mid,
                    const int32_t *imap_dev, const int32_t *omap_dev, const int32_t *kpos_dev,
                    const int32_t *qkpos_dev, int64_t qsum, float *grad_w_f32_dev, pce_stream_t stream);
+/* The same without the zeroing: the sums are added to what grad_w holds. */
+int pce_conv_wgrad_add(const void *in_feats, const void *grad_out, int32_t dtype, int64_t n_in,
+                       int64_t n_out, int32_t c_in, int32_t c_out, int32_t kv, int32_t mid,
+                       const int32_t *imap_dev, const int32_t *omap_dev, const int32_t *kpos_dev,
+                       const int32_t *qkpos_dev, int64_t qsum, float *grad_w_f32_dev, pce_stream_t stream);
 
 /* Per-layer dataflow choice from map density (pairs per output row), channel widths and the layer's kind:
  * `mid` as in the forward entry points (the centre offset of a submanifold layer, -1 otherwise), `transposed`

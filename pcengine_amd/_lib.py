@@ -147,6 +147,7 @@ _SIGNATURES = {
     "pce_packed_weight_bytes": (c_int64, [c_int32, c_int32, c_int32, c_int32]),
     "pce_pack_weights": (c_int32, [c_void_p, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p]),
     "pce_prepare_weights": (c_int32, [c_void_p] + [c_int32] * 7 + [c_void_p, c_void_p, c_void_p]),
+    "pce_prepare_weights_zero": (c_int32, [c_void_p] + [c_int32] * 7 + [c_void_p, c_void_p, c_void_p, c_void_p]),
     "pce_conv_fwd_fds": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32,
                                    c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, POINTER(c_int32), POINTER(c_int32), c_void_p, c_void_p,
                                    c_int64, c_int64, c_void_p, c_int64, POINTER(Epilogue), c_void_p]),
@@ -180,6 +181,8 @@ _SIGNATURES = {
     "pce_row_order_elems": (c_int64, [c_int64]),
     "pce_conv_fwd_dense": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int32, c_int32, POINTER(Epilogue), c_void_p]),
     "pce_conv_wgrad": (c_int32, [c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p,
+                                 c_void_p, c_void_p, c_int64, c_void_p, c_void_p]),
+    "pce_conv_wgrad_add": (c_int32, [c_void_p, c_void_p, c_int32, c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p,
                                  c_void_p, c_void_p, c_int64, c_void_p, c_void_p]),
     "pce_pyramid_plan_sizeof": (c_int64, []),
     "pce_pyramid_plan": (c_int32, [c_int64, c_int32, POINTER(Geom), c_int32, POINTER(PyrRequest), c_int32, POINTER(PyrPlan)]),

@@ -1016,19 +1016,28 @@ def pack_weights(weight: torch.Tensor) -> Optional[torch.Tensor]:
     return packed
 
 
-def prepare_weights(weight: torch.Tensor, dtype: torch.dtype, transpose: bool = False, flip: bool = False):
+def prepare_weights(weight: torch.Tensor, dtype: torch.dtype, transpose: bool = False, flip: bool = False,
+                    zero: Optional[torch.Tensor] = None):
     """(kernel, packed copy or None) of a layer of a training step in one launch: ``weight`` [kv, c_in, c_out] (or
-    [c_in, c_out]) in ``dtype``, every offset's matrix transposed and / or the offsets in reverse order on request."""
+    [c_in, c_out]) in ``dtype``, every offset's matrix transposed and / or the offsets in reverse order on request.
+    ``zero``: an fp32 array of as many elements that the launch clears."""
     half = dtype == torch.float16
     if not weight.is_cuda or weight.numel() == 0 or not (weight.dtype == dtype and (half or dtype == torch.float32)
                                                          or half and weight.dtype == torch.float32):
+        if zero is not None:
+            zero.zero_()
         w = weight.to(dtype)
         w = w.transpose(-2, -1) if transpose else w
         w = (w.flip(0) if flip and w.dim() == 3 else w).contiguous()
         return w, pack_weights(w) if half else None
     weight = weight.contiguous()
     if weight.dtype == dtype and not (transpose or flip):
+        if zero is not None:
+            zero.zero_()
         return weight, pack_weights(weight)
+    if zero is not None and (zero.dtype != torch.float32 or zero.numel() != weight.numel() or not zero.is_contiguous()
+                             or zero.device != weight.device):
+        raise ValueError("the array to clear must be a contiguous fp32 one of the kernel's size")
     lib = _lib.load()
     kv = weight.shape[0] if weight.dim() == 3 else 1
     c_in, c_out = weight.shape[-2:]
@@ -1037,8 +1046,8 @@ def prepare_weights(weight: torch.Tensor, dtype: torch.dtype, transpose: bool = 
     packed = None
     if half:
         packed = torch.empty(lib.pce_packed_weight_bytes(PCE_F16, kv, rows, cols), dtype=torch.uint8, device=weight.device)
-    _lib.check(lib.pce_prepare_weights(weight.data_ptr(), _dtype_code(weight), PCE_F16 if half else PCE_F32, kv, c_in, c_out,
-                                       int(transpose), int(flip), out.data_ptr(), _ptr(packed), _stream(weight.device)))
+    _lib.check(lib.pce_prepare_weights_zero(weight.data_ptr(), _dtype_code(weight), PCE_F16 if half else PCE_F32, kv, c_in, c_out,
+                                            int(transpose), int(flip), out.data_ptr(), _ptr(packed), _ptr(zero), _stream(weight.device)))
     return out, packed
 
 
@@ -1501,13 +1510,15 @@ def bn_backward(x: torch.Tensor, dy: torch.Tensor, weight, save_mean: torch.Tens
     return (dx, grads[0], grads[1]) + ((dm,) if masked else ())
 
 
-def conv_wgrad(feats: torch.Tensor, grad_out: torch.Tensor, km: KernelMap, transposed: bool = False) -> torch.Tensor:
-    """Gradient of ``conv_forward`` with respect to the kernel: fp32 [kv, c_in, c_out]."""
+def conv_wgrad(feats: torch.Tensor, grad_out: torch.Tensor, km: KernelMap, transposed: bool = False,
+               zeros: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Gradient of ``conv_forward`` with respect to the kernel: fp32 [kv, c_in, c_out], in ``zeros`` (fp32 of that shape, cleared
+    already) where that is given."""
     lib = _lib.load()
     _require_cuda(feats, "feats")
     a, b = (km.omap, km.imap) if transposed else (km.imap, km.omap)
     done = _lib.wgrad(feats, grad_out, a, b, km.kpos, km.qkpos, km.n_out if transposed else km.n_in, km.n_in if transposed else km.n_out,
-                      km.kv, _mid(km.ks) if km.subm else -1, km.qsum, _stream(feats.device))
+                      km.kv, _mid(km.ks) if km.subm else -1, km.qsum, _stream(feats.device), zeros)
     if done is not None:
         return done if type(done) is not int else _lib.check(done)
     feats, grad_out = feats.contiguous(), grad_out.contiguous()
@@ -1518,19 +1529,22 @@ def conv_wgrad(feats: torch.Tensor, grad_out: torch.Tensor, km: KernelMap, trans
         raise ValueError(f"the map expects {n_in} feature rows and {n_out} gradient rows")
     imap, omap = (km.omap, km.imap) if transposed else (km.imap, km.omap)
     c_in, c_out = feats.shape[1], grad_out.shape[1]
-    gw = torch.empty((km.kv, c_in, c_out), dtype=torch.float32, device=feats.device)
-    _lib.check(lib.pce_conv_wgrad(feats.data_ptr(), grad_out.data_ptr(), _dtype_code(feats), n_in, n_out, c_in, c_out, km.kv,
-                                  _mid(km.ks) if km.subm else -1, imap.data_ptr(), omap.data_ptr(), km.kpos.data_ptr(),
-                                  km.qkpos.data_ptr(), km.qsum, gw.data_ptr(), _stream(feats.device)))
+    if zeros is not None and (zeros.dtype != torch.float32 or tuple(zeros.shape) != (km.kv, c_in, c_out) or not zeros.is_contiguous()
+                              or zeros.device != feats.device):
+        raise ValueError(f"the gradient goes to a contiguous fp32 array [{km.kv}, {c_in}, {c_out}]")
+    gw = zeros if zeros is not None else torch.empty((km.kv, c_in, c_out), dtype=torch.float32, device=feats.device)
+    wgrad = lib.pce_conv_wgrad if zeros is None else lib.pce_conv_wgrad_add
+    _lib.check(wgrad(feats.data_ptr(), grad_out.data_ptr(), _dtype_code(feats), n_in, n_out, c_in, c_out, km.kv, _mid(km.ks) if km.subm else -1,
+                     imap.data_ptr(), omap.data_ptr(), km.kpos.data_ptr(), km.qkpos.data_ptr(), km.qsum, gw.data_ptr(), _stream(feats.device)))
     return gw
 
 
 _ZERO_POS = {}
 
 
-def dense_wgrad(feats: torch.Tensor, grad_out: torch.Tensor) -> torch.Tensor:
+def dense_wgrad(feats: torch.Tensor, grad_out: torch.Tensor, zeros: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Gradient of ``dense_forward`` with respect to its [c_in, c_out] matrix, in fp32: the kernel-gradient
-    kernel run over row tiles only (one offset, every row paired with itself, no pair list)."""
+    kernel run over row tiles only (one offset, every row paired with itself, no pair list).  ``zeros`` as for ``conv_wgrad``."""
     lib = _lib.load()
     _require_cuda(feats, "feats")
     feats, grad_out = feats.contiguous(), grad_out.contiguous()
@@ -1544,9 +1558,13 @@ def dense_wgrad(feats: torch.Tensor, grad_out: torch.Tensor) -> torch.Tensor:
         pos = _ZERO_POS[feats.device] = torch.zeros(2, dtype=torch.int32, device=feats.device)
     if n == 0:  # empty tensors have no data pointer to hand over
         return torch.zeros((c_in, c_out), dtype=torch.float32, device=feats.device)
-    gw = torch.empty((c_in, c_out), dtype=torch.float32, device=feats.device)
-    _lib.check(lib.pce_conv_wgrad(feats.data_ptr(), grad_out.data_ptr(), _dtype_code(feats), n, n, c_in, c_out, 1, 0, None, None,
-                                  pos.data_ptr(), pos.data_ptr(), 0, gw.data_ptr(), _stream(feats.device)))
+    if zeros is not None and (zeros.dtype != torch.float32 or tuple(zeros.shape) != (c_in, c_out) or not zeros.is_contiguous()
+                              or zeros.device != feats.device):
+        raise ValueError(f"the gradient goes to a contiguous fp32 array [{c_in}, {c_out}]")
+    gw = zeros if zeros is not None else torch.empty((c_in, c_out), dtype=torch.float32, device=feats.device)
+    wgrad = lib.pce_conv_wgrad if zeros is None else lib.pce_conv_wgrad_add
+    _lib.check(wgrad(feats.data_ptr(), grad_out.data_ptr(), _dtype_code(feats), n, n, c_in, c_out, 1, 0, None, None,
+                     pos.data_ptr(), pos.data_ptr(), 0, gw.data_ptr(), _stream(feats.device)))
     return gw
 
 
@@ -1557,7 +1575,7 @@ def conv_backward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, grad
     ``grad_out`` with the per-offset transposed kernel over the same pairs with the roles swapped,
     run by the forward kernels; the kernel gradient comes from ``pce_conv_wgrad`` (fp32 sums,
     returned in ``weight_dtype``, by default the kernel's)."""
-    gf = gw = None
+    gf = gw = zeros = None
     if need_feats:
         w3 = weight if weight.dim() == 3 else weight.unsqueeze(0)
         c_out, c_in = w3.shape[1:]
@@ -1565,11 +1583,13 @@ def conv_backward(feats: torch.Tensor, weight: torch.Tensor, km: KernelMap, grad
         # over a map that is its own mirror image the swapped layer is the plain one with the offsets reversed (see
         # conv_forward): they are reversed in the launch that transposes them
         mirror = not transposed and km.subm and all(k % 2 == 1 for k in km.ks)
-        wt, packed = prepare_weights(w3, w3.dtype, transpose=True, flip=mirror)
+        if need_weight and w3.is_cuda and tuple(w3.shape) == (km.kv, feats.shape[1], grad_out.shape[1]):      # the launch that transposes the kernel clears its gradient's array
+            zeros = torch.empty(w3.shape, dtype=torch.float32, device=w3.device)
+        wt, packed = prepare_weights(w3, w3.dtype, transpose=True, flip=mirror, zero=zeros)
         gf = conv_forward(grad_out.contiguous(), wt, km, df, transposed=not transposed and not mirror, packed=packed,
                           split_offsets=False)
     if need_weight:
-        gw = conv_wgrad(feats, grad_out, km, transposed).to(weight_dtype or weight.dtype).reshape(weight.shape)
+        gw = conv_wgrad(feats, grad_out, km, transposed, zeros).to(weight_dtype or weight.dtype).reshape(weight.shape)
     return gf, gw
 
 

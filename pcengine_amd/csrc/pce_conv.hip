@@ -52,11 +52,12 @@ __global__ void __launch_bounds__(256) pack_weights_kernel(const half_t *__restr
 // for fp16 the packed copy beside it.  A workgroup takes a 32 x 32 tile of one offset through LDS, so that rows are
 // read and written along memory in either orientation (row stride 33: no bank conflicts down a column).  Bound by
 // launches: a 27 x 256 x 256 kernel is 10 MB in and out.  As a cast, a transposing copy, a reversal and one or two packing
-// launches the same took a step of a U-Net on a 100 k-voxel scan 1740 us in 330 launches, now 525 in 99.
+// launches the same took a step of a U-Net on a 100 k-voxel scan 1740 us in 330 launches, now 525 in 99.  `zero`: an array shaped like
+// W that is cleared by the way, the kernel gradient's (a launch of its own: 50 more a step, 3.4 us each and the gaps between).
 template <typename TS, typename TD>
 __global__ void __launch_bounds__(256) prepare_weights_kernel(const TS *__restrict__ W, TD *__restrict__ out, half_t *__restrict__ P,
                                                               int kv, int c_in, int c_out, int transpose, int flip,
-                                                              int k8_total, int n_pad, int bi, int bo) {
+                                                              int k8_total, int n_pad, int bi, int bo, float *__restrict__ zero) {
   __shared__ TD tile[32][33];   // [row k][column n] of the result
   const int kp = blockIdx.x / (bi * bo), rest = blockIdx.x % (bi * bo);
   const int i0 = (rest / bo) * 32, o0 = (rest % bo) * 32;   // input and output channels of the tile
@@ -64,7 +65,10 @@ __global__ void __launch_bounds__(256) prepare_weights_kernel(const TS *__restri
 #pragma unroll
   for (int y = y0; y < 32; y += 8) {
     TD v = (TD)0.f;
-    if (i0 + y < c_in && o0 + x < c_out) v = (TD)W[((long long)kp * c_in + i0 + y) * c_out + o0 + x];
+    const long long at = ((long long)kp * c_in + i0 + y) * c_out + o0 + x;
+    const bool in = i0 + y < c_in && o0 + x < c_out;
+    if (in) v = (TD)W[at];
+    if (in && zero) zero[at] = 0.f;
     if (transpose)
       tile[x][y] = v;
     else
@@ -1737,8 +1741,8 @@ extern "C" int pce_pack_weights(const void *w, int32_t dtype, int32_t kv, int32_
   return PCE_OK;
 }
 
-extern "C" int pce_prepare_weights(const void *w, int32_t dtype_w, int32_t dtype, int32_t kv, int32_t c_in, int32_t c_out,
-                                   int32_t transpose, int32_t flip, void *out, void *packed, pce_stream_t stream) {
+extern "C" int pce_prepare_weights_zero(const void *w, int32_t dtype_w, int32_t dtype, int32_t kv, int32_t c_in, int32_t c_out,
+                                        int32_t transpose, int32_t flip, void *out, void *packed, float *zero, pce_stream_t stream) {
   if (!w || !out || kv <= 0 || c_in <= 0 || c_out <= 0) PCE_FAIL(PCE_EINVAL, "pce_prepare_weights: bad argument");
   if ((dtype_w != PCE_F16 && dtype_w != PCE_F32) || (dtype != dtype_w && dtype != PCE_F16))
     PCE_FAIL(PCE_EINVAL, "pce_prepare_weights: dtype %d from %d", (int)dtype, (int)dtype_w);
@@ -1751,7 +1755,7 @@ extern "C" int pce_prepare_weights(const void *w, int32_t dtype_w, int32_t dtype
   if (blocks >= (1ll << 31)) PCE_FAIL(PCE_ECAPACITY, "pce_prepare_weights: %lld workgroups exceed the grid limit", blocks);
 #define PCE_PREP(TS_, TD_)                                                                                                       \
   hipLaunchKernelGGL((prepare_weights_kernel<TS_, TD_>), dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (const TS_ *)w, \
-                     (TD_ *)out, (half_t *)packed, kv, c_in, c_out, transpose, flip, k8_total, n_pad, bi, bo)
+                     (TD_ *)out, (half_t *)packed, kv, c_in, c_out, transpose, flip, k8_total, n_pad, bi, bo, zero)
   if (dtype_w == PCE_F16)
     PCE_PREP(half_t, half_t);
   else if (dtype == PCE_F16)
@@ -1761,6 +1765,11 @@ extern "C" int pce_prepare_weights(const void *w, int32_t dtype_w, int32_t dtype
 #undef PCE_PREP
   PCE_LAUNCH_CHECK("prepare_weights");
   return PCE_OK;
+}
+
+extern "C" int pce_prepare_weights(const void *w, int32_t dtype_w, int32_t dtype, int32_t kv, int32_t c_in, int32_t c_out,
+                                   int32_t transpose, int32_t flip, void *out, void *packed, pce_stream_t stream) {
+  return pce_prepare_weights_zero(w, dtype_w, dtype, kv, c_in, c_out, transpose, flip, out, packed, nullptr, stream);
 }
 
 extern "C" int64_t pce_conv_fod_workspace_bytes(int64_t n_out, int32_t c_out, int32_t dtype) {
@@ -4002,16 +4011,18 @@ __global__ void __launch_bounds__(256) wgrad_kernel(const T *__restrict__ in, co
   if (cur >= 0) flush(cur);
 }
 
-extern "C" int pce_conv_wgrad(const void *in, const void *gout, int32_t dtype, int64_t n_in, int64_t n_out, int32_t c_in,
-                              int32_t c_out, int32_t kv, int32_t mid, const int32_t *imap, const int32_t *omap,
-                              const int32_t *kpos, const int32_t *qkpos, int64_t qsum, float *gw, pce_stream_t stream) {
+static int wgrad_impl(bool clear, const void *in, const void *gout, int32_t dtype, int64_t n_in, int64_t n_out, int32_t c_in,
+                      int32_t c_out, int32_t kv, int32_t mid, const int32_t *imap, const int32_t *omap,
+                      const int32_t *kpos, const int32_t *qkpos, int64_t qsum, float *gw, pce_stream_t stream) {
   int rc = check_common("pce_conv_wgrad", in, gout, gw, dtype, n_in, n_out, c_in, c_out, kv, mid);
   if (rc || (rc = check_qsum("pce_conv_wgrad", qsum))) return rc;
   if (!kpos || !qkpos || (qsum > 0 && (!imap || !omap))) PCE_FAIL(PCE_EINVAL, "pce_conv_wgrad: null map pointer");
   hipStream_t s = (hipStream_t)stream;
   long long total = (long long)kv * c_in * c_out;
-  hipLaunchKernelGGL(zero_f32_kernel, dim3((unsigned)pce_div_up(total, 1024)), dim3(256), 0, s, gw, total);
-  PCE_LAUNCH_CHECK("zero_f32");
+  if (clear) {
+    hipLaunchKernelGGL(zero_f32_kernel, dim3((unsigned)pce_div_up(total, 1024)), dim3(256), 0, s, gw, total);
+    PCE_LAUNCH_CHECK("zero_f32");
+  }
   long long pair_tiles = qsum / PCE_QUANTUM;
   long long tiles = pair_tiles + (mid >= 0 ? pce_div_up(n_out, 128) : 0);
   if (tiles <= 0) return PCE_OK;
@@ -4064,6 +4075,17 @@ extern "C" int pce_conv_wgrad(const void *in, const void *gout, int32_t dtype, i
 #undef PCE_WGRAD16
   PCE_LAUNCH_CHECK("wgrad");
   return PCE_OK;
+}
+
+extern "C" int pce_conv_wgrad(const void *in, const void *gout, int32_t dtype, int64_t n_in, int64_t n_out, int32_t c_in,
+                              int32_t c_out, int32_t kv, int32_t mid, const int32_t *imap, const int32_t *omap,
+                              const int32_t *kpos, const int32_t *qkpos, int64_t qsum, float *gw, pce_stream_t stream) {
+  return wgrad_impl(true, in, gout, dtype, n_in, n_out, c_in, c_out, kv, mid, imap, omap, kpos, qkpos, qsum, gw, stream);
+}
+extern "C" int pce_conv_wgrad_add(const void *in, const void *gout, int32_t dtype, int64_t n_in, int64_t n_out, int32_t c_in,
+                                  int32_t c_out, int32_t kv, int32_t mid, const int32_t *imap, const int32_t *omap,
+                                  const int32_t *kpos, const int32_t *qkpos, int64_t qsum, float *gw, pce_stream_t stream) {
+  return wgrad_impl(false, in, gout, dtype, n_in, n_out, c_in, c_out, kv, mid, imap, omap, kpos, qkpos, qsum, gw, stream);
 }
 
 // ---- batch normalisation over the rows of a feature matrix (script/batchnorm.py:7-10) -----------------

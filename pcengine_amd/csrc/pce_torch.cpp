@@ -16,6 +16,7 @@
 // entry points that a library beside this extension may be without: the calls that need them are then declined
 #pragma weak pce_bn_forward_counted
 #pragma weak pce_bn_backward_masked
+#pragma weak pce_conv_wgrad_add
 
 namespace {
 
@@ -324,11 +325,12 @@ PyObject *bn_backward(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   END_HANDLE_TH_ERRORS
 }
 
-// wgrad(features, output gradient, imap, omap, kpos, qkpos, n_in, n_out, kv, mid, qsum, stream) -> fp32 [kv, c_in, c_out], None or an error code
+// wgrad(features, output gradient, imap, omap, kpos, qkpos, n_in, n_out, kv, mid, qsum, stream[, zeros to add to])
+//   -> fp32 [kv, c_in, c_out], None or an error code
 PyObject *wgrad(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  if (n_args != 12) {
-    PyErr_SetString(PyExc_TypeError, "wgrad: twelve arguments");
+  if (n_args != 12 && n_args != 13) {
+    PyErr_SetString(PyExc_TypeError, "wgrad: twelve or thirteen arguments");
     return nullptr;
   }
   const at::Tensor *x = rows_of(args[0]), *g = rows_of(args[1]);
@@ -346,16 +348,27 @@ PyObject *wgrad(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   Py_DECREF(tuple);   // (the caller holds the tensors)
   if (v.bad || num[2] <= 0) Py_RETURN_NONE;
   const int64_t c_in = x->size(1), c_out = g->size(1);
+  const at::Tensor *zeros = nullptr;
+  if (n_args == 13 && args[12] != Py_None) {
+    zeros = plain(args[12]);
+    if (!zeros || zeros->scalar_type() != at::kFloat || zeros->device() != x->device() || !zeros->is_contiguous() ||
+        zeros->numel() != num[2] * c_in * c_out || !pce_conv_wgrad_add)
+      Py_RETURN_NONE;
+  }
   at::Tensor gw;
   int rc;
   {
     Unlocked unlocked;
-    gw = at::empty({num[2], c_in, c_out}, x->options().dtype(at::kFloat));
-    rc = pce_conv_wgrad(x->data_ptr(), g->data_ptr(), x->scalar_type() == at::kHalf ? PCE_F16 : PCE_F32, num[0], num[1], (int32_t)c_in, (int32_t)c_out,
-                        (int32_t)num[2], (int32_t)num[3], m[0], m[1], m[2], m[3], num[4], gw.data_ptr<float>(), stream);
+    if (!zeros) gw = at::empty({num[2], c_in, c_out}, x->options().dtype(at::kFloat));
+    float *to = zeros ? zeros->data_ptr<float>() : gw.data_ptr<float>();
+    const int dt = x->scalar_type() == at::kHalf ? PCE_F16 : PCE_F32, ci = (int)c_in, co = (int)c_out, kv = (int)num[2], mid = (int)num[3];
+    rc = zeros ? pce_conv_wgrad_add(x->data_ptr(), g->data_ptr(), dt, num[0], num[1], ci, co, kv, mid, m[0], m[1], m[2], m[3], num[4], to, stream)
+               : pce_conv_wgrad(x->data_ptr(), g->data_ptr(), dt, num[0], num[1], ci, co, kv, mid, m[0], m[1], m[2], m[3], num[4], to, stream);
   }
   if (rc != PCE_OK) return PyLong_FromLong(rc);
-  return THPVariable_Wrap(std::move(gw));
+  if (!zeros) return THPVariable_Wrap(std::move(gw));
+  Py_INCREF(args[12]);
+  return args[12];
   END_HANDLE_TH_ERRORS
 }
 

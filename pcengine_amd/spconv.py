@@ -228,12 +228,14 @@ class _DenseFunction(torch.autograd.Function):
     def backward(ctx, grad_out):
         feats, kernel = ctx.saved_tensors
         grad_out = grad_out.contiguous()
-        gf = gw = None
+        gf = gw = zeros = None
         if ctx.needs_input_grad[0]:
-            kt, packed = backend.prepare_weights(kernel.detach(), kernel.dtype, transpose=True)
+            if ctx.needs_input_grad[1] and kernel.is_cuda and feats.shape[0] > 0:     # cleared in the launch that transposes the kernel
+                zeros = torch.empty(kernel.shape, dtype=torch.float32, device=kernel.device)
+            kt, packed = backend.prepare_weights(kernel.detach(), kernel.dtype, transpose=True, zero=zeros)
             gf = backend.dense_forward(grad_out, kt, packed)
         if ctx.needs_input_grad[1]:
-            gw = backend.dense_wgrad(feats.detach(), grad_out).to(ctx.kernel_dtype)
+            gw = backend.dense_wgrad(feats.detach(), grad_out, zeros).to(ctx.kernel_dtype)
         gb = grad_out.sum(0) if (ctx.has_bias and ctx.needs_input_grad[2]) else None
         return gf, gw, gb
 
