@@ -180,6 +180,11 @@ int pce_voxelize_emit3(const void *ws_dev, int64_t n_points, int64_t n_voxels,
                        const int32_t *coords_min3_host, const int32_t *coords_max3_host, int32_t *coords_out_dev,
                        int64_t *index_out_dev, int64_t *inverse_out_dev, pce_stream_t stream);
 
+/* Maxima of the columns behind the first of rows_dev[n][width] (width 2 to 4), to upper_host[width - 1]; one wait of the host. */
+int64_t pce_column_max_workspace_bytes(void);
+int pce_column_max(const int32_t *rows_dev, int64_t n, int32_t width, void *ws_dev, int64_t ws_bytes, int32_t *upper_host,
+                   pce_stream_t stream);
+
 /* ---- collation -------------------------------------------------------------------------------- *
  * The coordinates of a batch (sparse_collate, script/utils.py:167-196): sample k's rows[k] rows of (x, y, z) at
  * coords_dev[k] become out_dev[total,4] = (k, x, y, z), in order; upper3_host receives the maxima of the three

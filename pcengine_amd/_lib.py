@@ -123,6 +123,8 @@ _SIGNATURES = {
                                      c_void_p]),
     "pce_collate_workspace_bytes": (c_int64, []),
     "pce_collate": (c_int32, [POINTER(c_void_p), POINTER(c_int64), c_int32, c_void_p, c_void_p, c_int64, POINTER(c_int32), c_void_p]),
+    "pce_column_max_workspace_bytes": (c_int64, []),
+    "pce_column_max": (c_int32, [c_void_p, c_int64, c_int32, c_void_p, c_int64, POINTER(c_int32), c_void_p]),
     "pce_col_sums_workspace_bytes": (c_int64, [c_int64, c_int32]),
     "pce_col_sums": (c_int32, [c_void_p, c_void_p, c_int32, c_int64, c_int32, c_void_p, c_int64, c_void_p, c_void_p]),
     "pce_col_affine": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_int32,

@@ -293,6 +293,19 @@ def voxelize(points: torch.Tensor, voxel_size, batch_index: Optional[int] = 0, r
     return tuple(outs)
 
 
+def coords_upper(coords: torch.Tensor) -> list:
+    """Maxima of the columns behind the first, as a list (one read-back)."""
+    if not (type(coords) is torch.Tensor and coords.is_cuda and coords.dtype == torch.int32 and coords.dim() == 2 and 2 <= coords.shape[1] <= 4
+            and coords.shape[0] > 0 and coords.is_contiguous() and coords.device.index == torch.cuda.current_device()):
+        return coords[:, 1:].max(dim=0).values.cpu().tolist()
+    lib = _lib.load()
+    ws_bytes = lib.pce_column_max_workspace_bytes()
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=coords.device)
+    upper = (_lib.c_int32 * (coords.shape[1] - 1))()
+    _lib.check(lib.pce_column_max(coords.data_ptr(), coords.shape[0], coords.shape[1], ws.data_ptr(), ws_bytes, upper, _stream(coords.device)))
+    return list(upper)
+
+
 def collate_coords(coords: Sequence[torch.Tensor]):
     """(int32 [N, 4] = (sample, x, y, z), maxima of x, y, z as a list) of the samples' int32 [n, 3] coordinates in one
     launch, or None where the kernel does not take them (other layouts or dtypes, another device than the current one, no

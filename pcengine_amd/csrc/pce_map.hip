@@ -1575,6 +1575,62 @@ __global__ void __launch_bounds__(256) collate_kernel(CollateArgs a, int4 *__res
   }
 }
 
+// upper[block]: maxima of the columns behind the first of rows of `width` ints (a sample's: y and z of x, y, z; a batch's: x, y and
+// z), over the rows that the workgroup reads.  Bound by the launch: torch's reduction of the view is a fill of 4 us and a
+// kernel of one workgroup, 9 to 12 on 150 k rows; 6 in all this way.
+__global__ void __launch_bounds__(256) column_max_kernel(const int *__restrict__ rows, long long n, int width, int *__restrict__ upper) {
+  __shared__ int part[4][3];
+  int m[3] = {(int)0x80000000, (int)0x80000000, (int)0x80000000};
+  for (long long r0 = (long long)blockIdx.x * 1024 + threadIdx.x; r0 < n; r0 += (long long)gridDim.x * 1024) {
+    int c[4][3];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {   // four rows out together, the last one again behind the end
+      const long long r = r0 + 256 * k < n ? r0 + 256 * k : n - 1;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) c[k][d] = rows[r * width + (d + 1 < width ? d + 1 : 1)];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) m[d] = c[k][d] > m[d] ? c[k][d] : m[d];
+  }
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    for (int o = 32; o >= 1; o >>= 1) {
+      const int v = __shfl_xor(m[d], o, PCE_WAVE);
+      m[d] = v > m[d] ? v : m[d];
+    }
+    if (__lane_id() == 0) part[threadIdx.x >> 6][d] = m[d];
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    int v = part[0][threadIdx.x];
+    for (int w = 1; w < 4; ++w) v = part[w][threadIdx.x] > v ? part[w][threadIdx.x] : v;
+    upper[blockIdx.x * 4 + threadIdx.x] = v;
+  }
+}
+
+extern "C" int64_t pce_column_max_workspace_bytes(void) { return COLLATE_BLOCKS * 16; }
+
+extern "C" int pce_column_max(const int32_t *rows, int64_t n, int32_t width, void *ws, int64_t ws_bytes, int32_t *upper_host,
+                              pce_stream_t stream) {
+  if (!rows || !ws || !upper_host) PCE_FAIL(PCE_EINVAL, "pce_column_max: null pointer");
+  if (n <= 0 || width < 2 || width > 4) PCE_FAIL(PCE_EINVAL, "pce_column_max: %lld rows of %d (2..4)", (long long)n, (int)width);
+  if (ws_bytes < pce_column_max_workspace_bytes()) PCE_FAIL(PCE_EWORKSPACE, "pce_column_max: workspace %lld", (long long)ws_bytes);
+  hipStream_t s = (hipStream_t)stream;
+  const unsigned blocks = (unsigned)(pce_div_up(n, 1024) < COLLATE_BLOCKS ? pce_div_up(n, 1024) : COLLATE_BLOCKS);
+  hipLaunchKernelGGL(column_max_kernel, dim3(blocks), dim3(256), 0, s, rows, (long long)n, (int)width, (int *)ws);
+  PCE_LAUNCH_CHECK("column_max");
+  int host[COLLATE_BLOCKS][4];
+  PCE_HIP(hipMemcpyAsync(host, ws, (size_t)blocks * sizeof(host[0]), hipMemcpyDeviceToHost, s));
+  PCE_HIP(hipStreamSynchronize(s));
+  for (int d = 0; d + 1 < width; ++d) {
+    upper_host[d] = host[0][d];
+    for (unsigned b = 1; b < blocks; ++b) upper_host[d] = host[b][d] > upper_host[d] ? host[b][d] : upper_host[d];
+  }
+  return PCE_OK;
+}
+
 extern "C" int64_t pce_collate_workspace_bytes(void) { return COLLATE_BLOCKS * 16; }
 
 extern "C" int pce_collate(const int32_t *const *coords, const int64_t *rows, int32_t samples, int32_t *out, void *ws,
