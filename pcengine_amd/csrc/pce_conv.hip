@@ -3469,11 +3469,11 @@ extern "C" int pce_conv_fwd_dense(const void *in, const void *w, const void *wp,
 // (ConvolutionBackwardD1's per-offset GEMM, backend/spconv.cu:400-629): per offset a GEMM whose reduction
 // runs over the pairs.  A workgroup owns a BLK x BLK block of (ci, co) and a run of consecutive 128-pair
 // quanta (then 128-row tiles of the centre offset); its four wavefronts hold (BLK/2) x (BLK/2) each in
-// fp32 MFMA accumulators (v_mfma_f32_32x32x2_f32, also for fp16 tensors: they are widened when staged, and
-// with the pair index as the reduction index the fp16 MFMA would need its operands transposed).  Rows
-// are staged in LDS 32 pairs at a time.  The accumulators are added to the fp32 result with atomics only
-// when the offset changes or the run ends: one atomic per element per run instead of one per quantum (the
-// order of the additions, and so the last bits, still vary from run to run).
+// fp32 MFMA accumulators (v_mfma_f32_32x32x2_f32).  Rows are staged in LDS 32 pairs at a time.  The accumulators
+// are added to the fp32 result with atomics only when the offset changes or the run ends: one atomic per element
+// per run instead of one per quantum (the order of the additions, and so the last bits, still vary from run to run).
+// fp32 rows that are not whole 16-byte pieces, or lie beyond 3.75 GB, come this way; the others have
+// wgrad_f32_ring_kernel.
 #define WGRAD_KP 32   // pairs per LDS stage
 
 // PER consecutive channels of one row as fp32 (zeros for a missing row or past the last channel); the vector
@@ -3711,6 +3711,46 @@ __device__ __forceinline__ u32x4 byte_range(const void *p, unsigned bytes) {
   return (u32x4){(unsigned)(uintptr_t)p, (unsigned)((uintptr_t)p >> 32), bytes, 0x00020000u};
 }
 
+// A tile: its offset (-1: none), its first pair or row, how many, and whether rows pair with themselves.
+struct WgradTile {
+  int w, first, count, same;
+};
+// The tiles of a run, one after the other.  What it returns is uniform and in scalar registers.
+struct WgradWalk {
+  long long tile, end, pair_tiles, n_rows;
+  int kv, mid, lw;
+  const int *kpos, *qkpos;
+  __device__ __forceinline__ WgradWalk(long long t_begin, int n_tiles, long long pair_tiles, long long n_rows, int kv, int mid, const int *kpos, const int *qkpos)
+      : tile(t_begin), end(t_begin + n_tiles), pair_tiles(pair_tiles), n_rows(n_rows), kv(kv), mid(mid), lw(0), kpos(kpos), qkpos(qkpos) {
+    if (tile < pair_tiles)
+      for (int i = 0; i < kv; ++i) lw += ((long long)qkpos[i + 1] <= tile * 128) ? 1 : 0;
+  }
+  __device__ __forceinline__ WgradTile next() {
+    WgradTile d = {-1, 0, 0, 1};
+    const long long at = tile++;
+    if (at >= end) return d;
+    if (at < pair_tiles) {
+      while (lw < kv && (long long)qkpos[lw + 1] <= at * 128) ++lw;
+      if (lw >= kv) return d;
+      d.w = lw;
+      d.first = (int)(at * 128 - qkpos[lw]) + kpos[lw];
+      d.count = kpos[lw + 1] - d.first;
+      d.same = 0;
+    } else {
+      d.w = mid;
+      d.first = (int)((at - pair_tiles) * 128);
+      d.count = (int)(n_rows - d.first);
+    }
+    d.count = d.count < 128 ? (d.count > 0 ? d.count : 0) : 128;
+    d.w = __builtin_amdgcn_readfirstlane(d.w);
+    d.first = __builtin_amdgcn_readfirstlane(d.first);
+    d.count = __builtin_amdgcn_readfirstlane(d.count);
+    d.same = __builtin_amdgcn_readfirstlane(d.same);
+    lw = __builtin_amdgcn_readfirstlane(lw);
+    return d;
+  }
+};
+
 __global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__restrict__ in, const half_t *__restrict__ gout, long long n_rows,
                                                             unsigned in_bytes, unsigned out_bytes, int c_in, int c_out, int kv, int mid,
                                                             const int *__restrict__ imap, const int *__restrict__ omap,
@@ -3770,42 +3810,11 @@ __global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__rest
         for (int e = 0; e < 16; ++e) sum[i][j][e] = 0.f;
   };
 
-  // a tile: its offset (-1: none), its first pair or row, how many, and whether rows pair with themselves
-  struct Tile {
-    int w, first, count, same;
-  };
-  int lw = 0;
-  if (t_begin < pair_tiles)
-    for (int i = 0; i < kv; ++i) lw += ((long long)qkpos[i + 1] <= t_begin * 128) ? 1 : 0;
-  auto describe = [&](int t) {   // called for consecutive tiles
-    Tile d = {-1, 0, 0, 1};
-    const long long tile = t_begin + t;
-    if (t >= n_tiles) return d;
-    if (tile < pair_tiles) {
-      while (lw < kv && (long long)qkpos[lw + 1] <= tile * 128) ++lw;
-      if (lw >= kv) return d;
-      d.w = lw;
-      d.first = (int)(tile * 128 - qkpos[lw]) + kpos[lw];
-      d.count = kpos[lw + 1] - d.first;
-      d.same = 0;
-    } else {
-      d.w = mid;
-      d.first = (int)((tile - pair_tiles) * 128);
-      d.count = (int)(n_rows - d.first);
-    }
-    d.count = d.count < 128 ? (d.count > 0 ? d.count : 0) : 128;
-    // (uniform: in scalar registers from here on)
-    d.w = __builtin_amdgcn_readfirstlane(d.w);
-    d.first = __builtin_amdgcn_readfirstlane(d.first);
-    d.count = __builtin_amdgcn_readfirstlane(d.count);
-    d.same = __builtin_amdgcn_readfirstlane(d.same);
-    lw = __builtin_amdgcn_readfirstlane(lw);
-    return d;
-  };
+  WgradWalk walk(t_begin, n_tiles, pair_tiles, n_rows, kv, mid, kpos, qkpos);
   const u32x4 in_rows = byte_range(in, in_bytes), out_rows = byte_range(gout, out_bytes);
   const unsigned lds0 = (unsigned)(uintptr_t)(lds_char *)lds, rows0 = (unsigned)(uintptr_t)(lds_char *)(char *)rows;
   // the row indices of a tile of pairs: wavefronts 0 and 1 the input rows, 2 and 3 the output rows, 64 each
-  auto fetch_rows = [&](const Tile &d, int slot_) {
+  auto fetch_rows = [&](const WgradTile &d, int slot_) {
     const int *list = (wave < 2 ? imap : omap) + d.first;
     const int part = (wave & 1) * 64;
     copy_to_lds<4>(byte_range(list, d.same ? 0u : (unsigned)d.count * 4u), (part + lane) * 4,
@@ -3815,7 +3824,7 @@ __global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__rest
   const int piece = (lane & 15) ^ ((lane >> 4) << 2);
   const unsigned in_at = (unsigned)(ci0 + piece * 8) * 2u, in_gone = ci0 + piece * 8 < c_in ? 0u : ~0u;
   const unsigned out_at = (unsigned)(co0 + piece * 8) * 2u, out_gone = co0 + piece * 8 < c_out ? 0u : ~0u;
-  auto issue = [&](const Tile &d, int slot_, int stage, int buf) {
+  auto issue = [&](const WgradTile &d, int slot_, int stage, int buf) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int r = wave * 8 + t * 4 + (lane >> 4), pos = stage * WP_PAIRS + r;
@@ -3861,7 +3870,7 @@ __global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__rest
     }
   };
 #define WP_LANDED() asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory")
-  Tile d = describe(0), next = describe(1);
+  WgradTile d = walk.next(), next = walk.next();
   fetch_rows(d, 0);
   fetch_rows(next, 1);
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
@@ -3886,18 +3895,156 @@ __global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__rest
     multiply(1);
     WP_LANDED();
     issue(d, (t + 1) & 1, 1, 1);
-    next = describe(t + 2);
+    next = walk.next();
     fetch_rows(next, t & 1);
     multiply(2);
     WP_LANDED();
     issue(d, (t + 1) & 1, 2, 2);
     multiply(3);
   }
-#undef WP_LANDED
   end_chain();
   if (cur >= 0) flush(cur);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the copies behind the last stage end before the LDS is given back
 }
+
+// The same ring for fp32 rows of a multiple of four channels: stages of 16 pairs, copied three ahead, 512 bytes a pair and operand
+// whatever the block's width.  A wavefront holds TI x TO tiles of v_mfma_f32_16x16x4_f32, so that a block is 64, 96 or 128 channels
+// wide (32 TI, 32 TO).  A fragment is sixteen channels of four pairs; the 16-byte pieces of a row are exchanged by its pair index
+// (piece ^ (pair & 3) * 4), which puts the four into different banks.  Every tile is a chain of sums of its own (128 -> 128 on 19 k rows
+// of 14 pairs: relative error 2.2e-7, 6.0e-7 as one chain over a run).
+// Bound by the matrix cores where the tiles are many (a stage is 2048 of their clocks for 128 x 128 and 32 LDS reads), by the
+// sums' atomics and the first gathers where they are few.  wgrad_kernel, whose stages' gathers nothing hid -> this one: 96 -> 96 on
+// 21 k rows of 5 pairs 79 us -> 35, 128 -> 128 85 -> 55, 256 -> 256 207 -> 145, on 35 k of 5 415 -> 253 (90 TFLOP/s), 96 -> 96 on 19 k
+// of 14 197 -> 63; 64 -> 64 on 21 k 33 -> 24; 128 -> 128 on 800 rows 24 -> 16.
+template <int TI, int TO>
+__global__ void __launch_bounds__(256, 2) wgrad_f32_ring_kernel(const float *__restrict__ in, const float *__restrict__ gout, long long n_rows,
+                                                                unsigned in_bytes, unsigned out_bytes, int c_in, int c_out, int kv, int mid,
+                                                                const int *__restrict__ imap, const int *__restrict__ omap,
+                                                                const int *__restrict__ kpos, const int *__restrict__ qkpos,
+                                                                long long pair_tiles, long long tiles, int run, int ci_blocks,
+                                                                int co_blocks, float *__restrict__ gw) {
+  constexpr int PAIRS = 16, ROW = 512, OP = PAIRS * ROW, STAGE = 2 * OP, ST = 4;   // (bytes)
+  __shared__ __attribute__((aligned(1024))) char lds[ST * STAGE];
+  __shared__ __attribute__((aligned(16))) int rows[2][2][128];   // input and output rows of a tile, for two tiles
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, q = lane >> 4, wr = wave >> 1, wc = wave & 1;
+  // (the blocks of one run of tiles go to one XCD, as in wgrad_f16_kernel)
+  const long long slot = blockIdx.x >> 3;
+  const int rest = (int)(slot % (ci_blocks * co_blocks));
+  const long long grp = (slot / (ci_blocks * co_blocks)) * 8 + (blockIdx.x & 7);
+  const int ci0 = (rest / co_blocks) * (32 * TI), co0 = (rest % co_blocks) * (32 * TO);
+  const long long t_begin = grp * run, t_end = (grp + 1) * run < tiles ? (grp + 1) * run : tiles;
+  if (t_begin >= t_end) return;
+  const int n_tiles = (int)(t_end - t_begin);
+
+  f32x4 acc[TI][TO], sum[TI][TO];   // of the tile, and of the tiles of this offset before it
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TO; ++j) acc[i][j] = sum[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  auto end_tile = [&] {
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TO; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          sum[i][j][e] += acc[i][j][e];
+          acc[i][j][e] = 0.f;
+        }
+  };
+  auto flush = [&](int widx) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+      const int ci = ci0 + (wr * TI + i) * 16 + q * 4;   // four input channels at a time are there or not
+      float *dst = gw + ((long long)widx * c_in + ci) * c_out;
+#pragma unroll
+      for (int j = 0; j < TO; ++j) {
+        const int co = co0 + (wc * TO + j) * 16 + l16;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (ci < c_in && co < c_out) unsafeAtomicAdd(dst + (long long)e * c_out + co, sum[i][j][e]);
+        sum[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  };
+
+  WgradWalk walk(t_begin, n_tiles, pair_tiles, n_rows, kv, mid, kpos, qkpos);
+  const u32x4 in_rows = byte_range(in, in_bytes), out_rows = byte_range(gout, out_bytes);
+  const unsigned lds0 = (unsigned)(uintptr_t)(lds_char *)lds, rows0 = (unsigned)(uintptr_t)(lds_char *)(char *)rows;
+  // the row indices of a tile of pairs: wavefronts 0 and 1 the input rows, 2 and 3 the output rows, 64 each
+  auto fetch_rows = [&](const WgradTile &d, int slot_) {
+    const int *list = (wave < 2 ? imap : omap) + d.first;
+    const int part = (wave & 1) * 64;
+    copy_to_lds<4>(byte_range(list, d.same ? 0u : (unsigned)d.count * 4u), (part + lane) * 4,
+                   rows0 + ((slot_ * 2 + (wave >> 1)) * 128 + part) * 4);
+  };
+  // pairs 4 wave .. + 3 of a stage of both operands, two an instruction: this lane's row and its piece of it
+  auto issue = [&](const WgradTile &d, int slot_, int stage) {
+    const int buf = stage & (ST - 1);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int r = t * 2 + (lane >> 5), pos = stage * PAIRS + wave * 4 + r, ch = ((lane & 31) ^ (r << 2)) * 4;
+      const int li = rows[slot_][0][pos], lo = rows[slot_][1][pos], own = d.first + pos;
+      const unsigned x = (unsigned)(d.same ? own : li) * (unsigned)(c_in * 4) + (unsigned)(ci0 + ch) * 4u;
+      const unsigned y = (unsigned)(d.same ? own : lo) * (unsigned)(c_out * 4) + (unsigned)(co0 + ch) * 4u;
+      const unsigned gone = pos < d.count ? 0u : ~0u;
+      const unsigned in_gone = ch < 32 * TI && ci0 + ch < c_in ? gone : ~0u, out_gone = ch < 32 * TO && co0 + ch < c_out ? gone : ~0u;
+      copy_to_lds<16>(in_rows, x | in_gone, lds0 + buf * STAGE + (wave * 4 + t * 2) * ROW);
+      copy_to_lds<16>(out_rows, y | out_gone, lds0 + buf * STAGE + OP + (wave * 4 + t * 2) * ROW);
+    }
+  };
+  // where a lane's channel of the sixteen from c on lies, for pair q of four
+  auto frag_at = [&](int c) { return q * ROW + ((c / 4) ^ (q << 2)) * 16 + l16 * 4; };
+  int a_at[TI], b_at[TO];
+#pragma unroll
+  for (int i = 0; i < TI; ++i) a_at[i] = frag_at((wr * TI + i) * 16);
+#pragma unroll
+  for (int j = 0; j < TO; ++j) b_at[j] = OP + frag_at((wc * TO + j) * 16);
+  auto multiply = [&](int buf) {
+#pragma unroll
+    for (int k = 0; k < PAIRS; k += 4) {
+      float av[TI], bv[TO];
+#pragma unroll
+      for (int i = 0; i < TI; ++i) av[i] = *reinterpret_cast<const float *>(lds + buf * STAGE + k * ROW + a_at[i]);
+#pragma unroll
+      for (int j = 0; j < TO; ++j) bv[j] = *reinterpret_cast<const float *>(lds + buf * STAGE + k * ROW + b_at[j]);
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TO; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+    }
+  };
+  WgradTile d = walk.next(), next = walk.next();
+  fetch_rows(d, 0);
+  fetch_rows(next, 1);
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  for (int st = 0; st < 3; ++st) issue(d, 0, st);
+  int cur = -1;
+  for (int t = 0; t < n_tiles; ++t) {
+    end_tile();
+    if (d.w != cur) {
+      if (cur >= 0) flush(cur);
+      cur = d.w;
+    }
+    // stages 3 .. 7 of this tile, then the first three of the next one
+#pragma unroll
+    for (int st = 0; st < 8; ++st) {
+      WP_LANDED();   // (from st = 5 on every wavefront has issued this tile's last copies: its row indices are not read any more)
+      if (st == 5) d = next;
+      issue(d, st < 5 ? t & 1 : (t + 1) & 1, (st + 3) & 7);
+      if (st == 6) {
+        next = walk.next();
+        fetch_rows(next, t & 1);
+      }
+      multiply(st & (ST - 1));
+    }
+  }
+  end_tile();
+  if (cur >= 0) flush(cur);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the copies behind the last stage end before the LDS is given back
+}
+#undef WP_LANDED
 
 template <typename T, int BLK>
 __global__ void __launch_bounds__(256) wgrad_kernel(const T *__restrict__ in, const T *__restrict__ gout, long long n_rows,
@@ -4011,6 +4158,15 @@ __global__ void __launch_bounds__(256) wgrad_kernel(const T *__restrict__ in, co
   if (cur >= 0) flush(cur);
 }
 
+// width of a wgrad_f32_ring_kernel block for c channels, in 32 of them: the least padding, then the fewest gathers (192 -> 96 on 21 k
+// rows of 5 pairs: 56 us with blocks of 96, 154 with the 128 of wgrad_kernel)
+static int ring_tiles(int c) {
+  int best = 2;
+  for (int t = 3; t <= 4; ++t)
+    if (pce_div_up(c, 32 * t) * (32 * t + 16) < pce_div_up(c, 32 * best) * (32 * best + 16)) best = t;
+  return best;
+}
+
 static int wgrad_impl(bool clear, const void *in, const void *gout, int32_t dtype, int64_t n_in, int64_t n_out, int32_t c_in,
                       int32_t c_out, int32_t kv, int32_t mid, const int32_t *imap, const int32_t *omap,
                       const int32_t *kpos, const int32_t *qkpos, int64_t qsum, float *gw, pce_stream_t stream) {
@@ -4041,6 +4197,9 @@ static int wgrad_impl(bool clear, const void *in, const void *gout, int32_t dtyp
   const int64_t in_bytes = n_in * c_in * 2, out_bytes = n_out * c_out * 2;
   const bool pipe = dtype == PCE_F16 && blk == 128 && c_in % 8 == 0 && c_out % 8 == 0 && aligned16(in) && aligned16(gout) &&
                     in_bytes < WP_MAX_BYTES && out_bytes < WP_MAX_BYTES;
+  const int64_t ring_in_bytes = n_in * c_in * 4, ring_out_bytes = n_out * c_out * 4;
+  const bool ring = dtype == PCE_F32 && c_in % 4 == 0 && c_out % 4 == 0 && aligned16(in) && aligned16(gout) &&
+                    ring_in_bytes < WP_MAX_BYTES && ring_out_bytes < WP_MAX_BYTES;
   const int fold = (int)(run < 1 ? 1 : (run > 8 ? 8 : run));   // wgrad_pipe_kernel: chains no longer than that run, nor than eight tiles
   if (pipe) {
     // one workgroup per compute unit, as many runs on every XCD (256 -> 256 on 27 k rows of 19 pairs 117 us with 256 workgroups,
@@ -4055,11 +4214,45 @@ static int wgrad_impl(bool clear, const void *in, const void *gout, int32_t dtyp
   hipLaunchKernelGGL((wgrad_kernel<T_, BLK_>), dim3((unsigned)blocks), dim3(256), 0, s, (const T_ *)in, (const T_ *)gout, \
                      (long long)n_out, c_in, c_out, kv, mid, imap, omap, kpos, qkpos, pair_tiles, tiles, (int)run,       \
                      ci_blocks, co_blocks, gw)
+#define PCE_WGRAD_RING(TI_, TO_)                                                                                                  \
+  hipLaunchKernelGGL((wgrad_f32_ring_kernel<TI_, TO_>), dim3((unsigned)ring_wgs), dim3(256), 0, s, (const float *)in,               \
+                     (const float *)gout, (long long)n_out, (unsigned)ring_in_bytes, (unsigned)ring_out_bytes, c_in, c_out, kv, mid, \
+                     imap, omap, kpos, qkpos, pair_tiles, tiles, (int)ring_run, ring_ci, ring_co, gw)
 #define PCE_WGRAD16(BLK_)                                                                                            \
   hipLaunchKernelGGL((wgrad_f16_kernel<BLK_>), dim3((unsigned)blocks), dim3(256), 0, s, (const half_t *)in,            \
                      (const half_t *)gout, (long long)n_out, c_in, c_out, kv, mid, imap, omap, kpos, qkpos, pair_tiles, \
                      tiles, (int)run, ci_blocks, co_blocks, gw)
-  if (pipe)
+  if (ring) {
+    // Where a run is one or two tiles, a block's products and its atomics are a chain that nothing runs beside: blocks of 64 channels
+    // there, four times as many (128 -> 128 on 246 tiles 24.3 -> 18.6 us, on 373 39 -> 25, on 8 15.6 -> 9.7; 96 -> 96 on 36 11.6 -> 9.6,
+    // but on 246 15.2 -> 17.5)
+    int ti = ring_tiles(c_in), to = ring_tiles(c_out);
+    const long long wide = tiles * pce_div_up(c_in, 32 * ti) * pce_div_up(c_out, 32 * to);
+    if (wide < 64 || (wide < 512 && ti == 4)) ti = 2;
+    if (wide < 64 || (wide < 512 && to == 4)) to = 2;
+    const int ring_ci = (int)pce_div_up(c_in, 32 * ti), ring_co = (int)pce_div_up(c_out, 32 * to);
+    // one workgroup per compute unit, two where the tiles are many: their waits overlap, their atomics are twice as many (256 and 512:
+    // 128 -> 128 on 931 tiles 55 and 63 us, on 1854 88 and 83; 384 -> 256 on 860 206 and 192)
+    const bool two = tiles * ring_ci * ring_co >= (ti == 2 && to == 2 && ring_ci * ring_co > 1 ? 1024 : 1536);
+    const long long runs = (two ? 512 : 256) / (ring_ci * ring_co) / 8 * 8, ring_run = pce_div_up(tiles, runs < 8 ? 8 : runs);
+    const long long ring_wgs = pce_div_up(pce_div_up(tiles, ring_run), 8) * 8 * ring_ci * ring_co;
+    if (ring_wgs >= (1ll << 31)) PCE_FAIL(PCE_ECAPACITY, "pce_conv_wgrad: %lld workgroups exceed the grid limit", ring_wgs);
+#define PCE_WGRAD_RING_(TI_) \
+    if (to == 2)             \
+      PCE_WGRAD_RING(TI_, 2); \
+    else if (to == 3)        \
+      PCE_WGRAD_RING(TI_, 3); \
+    else                     \
+      PCE_WGRAD_RING(TI_, 4)
+    if (ti == 2) {
+      PCE_WGRAD_RING_(2);
+    } else if (ti == 3) {
+      PCE_WGRAD_RING_(3);
+    } else {
+      PCE_WGRAD_RING_(4);
+    }
+#undef PCE_WGRAD_RING_
+  } else if (pipe)
     hipLaunchKernelGGL(wgrad_pipe_kernel, dim3((unsigned)blocks), dim3(256), 0, s, (const half_t *)in, (const half_t *)gout, (long long)n_out,
                        (unsigned)in_bytes, (unsigned)out_bytes, c_in, c_out, kv, mid, imap, omap, kpos, qkpos, pair_tiles, tiles, (int)run,
                        fold, ci_blocks, co_blocks, gw);
@@ -4073,6 +4266,7 @@ static int wgrad_impl(bool clear, const void *in, const void *gout, int32_t dtyp
     PCE_WGRAD(float, 64);
 #undef PCE_WGRAD
 #undef PCE_WGRAD16
+#undef PCE_WGRAD_RING
   PCE_LAUNCH_CHECK("wgrad");
   return PCE_OK;
 }
