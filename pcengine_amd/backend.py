@@ -768,6 +768,7 @@ def build_pyramid(in_coords: torch.Tensor, strided: Sequence[Geom], requests: Se
         raise PlanNotApplicable()
     if in_coords.shape[0] == 0 or in_coords.dtype != torch.int32 or in_coords.dim() != 2 or in_coords.shape[1] != 4 or not in_coords.is_contiguous():
         raise PlanNotApplicable()
+    reqs, args = _pyramid_requests(requests)      # (in front of the chain: a kernel too large for a plan costs no launch)
     coords = [in_coords]
     if levels:
         try:
@@ -777,7 +778,6 @@ def build_pyramid(in_coords: torch.Tensor, strided: Sequence[Geom], requests: Se
         if outs is None or any(c.shape[0] == 0 for c in outs):
             raise PlanNotApplicable()
         coords += outs
-    reqs, args = _pyramid_requests(requests)
     plan = _lib.PyrPlan()
     if lib.pce_pyramid_plan_levels((_lib.c_int64 * (levels + 1))(*[c.shape[0] for c in coords]), levels, int(n_batch), reqs, len(requests),
                                    plan) != _lib.PCE_OK:

@@ -89,6 +89,22 @@ def test_what_it_does_not_take(kind, monkeypatch):
             assert k == k2 and m == m2 and torch.equal(i, i2) and torch.equal(o, o2)
 
 
+def counted(monkeypatch):
+    """Calls of the chained output coordinates and the maps that were built one by one, from here on."""
+    chains, singles = [], []
+    chain, build = backend.build_out_coords_chain, backend.build_kernel_maps
+    monkeypatch.setattr(backend, "build_out_coords_chain", lambda *a: (chains.append(1), chain(*a))[1])
+    monkeypatch.setattr(backend, "build_kernel_maps", lambda jobs, *a, **k: (singles.extend(jobs), build(jobs, *a, **k))[1])
+    return chains, singles
+
+
+def test_a_kernel_too_large_for_a_plan_costs_no_second_chain(monkeypatch):
+    x = tensor(CLOUDS["lidar"]())
+    chains, singles = counted(monkeypatch)
+    spconv.prebuild_maps(x, [(5, 1, 0), (2, 2, 0), (3, 1, 0), (2, 2, 0), (3, 1, 0)])
+    assert len(chains) == 1 and len(singles) == 5 == len(x.kmaps)
+
+
 def test_memory_of_maps_built_on_another_stream_is_told():
     x = tensor(CLOUDS["lidar"]())
     spconv.prebuild_maps(x, UNET)
