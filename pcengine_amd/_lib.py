@@ -315,4 +315,6 @@ def check(rc: int) -> None:
         raise ValueError(msg)
     if rc == PCE_ECAPACITY:
         raise OverflowError(msg)
-    raise PCEError(f"[pce status {rc}] {msg}")
+    error = PCEError(f"[pce status {rc}] {msg}")
+    error.status = rc
+    raise error

@@ -754,11 +754,19 @@ def _pyramid_maps(plan, args, arena: torch.Tensor, a32: torch.Tensor, coords: Se
     return maps
 
 
+def _check_or_decline(rc: int) -> None:
+    """``PlanNotApplicable`` for a cloud that the general path takes or refuses in its own words, the error for everything else."""
+    if rc in (_lib.PYR_UNSORTED, _lib.PCE_ECOORD, _lib.PCE_ECAPACITY):
+        raise PlanNotApplicable()
+    _lib.check(rc)
+
+
 def build_pyramid(in_coords: torch.Tensor, strided: Sequence[Geom], requests: Sequence[tuple], n_batch: int):
     """(coordinates of every level, the maps in request order) of one cloud, laid out for exactly its rows and kept by nobody else:
     the output coordinates of the strided levels (``build_out_coords_chain``, one wait), then every map in one library call
     (one wait).  Arguments as ``PyramidPlan``'s.  The general path of a map at a time takes the host 0.3 ms more for nine maps.
-    Raises ``PlanNotApplicable`` where the library does not take the cloud, or refuses it: the general path words the error."""
+    Raises ``PlanNotApplicable`` where the library does not take the cloud, or refuses its coordinates or its size: the general
+    path words the error."""
     lib = _lib.load()
     _require_cuda(in_coords, "coords")
     if lib.pce_pyramid_plan_sizeof() != _lib.ctypes.sizeof(_lib.PyrPlan):
@@ -773,19 +781,21 @@ def build_pyramid(in_coords: torch.Tensor, strided: Sequence[Geom], requests: Se
     if levels:
         try:
             outs = build_out_coords_chain(in_coords, strided, n_batch)
-        except (_lib.PCEError, ValueError, OverflowError):
-            outs = None
+        except OverflowError:
+            raise PlanNotApplicable()
+        except _lib.PCEError as error:
+            if getattr(error, "status", None) != _lib.PCE_ECOORD:
+                raise
+            raise PlanNotApplicable()
         if outs is None or any(c.shape[0] == 0 for c in outs):
             raise PlanNotApplicable()
         coords += outs
     plan = _lib.PyrPlan()
-    if lib.pce_pyramid_plan_levels((_lib.c_int64 * (levels + 1))(*[c.shape[0] for c in coords]), levels, int(n_batch), reqs, len(requests),
-                                   plan) != _lib.PCE_OK:
-        raise PlanNotApplicable()
+    _check_or_decline(lib.pce_pyramid_plan_levels((_lib.c_int64 * (levels + 1))(*[c.shape[0] for c in coords]), levels, int(n_batch), reqs,
+                                                  len(requests), plan))
     arena = torch.empty(plan.arena_bytes, dtype=torch.uint8, device=in_coords.device)
-    if lib.pce_pyramid_maps(plan, (_lib.ctypes.c_void_p * (levels + 1))(*[c.data_ptr() for c in coords]), arena.data_ptr(), arena.numel(),
-                            _stream(in_coords.device)) != _lib.PCE_OK:
-        raise PlanNotApplicable()
+    _check_or_decline(lib.pce_pyramid_maps(plan, (_lib.ctypes.c_void_p * (levels + 1))(*[c.data_ptr() for c in coords]), arena.data_ptr(),
+                                           arena.numel(), _stream(in_coords.device)))
     return coords, _pyramid_maps(plan, args, arena, arena.view(torch.int32), coords, int(n_batch), None)
 
 

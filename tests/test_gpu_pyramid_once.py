@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import pcengine_amd as pe
-from pcengine_amd import backend, spconv, synth
+from pcengine_amd import _lib, backend, spconv, synth
 from tests.util import DEV, dev_coords
 
 pytestmark = pytest.mark.gpu
@@ -103,6 +103,28 @@ def test_a_kernel_too_large_for_a_plan_costs_no_second_chain(monkeypatch):
     chains, singles = counted(monkeypatch)
     spconv.prebuild_maps(x, [(5, 1, 0), (2, 2, 0), (3, 1, 0), (2, 2, 0), (3, 1, 0)])
     assert len(chains) == 1 and len(singles) == 5 == len(x.kmaps)
+
+
+@pytest.mark.parametrize("call", ["pce_outcoords_chain", "pce_pyramid_plan_levels", "pce_pyramid_maps"])
+@pytest.mark.parametrize("status", [_lib.PCE_EHIP, _lib.PCE_EWORKSPACE])
+def test_a_failed_launch_is_an_error(call, status, monkeypatch):
+    """What is not the cloud's fault is raised and nothing is built again (the status is made up on the host, no launch fails)."""
+    x = tensor(CLOUDS["lidar"]())
+    chains, singles = counted(monkeypatch)
+    monkeypatch.setattr(_lib.load(), call, lambda *a: status)
+    with pytest.raises(_lib.PCEError, match=f"pce status {status}"):
+        spconv.prebuild_maps(x, UNET)
+    assert len(chains) == 1 and not singles and not x.kmaps
+
+
+@pytest.mark.parametrize("call", ["pce_outcoords_chain", "pce_pyramid_plan_levels", "pce_pyramid_maps"])
+@pytest.mark.parametrize("status", [_lib.PCE_ECOORD, _lib.PCE_ECAPACITY])
+def test_a_refused_cloud_is_built_map_by_map(call, status, monkeypatch):
+    x = tensor(CLOUDS["lidar"]())
+    real, done = getattr(_lib.load(), call), []
+    monkeypatch.setattr(_lib.load(), call, lambda *a: (done.append(1), status if len(done) == 1 else real(*a))[1])
+    spconv.prebuild_maps(x, UNET)
+    assert len(x.kmaps) == 9 and not any(km.__dict__.get("_arena") is not None for km in x.kmaps.values())
 
 
 def test_memory_of_maps_built_on_another_stream_is_told():
