@@ -323,7 +323,8 @@ int pce_pyramid_plan(int64_t n_cap, int32_t n_levels, const pce_geom_t *strided,
 int pce_pyramid_build(pce_pyr_plan_t *plan, const int32_t *in_coords_dev, int64_t n_in, void *arena_dev, int64_t arena_bytes,
                       pce_stream_t stream);
 /* The same for one cloud whose levels' coordinates are there already: pce_pyramid_plan_levels lays out the maps alone, for exactly
- * level_n[0 .. n_levels] rows, and pce_pyramid_maps builds them from level_coords_dev[0 .. n_levels] (one wait). */
+ * level_n[0 .. n_levels] rows, and pce_pyramid_maps builds them from level_coords_dev[0 .. n_levels] (one wait; a second one where
+ * rows are out of order or outside the stated box: the maps of those are built again, through the hash table). */
 int pce_pyramid_plan_levels(const int64_t *level_n, int32_t n_levels, int32_t n_batch, const pce_pyr_request_t *requests,
                             int32_t n_requests, pce_pyr_plan_t *plan_out);
 int pce_pyramid_maps(pce_pyr_plan_t *plan, const int32_t *const *level_coords_dev, void *arena_dev, int64_t arena_bytes,

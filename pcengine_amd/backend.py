@@ -756,7 +756,7 @@ def _pyramid_maps(plan, args, arena: torch.Tensor, a32: torch.Tensor, coords: Se
 
 def _check_or_decline(rc: int) -> None:
     """``PlanNotApplicable`` for a cloud that the general path takes or refuses in its own words, the error for everything else."""
-    if rc in (_lib.PYR_UNSORTED, _lib.PCE_ECOORD, _lib.PCE_ECAPACITY):
+    if rc in (_lib.PCE_ECOORD, _lib.PCE_ECAPACITY):
         raise PlanNotApplicable()
     _lib.check(rc)
 
@@ -764,7 +764,8 @@ def _check_or_decline(rc: int) -> None:
 def build_pyramid(in_coords: torch.Tensor, strided: Sequence[Geom], requests: Sequence[tuple], n_batch: int):
     """(coordinates of every level, the maps in request order) of one cloud, laid out for exactly its rows and kept by nobody else:
     the output coordinates of the strided levels (``build_out_coords_chain``, one wait), then every map in one library call
-    (one wait).  Arguments as ``PyramidPlan``'s.  The general path of a map at a time takes the host 0.3 ms more for nine maps.
+    (one wait, two where rows are not sorted or not inside the stated box: their maps go through the hash table).
+    Arguments as ``PyramidPlan``'s.  The general path of a map at a time takes the host 0.3 ms more for nine maps.
     Raises ``PlanNotApplicable`` where the library does not take the cloud, or refuses its coordinates or its size: the general
     path words the error."""
     lib = _lib.load()

@@ -121,8 +121,10 @@ extern "C" int pce_pyramid_plan_levels(const int64_t *level_n, int32_t n_levels,
   return lay_out_maps(plan, requests, 0);
 }
 
-// every map of the plan, from the coordinates of its levels; one wait, for the counts
-static int build_maps(pce_pyr_plan_t *plan, const int32_t *const *coords, char *base, hipStream_t s) {
+// Every map of the plan, from the coordinates of its levels; one wait, for the counts.  Maps whose rows the column grid refused (out
+// of order, or outside the stated box) are built again through the hash table, together and with a second wait (rehash), or the
+// answer is PCE_PYR_UNSORTED.
+static int build_maps(pce_pyr_plan_t *plan, const int32_t *const *coords, char *base, bool rehash, hipStream_t s) {
   PCE_HIP(hipMemsetAsync(base + plan->off_meta, 0, (size_t)plan->meta_bytes, s));
   pce_kmap_problem_t probs[PCE_PYR_MAX_MAPS];
   memset(probs, 0, sizeof(probs));
@@ -160,25 +162,34 @@ static int build_maps(pce_pyr_plan_t *plan, const int32_t *const *coords, char *
     u.n_batch = plan->n_batch;
     u.flags = r.table_only ? PCE_KMAP_TABLE_ONLY : 0;
   }
-  const int rc = pce_kmap_build_batch(probs, plan->n_maps, (pce_stream_t)s);
+  int rc = pce_kmap_build_batch(probs, plan->n_maps, (pce_stream_t)s);
   if (rc) return rc;
   int32_t host[PCE_PYR_MAX_MAPS * (3 * 31 + 2 + META_STATUS)];
-  PCE_HIP(hipMemcpyAsync(host, base + plan->off_meta, (size_t)plan->meta_bytes, hipMemcpyDeviceToHost, s));
-  PCE_HIP(hipStreamSynchronize(s));
-  int fallback = 0;
-  for (int i = 0; i < plan->n_maps; ++i) {
-    pce_pyr_map_t &m = plan->map[i];
-    const int32_t *h = host + (m.off[PCE_PYR_META] - plan->off_meta) / 4;
-    memcpy(m.meta, h, (size_t)meta_ints(m.kv) * 4);
-    const int32_t *st = h + 3 * m.kv + 2;
-    if (st[0]) PCE_FAIL(PCE_ECOORD, "pce_pyramid_build: a coordinate of map %d is outside the supported range", i);
-    if (st[1]) PCE_FAIL(PCE_ECAPACITY, "pce_pyramid_build: hash table of map %d exhausted", i);
-    if (st[2]) PCE_FAIL(PCE_ECAPACITY, "pce_pyramid_build: an offset of map %d holds too many pairs for the CSR code", i);
-    if (st[3]) fallback = 1;   // unsorted rows or rows outside the stated box: the caller builds this cloud map by map
-    m.n_pairs = h[2 * m.kv];
-    m.qsum = h[3 * m.kv + 1];
-  }
-  return fallback ? PCE_PYR_UNSORTED : PCE_OK;
+  int refused = 0;   // their problems are the first of probs
+  do {
+    PCE_HIP(hipMemcpyAsync(host, base + plan->off_meta, (size_t)plan->meta_bytes, hipMemcpyDeviceToHost, s));
+    PCE_HIP(hipStreamSynchronize(s));
+    const bool again = refused != 0;
+    refused = 0;
+    for (int i = 0; i < plan->n_maps; ++i) {
+      pce_pyr_map_t &m = plan->map[i];
+      const int32_t *h = host + (m.off[PCE_PYR_META] - plan->off_meta) / 4;
+      memcpy(m.meta, h, (size_t)meta_ints(m.kv) * 4);
+      const int32_t *st = h + 3 * m.kv + 2;
+      if (st[0]) PCE_FAIL(PCE_ECOORD, "pce_pyramid_build: a coordinate of map %d is outside the supported range", i);
+      if (st[1]) PCE_FAIL(PCE_ECAPACITY, "pce_pyramid_build: hash table of map %d exhausted", i);
+      if (st[2]) PCE_FAIL(PCE_ECAPACITY, "pce_pyramid_build: an offset of map %d holds too many pairs for the CSR code", i);
+      m.n_pairs = h[2 * m.kv];
+      m.qsum = h[3 * m.kv + 1];
+      if (!st[3] || again) continue;
+      probs[refused] = probs[i];   // (at or in front of i)
+      probs[refused++].flags |= PCE_KMAP_NO_GRID;
+      if (rehash) PCE_HIP(hipMemsetAsync(base + m.off[PCE_PYR_META], 0, (size_t)meta_ints(m.kv) * 4, s));
+    }
+    if (refused && !rehash) return PCE_PYR_UNSORTED;   // the caller builds this cloud map by map
+    if (refused && (rc = pce_kmap_build_batch(probs, refused, (pce_stream_t)s))) return rc;
+  } while (refused);
+  return PCE_OK;
 }
 
 extern "C" int pce_pyramid_build(pce_pyr_plan_t *plan, const int32_t *in_coords, int64_t n_in, void *arena, int64_t arena_bytes,
@@ -213,7 +224,7 @@ extern "C" int pce_pyramid_build(pce_pyr_plan_t *plan, const int32_t *in_coords,
       plan->level_n[l + 1] = n_out[l];
     }
   }
-  return build_maps(plan, coords, base, s);
+  return build_maps(plan, coords, base, false, s);
 }
 
 extern "C" int pce_pyramid_maps(pce_pyr_plan_t *plan, const int32_t *const *level_coords, void *arena, int64_t arena_bytes, pce_stream_t stream) {
@@ -223,5 +234,5 @@ extern "C" int pce_pyramid_maps(pce_pyr_plan_t *plan, const int32_t *const *leve
   if (arena_bytes < plan->arena_bytes || ((uintptr_t)arena & 255))
     PCE_FAIL(PCE_EWORKSPACE, "pce_pyramid_maps: the arena holds %lld bytes, the plan needs %lld (256-byte aligned)", (long long)arena_bytes,
              (long long)plan->arena_bytes);
-  return build_maps(plan, level_coords, (char *)arena, (hipStream_t)stream);
+  return build_maps(plan, level_coords, (char *)arena, true, (hipStream_t)stream);
 }

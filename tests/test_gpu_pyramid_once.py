@@ -127,6 +127,48 @@ def test_a_refused_cloud_is_built_map_by_map(call, status, monkeypatch):
     assert len(x.kmaps) == 9 and not any(km.__dict__.get("_arena") is not None for km in x.kmaps.values())
 
 
+@pytest.mark.parametrize("kind", ["unsorted", "outside the box"])
+@pytest.mark.parametrize("layers", ["unet", "lean", "one", "down", "threes"])
+def test_rows_that_the_column_grid_refuses(kind, layers, monkeypatch):
+    """They go through the hash table, and nothing that has been built is built again on the general path."""
+    c = CLOUDS["lidar"]()
+    cmax = c[:, 1:].max(0).tolist()
+    if kind == "unsorted":
+        c = c[np.random.default_rng(0).permutation(len(c))]
+    else:
+        cmax[0] //= 2
+    make = lambda: pe.spTensor(torch.zeros((len(c), 1), device=DEV), dev_coords(c), None, [0, 0, 0], list(cmax), batchsize=1)
+    a, b = make(), make()
+    with monkeypatch.context() as m:
+        chains, singles = counted(m)
+        spconv.prebuild_maps(a, LISTS[layers])
+        assert len(chains) <= 1 and not singles
+    general(monkeypatch)
+    spconv.prebuild_maps(b, LISTS[layers])
+    assert list(a.kmaps) == list(b.kmaps) and set(a.cbook) == set(b.cbook)
+    for s in a.cbook:
+        assert torch.equal(a.cbook[s], b.cbook[s])
+    for key in a.kmaps:
+        p, q = a.kmaps[key], b.kmaps[key]
+        for name in ("n_in", "n_out", "kv", "M", "qsum", "order_heavy", "order_nonzero", "order_single", "tag", "has_pairs", "batchsize", "_cmin", "_cmax"):
+            assert getattr(p, name) == getattr(q, name), name
+        assert list(p.kpos_host) == list(q.kpos_host) and list(p.qkpos_host) == list(q.qkpos_host)
+        for name in ("knnz", "kpos", "qkpos", "out_coords", "nbr_out", "nbr_in", "icsr", "ocsr", "icode", "ocode", "islot", "oslot"):
+            x, y = getattr(p, name), getattr(q, name)
+            assert (x is None) == (y is None), name
+            assert x is None or torch.equal(x.reshape(-1), y.reshape(-1)), name
+        if p.has_pairs:
+            assert torch.equal(p.imap, q.imap) and torch.equal(p.omap, q.omap)
+        if p.order is not None:
+            n = p.n_out
+            assert torch.equal(p.order[n:2 * n], q.order[n:2 * n])
+            assert torch.equal(p.order[:n].sort().values, q.order[:n].sort().values)
+        spans = [(t.untyped_storage().data_ptr(), t.untyped_storage().nbytes()) for t in p.device_tensors()]
+        for name in ("nbr_out", "out_coords", "kpos"):
+            at = getattr(p, name).data_ptr()
+            assert any(lo <= at < lo + size for lo, size in spans), name
+
+
 def test_memory_of_maps_built_on_another_stream_is_told():
     x = tensor(CLOUDS["lidar"]())
     spconv.prebuild_maps(x, UNET)
