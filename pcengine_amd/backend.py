@@ -637,7 +637,13 @@ def _scratch(buffer: Optional[torch.Tensor], need: int, device) -> Optional[torc
 
 class PlanNotApplicable(Exception):
     """The native planner does not take this pyramid (a level that is not a bitmap chain, an unsorted cloud): the
-    caller builds map by map."""
+    caller builds map by map.  ``chain``: what ``build_out_coords_chain`` gave for its strided levels, where that was asked already."""
+
+    def __init__(self, *chain):
+        self.chain = chain
+
+
+PYRAMID_MAX_KV = 31     # offsets of a map in a plan (pce_pyr_map_t)
 
 
 class PyramidPlan:
@@ -711,7 +717,7 @@ def _pyramid_requests(requests: Sequence[tuple]):
     reqs, args = (_lib.PyrRequest * len(requests))(), []
     for r, (lin, lout, ks, stride, pad, cmin, cmax_out, subm, want_csr, want_nbr_in, table_only) in zip(reqs, requests):
         kv = int(ks[0]) * int(ks[1]) * int(ks[2])
-        if kv > 31:
+        if kv > PYRAMID_MAX_KV:
             raise PlanNotApplicable()
         r.level_in, r.level_out = lin, lout
         r.geom = Geom.make(ks, stride, pad, cmin, cmax_out, subm)
@@ -754,16 +760,16 @@ def _pyramid_maps(plan, args, arena: torch.Tensor, a32: torch.Tensor, coords: Se
     return maps
 
 
-def _check_or_decline(rc: int) -> None:
+def _check_or_decline(rc: int, chain: tuple) -> None:
     """``PlanNotApplicable`` for a cloud that the general path takes or refuses in its own words, the error for everything else."""
     if rc in (_lib.PCE_ECOORD, _lib.PCE_ECAPACITY):
-        raise PlanNotApplicable()
+        raise PlanNotApplicable(*chain)
     _lib.check(rc)
 
 
 def build_pyramid(in_coords: torch.Tensor, strided: Sequence[Geom], requests: Sequence[tuple], n_batch: int):
     """(coordinates of every level, the maps in request order) of one cloud, laid out for exactly its rows and kept by nobody else:
-    the output coordinates of the strided levels (``build_out_coords_chain``, one wait), then every map in one library call
+    the output coordinates of the strided levels (``build_out_coords_chain``; one wait), then every map in one library call
     (one wait, two where rows are not sorted or not inside the stated box: their maps go through the hash table).
     Arguments as ``PyramidPlan``'s.  The general path of a map at a time takes the host 0.3 ms more for nine maps.
     Raises ``PlanNotApplicable`` where the library does not take the cloud, or refuses its coordinates or its size: the general
@@ -777,9 +783,12 @@ def build_pyramid(in_coords: torch.Tensor, strided: Sequence[Geom], requests: Se
         raise PlanNotApplicable()
     if in_coords.shape[0] == 0 or in_coords.dtype != torch.int32 or in_coords.dim() != 2 or in_coords.shape[1] != 4 or not in_coords.is_contiguous():
         raise PlanNotApplicable()
-    reqs, args = _pyramid_requests(requests)      # (in front of the chain: a kernel too large for a plan costs no launch)
-    coords = [in_coords]
-    if levels:
+    coords, chain = [in_coords], ()
+    if levels == 1:       # (with one wait either way, and behind it the rows are written while the host goes on)
+        coords.append(build_out_coords(in_coords, strided[0], n_batch))
+        if coords[1].shape[0] == 0:
+            raise PlanNotApplicable()
+    elif levels:
         try:
             outs = build_out_coords_chain(in_coords, strided, n_batch)
         except OverflowError:
@@ -788,15 +797,17 @@ def build_pyramid(in_coords: torch.Tensor, strided: Sequence[Geom], requests: Se
             if getattr(error, "status", None) != _lib.PCE_ECOORD:
                 raise
             raise PlanNotApplicable()
+        chain = (outs,)
         if outs is None or any(c.shape[0] == 0 for c in outs):
-            raise PlanNotApplicable()
+            raise PlanNotApplicable(*chain)
         coords += outs
+    reqs, args = _pyramid_requests(requests)
     plan = _lib.PyrPlan()
     _check_or_decline(lib.pce_pyramid_plan_levels((_lib.c_int64 * (levels + 1))(*[c.shape[0] for c in coords]), levels, int(n_batch), reqs,
-                                                  len(requests), plan))
+                                                  len(requests), plan), chain)
     arena = torch.empty(plan.arena_bytes, dtype=torch.uint8, device=in_coords.device)
     _check_or_decline(lib.pce_pyramid_maps(plan, (_lib.ctypes.c_void_p * (levels + 1))(*[c.data_ptr() for c in coords]), arena.data_ptr(),
-                                           arena.numel(), _stream(in_coords.device)))
+                                           arena.numel(), _stream(in_coords.device)), chain)
     return coords, _pyramid_maps(plan, args, arena, arena.view(torch.int32), coords, int(n_batch), None)
 
 

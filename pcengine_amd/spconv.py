@@ -21,6 +21,7 @@ from __future__ import annotations
 
 import math
 import os
+from functools import lru_cache
 from typing import List, Optional, Union
 
 import numpy as np
@@ -355,12 +356,11 @@ def _chain_out_coords(input: spTensor, layers) -> dict:
     stride, cmax, cmin = input.stride, list(input.coords_max[:3]), list(input.coords_min[:3])
     for i, entry in enumerate(layers):
         ks, st, pad, _ = _layer_entry(entry)
-        ksc, sc, pc = (conv_info_encoder(_triple(v, "layer")) for v in (ks, st, pad))
+        (ksc, sc, _), (k3, s3, p3) = _layer_codes(ks, st, pad)
         if sc == _UNIT:
             continue
         if (ksc, stride, sc) in input.kmaps:
             return {}
-        k3, s3, p3 = conv_info_decoder(ksc), conv_info_decoder(sc), conv_info_decoder(pc)
         cmax = backend.strided_coords_max(cmax, k3, s3, p3)
         geoms.append(backend.Geom.make(k3, s3, p3, cmin, cmax, False))
         idx.append(i)
@@ -380,6 +380,20 @@ def _layer_entry(entry):
         return entry[0], entry[1], entry[2], bool(entry[3])
     ks, stride, pad = entry
     return ks, stride, pad, False
+
+
+def _layer_codes(ks, st, pad):
+    """(codes, decoded triples) of a layer's kernel size, stride and padding: (ksc, sc, pc), (k3, s3, p3)."""
+    if type(ks) is int and type(st) is int and type(pad) is int:
+        return _layer_codes_of_ints(ks, st, pad)
+    codes = tuple(conv_info_encoder(_triple(v, "layer")) for v in (ks, st, pad))
+    return codes, tuple(map(conv_info_decoder, codes))
+
+
+@lru_cache(maxsize=256)
+def _layer_codes_of_ints(ks, st, pad):      # (plain numbers: a network's list holds two kinds of layers, and is gone through for every cloud)
+    codes = tuple(conv_info_encoder(_triple(v, "layer")) for v in (ks, st, pad))
+    return codes, tuple(map(conv_info_decoder, codes))
 
 
 class MapPlanner:
@@ -402,26 +416,25 @@ class MapPlanner:
 
 
 def _prebuild_planned(input: spTensor, layers, planner: Optional[MapPlanner]):
-    """The maps `layers` asks for in one library call, in the allocation of a plan that `planner` keeps or (None) in one of their own,
-    or None where that does not apply (a map already cached,
-    reference tags, no batch count, a strided layer whose kernel differs from its stride or that is padded, a cloud
+    """(the maps `layers` asks for in one library call, in the allocation of a plan that `planner` keeps or (None) in one of their own,
+    None), or (None, what ``_chain_out_coords`` gives or None) where that does not apply (a map already cached,
+    reference tags, no batch count, a strided layer whose kernel differs from its stride or that is padded; with a planner, a cloud
     that is not sorted): the caller then builds them map by map.  Same maps, same cache entries."""
     if not input.coords.is_cuda or not input.batchsize or input.batchsize <= 0:
-        return None
+        return None, None
     if input.init_tag and input.init_tag[0] not in ('end', 'auto'):      # the reference's D1 / D2 tags: map by map
-        return None
-    entries, strided, requests = [], [], []
+        return None, None
+    entries, strided, places, requests = [], [], [], []
     stride_code, cmin, cmax, level = input.stride, list(input.coords_min[:3]), list(input.coords_max[:3]), 0
     seen = {}
-    for entry in layers:
+    for i, entry in enumerate(layers):
         ks, st, pad, table_only = _layer_entry(entry)
-        ksc, sc, pc = (conv_info_encoder(_triple(v, "layer")) for v in (ks, st, pad))
+        (ksc, sc, pc), (k3, s3, p3) = _layer_codes(ks, st, pad)
         if ksc == _UNIT and sc == _UNIT:
             continue
         key = (ksc, stride_code, sc)
-        if key in input.kmaps:
-            return None
-        k3, s3, p3 = conv_info_decoder(ksc), conv_info_decoder(sc), conv_info_decoder(pc)
+        if key in input.kmaps or k3[0] * k3[1] * k3[2] > backend.PYRAMID_MAX_KV:
+            return None, None
         subm = sc == _UNIT
         if subm:
             if key not in seen:
@@ -431,32 +444,35 @@ def _prebuild_planned(input: spTensor, layers, planner: Optional[MapPlanner]):
                 entries.append((key, stride_code, level, level))
             continue
         if k3 != s3 or any(p3) or key in seen:
-            return None
+            return None, None
         cmax = backend.strided_coords_max(cmax, k3, s3, p3)
         out_stride = output_stride_compute(sc, stride_code, 0)
         strided.append(backend.Geom.make(k3, s3, p3, cmin, cmax, False))
+        places.append(i)
         seen[key] = len(requests)
         requests.append((level, level + 1, k3, s3, p3, cmin, cmax, False, True, True, False))
         entries.append((key, out_stride, level, level + 1))
         stride_code, level = out_stride, level + 1
     if not requests:
-        return None
+        return None, None
     coords = input.coords if input.coords.is_contiguous() else input.coords.contiguous()
     n = coords.shape[0]
     if planner is None:
         try:
             level_coords, maps = backend.build_pyramid(coords, strided, requests, input.batchsize)
-        except backend.PlanNotApplicable:
-            return None
-        return _pyramid_store(input, entries, level_coords, maps)
+        except backend.PlanNotApplicable as refusal:
+            if not refusal.chain:
+                return None, None
+            return None, {} if refusal.chain[0] is None else dict(zip(places, refusal.chain[0]))
+        return _pyramid_store(input, entries, level_coords, maps), None
     pkey = (tuple(map(tuple, ((r[0], r[1], r[10]) + tuple(r[2]) + tuple(r[6]) for r in requests))), tuple(input.coords_min[:3]),
             int(input.batchsize), coords.device)
     try:
         plan = planner.plan_for(pkey, n, lambda cap: backend.PyramidPlan(cap, strided, requests, input.batchsize, coords.device))
         level_coords, maps = plan.build(coords)
     except backend.PlanNotApplicable:
-        return None
-    return _pyramid_store(input, entries, level_coords, maps)
+        return None, None
+    return _pyramid_store(input, entries, level_coords, maps), None
 
 
 def _pyramid_store(input: spTensor, entries, level_coords, maps):
@@ -475,16 +491,17 @@ def _prebuild(input: spTensor, layers, planner: Optional[MapPlanner] = None):
     """Builds the maps `layers` asks for, starting at `input`.  Returns (the tensor at the coordinates the last
     entry leaves, the maps that were built now)."""
     layers = list(layers)
-    built = _prebuild_planned(input, layers, planner)
+    built, chained = _prebuild_planned(input, layers, planner)
     if built is not None:
         return input, built
     x = input
     pending, done = [], []
-    chained = _chain_out_coords(input, layers)
+    if chained is None:
+        chained = _chain_out_coords(input, layers)
     try:
         for i, entry in enumerate(layers):
             ks, stride, pad, table_only = _layer_entry(entry)
-            ksc, sc, pc = (conv_info_encoder(_triple(v, "layer")) for v in (ks, stride, pad))
+            (ksc, sc, pc), _ = _layer_codes(ks, stride, pad)
             if ksc == _UNIT and sc == _UNIT:
                 continue
             km, request, key, tag, out_stride, cmin, cmax = _map_request(x, ksc, sc, pc)

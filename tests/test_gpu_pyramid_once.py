@@ -127,6 +127,25 @@ def test_a_refused_cloud_is_built_map_by_map(call, status, monkeypatch):
     assert len(x.kmaps) == 9 and not any(km.__dict__.get("_arena") is not None for km in x.kmaps.values())
 
 
+@pytest.mark.parametrize("kind", ["too empty", "refused maps"])
+def test_the_chain_of_a_declined_cloud_is_not_asked_again(kind, monkeypatch):
+    """The general path goes on from the levels' coordinates, or from the answer that the chain does not take the cloud."""
+    c = CLOUDS["lidar"]() if kind == "refused maps" else synth.lidar_cloud(seed=2, azimuths=40, n_ground=400, voxel=0.1)
+    a, b = tensor(c), tensor(c)
+    with monkeypatch.context() as m:
+        chains, singles = counted(m)
+        if kind == "refused maps":
+            m.setattr(_lib.load(), "pce_pyramid_maps", lambda *args: _lib.PCE_ECAPACITY)
+        spconv.prebuild_maps(a, UNET)
+        assert len(chains) == 1 and len(singles) == 9
+    general(monkeypatch)
+    spconv.prebuild_maps(b, UNET)
+    assert list(a.kmaps) == list(b.kmaps)
+    for key in a.kmaps:
+        p, q = a.kmaps[key], b.kmaps[key]
+        assert p.M == q.M and torch.equal(p.out_coords, q.out_coords) and torch.equal(p.imap, q.imap) and torch.equal(p.omap, q.omap)
+
+
 @pytest.mark.parametrize("kind", ["unsorted", "outside the box"])
 @pytest.mark.parametrize("layers", ["unet", "lean", "one", "down", "threes"])
 def test_rows_that_the_column_grid_refuses(kind, layers, monkeypatch):

@@ -417,6 +417,19 @@ def test_output_stride_of_numbers_and_arrays():
     assert int(output_stride_compute(two, code)) == four
 
 
+def test_codes_of_a_layer_of_numbers_and_lists():
+    from pcengine_amd.spconv import _layer_codes
+    from pcengine_amd.utils import conv_info_decoder, conv_info_encoder
+    for layer in ((3, 1, 0), (2, 2, 0), (3, 2, 1), ([3, 3, 3], 1, 0), ([1, 3, 5], [1, 2, 1], [0, 1, 2]), (True, 1, False)):
+        for _ in range(2):
+            codes, triples = _layer_codes(*layer)
+            want = [v if isinstance(v, list) else [int(v)] * 3 for v in layer]
+            assert codes == tuple(map(conv_info_encoder, want)) and triples == tuple(map(tuple, want)) == tuple(map(conv_info_decoder, codes))
+    for layer in ((3.0, 1, 0), (3, 1.0, 0), ((3, 3, 3), 1, 0), ("3", 1, 0)):
+        with pytest.raises(NotImplementedError):
+            _layer_codes(*layer)
+
+
 def test_voxel_workspace_is_the_sorts_and_two_bitmaps():
     """Beyond the points whose blocks' cells fit the largest bitmap the workspace grows by what a sorted point takes."""
     for n in (1, 1000, 1 << 20, 1 << 22, (1 << 22) + 1, 10 ** 7, 1 << 25, 1 << 26, (1 << 26) + 1, 1 << 28):
