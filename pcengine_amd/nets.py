@@ -17,7 +17,7 @@ from torch import nn
 from . import backend
 from .activation import ReLU
 from .batchnorm import BatchNorm
-from .spconv import _pick_dataflow, conv3d, prebuild_maps
+from .spconv import _pick_dataflow, conv3d, dataflow_of_environment, prebuild_maps
 from .sptensor import spTensor
 from .utils import cat, conv_info_encoder, output_stride_compute
 
@@ -104,7 +104,6 @@ class SparseResUNet(nn.Module):
             if isinstance(m, ConvBN):
                 m.fuse()
         self._in_place_ok = None
-        self._block_layers = None
         return self
 
     def use_planner(self, on: bool = True) -> "SparseResUNet":
@@ -164,10 +163,10 @@ class SparseResUNet(nn.Module):
         # laid out and built by the library in one allocation
         inference = not (torch.is_grad_enabled() and (x.feats.requires_grad or any(p.requires_grad for p in self.parameters())))
         prebuild_maps(x, self.map_plan(x.feats.dtype if inference else None), planner)
-        self._prebuild_block_orders(x)
         if self._skips_in_place(x):
             return self._forward_skips_in_place(x)
         x = self.stem(x)
+        self._prebuild_block_orders(x)
         feats = [x]
         for down, enc in zip(self.down, self.enc):
             x = enc(down(x))
@@ -179,29 +178,47 @@ class SparseResUNet(nn.Module):
         return self.head(x)
 
     def _prebuild_block_orders(self, x: spTensor) -> None:
-        """The block orders that the network's layers will ask for, together and before the first layer: the GPU has little to do
-        while the host queues the narrow layers of the first level.  What is missed here is built when its layer asks for it."""
+        """The block orders that the layers behind the stem will ask for, together and while the GPU runs the stem.  What is missed here
+        is built when its layer asks for it."""
         dtype = x.feats.dtype
         if dtype != torch.float16 or not x.feats.is_cuda:
             return
-        layers = getattr(self, "_block_layers", None)
-        if layers is None:      # the different wide layers of every level; what the modules' widths say, looked up once
-            layers, depth = {}, len(self.down)
-            for level, module in [(l + 1, m) for l, m in enumerate(self.enc)] + [(l, m) for l, m in enumerate(self.down)] + \
-                    [(depth - 1 - i, m) for ms in (self.up, self.dec) for i, m in enumerate(ms)]:
-                for m in module.modules():
-                    if isinstance(m, conv3d) and m.kernel_volume > 1 and backend.osb_takes(m.kernel_volume, m.in_channels, m.out_channels, dtype):
-                        layers[(level, m.kernel_size_code, m.stride_code, m.in_channels, m.out_channels, m.dataflow, m.transposed)] = None
-            layers = self._block_layers = list(layers)
-        strides, wanted = [x.stride], {}
+        known = getattr(self, "_block_layers", None)
+        if known is None or any(children.get(name) is not m for children, name, m in known[0]) or any(m.dataflow != df for m, df in known[1]):
+            known = self._block_layers = self._find_block_layers(dtype)
+        strides, env = [x.stride], dataflow_of_environment()
         for _ in self.down:
             strides.append(output_stride_compute(_TWO, strides[-1], False))
-        for level, size, stride, c_in, c_out, dataflow, transposed in layers:
+        wanted = []
+        for (level, size, stride, transposed), widths in known[2]:
             km = x.kmaps.get((size, strides[level], stride))
-            if isinstance(km, backend.KernelMap) and (id(km), transposed) not in wanted and \
-                    _pick_dataflow(km, dataflow, c_in, c_out, dtype, transposed) == backend.DATAFLOW_OS:
-                wanted[(id(km), transposed)] = (km, transposed)
-        backend.block_orders(list(wanted.values()))
+            if isinstance(km, backend.KernelMap) and any(_pick_dataflow(km, dataflow, c_in, c_out, dtype, transposed, env) == backend.DATAFLOW_OS
+                                                         for c_in, c_out, dataflow in widths):
+                wanted.append((km, transposed))
+        backend.block_orders(wanted)
+
+    def _find_block_layers(self, dtype):
+        """(every module on the way to a layer wide enough for the block kernel, as (its parent's children, name, module); the layers
+        with their dataflows; [(the map a layer reads, [the widths and dataflows of the layers that read it])])."""
+        path, layers, maps = {}, [], {}
+
+        def visit(parent, level, way):
+            for name, m in parent._modules.items():
+                here = way + ((parent._modules, name, m),)
+                if isinstance(m, conv3d):
+                    if m.kernel_volume > 1 and backend.osb_takes(m.kernel_volume, m.in_channels, m.out_channels, dtype):
+                        path.update(((id(children), child), (children, child, module)) for children, child, module in here)
+                        layers.append((m, m.dataflow))
+                        maps.setdefault((level, m.kernel_size_code, m.stride_code, m.transposed), {})[m.in_channels, m.out_channels, m.dataflow] = None
+                elif m is not None:
+                    visit(m, level, here)
+
+        depth = len(self.down)
+        for name, first, step in (("enc", 1, 1), ("down", 0, 1), ("up", depth - 1, -1), ("dec", depth - 1, -1)):
+            stages = self._modules[name]
+            for i, m in enumerate(stages):
+                visit(m, first + step * i, ((self._modules, name, stages), (stages._modules, str(i), m)))
+        return list(path.values()), layers, [(key, list(widths)) for key, widths in maps.items()]
 
     def _skips_in_place(self, x: spTensor) -> bool:
         """Inference with every norm folded, on the GPU, all widths multiples of 8 channels: the two producers of
@@ -230,6 +247,7 @@ class SparseResUNet(nn.Module):
         x = self.stem[0](x)
         buf = joined(x.feats.shape[0], x.feats, ups[0], self.stem[1].conv.out_channels)
         x = self.stem[1](x, out=buf[:, ups[0]:])
+        self._prebuild_block_orders(x)
         bufs = [buf]
         last = len(self.enc) - 1
         for lv, (down, enc) in enumerate(zip(self.down, self.enc)):

@@ -170,9 +170,13 @@ class conv3d(nn.Module):
         return result
 
 
-def _pick_dataflow(km: backend.KernelMap, requested: str, c_in: int, c_out: int, dtype, transposed: bool) -> int:
-    env = os.environ.get("PCENGINE_DATAFLOW", "").lower()
-    forced = _DATAFLOWS.get(env, _DATAFLOWS.get(requested))
+def dataflow_of_environment() -> str:
+    return os.environ.get("PCENGINE_DATAFLOW", "").lower()
+
+
+def _pick_dataflow(km: backend.KernelMap, requested: str, c_in: int, c_out: int, dtype, transposed: bool, env: Optional[str] = None) -> int:
+    """``env``: ``dataflow_of_environment()`` where it is known already."""
+    forced = _DATAFLOWS.get(dataflow_of_environment() if env is None else env, _DATAFLOWS.get(requested))
     if forced is not None:
         if forced == DATAFLOW_OSO and not backend.oso_takes(km, c_in, c_out, dtype, transposed):
             return DATAFLOW_FDS     # the ordered dataflow exists for narrow layers only (backend.oso_takes)

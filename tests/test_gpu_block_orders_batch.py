@@ -82,3 +82,39 @@ def test_network_builds_its_orders_ahead(planned, monkeypatch):
         monkeypatch.setattr(nets.SparseResUNet, "_prebuild_block_orders", lambda self, x: None)
         want = model(make()).feats
         assert "blocks" in single and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("change", ["dataflows", "a stage", "a width"])
+def test_orders_follow_the_modules(change):
+    """Layers that are set to another dataflow, or replaced, after a forward: no order is built that none of them reads, and those
+    that they read are there ahead of them."""
+    torch.manual_seed(3)
+    model = nets.SparseResUNet(4, 20).to(DEV).eval().half()
+    coords = synth.random_cloud(seed=5, n=40000, extent=40)
+    f = torch.as_tensor(synth.features(4, len(coords), 4), device=DEV).half()
+    make = lambda: pe.spTensor(f, dev_coords(coords), None, [0, 0, 0], coords[:, 1:].max(0).tolist(), batchsize=1)
+
+    def orders():
+        x = make()
+        with torch.no_grad():
+            model(x)
+        return {key for key, km in x.kmaps.items() if km.__dict__.get("_blocks")}
+
+    first = orders()
+    deep = [key for key in first if key[1] == max(k[1] for k in first)]
+    assert len(first) > 1 and len(deep) >= 1
+    if change == "dataflows":
+        for m in model.modules():
+            if isinstance(m, pe.conv3d):
+                m.dataflow = "fds"
+        assert orders() == set()
+        for m in model.modules():
+            if isinstance(m, pe.conv3d):
+                m.dataflow = "auto"
+        assert orders() == first
+    elif change == "a stage":
+        model.enc[-1] = torch.nn.Sequential(nets.ResidualBlock(128, 256, "fds"), nets.ResidualBlock(256, 256, "fds")).to(DEV).eval().half()
+        assert orders() == first - set(deep)
+    else:
+        model.dec[-1][1].b.conv = pe.conv3d(96, 96, 3).to(DEV).half()
+        assert orders() == first
