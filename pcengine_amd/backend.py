@@ -65,6 +65,13 @@ def _mid(ks: Sequence[int]) -> int:
     return (ks[0] - 1) // 2 * ks[1] * ks[2] + (ks[1] - 1) // 2 * ks[2] + (ks[2] - 1) // 2
 
 
+def _cut(array: torch.Tensor, first: int, count: int) -> torch.Tensor:
+    """array[first:first + count], natively (a slice takes the host 1.2 us, and several between work of another kind: the first
+    layer over a new map reads up to eight arrays)."""
+    part = _lib.host().cut(array, first, count) if array.is_cuda else None
+    return array[first:first + count] if part is None else part
+
+
 class _Cut:
     """A per-pair array of a map: allocated for the largest possible pair count and cut to the real one on first
     use (a network reads a few of the six arrays of each of its maps; cutting all of them up front is Python time
@@ -87,10 +94,9 @@ class _Cut:
         v = obj.__dict__.get(self.slot)
         if isinstance(v, tuple):
             if len(v) == 2:              # (array at capacity, count)
-                v = v[0][:v[1]]
-            else:                        # (int32 view of an arena, first element, count[, shape]): a map of a PyramidPlan
-                t = v[0][v[1]:v[1] + v[2]]
-                v = t.view(v[3]) if len(v) > 3 else t
+                v = _cut(v[0], 0, v[1])
+            else:                        # (int32 view of an arena, first element, count): a map of a PyramidPlan
+                v = _cut(*v)
             obj.__dict__[self.slot] = v
         return v
 

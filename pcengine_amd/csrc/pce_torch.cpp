@@ -394,11 +394,27 @@ PyObject *piece(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
   END_HANDLE_TH_ERRORS
 }
 
+// cut(array, first, count) -> elements `first` .. of a vector of int32, in its memory; None where the caller has to slice it
+PyObject *cut(PyObject *, PyObject *const *args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  if (n_args != 3) {
+    PyErr_SetString(PyExc_TypeError, "cut: a tensor and two numbers");
+    return nullptr;
+  }
+  const at::Tensor *t = plain(args[0]);
+  const int64_t first = PyLong_AsLongLong(args[1]), count = PyLong_AsLongLong(args[2]);
+  if (PyErr_Occurred()) return nullptr;
+  if (!t || t->scalar_type() != at::kInt || t->dim() != 1 || !t->is_contiguous() || first < 0 || count < 0 || first > t->numel() - count) Py_RETURN_NONE;
+  return THPVariable_Wrap(part(*t, first, count));
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {{"layer", (PyCFunction)(void (*)())layer, METH_FASTCALL, nullptr},
                          {"bn_forward", (PyCFunction)(void (*)())bn_forward, METH_FASTCALL, nullptr},
                          {"bn_backward", (PyCFunction)(void (*)())bn_backward, METH_FASTCALL, nullptr},
                          {"wgrad", (PyCFunction)(void (*)())wgrad, METH_FASTCALL, nullptr},
                          {"piece", (PyCFunction)(void (*)())piece, METH_FASTCALL, nullptr},
+                         {"cut", (PyCFunction)(void (*)())cut, METH_FASTCALL, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "Host side of a forward layer", -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -196,3 +196,29 @@ def test_memory_of_maps_built_on_another_stream_is_told():
         for name in ("imap", "nbr_out", "order", "out_coords", "kpos"):
             at = getattr(km, name).data_ptr()
             assert any(lo <= at < lo + n for lo, n in spans), name
+
+
+def test_arrays_are_cut_natively():
+    """The arrays of a map are parts of its allocation; what the extension does not take is sliced."""
+    whole = torch.arange(1000, dtype=torch.int32, device=DEV)
+    for array, first, count in ((whole, 0, 1000), (whole, 0, 0), (whole, 1000, 0), (whole, 3, 17), (whole[100:], 5, 895), (whole, 999, 1)):
+        part = _lib.host().cut(array, first, count)
+        want = array[first:first + count]
+        assert torch.equal(part, want) and part.shape == want.shape and part.stride() == want.stride() and part.data_ptr() == want.data_ptr()
+        assert part.untyped_storage().data_ptr() == whole.untyped_storage().data_ptr() and not part.requires_grad
+    for array, first, count in ((whole, 1, 1000), (whole, 1001, 0), (whole[::2], 0, 5), (whole.view(10, 100), 0, 5), (whole.long(), 0, 5), (whole.cpu(), 0, 5)):
+        assert _lib.host().cut(array, first, count) is None
+        assert torch.equal(backend._cut(array, first, count), array[first:first + count])
+    for array, first, count in ((whole, -3, 2), (whole, 3, -1), (whole, 2 ** 62, 2 ** 62)):
+        assert _lib.host().cut(array, first, count) is None
+    with pytest.raises(TypeError):
+        _lib.host().cut(whole, 1)
+    with pytest.raises(OverflowError):
+        _lib.host().cut(whole, 2 ** 70, 1)
+    with torch.inference_mode():
+        other = torch.arange(10, dtype=torch.int32, device=DEV)
+        assert torch.equal(backend._cut(other, 2, 3), other[2:5])
+    x = tensor(CLOUDS["lidar"]())
+    spconv.prebuild_maps(x, UNET)
+    for km in x.kmaps.values():
+        assert km.imap.numel() == km.omap.numel() == km.M and km.imap is km.imap and km.nbr_out.numel() == km.kv * km.n_out
