@@ -4233,7 +4233,12 @@ static int wgrad_impl(bool clear, const void *in, const void *gout, int32_t dtyp
     const int ring_ci = (int)pce_div_up(c_in, 32 * ti), ring_co = (int)pce_div_up(c_out, 32 * to);
     // one workgroup per compute unit, two where the tiles are many: their waits overlap, their atomics are twice as many (256 and 512:
     // 128 -> 128 on 931 tiles 55 and 63 us, on 1854 88 and 83; 384 -> 256 on 860 206 and 192)
-    const bool two = tiles * ring_ci * ring_co >= (ti == 2 && to == 2 && ring_ci * ring_co > 1 ? 1024 : 1536);
+    // A single block of 64 x 64 has few atomics: two from 512 tiles on (where one a unit has three tiles each), to 320 (where two tiles each
+    // take longer than the second round of workgroups), and at any number where the layer is narrow.  256 and 512, and wgrad_kernel
+    // before: 16 -> 16 on 273 tiles 13.1, 10.8 and 11.6 us, 428 13.2, 12.3 and 12.9, 832 20.1, 17.4 and 25.6, 1288 27.5, 22.9 and 41.2;
+    // 64 -> 64 on 273 14.0, 12.2 and 12.4, 428 14.7, 16.6 and 17.1, 519 18.0, 16.5 and 20.6, 1288 28.8, 26.6 and 44.5.
+    const bool two = ti == 2 && to == 2 && ring_ci * ring_co == 1 ? tiles >= 512 || tiles <= 320 || c_in * c_out <= 1024
+                                                                  : tiles * ring_ci * ring_co >= (ti == 2 && to == 2 ? 1024 : 1536);
     const long long runs = (two ? 512 : 256) / (ring_ci * ring_co) / 8 * 8, ring_run = pce_div_up(tiles, runs < 8 ? 8 : runs);
     const long long ring_wgs = pce_div_up(pce_div_up(tiles, ring_run), 8) * 8 * ring_ci * ring_co;
     if (ring_wgs >= (1ll << 31)) PCE_FAIL(PCE_ECAPACITY, "pce_conv_wgrad: %lld workgroups exceed the grid limit", ring_wgs);

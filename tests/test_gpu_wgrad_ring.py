@@ -41,6 +41,19 @@ def test_kernel_gradient(n, extent, ks, stride, transposed, c_in, c_out):
     assert bool((got[empty] == 0).all())
 
 
+@pytest.mark.parametrize("n,extent", [(9000, 45), (10500, 48), (12600, 51), (16000, 54), (19000, 57), (21500, 59)])
+@pytest.mark.parametrize("c_in,c_out", [(4, 16), (32, 32), (32, 36), (64, 64)])
+def test_one_block_of_either_number_of_workgroups(n, extent, c_in, c_out):
+    """240 to 600 tiles in a single block of channels: where the number of workgroups changes with the tiles and the widths."""
+    km = gpu_map(synth.random_cloud(seed=n, n=n, extent=extent), (3, 3, 3))
+    x = torch.as_tensor(synth.features(1, km.n_in, c_in), device=DEV)
+    g = torch.as_tensor(synth.features(2, km.n_out, c_out), device=DEV)
+    want = reference(x, g, km, False)
+    # (as above; a run is at most three tiles, and an offset's runs no more than its tiles)
+    tol = 2 ** -24 * np.sqrt(2 * 128 + 3 + 256)
+    assert ((backend.conv_wgrad(x, g, km).double() - want).norm() / want.norm()).item() <= tol
+
+
 def test_infinite_and_nan_rows_reach_their_own_sums_only():
     km = gpu_map(synth.random_cloud(seed=3, n=700, extent=12), (3, 3, 3))
     x = torch.as_tensor(synth.features(1, km.n_in, 96), device=DEV)
