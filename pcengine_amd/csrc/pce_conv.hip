@@ -4373,15 +4373,27 @@ __device__ __forceinline__ void bn_group(const T *__restrict__ a, const T *__res
                                          long long n, int c, int col0, bool write, double (&s1)[VEC], double (&s2)[VEC]) {
   typedef typename VecOf<T, VEC>::type V;
   constexpr int ROWS = BnRows<GATE>::N;
-  // all loads are requested before the first is used
+  // All loads are requested before the first is used: from the last row behind the end, and what came from there is replaced
+  // afterwards (as a load on condition each, the gradients of 4200 x 2048 floats through an activation took 24.8 us, 21.4 so).
   V xs[ROWS], ys[ROWS], gs[GATE ? ROWS : 1];
   const V zero = vec_zero<T, VEC>();
+  long long at[ROWS];
 #pragma unroll
   for (int k = 0; k < ROWS; ++k) {
     const long long r = r0 + k * groups;
-    xs[k] = r < n ? *reinterpret_cast<const V *>(a + r * c + col0) : zero;
-    ys[k] = b ? (r < n ? *reinterpret_cast<const V *>(b + r * c + col0) : zero) : xs[k];
-    if (GATE) gs[k] = r < n ? *reinterpret_cast<const V *>((const T *)g.gate + r * c + col0) : zero;
+    at[k] = (r < n ? r : n - 1) * c + col0;
+    xs[k] = *reinterpret_cast<const V *>(a + at[k]);
+    if (GATE) gs[k] = *reinterpret_cast<const V *>((const T *)g.gate + at[k]);
+  }
+  if (b) {
+#pragma unroll
+    for (int k = 0; k < ROWS; ++k) ys[k] = *reinterpret_cast<const V *>(b + at[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < ROWS; ++k) {
+    const bool in = r0 + k * groups < n;
+    xs[k] = in ? xs[k] : zero;
+    ys[k] = !b ? xs[k] : in ? ys[k] : zero;
   }
   float f1[VEC], f2[VEC];
 #pragma unroll
@@ -4680,8 +4692,10 @@ __device__ __forceinline__ void load_columns(const float *__restrict__ from, flo
   }
 }
 
-// Bound by its bytes.  A thread keeps its columns' coefficients for ROWS rows, whose loads are out together (with one
-// row a thread the whole forward pass over 100 k x 256 in fp16 took 48.2 us, 45.1 so; 100 k x 96 27.7 and 25.8).  kd null: 1.
+// Bound by its bytes.  The threads of a workgroup lie over whole rows, so that nothing is divided (numbered through the matrix instead,
+// the whole forward pass over 100 k x 256 in fp16 took 43.7 us, 37.7 so; 100 k x 96 25.5 and 23.2).  A thread takes one row (two and
+// four with their loads out together: 37.9 and 38.8, 24.0 and 24.1), or AFFINE_ROWS where its columns are single ones (100 k x 100 in
+// fp16 53.0 us numbered through, 45.8 so).  kd null: 1.
 #define AFFINE_ROWS 4
 template <typename T, int VEC, int GATE, int ROWS>
 __global__ void __launch_bounds__(256) col_affine_kernel(const T *__restrict__ x, const T *__restrict__ d, T *__restrict__ y, long long n,
@@ -4690,12 +4704,12 @@ __global__ void __launch_bounds__(256) col_affine_kernel(const T *__restrict__ x
   typedef typename VecOf<T, VEC>::type V;
   const int tc = threadIdx.x % p.cpb, rl = threadIdx.x / p.cpb;
   const int col0 = (blockIdx.y * p.cpb + tc) * VEC;
-  if (rl >= p.lanes || col0 >= c) return;
   const long long r0 = (long long)blockIdx.x * p.lanes * ROWS + rl;
+  if (rl >= p.lanes || col0 >= c || r0 >= n) return;
   V xs[ROWS], ds[ROWS], gs[ROWS];
 #pragma unroll
   for (int k = 0; k < ROWS; ++k) {
-    const long long r = r0 + k * p.lanes, at = (r < n ? r : n - 1) * c + col0;
+    const long long r = r0 + k * p.lanes, at = (ROWS == 1 || r < n ? r : n - 1) * c + col0;
     xs[k] = *reinterpret_cast<const V *>(x + at);
     if (d) ds[k] = *reinterpret_cast<const V *>(d + at);
     if (GATE) gs[k] = *reinterpret_cast<const V *>((const T *)g.gate + at);
@@ -4709,7 +4723,7 @@ __global__ void __launch_bounds__(256) col_affine_kernel(const T *__restrict__ x
 #pragma unroll
   for (int k = 0; k < ROWS; ++k) {
     const long long r = r0 + k * p.lanes;
-    if (r < n)
+    if (ROWS == 1 || r < n)
       *reinterpret_cast<V *>(y + r * c + col0) = affine_vec<T, VEC, GATE>(xs[k], d != nullptr, ds[k], gs[k], cx, cd, c0, act, slope, g);
   }
 }
@@ -4721,32 +4735,31 @@ static int col_affine_launch(const char *who, const void *x, const void *d, void
   const int vec = aligned16(x) && aligned16(y) && aligned16(d) && aligned16(g.gate) && c % full == 0 ? full : 1;
   const int vcols = c / vec;
   const ColSplit p = col_split(vcols);
-  // one row a thread until that is eight workgroups a compute unit: below, the chain of a thread's rows is what takes the time (4096
-  // rows of 96 columns: 10.3 us for the whole backward pass, 11.1 with four)
-  const bool many = pce_div_up(n, (int64_t)p.lanes) * pce_div_up(vcols, p.cpb) >= 2048;
+  // several rows a thread from eight workgroups a compute unit on: below, the chain of a thread's rows is what takes the time
+  const bool many = vec == 1 && pce_div_up(n, (int64_t)p.lanes) * pce_div_up(vcols, p.cpb) >= 2048;
   const int64_t blocks = pce_div_up(n, (int64_t)p.lanes * (many ? AFFINE_ROWS : 1));
   if (blocks >= (1ll << 31)) PCE_FAIL(PCE_ECAPACITY, "%s: tensor too large for one launch", who);
   dim3 grid((unsigned)blocks, (unsigned)pce_div_up(vcols, p.cpb));
 #define PCE_AFFINE_(T_, V_, G_, R_)                                                                                                      \
   hipLaunchKernelGGL((col_affine_kernel<T_, V_, G_, R_>), grid, dim3(256), 0, s, (const T_ *)x, (const T_ *)d, (T_ *)y, (long long)n, c, \
                      p, kx, kd, k0, act, slope, g)
-#define PCE_AFFINE(T_, V_)                           \
-  if (g.gate && many)                                \
-    PCE_AFFINE_(T_, V_, GATE_SLOPE, AFFINE_ROWS);    \
-  else if (g.gate)                                   \
-    PCE_AFFINE_(T_, V_, GATE_SLOPE, 1);              \
-  else if (many)                                     \
-    PCE_AFFINE_(T_, V_, GATE_NONE, AFFINE_ROWS);     \
-  else                                               \
-    PCE_AFFINE_(T_, V_, GATE_NONE, 1)
+#define PCE_AFFINE(T_, V_, R_)                 \
+  if (g.gate)                                  \
+    PCE_AFFINE_(T_, V_, GATE_SLOPE, R_);       \
+  else                                         \
+    PCE_AFFINE_(T_, V_, GATE_NONE, R_)
   if (dtype == PCE_F16 && vec == 8) {
-    PCE_AFFINE(half_t, 8);
+    PCE_AFFINE(half_t, 8, 1);
+  } else if (dtype == PCE_F16 && many) {
+    PCE_AFFINE(half_t, 1, AFFINE_ROWS);
   } else if (dtype == PCE_F16) {
-    PCE_AFFINE(half_t, 1);
+    PCE_AFFINE(half_t, 1, 1);
   } else if (vec == 4) {
-    PCE_AFFINE(float, 4);
+    PCE_AFFINE(float, 4, 1);
+  } else if (many) {
+    PCE_AFFINE(float, 1, AFFINE_ROWS);
   } else {
-    PCE_AFFINE(float, 1);
+    PCE_AFFINE(float, 1, 1);
   }
 #undef PCE_AFFINE
 #undef PCE_AFFINE_
@@ -4763,6 +4776,7 @@ static int col_affine_launch(const char *who, const void *x, const void *d, void
 #define BN_SMALL_COLS 2
 #define BN_SMALL_LANES (BN_SMALL_THREADS / BN_SMALL_COLS)
 #define BN_SMALL_WORKGROUPS 128
+#define BN_SMALL_ROWS 4   // rows of a thread whose loads are out together
 // both sums of every column over the row lanes, in red[0], red[1]; the wavefronts halve their lanes' values and lanes together
 template <int VEC>
 __device__ __forceinline__ void bn_small_sums(double (&v)[2 * VEC], double (*red)[BN_SMALL_COLS * VEC]) {
@@ -4841,10 +4855,10 @@ __global__ void __launch_bounds__(BN_SMALL_THREADS) bn_small_kernel(const T *__r
     cd[j] = FORWARD ? 1.f : coef[1][tc * VEC + j];
     c0[j] = coef[2][tc * VEC + j];
   }
-  for (int r0 = lo + rl; r0 < hi; r0 += BN_SMALL_LANES * AFFINE_ROWS) {
-    V xs[AFFINE_ROWS], ds[AFFINE_ROWS], gs[AFFINE_ROWS];
+  for (int r0 = lo + rl; r0 < hi; r0 += BN_SMALL_LANES * BN_SMALL_ROWS) {
+    V xs[BN_SMALL_ROWS], ds[BN_SMALL_ROWS], gs[BN_SMALL_ROWS];
 #pragma unroll
-    for (int k = 0; k < AFFINE_ROWS; ++k) {
+    for (int k = 0; k < BN_SMALL_ROWS; ++k) {
       const int r = r0 + k * BN_SMALL_LANES;
       const long long at = (long long)(r < hi ? r : hi - 1) * c + col0;
       xs[k] = *reinterpret_cast<const V *>(x + at);
@@ -4852,7 +4866,7 @@ __global__ void __launch_bounds__(BN_SMALL_THREADS) bn_small_kernel(const T *__r
       if (GATE) gs[k] = *reinterpret_cast<const V *>((const T *)g.gate + at);
     }
 #pragma unroll
-    for (int k = 0; k < AFFINE_ROWS; ++k) {
+    for (int k = 0; k < BN_SMALL_ROWS; ++k) {
       const int r = r0 + k * BN_SMALL_LANES;
       const long long at = (long long)r * c + col0;
       V in = xs[k];

@@ -123,3 +123,34 @@ def test_module_counts_its_batches_on_the_device():
         assert int(bn.num_batches_tracked) == 3
     with pytest.raises(ValueError):
         backend.bn_backward(x.feats.detach(), x.feats.detach(), None, torch.zeros(16, device=DEV), torch.ones(16, device=DEV), True, masked=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("n,c", [(1, 8), (1025, 8), (1025, 5), (5003, 64), (20001, 33), (70001, 20), (60000, 24)])
+def test_rows_behind_the_last_one_add_nothing(n, c, dtype):
+    """Sums and maps of many rows, by full vectors and single columns: the last row, which stands in for rows that are not there, counts
+    once, also where it is infinite."""
+    x, dy, _, w, b = data(n, c, dtype)
+    x[-1, 0], dy[-1, 0] = float("inf"), 1.0
+    x[-1, 1], dy[-1, 1] = 3.0, float("inf")
+    s = backend.col_sums(x, dy).double()
+    want = torch.stack([x.double().sum(0), (x.double() * dy.double()).sum(0)])
+    scale = torch.stack([x.double().abs().sum(0), (x.double() * dy.double()).abs().sum(0)])
+    assert torch.equal(torch.isnan(s.view(2, c)), torch.isnan(want)) and torch.equal(torch.isinf(s.view(2, c)), torch.isinf(want))
+    ok = torch.isfinite(want)
+    # fp32 sums over eight rows, fp64 above, one rounding to fp32: at most 2^-24 (8 + 1 + 1) of the terms' sum
+    assert ((s.view(2, c) - want).abs()[ok] <= 10 * 2.0 ** -24 * scale[ok]).all()
+    y = torch.empty_like(x)
+    k = torch.randn(3, c, device=DEV)
+    lib = _lib.load()
+    for d, kd in ((None, None), (dy, k[2])):
+        whole = torch.full((n + 2, c), 7.0, device=DEV).to(dtype)
+        y = whole[1:-1]
+        if y.data_ptr() % 16 and c % 8 == 0:
+            continue
+        _lib.check(lib.pce_col_affine(x.data_ptr(), None if d is None else d.data_ptr(), y.data_ptr(), CODE[dtype], n, c, k[0].data_ptr(),
+                                      None if kd is None else kd.data_ptr(), k[1].data_ptr(), _lib.ACT_NONE, 0.0,
+                                      torch.cuda.current_stream().cuda_stream))
+        want = x.double() * k[0].double() + k[1].double() + (0 if d is None else d.double() * kd.double())
+        assert rel(y[:-1], want[:-1]) <= BAR[dtype] and rel(y[-1:, 2:], want[-1:, 2:]) <= 3 * BAR[dtype]
+        assert bool((whole[0] == 7).all()) and bool((whole[-1] == 7).all())
