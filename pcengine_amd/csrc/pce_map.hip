@@ -751,6 +751,10 @@ __global__ void __launch_bounds__(256) chain_fill_kernel(ChainDev d) {
 
 // Bound by its atomics, which all end at the memory side.  Four levels of eight indoor scenes (954 k rows) 96 us with one a row at the
 // first level and none combined across more than four words of a wavefront, 26 so; of a 100 k-voxel scan, whose runs are short, 21 and 9.
+// From CHAIN_CROWDED rows a word on the runs of a wavefront are combined further: the whole call for four levels of 246 k rows in a box
+// of 90^3 136 us that older way, 181 with runs alone, 116 so, their rows in random order 519, 828 and 501; of a 37 k-voxel surface 80, 100
+// and 81 (from 64 rows a word on the same within 1 us, but the scenes 126 in place of 124).
+#define CHAIN_CROWDED 256
 __global__ void __launch_bounds__(256) chain_mark_kernel(const int4 *__restrict__ coords, long long n_in, ChainDev d) {
   // no lane leaves early: the lanes of a wavefront combine their bits below
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -797,7 +801,24 @@ __global__ void __launch_bounds__(256) chain_mark_kernel(const int4 *__restrict_
       if (lane + d < PCE_WAVE && there == at) run |= bits;
     }
     const unsigned before = (unsigned)__shfl_up((int)at, 1, PCE_WAVE);
-    if (live && (lane == 0 || before != at)) atomicOr(&v.bits[word], run);
+    bool pending = live && (lane == 0 || before != at);
+    if (n_in >= CHAIN_CROWDED * v.words) {
+      // A wavefront has several runs of the few words there are, and all wavefronts meet there: the runs of up to four words are
+      // combined, what is left goes alone.
+      unsigned long long todo = __ballot(pending);
+      for (int it = 0; it < 4 && todo; ++it) {
+        const int leader = __ffsll((long long)todo) - 1;
+        const unsigned lw = (unsigned)__shfl((int)at, leader, PCE_WAVE);
+        const bool same = pending && at == lw;
+        unsigned mm = same ? run : 0u;
+#pragma unroll
+        for (int dd = 1; dd < PCE_WAVE; dd <<= 1) mm |= (unsigned)__shfl_xor((int)mm, dd, PCE_WAVE);
+        if (lane == leader) atomicOr(&v.bits[lw], mm);
+        if (same) pending = false;
+        todo &= ~__ballot(same);
+      }
+    }
+    if (pending) atomicOr(&v.bits[word], run);
   }
 }
 
