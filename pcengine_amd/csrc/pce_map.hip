@@ -1777,8 +1777,8 @@ struct ProbDev {
 struct Job {
   unsigned blk0;
   int prob;
-  int kind;
-  int per;   // row order: rows per workgroup, in 256s
+  short kind;
+  short per;   // row order: rows per workgroup, in 256s
 };
 enum { JOB_CSR_SUBM = 0, JOB_CSR_IN = 1, JOB_CSR_COUNT_OUT = 2, JOB_CSR_OUT = 3, JOB_ORDER_SCATTER = 4, JOB_FILL_VIEWS = 5, JOB_FILL_FULL3 = 6 };
 
@@ -2933,6 +2933,9 @@ struct BatchImage {
   FillRegion fills[5 * PCE_MAX_BATCH];
   ScanArr scans[2][2 * PCE_MAX_BATCH];  // first scan (segments, input rows), second scan (output rows)
 };
+// The runtime gives copies of more than 16 KB to a copy engine, and the kernels behind wait for its signal: with 16.2 KB every build of
+// maps took 10 to 20 us more (the map of a 5x5x5 layer on 4.5 k voxels 289 us, 302 so).
+static_assert(sizeof(BatchImage) <= 16384, "the descriptors go in one copy of a kernel");
 
 // The descriptor block travels from pinned host memory, so the copy is queued like a kernel and the
 // host does not wait for earlier work on the stream.  A small ring of pinned blocks per device; a
@@ -2985,8 +2988,8 @@ extern "C" int pce_kmap_build_batch(const pce_kmap_problem_t *probs, int32_t n_p
     Job &j = img.jobs[stage][img.n_jobs[stage]++];
     j.blk0 = blk[stage];
     j.prob = prob;
-    j.kind = kind;
-    j.per = per;
+    j.kind = (short)kind;
+    j.per = (short)per;   // (at most 2^30 / (256 ORDER_PLAIN_COUNTS))
     blk[stage] += (unsigned)pce_div_up(items, 256 * per);
   };
   auto add_fill = [&](void *p, long long words, unsigned zero = 0) {
