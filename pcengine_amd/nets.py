@@ -200,25 +200,31 @@ class SparseResUNet(nn.Module):
     def _find_block_layers(self, dtype):
         """(every module on the way to a layer wide enough for the block kernel, as (its parent's children, name, module); the layers
         with their dataflows; [(the map a layer reads, [the widths and dataflows of the layers that read it])])."""
-        path, layers, maps = {}, [], {}
+        path, layers, maps = [], [], {}
 
-        def visit(parent, level, way):
-            for name, m in parent._modules.items():
-                here = way + ((parent._modules, name, m),)
+        def visit(children, level) -> bool:
+            found = False
+            for name, m in children.items():
                 if isinstance(m, conv3d):
-                    if m.kernel_volume > 1 and backend.osb_takes(m.kernel_volume, m.in_channels, m.out_channels, dtype):
-                        path.update(((id(children), child), (children, child, module)) for children, child, module in here)
+                    here = m.kernel_volume > 1 and backend.osb_takes(m.kernel_volume, m.in_channels, m.out_channels, dtype)
+                    if here:
                         layers.append((m, m.dataflow))
                         maps.setdefault((level, m.kernel_size_code, m.stride_code, m.transposed), {})[m.in_channels, m.out_channels, m.dataflow] = None
-                elif m is not None:
-                    visit(m, level, here)
+                else:
+                    here = m is not None and len(m._modules) > 0 and visit(m._modules, level)
+                if here:
+                    path.append((children, name, m))
+                    found = True
+            return found
 
         depth = len(self.down)
         for name, first, step in (("enc", 1, 1), ("down", 0, 1), ("up", depth - 1, -1), ("dec", depth - 1, -1)):
-            stages = self._modules[name]
-            for i, m in enumerate(stages):
-                visit(m, first + step * i, ((self._modules, name, stages), (stages._modules, str(i), m)))
-        return list(path.values()), layers, [(key, list(widths)) for key, widths in maps.items()]
+            stages = self._modules[name]._modules
+            for i, (index, m) in enumerate(stages.items()):
+                if visit(m._modules, first + step * i):
+                    path.append((stages, index, m))
+            path.append((self._modules, name, self._modules[name]))
+        return path, layers, [(key, list(widths)) for key, widths in maps.items()]
 
     def _skips_in_place(self, x: spTensor) -> bool:
         """Inference with every norm folded, on the GPU, all widths multiples of 8 channels: the two producers of
