@@ -72,6 +72,32 @@ def test_order_of_a_table(n, kv, mid, share):
     _check(order.cpu().numpy(), nbr, mid, tuple(counts))
 
 
+def test_order_of_rows_beyond_sixteen_times_the_workgroups():
+    """More rows than the places of the counts allow at 16 times 256 rows a workgroup: longer workgroups."""
+    kv, n = 8, 256 * 16 * 2040 + 5
+    g = torch.Generator(device=DEV).manual_seed(1)
+    nbr = torch.where(torch.rand((kv, n), generator=g, device=DEV) < 0.05, 0, -1).int()
+    lib = _lib.load()
+    order = torch.empty(lib.pce_row_order_elems(n), dtype=torch.int32, device=DEV)
+    counts = (_lib.c_int64 * 3)()
+    _lib.check(lib.pce_row_order(nbr.data_ptr(), kv, n, -1, order.data_ptr(), order.numel(), counts, torch.cuda.current_stream().cuda_stream))
+    masks = torch.zeros(n, dtype=torch.int32, device=DEV)
+    pairs = torch.zeros(n, dtype=torch.int32, device=DEV)
+    for k in range(kv):
+        masks |= (nbr[k] >= 0).int() << k
+        pairs += (nbr[k] >= 0).int()
+    assert tuple(counts) == (int((pairs >= 3).sum()), int((pairs >= 1).sum()), int((pairs == 1).sum()))
+    plain = n - counts[1]
+    perm = order[:n].long()
+    assert torch.equal(order[n:2 * n], masks) and torch.equal(perm.sort().values, torch.arange(n, device=DEV))
+    sect = masks[perm]
+    assert bool((sect[:plain] == 0).all()) and bool((sect[plain:] != 0).all()) and bool((perm[:plain].diff() > 0).all())
+    assert (np.diff(_keys(sect[plain:].cpu().numpy().astype(np.int64))) >= 0).all()
+    at = (2 * n + TAIL + 3) // 4 * 4
+    rec = order[at:at + 4 * n].view(n, 4)[plain:]
+    assert torch.equal(rec[:, 0], order[plain:n]) and torch.equal(rec[:, 1], sect[plain:]) and bool((rec[:, 2] == 0).all())
+
+
 @pytest.mark.parametrize("sorted_rows", [True, False])
 @pytest.mark.parametrize("cloud", ["lidar", "rooms"])
 def test_order_built_with_a_map_of_many_rows(cloud, sorted_rows):
