@@ -3915,7 +3915,9 @@ __global__ void __launch_bounds__(256, 2) wgrad_pipe_kernel(const half_t *__rest
 // Bound by the matrix cores where the tiles are many (a stage is 2048 of their clocks for 128 x 128 and 32 LDS reads), by the
 // sums' atomics and the first gathers where they are few.  wgrad_kernel, whose stages' gathers nothing hid -> this one: 96 -> 96 on
 // 21 k rows of 5 pairs 79 us -> 35, 128 -> 128 85 -> 55, 256 -> 256 207 -> 145, on 35 k of 5 415 -> 253 (90 TFLOP/s), 96 -> 96 on 19 k
-// of 14 197 -> 63; 64 -> 64 on 21 k 33 -> 24; 128 -> 128 on 800 rows 24 -> 16.
+// of 14 197 -> 63; 64 -> 64 on 18 k of 5.5 32 -> 21; 128 -> 128 on 800 rows 24 -> 16.  Narrower layers, whose blocks are padded to 64
+// channels: 16 -> 16 on 10 k rows of 2.3 pairs 11.5 -> 10.8, on 18 k of 5.5 27 -> 17, on 66 k of 9 90 -> 59; 4 -> 32 on 99 k of 0.1
+// 27 -> 23.
 template <int TI, int TO>
 __global__ void __launch_bounds__(256, 2) wgrad_f32_ring_kernel(const float *__restrict__ in, const float *__restrict__ gout, long long n_rows,
                                                                 unsigned in_bytes, unsigned out_bytes, int c_in, int c_out, int kv, int mid,

@@ -1598,7 +1598,8 @@ __global__ void __launch_bounds__(256) collate_kernel(CollateArgs a, int4 *__res
 
 // upper[block]: maxima of the columns behind the first of rows of `width` ints (a sample's: y and z of x, y, z; a batch's: x, y and
 // z), over the rows that the workgroup reads.  Bound by the launch: torch's reduction of the view is a fill of 4 us and a
-// kernel of one workgroup, 9 to 12 on 150 k rows; 6 in all this way.
+// kernel of one workgroup, 9 to 12 on 150 k rows; 6 in all this way.  With the wait, a tensor over rows without bounds 31 us of torch's
+// and 29 so on 3 k rows, 35 and 30 on 15 k, 55 and 30 on 99 k.
 __global__ void __launch_bounds__(256) column_max_kernel(const int *__restrict__ rows, long long n, int width, int *__restrict__ upper) {
   __shared__ int part[4][3];
   int m[3] = {(int)0x80000000, (int)0x80000000, (int)0x80000000};

@@ -13,7 +13,8 @@
 
 #include "pcengine_amd.h"
 
-// entry points that a library beside this extension may be without: the calls that need them are then declined
+// entry points that a library beside this extension may be without, as the stubs are that its host side is tested beside (the library
+// that the package loads has all of them, or is refused): the calls that need them are then declined
 #pragma weak pce_bn_forward_counted
 #pragma weak pce_bn_backward_masked
 #pragma weak pce_conv_wgrad_add
